@@ -32,6 +32,7 @@ SOURCES = {
     "attn_bwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "mla_glue.hip": [],
     "block_train.hip": [],
+    "linear_bwd.hip": [],
 }
 
 COMMON_FLAGS = [

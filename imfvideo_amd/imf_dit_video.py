@@ -21,9 +21,75 @@ __all__ = ["RMSNorm", "SituAndMul", "SwiGLUMlp", "MLAAttention", "TransformerBlo
            "sdpa_math_attention"]
 
 
+class _LinearFunction(torch.autograd.Function):
+    """x @ weight^T for a 16-bit x and an fp32 weight, as nn.Linear under a 16-bit
+    autocast, with the weight gradient from sla2h_linear_wgrad: fp32, summed
+    over all rows in fp32 (autocast's is rounded to 16 bits on its way)."""
+
+    @staticmethod
+    def forward(ctx, x, weight):
+        w16 = weight.to(x.dtype)
+        ctx.save_for_backward(x, w16)
+        ctx.weight, ctx.version = weight, weight._version
+        return F.linear(x, w16)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, w16 = ctx.saved_tensors
+        need_x, need_w = ctx.needs_input_grad
+        if torch.is_grad_enabled():  # create_graph: torch ops, differentiable again
+            if ctx.weight._version != ctx.version:
+                raise RuntimeError("a linear layer's weight was modified in place before its "
+                                   "double backward")
+            dw = dy.flatten(0, -2).t() @ x.flatten(0, -2) if need_w else None
+            return (dy @ ctx.weight.to(x.dtype) if need_x else None,
+                    dw.to(ctx.weight.dtype) if need_w else None)
+        from . import ops
+        return dy @ w16 if need_x else None, ops.linear_wgrad(dy, x) if need_w else None
+
+
+# Weights of at most this many 128 x 128 tiles take the split-row gradient
+# kernel: with few output tiles the library's kernel for the same product leaves
+# most CUs idle (2048 x 512, 64 tiles: 110 us against 46 us at 16,384 rows, 284
+# against 157 us at 59,904), with many it is as fast or faster (4096 x 1024, 256
+# tiles: 555 against 622 us at 59,904 rows).
+_WGRAD_MAX_TILES = 64
+
+
+def _own_wgrad(x, weight, bias):
+    """The weight gradient of this call can come from sla2h_linear_wgrad: plain
+    GPU tensors under a 16-bit autocast, eager first-order reverse mode."""
+    if not (bias is None and type(x) is torch.Tensor and x.is_cuda and x.dim() >= 2
+            and type(weight) in (nn.Parameter, torch.Tensor) and weight.device == x.device
+            and weight.dtype == torch.float32 and weight.requires_grad
+            and torch.is_grad_enabled() and torch.is_autocast_enabled("cuda")
+            and torch.get_autocast_dtype("cuda") in (torch.bfloat16, torch.float16)
+            and x.dtype in (torch.float32, torch.bfloat16, torch.float16)):
+        return False
+    if (torch.compiler.is_compiling() or torch.jit.is_tracing()
+            or torch._C._are_functorch_transforms_active()
+            or torch.autograd.forward_ad._current_level >= 0):
+        return False
+    M, N = weight.shape
+    if x.shape[-1] != N or -(-M // 128) * -(-N // 128) > _WGRAD_MAX_TILES:
+        return False
+    from . import ops
+    return ops.linear_wgrad_ok(x.numel() // N, M, N)
+
+
+class _Linear(nn.Linear):
+    """nn.Linear whose weight gradient, under a 16-bit autocast on the GPU, comes
+    from this package's kernel (_LinearFunction); otherwise nn.Linear's."""
+
+    def forward(self, x):
+        if _own_wgrad(x, self.weight, self.bias):
+            return _LinearFunction.apply(x.to(torch.get_autocast_dtype("cuda")), self.weight)
+        return super().forward(x)
+
+
 def scaled_variance_linear(in_features, out_features, bias=True, init_constant=1.0):
     """nn.Linear with weights N(0, init_constant / sqrt(in_features))."""
-    linear = nn.Linear(in_features, out_features, bias=bias)
+    linear = _Linear(in_features, out_features, bias=bias)
     nn.init.normal_(linear.weight, std=init_constant / math.sqrt(in_features))
     if bias:
         nn.init.zeros_(linear.bias)

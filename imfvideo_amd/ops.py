@@ -1086,3 +1086,43 @@ def residual_scale_bwd(dy, a, s):
         da.data_ptr(), ds.data_ptr(), ws.data_ptr(), _stream(a.device)),
         "sla2h_residual_scale_bwd")
     return da, ds
+
+
+# ---------------------------------------------------------------------------
+# DiT block, training backward: weight gradients of the linear layers
+# ---------------------------------------------------------------------------
+def linear_wgrad_ok(rows, M, N):
+    """Sizes that sla2h_linear_wgrad takes: M and N multiples of 8, 32-bit byte offsets."""
+    return (rows > 0 and M > 0 and N > 0 and M % 8 == 0 and N % 8 == 0
+            and (rows + 144) * max(M, N) * 2 + 256 < 2 ** 31)
+
+
+def linear_wgrad(dy, x):
+    """dW = dY^T X (M, N) fp32 from dy (..., M) and x (..., N) of one 16-bit dtype
+    and the same leading dimensions; fp32 accumulation, not rounded to 16 bits."""
+    _need_gpu(dy, x)
+    if dy.dtype != x.dtype or dy.shape[:-1] != x.shape[:-1]:
+        raise ValueError("linear_wgrad: dy and x must share dtype and leading dimensions")
+    code = _dtype_code(x)
+    dy2, M, ldy = _rows16(dy)
+    x2, N, ldx = _rows16(x)
+    rows = x2.shape[0]
+    if not linear_wgrad_ok(rows, max(M, ldy), max(N, ldx)):
+        raise ValueError(f"linear_wgrad: unsupported sizes {tuple(dy.shape)}, {tuple(x.shape)}")
+    lib = _lib.load()
+    dw = torch.empty(M, N, device=x.device, dtype=torch.float32)
+    need = lib.sla2h_linear_wgrad_workspace_bytes(rows, M, N)
+    ws = torch.empty(need, device=x.device, dtype=torch.uint8) if need else None
+    _lib.check(lib.sla2h_linear_wgrad(dy2.data_ptr(), ldy, x2.data_ptr(), ldx, code, rows, M, N,
+                                      _ptr(ws), dw.data_ptr(), _stream(x.device)),
+               "sla2h_linear_wgrad")
+    return dw
+
+
+def _rows16(t):
+    """_rows_view with 16-byte aligned rows (copied when they are not)."""
+    v, F, s = _rows_view(t)
+    if v.data_ptr() % 16 or s % 8:
+        v = v.clone(memory_format=torch.contiguous_format)
+        s = F
+    return v, F, s

@@ -686,6 +686,21 @@ int sla2h_lin_fwd3(const void* qphi, const void* comp, const void* o_s, const fl
                    int alpha_stride, int dtype, int B, int H, int64_t L, int D, int bq,
                    float eps_l, void* o, void* stream);
 
+/*
+ * Weight gradient of a linear layer, dw[m][n] = sum over rows t of dy[t][m] x[t][n],
+ * 16-bit dy (rows, M; row stride ldy) and x (rows, N; row stride ldx), fp32
+ * accumulation and result (M, N).  M, N, ldy, ldx multiples of 8, 16-byte
+ * aligned pointers, (rows + 144) * ld * 2 + 256 < 2^31.  The rows are summed in
+ * ranges (partial results in `workspace`, of
+ * sla2h_linear_wgrad_workspace_bytes, NULL when that is 0) that are added in
+ * order: the result is deterministic.
+ * Replaces torch autograd of the nn.Linear layers (models/imf_dit_video.py:174-187,
+ * 422-467) for their fp32 weights under a 16-bit autocast.
+ */
+size_t sla2h_linear_wgrad_workspace_bytes(int64_t rows, int M, int N);
+int sla2h_linear_wgrad(const void* dy, int64_t ldy, const void* x, int64_t ldx, int dtype,
+                       int64_t rows, int M, int N, void* workspace, float* dw, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

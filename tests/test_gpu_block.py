@@ -443,3 +443,63 @@ def test_block_fused_attention_path_matches_eager_layout():
     assert g1.keys() == g0.keys() and len(g0) > 10
     for k in g0:
         assert rel(g1[k], g0[k]) < 1e-3, k
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,M,N", [(1, 8, 8), (31, 128, 128), (33, 136, 120), (257, 160, 512),
+                                      (1000, 512, 264), (4099, 768, 128), (16417, 256, 512)])
+def test_linear_wgrad(dt, rows, M, N):
+    """dW = dY^T X against float64: products of 16-bit values are exact in fp32, so
+    the only error is fp32 summation, at most rows * 2^-24 of sum |dy| |x| per
+    element (twice that allowed for the matrix core's own rounding).  dy is a
+    column slice of a wider tensor (row stride), x contiguous."""
+    from imfvideo_amd import ops
+    say("linear_wgrad", dt, rows, M, N)
+    g = torch.Generator().manual_seed(rows + M)
+    wide = torch.randn(rows, M + 16, generator=g).to(dt).cuda()
+    dy, x = wide[:, 8:8 + M], torch.randn(rows, N, generator=g).to(dt).cuda()
+    dw = ops.linear_wgrad(dy, x)
+    assert dw.dtype == torch.float32 and dw.shape == (M, N)
+    d64, x64 = dy.double(), x.double()
+    bound = 2 * rows * 2.0 ** -24 * (d64.abs().t().contiguous() @ x64.abs())
+    assert bool(((dw.double() - d64.t().contiguous() @ x64).abs() <= bound).all())
+    assert torch.equal(dw, ops.linear_wgrad(dy, x))
+
+
+@pytest.mark.parametrize("shape", [(2, 300, 64), (65, 64), (1, 1, 64)])
+def test_linear_module_matches_nn_linear(shape):
+    """The block's linear against nn.Linear under autocast: same output and input
+    gradient bit for bit, the weight gradient within the 16-bit rounding that
+    nn.Linear's carries; and without autocast, in a double backward and under
+    torch.func the plain layer's results."""
+    from imfvideo_amd.imf_dit_video import scaled_variance_linear
+    say("linear module", shape)
+    torch.manual_seed(1)
+    own = scaled_variance_linear(64, 96, bias=False).cuda()
+    ref = torch.nn.Linear(64, 96, bias=False).cuda()
+    ref.load_state_dict(own.state_dict())
+    x = torch.randn(shape, device="cuda")
+    dy = torch.randn(*shape[:-1], 96, device="cuda", dtype=torch.bfloat16)
+    res = []
+    for m in (own, ref):
+        xi = x.clone().requires_grad_()
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = m(xi)
+        res.append((y, *torch.autograd.grad(y, [xi, m.weight], dy)))
+    (y0, dx0, dw0), (y1, dx1, dw1) = res
+    assert y0.dtype == y1.dtype and torch.equal(y0, y1) and torch.equal(dx0, dx1)
+    assert dw0.dtype == dw1.dtype == torch.float32
+    # one bf16 rounding (2^-9 of each element) plus fp32 summation order
+    assert bool(((dw0 - dw1).abs() <= 2.0 ** -8 * dw1.abs() + 1e-4).all())
+    assert torch.equal(own(x), ref(x))
+    gg = []
+    for m in (own, ref):
+        xi = x.clone().requires_grad_()
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = m(xi)
+        g1, = torch.autograd.grad(y.float().pow(2).sum(), xi, create_graph=True)
+        gg.append(torch.autograd.grad(g1.float().sum(), m.weight)[0])
+    assert (gg[0] - gg[1]).norm() <= 2e-2 * gg[1].norm()  # two bf16 products deep
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        j0, j1 = (torch.func.jvp(m, (x,), (x,))[1] for m in (own, ref))
+    assert torch.equal(j0, j1)
