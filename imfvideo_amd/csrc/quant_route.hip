@@ -458,45 +458,48 @@ __global__ __launch_bounds__(256) void route_topk_kernel(const float* __restrict
   }
 }
 
-// Top-T of each row by wave-wide radix selection (T <= 64): one wave per
-// query block, NK keys per lane (tile n = lane + 64 i), R rows per wave.
+// Top-T of each row by wave-wide radix selection (T <= CAP): one wave per query
+// block, NK keys per lane (tile n = lane + 64 i).
 //   1. scores, same sequential fp32 order as route_topk_kernel;
-//   2. s* = the T-th largest order-preserving score word (32-bit binary
-//      search with ballot counts); if several keys share s*, the lowest
-//      indices among them fill up to T (a 12-bit binary search over n);
-//   3. the T winners are compacted through LDS and bitonic-sorted across
-//      the lanes by their 64-bit keys (score word, then lower index first).
-template <int NK, int R, bool V4>
+//   2. a score word s* that exactly T keys reach, by a 32-bit binary search
+//      with ballot counts (it ends at the first bit where the count is T: with
+//      distinct scores about half-way); if several keys share the T-th
+//      largest word, the lowest indices among them fill up to T (a 13-bit
+//      binary search over n);
+//   3. the T winners are compacted through LDS and each is written at its
+//      rank, the number of winners with a larger 64-bit key (score word, then
+//      lower index first).
+// Bound by the wave's dependent chains (scores, ballots, ranks), not by
+// memory: NK is the smallest that holds Np, and rank counting replaced a
+// 64-lane bitonic sort (21 cross-lane exchanges whatever T) and, for T > 64,
+// the full sort of every row in LDS.  Heads x rows x Np, T: 4 x 5 x 4, 2:
+// 13.2 -> 4.2 us; 16 x 218 x 216, 6: 23.4 -> 11.9; 8 x 468 x 468, 46: 22.9 -> 20.3.
+template <int NK, int CAP, bool V4>
 __global__ __launch_bounds__(256) void route_select_kernel(const float* __restrict__ qpool,
                                                            const float* __restrict__ kpool_t,
                                                            int Mb, int Np, int T, float scale,
                                                            int32_t* __restrict__ lut,
                                                            uint8_t* __restrict__ mask) {
-  // pooled keys of the head, staged in chunks of DC channels (32 KB) that the
-  // four waves share
-  constexpr int DC = 128 / NK;
+  // pooled keys of the head, staged in chunks of DC channels (at most 32 KB)
+  // that the four waves share
+  constexpr int DC = NK == 1 ? kTile : 128 / NK;
   __shared__ float ksh[DC][64 * NK];
-  __shared__ uint64_t win[4][64];
+  __shared__ uint64_t win[4][CAP];
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int bh = blockIdx.y;
-  const int m0 = __builtin_amdgcn_readfirstlane((blockIdx.x * 4 + w) * R);
-  const bool active = m0 < Mb;  // uniform per wave; every wave takes the barriers
+  const int m = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + w);
+  const bool active = m < Mb;  // uniform per wave; every wave takes the barriers
 
   const float* kt = kpool_t + (int64_t)bh * kTile * Np;
-  float acc[R][NK];
+  float acc[NK];
 #pragma unroll
-  for (int rr = 0; rr < R; ++rr)
-#pragma unroll
-    for (int i = 0; i < NK; ++i) acc[rr][i] = 0.f;
+  for (int i = 0; i < NK; ++i) acc[i] = 0.f;
   // lane d holds q[row][d] (broadcast with readlane).  Key slots past Np
   // need no guard: their scores are never selected (ord = 0 below); the
   // buffer range check returns 0 past the end of this head's pooled keys.
-  const float* qrow = qpool + ((int64_t)bh * Mb + m0) * kTile;
-  float qlane[R];
-#pragma unroll
-  for (int rr = 0; rr < R; ++rr) qlane[rr] = (m0 + rr < Mb) ? qrow[rr * kTile + lane] : 0.f;
+  const float qlane = active ? qpool[((int64_t)bh * Mb + m) * kTile + lane] : 0.f;
   const auto rk = make_rsrc(kt, (int64_t)kTile * Np * 4);
   for (int d0 = 0; d0 < kTile; d0 += DC) {
     __syncthreads();  // the previous chunk is consumed
@@ -522,50 +525,42 @@ __global__ __launch_bounds__(256) void route_select_kernel(const float* __restri
     if (active) {
 #pragma unroll
       for (int dd = 0; dd < DC; ++dd) {
-        float kv[NK];
+        const float qv = __builtin_bit_cast(
+            float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, qlane), d0 + dd));
 #pragma unroll
-        for (int i = 0; i < NK; ++i) kv[i] = ksh[dd][lane + 64 * i];
-#pragma unroll
-        for (int rr = 0; rr < R; ++rr) {
-          const float qv = __builtin_bit_cast(
-              float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, qlane[rr]), d0 + dd));
-#pragma unroll
-          for (int i = 0; i < NK; ++i) acc[rr][i] = acc[rr][i] + qv * kv[i];
-        }
+        for (int i = 0; i < NK; ++i) acc[i] = acc[i] + qv * ksh[dd][lane + 64 * i];
       }
     }
   }
   if (!active) return;  // whole wave; no workgroup barrier below
 
+  uint32_t ord[NK];
 #pragma unroll
-  for (int rr = 0; rr < R; ++rr) {
-    const int m = m0 + rr;
-    if (m >= Mb) break;  // uniform
-    uint32_t ord[NK];
+  for (int i = 0; i < NK; ++i) {
+    const int n = lane + 64 * i;
+    ord[i] = n < Np ? (uint32_t)(score_key(acc[i] * scale, n) >> 32) : 0u;  // 0: below all
+  }
+  // wave-wide sum of per-lane counts 0..NK: one ballot per count bit
+  constexpr int kBits = NK == 1 ? 1 : NK == 2 ? 2 : NK == 4 ? 3 : NK == 8 ? 4
+                      : NK == 16 ? 5 : NK == 32 ? 6 : 7;
+  auto wave_sum = [&](int cl) {
+    int c = 0;
 #pragma unroll
-    for (int i = 0; i < NK; ++i) {
-      const int n = lane + 64 * i;
-      ord[i] = n < Np ? (uint32_t)(score_key(acc[rr][i] * scale, n) >> 32) : 0u;  // 0: below all
-    }
-    // wave-wide sum of per-lane counts 0..NK: one ballot per count bit
-    constexpr int kBits = NK == 8 ? 4 : (NK == 16 ? 5 : (NK == 32 ? 6 : 7));
-    auto wave_sum = [&](int cl) {
-      int c = 0;
+    for (int b = 0; b < kBits; ++b) c += __popcll(__ballot((cl >> b) & 1)) << b;
+    return c;
+  };
+  uint32_t sstar = 0, nstar = 0xffffffffu;  // keys at s* with n <= nstar are taken
+  bool exact = false;
+  for (int b = 31; b >= 0 && !exact; --b) {
+    const uint32_t cand = sstar | (1u << b);
+    int cl = 0;
 #pragma unroll
-      for (int b = 0; b < kBits; ++b) c += __popcll(__ballot((cl >> b) & 1)) << b;
-      return c;
-    };
-    auto count_ge = [&](uint32_t v) {
-      int cl = 0;
-#pragma unroll
-      for (int i = 0; i < NK; ++i) cl += ord[i] >= v ? 1 : 0;
-      return wave_sum(cl);
-    };
-    uint32_t sstar = 0;
-    for (int b = 31; b >= 0; --b) {
-      const uint32_t cand = sstar | (1u << b);
-      if (count_ge(cand) >= T) sstar = cand;
-    }
+    for (int i = 0; i < NK; ++i) cl += ord[i] >= cand ? 1 : 0;
+    const int c = wave_sum(cl);
+    if (c >= T) sstar = cand;
+    exact = c == T;
+  }
+  if (!exact) {
     int l_gt = 0, l_eq = 0;
 #pragma unroll
     for (int i = 0; i < NK; ++i) {
@@ -574,7 +569,6 @@ __global__ __launch_bounds__(256) void route_select_kernel(const float* __restri
     }
     const int c_gt = wave_sum(l_gt), c_eq = wave_sum(l_eq);
     const int need = T - c_gt;  // 1 <= need <= c_eq
-    uint32_t nstar = 0xffffffffu;  // tie keys with n <= nstar are taken
     if (need < c_eq) {
       uint32_t pre = 0;
       for (int b = 12; b >= 0; --b) {
@@ -586,40 +580,46 @@ __global__ __launch_bounds__(256) void route_select_kernel(const float* __restri
       }
       nstar = pre;
     }
-    // compact the T winners (any order), then sort them across the lanes
-    int base = 0;
+  }
+  // compact the T winners (any order)
+  int base = 0;
 #pragma unroll
-    for (int i = 0; i < NK; ++i) {
-      const uint32_t n = lane + 64 * i;
-      const bool sel = ord[i] > sstar || (ord[i] == sstar && n <= nstar);
-      const uint64_t bal = __ballot(sel);
-      if (sel) {
-        const int pos = base + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
-                                                         __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
-        win[w][pos] = ((uint64_t)ord[i] << 32) | (uint64_t)(0xffffffffu - n);
-      }
-      if (mask != nullptr && (int)n < Np) mask[((int64_t)bh * Mb + m) * Np + n] = sel ? 1 : 0;
-      base += __popcll(bal);
+  for (int i = 0; i < NK; ++i) {
+    const uint32_t n = lane + 64 * i;
+    const bool sel = ord[i] > sstar || (ord[i] == sstar && n <= nstar && (int)n < Np);
+    const uint64_t bal = __ballot(sel);
+    if (sel) {
+      const int pos = base + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
+                                                       __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+      win[w][pos] = ((uint64_t)ord[i] << 32) | (uint64_t)(0xffffffffu - n);
     }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    uint64_t key = lane < T ? win[w][lane] : 0ull;
-    // bitonic sort, descending, over the 64 lanes
+    if (mask != nullptr && (int)n < Np) mask[((int64_t)bh * Mb + m) * Np + n] = sel ? 1 : 0;
+    base += __popcll(bal);
+  }
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  int32_t* row = lut + ((int64_t)bh * Mb + m) * T;
+  if constexpr (CAP == 64) {
+    const uint64_t key = lane < T ? win[w][lane] : 0ull;
+    const int klo = (int)(uint32_t)key, khi = (int)(uint32_t)(key >> 32);
+    int rank = 0;
+    for (int j = 0; j < T; j += 4) {  // lanes from T on hold key 0, above no winner
 #pragma unroll
-    for (int k = 2; k <= 64; k <<= 1) {
-#pragma unroll
-      for (int j = k >> 1; j > 0; j >>= 1) {
-        const uint32_t lo = __shfl_xor((uint32_t)key, j, 64);
-        const uint32_t hi = __shfl_xor((uint32_t)(key >> 32), j, 64);
-        const uint64_t other = ((uint64_t)hi << 32) | lo;
-        const bool desc = (lane & k) == 0;
-        const bool lower = (lane & j) == 0;  // this lane keeps the larger key in a desc run
-        const bool take = desc == lower ? other > key : other < key;
-        key = take ? other : key;
+      for (int u = 0; u < 4; ++u) {
+        const uint64_t other = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(khi, j + u) << 32) |
+                               (uint32_t)__builtin_amdgcn_readlane(klo, j + u);
+        rank += other > key ? 1 : 0;
       }
     }
-    if (lane < T) lut[((int64_t)bh * Mb + m) * T + lane] = (int32_t)(0xffffffffu - (uint32_t)key);
-    __builtin_amdgcn_wave_barrier();  // win[w] is reused by the next row
+    if (lane < T) row[rank] = (int32_t)(0xffffffffu - (uint32_t)key);
+  } else {
+    for (int i = lane; i < T; i += 64) {
+      const uint64_t key = win[w][i];
+      int rank = 0;
+#pragma unroll 8
+      for (int j = 0; j < T; ++j) rank += win[w][j] > key ? 1 : 0;
+      row[rank] = (int32_t)(0xffffffffu - (uint32_t)key);
+    }
   }
 }
 
@@ -882,24 +882,38 @@ extern "C" int sla2h_route_topk(const float* qpool, const float* kpool_t, int B,
   SLA2H_CHECK_ARG(B > 0 && H > 0 && B * H <= 65535 && Mb > 0);
   SLA2H_CHECK_ARG(Np > 0 && Np <= 4096 && T >= 1 && T <= Np);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (T <= 64) {
+  // The wave-wide selection up to 512 winners per row (456 rows of 456 tiles,
+  // T = 114: 95.8 -> 15.6 us against the full sort of every row).  Ranking the
+  // winners takes T^2 / 64 steps per wave, so with rows that the sort holds in
+  // 512 slots it stops paying at T = 448 (110 against 112 us; 512: 131 against
+  // 111), with longer rows it still does at 512 (Np = 600: 162 against 229 us).
+  if (T <= 448 || (T <= 512 && Np > 512)) {
     // one query block per wave: enough waves to hide the load latency
-    auto go = [&](auto nk, auto rows) {
-      constexpr int NK = decltype(nk)::value, R = decltype(rows)::value;
-      dim3 grid((Mb + 4 * R - 1) / (4 * R), B * H);
-      if (Np % 4 == 0)
-        route_select_kernel<NK, R, true><<<grid, 256, 0, st>>>(qpool, kpool_t, Mb, Np, T, scale, lut, mask);
+    auto go = [&](auto nk) {
+      constexpr int NK = decltype(nk)::value, BIG = NK == 1 ? 64 : 512;
+      dim3 grid((Mb + 3) / 4, B * H);
+      auto run = [&](auto kernel) {
+        kernel<<<grid, 256, 0, st>>>(qpool, kpool_t, Mb, Np, T, scale, lut, mask);
+      };
+      if (T <= 64)
+        Np % 4 == 0 ? run(route_select_kernel<NK, 64, true>) : run(route_select_kernel<NK, 64, false>);
       else
-        route_select_kernel<NK, R, false><<<grid, 256, 0, st>>>(qpool, kpool_t, Mb, Np, T, scale, lut, mask);
+        Np % 4 == 0 ? run(route_select_kernel<NK, BIG, true>) : run(route_select_kernel<NK, BIG, false>);
     };
-    if (Np <= 512)
-      go(std::integral_constant<int, 8>{}, std::integral_constant<int, 1>{});
+    if (Np <= 64)
+      go(std::integral_constant<int, 1>{});
+    else if (Np <= 128)
+      go(std::integral_constant<int, 2>{});
+    else if (Np <= 256)
+      go(std::integral_constant<int, 4>{});
+    else if (Np <= 512)
+      go(std::integral_constant<int, 8>{});
     else if (Np <= 1024)
-      go(std::integral_constant<int, 16>{}, std::integral_constant<int, 1>{});
+      go(std::integral_constant<int, 16>{});
     else if (Np <= 2048)
-      go(std::integral_constant<int, 32>{}, std::integral_constant<int, 1>{});
+      go(std::integral_constant<int, 32>{});
     else
-      go(std::integral_constant<int, 64>{}, std::integral_constant<int, 1>{});
+      go(std::integral_constant<int, 64>{});
     return (int)hipGetLastError();
   }
   int P2 = 1;

@@ -585,3 +585,33 @@ def test_fp16_clamp_follows_the_exact_maximum():
           flush=True)
     assert max_abs(o, eo) < TOL_MAX and rel_l2(o, eo) < TOL_REL
     assert rel_l2(do, edo) < 1e-3
+
+
+@pytest.mark.parametrize("Np,T", [(1, 1), (5, 2), (64, 64), (65, 65), (128, 3), (130, 127), (256, 64),
+                                  (257, 65), (468, 117), (512, 512), (700, 20), (1023, 300),
+                                  (1500, 512), (1500, 513), (2049, 100), (4095, 65)])
+@pytest.mark.parametrize("coarse", [False, True])
+def test_route_topk_selection_sizes(Np, T, coarse):
+    """The LUT over every selection kernel (keys per lane 1 .. 64, winners up to 64,
+    512 and the full sort beyond), against the oracle's order: bit-exact.
+    coarse: pooled values on a grid of quarters, so that most scores tie and the
+    lower tile id must win, with -0, NaN and infinite scores among them."""
+    from imfvideo_amd import ops
+    H, Mb = 2, 5
+    g = torch.Generator().manual_seed(Np * 7 + T)
+    qp, kp = torch.randn(1, H, Mb, 64, generator=g), torch.randn(1, H, Np, 64, generator=g)
+    if coarse:
+        qp, kp = (torch.zeros_like(t).index_copy_(3, torch.tensor([0]), (t[..., :1] * 4).round() / 4)
+                  for t in (qp, kp))
+        kp[0, 0, Np // 2] = float("nan")
+        kp[0, 1, Np // 3, 0] = float("inf")
+        qp[0, 0, 1], qp[0, 1, 2] = 0.0, -0.0
+    print("[case] route_topk", Np, T, coarse, flush=True)
+    lut, mask = ops.route_topk(qp.cuda(), kp.transpose(-1, -2).contiguous().cuda(), T, 0.125,
+                               with_mask=True)
+    with np.errstate(all="ignore"):
+        want = O.topk_rows(O.route_scores(qp.numpy(), kp.numpy(), 0.125), T)
+    assert np.array_equal(lut.cpu().numpy(), want)
+    wm = np.zeros((1, H, Mb, Np), np.uint8)
+    np.put_along_axis(wm, want.astype(np.int64), 1, -1)
+    assert np.array_equal(mask.cpu().numpy(), wm)
