@@ -59,22 +59,17 @@ _WGRAD_MAX_TILES = 64
 def _own_wgrad(x, weight, bias):
     """The weight gradient of this call can come from sla2h_linear_wgrad: plain
     GPU tensors under a 16-bit autocast, eager first-order reverse mode."""
-    if not (bias is None and type(x) is torch.Tensor and x.is_cuda and x.dim() >= 2
-            and type(weight) in (nn.Parameter, torch.Tensor) and weight.device == x.device
+    if not (bias is None and x.is_cuda and x.dim() >= 2 and weight.device == x.device
             and weight.dtype == torch.float32 and weight.requires_grad
             and torch.is_grad_enabled() and torch.is_autocast_enabled("cuda")
             and torch.get_autocast_dtype("cuda") in (torch.bfloat16, torch.float16)
             and x.dtype in (torch.float32, torch.bfloat16, torch.float16)):
         return False
-    if (torch.compiler.is_compiling() or torch.jit.is_tracing()
-            or torch._C._are_functorch_transforms_active()
-            or torch.autograd.forward_ad._current_level >= 0):
-        return False
     M, N = weight.shape
     if x.shape[-1] != N or -(-M // 128) * -(-N // 128) > _WGRAD_MAX_TILES:
         return False
     from . import ops
-    return ops.linear_wgrad_ok(x.numel() // N, M, N)
+    return ops.plain_eager(x, weight) and ops.linear_wgrad_ok(x.numel() // N, M, N)
 
 
 class _Linear(nn.Linear):

@@ -41,6 +41,16 @@ def _need_gpu(*ts):
             raise RuntimeError("sla2h ops run on the GPU only; got a tensor on " + str(t.device))
 
 
+def plain_eager(*ts):
+    """Plain tensors (no subclass) in eager mode, outside torch.func transforms,
+    forward-mode AD, tracing and compilation: what the autograd Functions that
+    replace torch's own ops are for."""
+    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in ts)
+            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+            and not torch._C._are_functorch_transforms_active()
+            and torch.autograd.forward_ad._current_level < 0)
+
+
 def _bhld(t, name):
     if t.dim() != 4 or t.shape[-1] != E_TILE:
         raise ValueError(f"{name}: expected (B, H, L, 64), got {tuple(t.shape)}")
@@ -1086,6 +1096,55 @@ def residual_scale_bwd(dy, a, s):
         da.data_ptr(), ds.data_ptr(), ws.data_ptr(), _stream(a.device)),
         "sla2h_residual_scale_bwd")
     return da, ds
+
+
+# ---------------------------------------------------------------------------
+# Token layout of the cube module: (B, L, H, 64) in model order <-> (B, H, L, 64)
+# fp16 rows in tile order (models/sla2_cube_qat.py:345-357, 433-439)
+# ---------------------------------------------------------------------------
+def rows_in_ok(xs):
+    """The tensors can go through rows_in: same (B, L, H, 64) shape, device and
+    16-bit or fp32 dtype, unit channel stride, 16-byte aligned rows."""
+    x0 = xs[0]
+    if x0.dim() != 4 or x0.shape[-1] != E_TILE or x0.dtype not in _SITU_DTYPES or not x0.numel():
+        return False
+    for x in xs:
+        if not (x.is_cuda and x.shape == x0.shape and x.dtype == x0.dtype
+                and x.device == x0.device and x.stride(3) == 1 and x.data_ptr() % 16 == 0):
+            return False
+        if any(s * x.element_size() % 16 for s in x.stride()[:3]):
+            return False
+    return True
+
+
+def rows_in(xs, idx):
+    """1 to 3 (B, L, H, 64) tensors (rows_in_ok) -> (B, H, L, 64) fp16, row l from
+    token idx[l] (int64 on their device; None: l itself)."""
+    x0 = xs[0]
+    B, L, H, D = x0.shape
+    n = len(xs)
+    outs = [torch.empty(B, H, L, D, device=x0.device, dtype=torch.float16) for _ in xs]
+    strides = [s for x in xs for s in x.stride()[:3]]
+    _lib.check(_lib.load().sla2h_rows_in(
+        _ptrs(xs), (_lib._c_i64 * (3 * n))(*strides), n, _SITU_DTYPES[x0.dtype],
+        _ptr(idx), B, H, L, _ptrs(outs), _stream(x0.device)), "sla2h_rows_in")
+    return outs
+
+
+def rows_out(xs, idx, dtype):
+    """1 to 3 (B, H, L, 64) fp16 tensors -> (B, L, H, 64) contiguous in dtype, token
+    l from row idx[l]."""
+    xs = [x.contiguous() for x in xs]
+    B, H, L, D = xs[0].shape
+    outs = [torch.empty(B, L, H, D, device=x.device, dtype=dtype) for x in xs]
+    _lib.check(_lib.load().sla2h_rows_out(
+        _ptrs(xs), len(xs), _SITU_DTYPES[dtype], _ptr(idx), B, H, L, _ptrs(outs),
+        _stream(xs[0].device)), "sla2h_rows_out")
+    return outs
+
+
+def _ptrs(ts):
+    return (_lib._p * len(ts))(*[t.data_ptr() for t in ts])
 
 
 # ---------------------------------------------------------------------------

@@ -135,6 +135,55 @@ class _CubeQATFunction(torch.autograd.Function):
         return (dq, dk, dv, d_alpha, None, None, None, None, None, None, None, None, None)
 
 
+class _RowsIn(torch.autograd.Function):
+    """(B, L, H, 64) tensors -> the op's (B, H, L, 64) fp16 rows, row l from token
+    idx[l] (None: l): the reference's permute, index and .half() in one kernel;
+    the backward is _RowsOut by the inverse permutation `inv`."""
+
+    @staticmethod
+    def forward(ctx, idx, inv, *xs):
+        ctx.save_for_backward(idx, inv)
+        ctx.dtype = xs[0].dtype
+        return tuple(ops.rows_in(xs, idx))
+
+    @staticmethod
+    def backward(ctx, *ds):
+        idx, inv = ctx.saved_tensors
+        if idx is None:  # no permutation: the transposed view is the gradient
+            return (None, None, *(None if d is None else d.permute(0, 2, 1, 3).to(ctx.dtype)
+                                  for d in ds))
+        have = [i for i, d in enumerate(ds) if d is not None]
+        grads = [None] * len(ds)
+        if have:
+            outs = _RowsOut.apply(inv, idx, ctx.dtype, *(ds[i].contiguous() for i in have))
+            for i, g in zip(have, outs):
+                grads[i] = g
+        return (None, None, *grads)
+
+
+class _RowsOut(torch.autograd.Function):
+    """(B, H, L, 64) fp16 rows -> (B, L, H, 64) in dtype, token l from row idx[l];
+    the backward is _RowsIn."""
+
+    @staticmethod
+    def forward(ctx, idx, inv, dtype, *xs):
+        ctx.save_for_backward(idx, inv)
+        return tuple(ops.rows_out(xs, idx, dtype))
+
+    @staticmethod
+    def backward(ctx, *ds):
+        idx, inv = ctx.saved_tensors
+        have = [i for i, d in enumerate(ds) if d is not None]
+        grads = [None] * len(ds)
+        if have:
+            xs = [ds[i] for i in have]
+            if not ops.rows_in_ok(xs):
+                xs = [x.clone(memory_format=torch.contiguous_format) for x in xs]
+            for i, g in zip(have, _RowsIn.apply(inv, idx, *xs)):
+                grads[i] = g
+        return (None, None, None, *grads)
+
+
 class SLA2CubeQATAttentionImpl(nn.Module):
     """The cube-tile SLA2 attention as a DiT ``attn_impl`` (reference :295-439).
 
@@ -192,9 +241,19 @@ class SLA2CubeQATAttentionImpl(nn.Module):
                 x = x[:, :, self.perm]
             return x.half().contiguous()
 
-        o = self.forward_tile_major(tm(q), tm(k), tm(v))
+        # one kernel for the three operands (and one for the output) where they
+        # are plain GPU tensors with 16-byte rows; else the torch form
+        own = (ops.plain_eager(q, k, v) and ops.rows_in_ok((q, k, v)) and self.perm.device == q.device
+               and (self.pre_permuted or self.perm.numel() == q.shape[1]))
+        perm, inv = (None, None) if self.pre_permuted else (self.perm, self.inv)
+        if own:
+            o = self.forward_tile_major(*_RowsIn.apply(perm, inv, q, k, v))
+        else:
+            o = self.forward_tile_major(tm(q), tm(k), tm(v))
         if self.pre_permuted:
             return o.permute(0, 2, 1, 3).to(q.dtype)
+        if own:
+            return _RowsOut.apply(inv, perm, q.dtype, o)[0]
         return o[:, :, self.inv].permute(0, 2, 1, 3).to(q.dtype)
 
     def forward_tile_major(self, qh, kh, vh):

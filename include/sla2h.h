@@ -687,6 +687,22 @@ int sla2h_lin_fwd3(const void* qphi, const void* comp, const void* o_s, const fl
                    float eps_l, void* o, void* stream);
 
 /*
+ * Token layout of the cube op, for n = 1 to 3 tensors of one dtype (0 / 1 / 2 =
+ * fp16 / bf16 / fp32).  rows_in: x[t] (B, L, H, 64), unit channel stride, strides
+ * of (b, l, h) in elements at strides[3 t ..], 16-byte aligned, to out[t]
+ * (B, H, L, 64) fp16, row l from token idx[l] (int64, NULL: l).  rows_out: x[t]
+ * (B, H, L, 64) fp16 to out[t] (B, L, H, 64) contiguous in dtype, token l from
+ * row idx[l].  x, strides and out are host arrays.  With idx a permutation and
+ * its inverse each is the other's backward.
+ * Replaces the index / permute / .half() of SLA2CubeQATAttentionImpl.forward
+ * (models/sla2_cube_qat.py:345-357, 433-439) and their backward.
+ */
+int sla2h_rows_in(const void* const* x, const int64_t* strides, int n, int dtype,
+                  const int64_t* idx, int B, int H, int64_t L, void* const* out, void* stream);
+int sla2h_rows_out(const void* const* x, int n, int dtype, const int64_t* idx, int B, int H,
+                   int64_t L, void* const* out, void* stream);
+
+/*
  * Weight gradient of a linear layer, dw[m][n] = sum over rows t of dy[t][m] x[t][n],
  * 16-bit dy (rows, M; row stride ldy) and x (rows, N; row stride ldx), fp32
  * accumulation and result (M, N).  M, N, ldy, ldx multiples of 8, 16-byte

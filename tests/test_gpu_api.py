@@ -273,3 +273,51 @@ def test_sublayer_jvp_pre_permuted_matches_model_order(monkeypatch):
         print(f"  {n} vs oracle: max {max_abs(got, w_):.2e} rel {rel_l2(got, w_):.2e}",
               flush=True)
         assert max_abs(got, w_) < bound and rel_l2(got, w_) < TOL_REL
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("layout", ["contiguous", "heads_first", "unaligned", "mixed"])
+@pytest.mark.parametrize("pre_permuted", [False, True])
+def test_module_token_layout_matches_torch(dt, layout, pre_permuted):
+    """The module's operand and output layout against torch's index / permute /
+    .half() on the same values: the rows, the output and every gradient's layout
+    pass equal to the bit, for each stride order the kernels take and for
+    layouts that go through torch (rows off 16 bytes, mixed dtypes)."""
+    from imfvideo_amd.sla2_cube_qat import SLA2CubeQATAttentionImpl
+    say = f"[case] module layout {dt} {layout} {pre_permuted}"
+    print(say, flush=True)
+    torch.manual_seed(3)
+    B, H, grid, P = 2, 3, (4, 8, 8), 18
+    L = 256 + P
+    mod = SLA2CubeQATAttentionImpl(64, L, H, grid, topk=0.5, pre_permuted=pre_permuted).cuda()
+    xs = []
+    for _ in range(3):
+        x = torch.randn(B, L, H, 64, device="cuda").to(dt)
+        if layout == "heads_first":
+            x = x.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3)
+        elif layout == "unaligned":
+            w = torch.empty(B, L, H, 65, device="cuda", dtype=dt)
+            w[..., 1:] = x
+            x = w[..., 1:]
+        xs.append(x)
+    if layout == "mixed":
+        xs[1] = xs[1].to(torch.float32 if dt != torch.float32 else torch.bfloat16)
+    seen = []
+
+    def fake(q, k, v):  # the op replaced by a differentiable function of its operands
+        seen.append((q, k, v))
+        return q * 2 + k * v
+
+    mod.forward_tile_major = fake
+    xs = [x.detach().requires_grad_() for x in xs]
+    o = mod(*xs)
+    do = torch.randn(o.shape, device="cuda").to(o.dtype)
+    grads = torch.autograd.grad(o, xs, do)
+    perm, inv = (slice(None), slice(None)) if pre_permuted else (mod.perm, mod.inv)
+    rows = [x.permute(0, 2, 1, 3)[:, :, perm].half().contiguous() for x in xs]
+    for a, b in zip(seen[0], rows):
+        assert a.dtype == b.dtype == torch.float16 and a.is_contiguous() and torch.equal(a, b)
+    want = (rows[0] * 2 + rows[1] * rows[2])[:, :, inv].permute(0, 2, 1, 3).to(xs[0].dtype)
+    assert o.dtype == want.dtype and torch.equal(o, want)
+    for g, gw in zip(grads, torch.autograd.grad(want, xs, do)):
+        assert g.dtype == gw.dtype and torch.equal(g, gw)
