@@ -39,6 +39,8 @@ SIGNATURES = {
                                _c_f, _c_f, _c_int, _p, _p, _p]),
     "sla2h_pool_blocks": (_c_int, [_p, _c_int, _c_i64, _c_i64, _c_int, _c_int, _p, _c_int, _p,
                                    _p]),
+    "sla2h_pool_qk": (_c_int, [_p, _p, _c_int, _c_int, _c_int, _c_i64, _c_int, _c_int, _c_int,
+                               _c_int, _p, _p, _p, _p, _p]),
     "sla2h_fwd_jvp_1d": (_c_int, [_p, _p, _p, _p, _p, _p, _c_int, _p, _c_int, _c_int, _c_int,
                                   _c_i64, _c_int, _c_int, _c_int, _c_int, _c_f, _c_f, _p, _p,
                                   _p]),

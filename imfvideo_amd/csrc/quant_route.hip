@@ -687,6 +687,138 @@ __global__ __launch_bounds__(64) void pool_blocks_kernel(const Raw* __restrict__
     out[((int64_t)bh * nblk + j) * kTile + d] = outv;
 }
 
+// The same block means and projections for a query and a key tensor of 16-bit
+// rows in one launch: half a wave per block (lane c: channels 2 c, 2 c + 1, one
+// 128-byte row per load, 64 rows of loads in flight ahead of the ordered adds
+// and beside the staging of the projection), eight blocks per workgroup.
+// Bound by the read of x where there is enough of it: 2 x 16 heads x 29,952 fp16
+// rows (123 MB) in 33.8 us (3.6 TB/s), where the quantising kernel that the
+// cube router borrowed also wrote 61 MB of INT8 rows (65.4 us); small ones by
+// the ordered sums' latency: 8 x 13,901 rows, 128-row query blocks 13.8 us (two
+// launches of pool_blocks_kernel: 17.2 us).
+struct PoolPairArgs {
+  const uint16_t* x[2];
+  const float* proj[2];  // (64, 64) or null
+  float* out[2];         // [0] (BH, n, 64), [1] transposed (BH, 64, n)
+  int blk[2], n[2];      // rows per block, blocks per head
+  int BH;
+  int64_t L;
+  int wg0;               // workgroups of tensor 0
+};
+
+template <typename T16>
+__global__ __launch_bounds__(256) void pool_pair_kernel(PoolPairArgs a) {
+  __shared__ __align__(16) float pt[kTile][kTile + 4];  // the projection [d][e]
+  __shared__ __align__(16) float mean[8][kTile];
+  const int tid = threadIdx.x;
+  const int hw = tid >> 5, c = tid & 31;
+  // workgroups of tensor 0, then of tensor 1 (one projection per workgroup)
+  const int t = (int)blockIdx.x >= a.wg0;
+  const int64_t jj = (int64_t)((int)blockIdx.x - (t ? a.wg0 : 0)) * 8 + hw;
+  const bool on = jj < (int64_t)a.BH * a.n[t];
+  const int64_t bh = on ? jj / a.n[t] : 0;
+  const int j = on ? (int)(jj - bh * a.n[t]) : 0;
+  const int64_t r0 = (int64_t)j * a.blk[t];
+  const int cnt = (int)(a.L - r0 < a.blk[t] ? a.L - r0 : a.blk[t]);
+  const uint32_t* src = reinterpret_cast<const uint32_t*>(a.x[t]) + (bh * a.L + r0) * 32 + c;
+  constexpr int kRows = 64;
+  uint32_t v[kRows];
+  auto load = [&](int rr) {  // rows past the block reload its last one
+#pragma unroll
+    for (int u = 0; u < kRows; ++u) {
+      const int row = rr + u < cnt ? rr + u : cnt - 1;
+      v[u] = src[row * 32];
+    }
+  };
+  load(0);
+  const float* proj = a.proj[t];
+  if (proj != nullptr) {
+    for (int i = tid; i < kTile * kTile; i += 256) pt[i & 63][i >> 6] = proj[i];
+    __syncthreads();
+  }
+  float s0 = 0.f, s1 = 0.f;
+  for (int rr = 0;;) {
+    if (rr + kRows <= cnt) {
+#pragma unroll
+      for (int u = 0; u < kRows; ++u) {
+        s0 = s0 + T16::to_f32((uint16_t)(v[u] & 0xffff));
+        s1 = s1 + T16::to_f32((uint16_t)(v[u] >> 16));
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < kRows; ++u) {
+        if (rr + u < cnt) {
+          s0 = s0 + T16::to_f32((uint16_t)(v[u] & 0xffff));
+          s1 = s1 + T16::to_f32((uint16_t)(v[u] >> 16));
+        }
+      }
+    }
+    rr += kRows;
+    if (rr >= cnt) break;
+    load(rr);
+  }
+  s0 = s0 / (float)cnt;
+  s1 = s1 / (float)cnt;
+  if (proj != nullptr) {
+    *reinterpret_cast<float2*>(&mean[hw][2 * c]) = make_float2(s0, s1);
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    float p0 = 0.f, p1 = 0.f;
+#pragma unroll 16
+    for (int d = 0; d < kTile; ++d) {
+      const float m = mean[hw][d];
+      const float2 w = *reinterpret_cast<const float2*>(&pt[d][2 * c]);
+      p0 = p0 + m * w.x;
+      p1 = p1 + m * w.y;
+    }
+    s0 = p0;
+    s1 = p1;
+  }
+  if (!on) return;
+  if (t) {
+    float* o = a.out[1] + (bh * kTile + 2 * c) * a.n[1] + j;
+    o[0] = s0;
+    o[a.n[1]] = s1;
+  } else {
+    *reinterpret_cast<float2*>(a.out[0] + jj * kTile + 2 * c) = make_float2(s0, s1);
+  }
+}
+
+extern "C" int sla2h_pool_qk(const void* q, const void* k, int dtype, int B, int H, int64_t L,
+                             int D, int bq, int bk, int Nk, const float* proj_q,
+                             const float* proj_k, float* qpool, float* kpool_t, void* stream) {
+  SLA2H_CHECK_ARG(q && k && qpool && kpool_t);
+  SLA2H_CHECK_ARG(D == kTile && bq >= 1 && bq <= 4096 && bk == kTile);
+  SLA2H_CHECK_ARG(dtype == SLA2H_DTYPE_F16 || dtype == SLA2H_DTYPE_BF16);
+  SLA2H_CHECK_ARG(B > 0 && H > 0 && (int64_t)B * H <= 65535 && L > 0);
+  SLA2H_CHECK_ARG(((uintptr_t)q | (uintptr_t)k) % 4 == 0 && (uintptr_t)qpool % 8 == 0);
+  const int64_t nq = (L + bq - 1) / bq;
+  SLA2H_CHECK_ARG(nq < (1ll << 31) && Nk > 0 && (int64_t)(Nk - 1) * bk < L);
+  PoolPairArgs a = {};
+  a.x[0] = static_cast<const uint16_t*>(q);
+  a.x[1] = static_cast<const uint16_t*>(k);
+  a.proj[0] = proj_q;
+  a.proj[1] = proj_k;
+  a.out[0] = qpool;
+  a.out[1] = kpool_t;
+  a.blk[0] = bq;
+  a.blk[1] = bk;
+  a.n[0] = (int)nq;
+  a.n[1] = Nk;
+  a.BH = B * H;
+  a.L = L;
+  const int64_t wq = ((int64_t)a.BH * nq + 7) / 8, wk = ((int64_t)a.BH * Nk + 7) / 8;
+  SLA2H_CHECK_ARG(wq + wk < (1ll << 31));
+  a.wg0 = (int)wq;
+  const unsigned grid = (unsigned)(wq + wk);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (dtype == SLA2H_DTYPE_BF16)
+    pool_pair_kernel<BF16><<<grid, 256, 0, st>>>(a);
+  else
+    pool_pair_kernel<F16><<<grid, 256, 0, st>>>(a);
+  return (int)hipGetLastError();
+}
+
 extern "C" int sla2h_pool_blocks(const void* x, int dtype, int64_t BH, int64_t L, int D, int blk,
                                  const float* proj, int transposed, float* out, void* stream) {
   SLA2H_CHECK_ARG(x && out);

@@ -3,7 +3,7 @@ reference's names and signatures (models/mla_video_sparse_jvp.py).
 
 On the gfx950 kernels:
   ``route_tiles`` (:268-295) and ``route_tiles_fast`` (:532-566): pooling,
-  projections, scores and the top-k behind ``sla2h_quant_pool_qk`` and
+  projections, scores and the top-k behind ``sla2h_pool_qk`` and
   ``sla2h_route_topk``, one pinned fp32 evaluation order, so the selected
   tile sets are reproducible bit for bit;
   ``mla_video_sparse_jvp`` (:403-454): the cube JVP with 16-bit primal
@@ -77,7 +77,9 @@ def route_tiles_fast(q, k, topk_frac, Np, E, prefix_len, proj_q=None, proj_k=Non
         kpool_t = ops.pool_blocks(k[:, :, :Np * E].contiguous(), E, proj_k, transposed=True)
     else:
         q, k = _to16(q), _to16(k)
-        _, _, _, _, qpool, kpool_t = ops.quant_pool_qk(q, k.to(q.dtype), Np, E, proj_q, proj_k)
+        if Np * E > L or 2 * B * H > 65535:
+            raise RuntimeError(f"route_tiles_fast: Np={Np} tiles of {E} in {L} tokens, {B * H} heads")
+        qpool, kpool_t = ops.pool_qk(q, k.to(q.dtype), E, Np, proj_q, proj_k, bk=E)
     T = ops.topk_count(topk_frac, Np)
     lut = ops.route_topk(qpool, kpool_t, T, D ** -0.5)
     return lut, T

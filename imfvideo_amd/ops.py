@@ -537,6 +537,25 @@ def pool_blocks(x, blk, proj=None, transposed=False):
     return out
 
 
+def pool_qk(q, k, bq, Nk, proj_q=None, proj_k=None, bk=E_TILE):
+    """pool_blocks of 16-bit q over bq rows (B,H,ceil(L/bq),64) and of k's first Nk
+    blocks of 64 rows, transposed (B,H,64,Nk), in one launch."""
+    _need_gpu(q, k, proj_q, proj_k)
+    q, k = _bhld(q, "q"), _bhld(k, "k")
+    if q.shape != k.shape or q.dtype != k.dtype:
+        raise ValueError("q and k must share shape and dtype")
+    B, H, L, D = q.shape
+    dev = q.device
+    pq, pk = (None if p is None else p.detach().to(dev, torch.float32).contiguous()
+              for p in (proj_q, proj_k))
+    qpool = torch.empty(B, H, -(-L // bq), D, device=dev, dtype=torch.float32)
+    kpool_t = torch.empty(B, H, D, Nk, device=dev, dtype=torch.float32)
+    _lib.check(_lib.load().sla2h_pool_qk(
+        q.data_ptr(), k.data_ptr(), _dtype_code(q), B, H, L, D, bq, bk, Nk, _ptr(pq), _ptr(pk),
+        qpool.data_ptr(), kpool_t.data_ptr(), _stream(dev)), "sla2h_pool_qk")
+    return qpool, kpool_t
+
+
 def route_1d(q, k, topk_frac, bq, bk=E_TILE, proj_q=None, proj_k=None):
     """1-D router: pooled-score hard top-k -> (lut (B,H,ceil(L/bq),T) int32, T)."""
     if bk != E_TILE:
@@ -544,8 +563,11 @@ def route_1d(q, k, topk_frac, bq, bk=E_TILE, proj_q=None, proj_k=None):
     B, H, L, D = q.shape
     nb = -(-L // bk)
     T = max(1, min(nb, int(topk_frac * nb)))
-    qpool = pool_blocks(q, bq, proj_q)
-    kpool_t = pool_blocks(k, bk, proj_k, transposed=True)
+    if q.dtype == k.dtype and q.dtype in _F16_CODES and q.shape == k.shape:
+        qpool, kpool_t = pool_qk(q, k, bq, nb, proj_q, proj_k)
+    else:
+        qpool = pool_blocks(q, bq, proj_q)
+        kpool_t = pool_blocks(k, bk, proj_k, transposed=True)
     return route_topk(qpool, kpool_t, T, D ** -0.5), T
 
 

@@ -202,6 +202,17 @@ int sla2h_pool_blocks(const void* x, int dtype, int64_t BH, int64_t L, int D, in
                       const float* proj, int transposed, float* out, void* stream);
 
 /*
+ * Both router inputs of 16-bit q and k (B,H,L,64) in one launch: qpool
+ * (B,H,ceil(L/bq),64) = means over bq rows, kpool_t (B,H,64,Nk) = means over the
+ * first Nk blocks of bk = 64 rows, transposed, each after its optional projection;
+ * sla2h_pool_blocks' arithmetic and order.  A block that reaches past L (only
+ * the last one can) averages its real rows.
+ */
+int sla2h_pool_qk(const void* q, const void* k, int dtype, int B, int H, int64_t L, int D, int bq,
+                  int bk, int Nk, const float* proj_q, const float* proj_k, float* qpool,
+                  float* kpool_t, void* stream);
+
+/*
  * 1-D SLA2 attention with forward-mode JVP (sla2_mla_jvp): as sla2h_fwd_jvp but
  * with 16-bit primal scores S = q.k^T (fp32 accumulate; no INT8), query blocks
  * of bq rows (bq = 64, 128 or 256; lut (B,H,ceil(L/bq),T), alpha (H,

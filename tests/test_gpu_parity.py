@@ -615,3 +615,26 @@ def test_route_topk_selection_sizes(Np, T, coarse):
     wm = np.zeros((1, H, Mb, Np), np.uint8)
     np.put_along_axis(wm, want.astype(np.int64), 1, -1)
     assert np.array_equal(mask.cpu().numpy(), wm)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("BH,L,bq,short", [(1, 1, 64, 0), (3, 63, 64, 0), (2, 274, 64, 1), (2, 583, 128, 0),
+                                           (5, 1000, 256, 0), (2, 4160, 128, 2), (40, 4100, 64, 1)])
+@pytest.mark.parametrize("proj", [False, True])
+def test_pool_qk_matches_pool_blocks(dt, BH, L, bq, short, proj):
+    """Both pooled tensors in one launch equal pool_blocks' per tensor (and, for one
+    size, the oracle's) to the bit: ragged last blocks, key blocks left out
+    (prefix tails), more blocks than one round of the grid."""
+    from imfvideo_amd import ops
+    print("[case] pool_qk", dt, BH, L, bq, short, proj, flush=True)
+    g = torch.Generator().manual_seed(L)
+    q, k = (torch.randn(1, BH, L, 64, generator=g).to(dt).cuda() for _ in range(2))
+    pq, pk = (torch.randn(64, 64, generator=g).cuda() if proj else None for _ in range(2))
+    Nk = -(-L // 64) - short
+    qp, kp = ops.pool_qk(q, k, bq, Nk, pq, pk)
+    assert torch.equal(qp, ops.pool_blocks(q, bq, pq))
+    assert torch.equal(kp, ops.pool_blocks(k, 64, pk, transposed=True)[..., :Nk])
+    if L == 583:
+        want = O.project_pool(O.pool_tiles(q.cpu().float(), -(-L // bq), L, block=bq),
+                              None if pq is None else pq.cpu())
+        assert np.array_equal(qp.cpu().numpy(), want)
