@@ -76,6 +76,29 @@ SIGNATURES = {
                                     _p, _p]),
     "sla2h_situ_mul_bwd": (_c_int, [_p, _p, _p, _c_int, _c_i64, _c_int, _c_i64, _c_i64, _c_f,
                                     _c_f, _p, _p, _p]),
+    "sla2h_cube_jvp_workspace_bytes": (ctypes.c_size_t, [_c_int, _c_int, _c_i64, _c_int, _c_int,
+                                                         _c_int]),
+    "sla2h_cube_jvp_quant": (_c_int, [_p, _p, _c_int, _c_int, _c_int, _c_i64, _c_int, _c_int,
+                                      _c_int, _p, _p, _p, _p, _p, _p]),
+    "sla2h_cube_jvp_attn": (_c_int, [_p, _p, _p, _p, _p, _p, _p, _c_int, _p, _c_int, _c_int,
+                                     _c_int, _c_i64, _c_int, _c_int, _c_f, _c_f, _p, _p, _p, _p]),
+    "sla2h_jvp16_workspace_bytes": (ctypes.c_size_t, [_c_int, _c_int, _c_i64, _c_int, _c_int,
+                                                      _c_int]),
+    "sla2h_jvp16": (_c_int, [_p, _p, _p, _p, _p, _p, _p, _c_int, _p, _c_int, _c_int, _c_int,
+                             _c_i64, _c_int, _c_int, _c_int, _c_f, _c_f, _p, _p, _p, _p]),
+    "sla2h_train_saved_bytes": (ctypes.c_size_t, [_c_int, _c_int, _c_i64, _c_int, _c_int, _c_int]),
+    "sla2h_train_fwd_workspace_bytes": (ctypes.c_size_t, [_c_int, _c_int, _c_i64, _c_int, _c_int,
+                                                          _c_int, _c_int]),
+    "sla2h_train_fwd": (_c_int, [_p, _p, _p, _p, _p, _c_int, _c_int, _c_int, _c_i64, _c_int,
+                                 _c_int, _c_int, _c_int, _c_f, _c_f, _p, _p, _p, _p, _p]),
+    "sla2h_train_bwd_workspace_bytes": (ctypes.c_size_t, [_c_int, _c_int, _c_i64, _c_int, _c_int,
+                                                          _c_int]),
+    "sla2h_train_bwd": (_c_int, [_p, _p, _p, _p, _p, _c_int, _c_int, _c_int, _c_i64, _c_int,
+                                 _c_int, _c_int, _c_f, _p, _p, _p, _p, _p, _p]),
+    "sla2h_sla2_infer_workspace_bytes": (ctypes.c_size_t, [_c_int, _c_int, _c_i64, _c_int, _c_int,
+                                                           _c_int]),
+    "sla2h_sla2_infer": (_c_int, [_p, _p, _p, _p, _c_int, _p, _c_int, _c_int, _c_int, _c_i64,
+                                  _c_int, _c_int, _c_int, _c_int, _c_f, _c_f, _p, _p, _p]),
     "sla2h_rows_in": (_c_int, [_p, _p, _c_int, _c_int, _p, _c_int, _c_int, _c_i64, _p, _p]),
     "sla2h_rows_out": (_c_int, [_p, _c_int, _c_int, _p, _c_int, _c_int, _c_i64, _p, _p]),
     "sla2h_linear_wgrad_workspace_bytes": (ctypes.c_size_t, [_c_i64, _c_int, _c_int]),

@@ -33,6 +33,7 @@ SOURCES = {
     "mla_glue.hip": [],
     "block_train.hip": [],
     "linear_bwd.hip": [],
+    "pipeline.hip": [],
 }
 
 COMMON_FLAGS = [

@@ -69,6 +69,7 @@ struct PrepArgs {
   uint16_t* g16;
   float* s;
   float* seg;
+  float* segp = nullptr;  // set: the block's segment sum is stored here, (BH, Nb)
   float* P;
   float* Pz;
   int64_t L;
@@ -159,8 +160,13 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(PrepArgs a) {
   for (int m = 32; m >= 1; m >>= 1) segp += __shfl_xor(segp, m, 64);
   if ((tid & 63) == 0) red[tid >> 6] = segp;
   __syncthreads();
-  if (tid == 0)
-    atomicAdd(a.seg + (int64_t)h * a.Mq + (blk >> a.qshift), (red[0] + red[1]) + (red[2] + red[3]));
+  if (tid == 0) {
+    const float sum = (red[0] + red[1]) + (red[2] + red[3]);
+    if (a.segp != nullptr)
+      a.segp[(int64_t)bh * a.Nb + blk] = sum;
+    else
+      atomicAdd(a.seg + (int64_t)h * a.Mq + (blk >> a.qshift), sum);
+  }
 
   // P[d][e] = sum_rows qphi[row][d] g[row][e] on fp32 MFMA, computed as P^T so
   // that a lane holds four consecutive e of one d (16-byte stores): wave w owns
@@ -866,13 +872,15 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_kernel(DkdvArgs a) {
 
 using namespace sla2h;
 
-extern "C" int sla2h_bwd_prep(const void* dout, const void* o_s, const void* o_l, const float* den,
-                              const void* qphi, const float* alpha, int alpha_stride, int dtype,
-                              int B, int H, int64_t L, int D, int E, void* dos, float* delta,
-                              void* g16, float* s, float* seg, float* P, float* Pz, void* stream) {
-  SLA2H_CHECK_ARG(dout && o_s && o_l && den && qphi && alpha && dos && delta && g16 && s && seg &&
-                  P && Pz);
-  SLA2H_CHECK_ARG(D == kT && (E == 64 || E == 128 || E == 256) && alpha_stride >= 0);
+namespace sla2h {
+namespace {
+int launch_bwd_prep(const void* dout, const void* o_s, const void* o_l, const float* den,
+                    const void* qphi, const float* alpha, int alpha_stride, int dtype, int B,
+                    int H, int64_t L, int E, void* dos, float* delta, void* g16, float* s,
+                    float* seg, float* segp, float* P, float* Pz, void* stream) {
+  SLA2H_CHECK_ARG(dout && o_s && o_l && den && qphi && alpha && dos && delta && g16 && s &&
+                  (seg || segp) && P && Pz);
+  SLA2H_CHECK_ARG((E == 64 || E == 128 || E == 256) && alpha_stride >= 0);
   SLA2H_CHECK_ARG(dtype == SLA2H_DTYPE_F16 || dtype == SLA2H_DTYPE_BF16);
   SLA2H_CHECK_ARG(B > 0 && H > 0 && B * H <= 65535 && L > 0);
   PrepArgs a;
@@ -889,6 +897,7 @@ extern "C" int sla2h_bwd_prep(const void* dout, const void* o_s, const void* o_l
   a.g16 = static_cast<uint16_t*>(g16);
   a.s = s;
   a.seg = seg;
+  a.segp = segp;
   a.P = P;
   a.Pz = Pz;
   a.L = L;
@@ -902,6 +911,25 @@ extern "C" int sla2h_bwd_prep(const void* dout, const void* o_s, const void* o_l
   else
     bwd_prep_kernel<F16><<<grid, 256, 0, st>>>(a);
   return (int)hipGetLastError();
+}
+}  // namespace
+
+int bwd_prep_segp(const void* dout, const void* o_s, const void* o_l, const float* den,
+                  const void* qphi, const float* alpha, int alpha_stride, int dtype, int B, int H,
+                  int64_t L, int E, void* dos, float* delta, void* g16, float* s, float* segp,
+                  float* P, float* Pz, void* stream) {
+  return launch_bwd_prep(dout, o_s, o_l, den, qphi, alpha, alpha_stride, dtype, B, H, L, E, dos,
+                         delta, g16, s, nullptr, segp, P, Pz, stream);
+}
+}  // namespace sla2h
+
+extern "C" int sla2h_bwd_prep(const void* dout, const void* o_s, const void* o_l, const float* den,
+                              const void* qphi, const float* alpha, int alpha_stride, int dtype,
+                              int B, int H, int64_t L, int D, int E, void* dos, float* delta,
+                              void* g16, float* s, float* seg, float* P, float* Pz, void* stream) {
+  SLA2H_CHECK_ARG(D == kT && seg);
+  return launch_bwd_prep(dout, o_s, o_l, den, qphi, alpha, alpha_stride, dtype, B, H, L, E, dos,
+                         delta, g16, s, seg, nullptr, P, Pz, stream);
 }
 
 extern "C" int sla2h_bwd_dq(const void* q, const void* k, const void* v, const void* dos,

@@ -1,0 +1,463 @@
+// Whole calls of the op in one host entry each: the stages' launches in order
+// on one stream, with their intermediates carved out of one caller-owned
+// workspace.  The stages are the entry points of include/sla2h.h; what is
+// added here are the small kernels between them that torch ran as chains of
+// elementwise launches (alpha from its logits, the LUT with the prefix tail,
+// the per-head maximum of lse, the alpha gradient).
+//
+// On small shapes the op is bound by the host: per stage a Python wrapper, its
+// output allocations and its launch.  One call per pass leaves the launches.
+#include "common.h"
+
+namespace sla2h {
+
+namespace {
+
+constexpr int kT = 64;
+constexpr size_t kRecBytes = 33280;
+
+// Consecutive 256-byte aligned pieces of one buffer; with base NULL only the
+// size is added up.
+struct Carve {
+  unsigned char* base;
+  size_t used = 0;
+  template <typename T>
+  T* take(size_t n) {
+    T* p = base == nullptr ? nullptr : reinterpret_cast<T*>(base + used);
+    used += (n * sizeof(T) + 255) / 256 * 256;
+    return p;
+  }
+};
+
+struct Dims {
+  int B, H;
+  int64_t L;
+  int Nb;  // 64-row blocks
+  int Np;  // routable blocks
+  int bq, Mq, T, J;  // query blocks of bq rows; LUT columns, with the tail J
+  size_t BH, rows, elems;
+  Dims(int B_, int H_, int64_t L_, int Np_, int bq_, int T_)
+      : B(B_), H(H_), L(L_), Nb((int)((L_ + kT - 1) / kT)), Np(Np_), bq(bq_),
+        Mq((int)((L_ + bq_ - 1) / bq_)), T(T_), J(T_ + Nb - Np_), BH((size_t)B_ * H_),
+        rows(BH * L_), elems(rows * kT) {}
+};
+
+bool dims_ok(int dtype, int B, int H, int64_t L, int Np, int bq, int T) {
+  return (dtype == SLA2H_DTYPE_F16 || dtype == SLA2H_DTYPE_BF16) && B > 0 && H > 0 &&
+         (int64_t)B * H <= 65535 && L > 0 && L * kT * 2 < (1ll << 31) && Np > 0 &&
+         (int64_t)(Np - 1) * kT < L && (bq == 64 || bq == 128 || bq == 256) && T >= 1 && T <= Np;
+}
+
+// alpha = sigmoid(logit); LUT rows with the tail blocks Np .. Nb - 1 appended;
+// stats = -inf.  Each part may be absent (n = 0 or NULL).
+__global__ __launch_bounds__(256) void train_setup_kernel(const float* __restrict__ logit, int na,
+                                                         float* __restrict__ alpha,
+                                                         const int32_t* __restrict__ lut,
+                                                         int64_t nl, int T, int J, int Np,
+                                                         int32_t* __restrict__ lut_aug,
+                                                         float* __restrict__ stats, int H) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < na) alpha[i] = 1.0f / (1.0f + expf(-logit[i]));
+  if (stats != nullptr && i < H) stats[i] = -INFINITY;
+  if (i < nl) {
+    const int64_t row = i / J;
+    const int j = (int)(i - row * J);
+    lut_aug[i] = j < T ? lut[row * T + j] : Np + (j - T);
+  }
+}
+
+// fp32 maximum by integer atomics: positive floats order as int, negative ones
+// in reverse as unsigned (NaN, made positive, above everything)
+__device__ inline void atomic_max_f32(float* p, float v) {
+  if (v != v) v = __builtin_bit_cast(float, 0x7fc00000);
+  if (__builtin_bit_cast(int, v) >= 0)
+    atomicMax(reinterpret_cast<int*>(p), __builtin_bit_cast(int, v));
+  else
+    atomicMin(reinterpret_cast<unsigned*>(p), __builtin_bit_cast(unsigned, v));
+}
+
+// stats[h] = max over batch and rows of lse (B, H, L); stats starts at -inf
+__global__ __launch_bounds__(256) void head_max_kernel(const float* __restrict__ lse, int64_t L,
+                                                      int H, float* __restrict__ stats) {
+  const float* src = lse + (int64_t)blockIdx.y * L;
+  float m = -INFINITY;
+  bool nan = false;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < L; i += (int64_t)gridDim.x * 256) {
+    const float x = src[i];
+    nan |= x != x;
+    m = fmaxf(m, x);
+  }
+#pragma unroll
+  for (int s = 32; s >= 1; s >>= 1) {
+    m = fmaxf(m, __shfl_xor(m, s, 64));
+    nan |= __shfl_xor((int)nan, s, 64) != 0;
+  }
+  if (nan) m = __builtin_bit_cast(float, 0x7fc00000);
+  if ((threadIdx.x & 63) == 0) atomic_max_f32(stats + blockIdx.y % H, m);
+}
+
+// d_logit[h][m] = seg a (1 - a), seg summed over the batches and the 64-row
+// blocks of query block m in order
+__global__ __launch_bounds__(256) void alpha_grad_kernel(const float* __restrict__ segp,
+                                                        const float* __restrict__ alpha, int B,
+                                                        int H, int Nb, int Mq, int sub,
+                                                        float* __restrict__ d) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= H * Mq) return;
+  const int h = i / Mq, m = i - h * Mq;
+  float s = 0.f;
+  for (int b = 0; b < B; ++b)
+    for (int n = m * sub; n < min(Nb, (m + 1) * sub); ++n)
+      s += segp[((int64_t)b * H + h) * Nb + n];
+  const float a = alpha[i];
+  d[i] = s * a * (1.0f - a);
+}
+
+struct JvpWs {
+  int8_t *q8, *k8;
+  float *qs, *ks, *kb, *Hb, *dHb, *zb, *dzb;
+  uint16_t *vt, *kt;
+  unsigned char *bits, *comp;
+  int32_t* lut;
+  size_t bytes;
+  // int8: the cube op's quantised scores; else 16-bit scores, LUT with its tail
+  JvpWs(void* p, const Dims& d, bool tan, bool int8) {
+    Carve c{static_cast<unsigned char*>(p)};
+    const size_t nb = d.BH * d.Nb, np = d.BH * d.Np;
+    if (int8) {
+      q8 = c.take<int8_t>(d.elems);
+      k8 = c.take<int8_t>(d.elems);
+      qs = c.take<float>(nb);
+      ks = c.take<float>(nb);
+      kb = c.take<float>(nb);
+    }
+    Hb = c.take<float>(np * kT * kT);
+    zb = c.take<float>(np * kT);
+    dHb = tan ? c.take<float>(np * kT * kT) : nullptr;
+    dzb = tan ? c.take<float>(np * kT) : nullptr;
+    vt = c.take<uint16_t>(nb * kT * kT * (tan ? 2 : 1));
+    kt = tan ? c.take<uint16_t>(nb * kT * kT * 2) : nullptr;
+    bits = c.take<unsigned char>(sla2h_complement_workspace_bytes(d.B, d.H, d.Mq, d.Np));
+    comp = c.take<unsigned char>(d.BH * d.Mq * kRecBytes);
+    lut = !int8 && d.J > d.T ? c.take<int32_t>(d.BH * d.Mq * d.J) : nullptr;
+    bytes = c.used;
+  }
+};
+
+// What the training forward keeps for the backward
+struct Saved {
+  uint16_t *o_s, *o_l, *qphi;
+  float *lse, *den, *Hall, *alpha;
+  unsigned char* comp;
+  int32_t* lut;
+  size_t bytes;
+  Saved(void* p, const Dims& d) {
+    Carve c{static_cast<unsigned char*>(p)};
+    o_s = c.take<uint16_t>(d.elems);
+    o_l = c.take<uint16_t>(d.elems);
+    qphi = c.take<uint16_t>(d.elems);
+    lse = c.take<float>(d.rows);
+    den = c.take<float>(d.rows);
+    Hall = c.take<float>(d.BH * kT * kT);
+    alpha = c.take<float>((size_t)d.H * d.Mq);
+    comp = c.take<unsigned char>(d.BH * d.Mq * kRecBytes);
+    lut = c.take<int32_t>(d.BH * d.Mq * d.J);
+    bytes = c.used;
+  }
+};
+
+struct FwdWs {
+  int8_t *q8, *k8, *v8f;
+  float *qs, *ks, *vs, *Hb, *zb, *zall;
+  uint16_t* vt;
+  unsigned char* bits;
+  size_t bytes;
+  FwdWs(void* p, const Dims& d, bool int8) {
+    Carve c{static_cast<unsigned char*>(p)};
+    const size_t nb = d.BH * d.Nb;
+    if (int8) {
+      q8 = c.take<int8_t>(d.elems);
+      k8 = c.take<int8_t>(d.elems);
+      v8f = c.take<int8_t>(nb * kT * kT);
+      qs = c.take<float>(nb);
+      ks = c.take<float>(nb);
+      vs = c.take<float>(nb);
+    }
+    vt = int8 ? nullptr : c.take<uint16_t>(nb * kT * kT);
+    Hb = c.take<float>(nb * kT * kT);
+    zb = c.take<float>(nb * kT);
+    zall = c.take<float>(d.BH * kT);
+    bits = c.take<unsigned char>(sla2h_complement_workspace_bytes(d.B, d.H, d.Mq, d.Nb));
+    bytes = c.used;
+  }
+};
+
+struct BwdWs {
+  uint16_t *dos, *g16;
+  float *delta, *s, *segp, *P, *Pz;
+  uint32_t* sel;
+  unsigned char *bits, *comp;
+  size_t bytes;
+  BwdWs(void* p, const Dims& d) {
+    Carve c{static_cast<unsigned char*>(p)};
+    const size_t nb = d.BH * d.Nb;
+    dos = c.take<uint16_t>(d.elems);
+    g16 = c.take<uint16_t>(d.elems);
+    delta = c.take<float>(d.rows);
+    s = c.take<float>(d.rows);
+    segp = c.take<float>(nb);
+    P = c.take<float>(nb * kT * kT);
+    Pz = c.take<float>(nb * kT);
+    sel = c.take<uint32_t>(nb * ((d.Nb + 31) / 32));
+    bits = c.take<unsigned char>(sla2h_complement_workspace_bytes(d.B, d.H, d.Nb, d.Nb));
+    comp = c.take<unsigned char>(nb * kRecBytes);
+    bytes = c.used;
+  }
+};
+
+int log2_of(int x) { return x == 64 ? 0 : (x == 128 ? 1 : 2); }
+
+}  // namespace
+
+// attn_bwd.hip: bwd_prep with each 64-row block's alpha segment sum stored to
+// segp[(b H + h) Nb + block] instead of added into seg
+int bwd_prep_segp(const void* dout, const void* o_s, const void* o_l, const float* den,
+                  const void* qphi, const float* alpha, int alpha_stride, int dtype, int B, int H,
+                  int64_t L, int E, void* dos, float* delta, void* g16, float* s, float* segp,
+                  float* P, float* Pz, void* stream);
+
+}  // namespace sla2h
+
+using namespace sla2h;
+
+#define SLA2H_TRY(call)              \
+  do {                               \
+    const int err_ = (call);         \
+    if (err_ != 0) return err_;      \
+  } while (0)
+
+extern "C" size_t sla2h_cube_jvp_workspace_bytes(int B, int H, int64_t L, int Np, int T,
+                                                 int tangent) {
+  if (!dims_ok(0, B, H, L, Np, kT, T)) return 0;
+  return JvpWs(nullptr, Dims(B, H, L, Np, kT, T), tangent != 0, true).bytes;
+}
+
+extern "C" int sla2h_cube_jvp_quant(const void* q, const void* k, int dtype, int B, int H,
+                                    int64_t L, int Np, int T, int tangent, const float* proj_q,
+                                    const float* proj_k, void* workspace, float* qpool,
+                                    float* kpool_t, void* stream) {
+  SLA2H_CHECK_ARG(workspace && dims_ok(dtype, B, H, L, Np, kT, T));
+  const JvpWs w(workspace, Dims(B, H, L, Np, kT, T), tangent != 0, true);
+  return sla2h_quant_pool_qk(q, k, dtype, B, H, L, kT, kT, Np, proj_q, proj_k, w.q8, w.qs, w.k8,
+                             w.ks, qpool, kpool_t, w.kb, stream);
+}
+
+extern "C" int sla2h_cube_jvp_attn(const void* q, const void* k, const void* v, const void* dq,
+                                   const void* dk, const void* dv, const float* alpha,
+                                   int alpha_stride, const int32_t* lut, int dtype, int B, int H,
+                                   int64_t L, int Np, int T, float scale, float eps_l,
+                                   void* workspace, float* o, float* d_o, void* stream) {
+  SLA2H_CHECK_ARG(workspace && lut && dims_ok(dtype, B, H, L, Np, kT, T));
+  const bool tan = dq != nullptr;
+  SLA2H_CHECK_ARG(!tan || (dk && dv && d_o));
+  const JvpWs w(workspace, Dims(B, H, L, Np, kT, T), tan, true);
+  SLA2H_TRY(sla2h_linear_states(k, tan ? dk : nullptr, v, tan ? dv : nullptr, dtype, B, H, L, kT,
+                                kT, Np, w.Hb, w.dHb, w.zb, w.dzb, nullptr, nullptr, nullptr,
+                                nullptr, w.vt, w.kt, stream));
+  const int Mb = (int)((L + kT - 1) / kT);
+  SLA2H_TRY(sla2h_complement(w.Hb, w.dHb, w.zb, w.dzb, lut, B, H, Mb, Np, kT, T, w.bits, w.comp,
+                             stream));
+  return sla2h_fwd_jvp(q, dq, w.kt, w.vt, w.q8, w.k8, w.qs, w.ks, w.kb, w.comp, alpha,
+                       alpha_stride, lut, dtype, B, H, L, kT, kT, Np, T, scale, eps_l, 0, o, d_o,
+                       stream);
+}
+
+extern "C" size_t sla2h_jvp16_workspace_bytes(int B, int H, int64_t L, int Np, int bq, int T) {
+  if (!dims_ok(0, B, H, L, Np, bq, T)) return 0;
+  return JvpWs(nullptr, Dims(B, H, L, Np, bq, T), true, false).bytes;
+}
+
+extern "C" int sla2h_jvp16(const void* q, const void* k, const void* v, const void* dq,
+                           const void* dk, const void* dv, const float* alpha, int alpha_stride,
+                           const int32_t* lut, int dtype, int B, int H, int64_t L, int Np, int bq,
+                           int T, float scale, float eps_l, void* workspace, float* o, float* d_o,
+                           void* stream) {
+  SLA2H_CHECK_ARG(workspace && lut && dq && dk && dv && dims_ok(dtype, B, H, L, Np, bq, T));
+  const Dims d(B, H, L, Np, bq, T);
+  const JvpWs w(workspace, d, true, false);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  SLA2H_TRY(sla2h_linear_states(k, dk, v, dv, dtype, B, H, L, kT, kT, Np, w.Hb, w.dHb, w.zb,
+                                w.dzb, nullptr, nullptr, nullptr, nullptr, w.vt, w.kt, stream));
+  SLA2H_TRY(sla2h_complement(w.Hb, w.dHb, w.zb, w.dzb, lut, B, H, d.Mq, Np, kT, T, w.bits, w.comp,
+                             stream));
+  if (d.J > T) {
+    const int64_t nl = (int64_t)d.BH * d.Mq * d.J;
+    train_setup_kernel<<<(unsigned)((nl + 255) / 256), 256, 0, st>>>(
+        nullptr, 0, nullptr, lut, nl, T, d.J, Np, w.lut, nullptr, 0);
+    SLA2H_TRY((int)hipGetLastError());
+    lut = w.lut;
+  }
+  return sla2h_fwd_jvp_1d(q, dq, w.kt, w.vt, w.comp, alpha, alpha_stride, lut, dtype, B, H, L, kT,
+                          bq, kT, d.J, scale, eps_l, o, d_o, stream);
+}
+
+extern "C" size_t sla2h_train_saved_bytes(int B, int H, int64_t L, int Np, int bq, int T) {
+  if (!dims_ok(0, B, H, L, Np, bq, T)) return 0;
+  return Saved(nullptr, Dims(B, H, L, Np, bq, T)).bytes;
+}
+
+extern "C" size_t sla2h_train_fwd_workspace_bytes(int B, int H, int64_t L, int Np, int bq, int T,
+                                                  int int8) {
+  if (!dims_ok(0, B, H, L, Np, bq, T)) return 0;
+  return FwdWs(nullptr, Dims(B, H, L, Np, bq, T), int8 != 0).bytes;
+}
+
+extern "C" int sla2h_train_fwd(const void* q, const void* k, const void* v,
+                               const float* alpha_logit, const int32_t* lut, int dtype, int B,
+                               int H, int64_t L, int Np, int bq, int T, int int8, float scale,
+                               float eps_l, void* saved, void* workspace, void* o, float* stats,
+                               void* stream) {
+  SLA2H_CHECK_ARG(q && k && v && alpha_logit && lut && saved && workspace && o);
+  SLA2H_CHECK_ARG(dims_ok(dtype, B, H, L, Np, bq, T));
+  const Dims d(B, H, L, Np, bq, T);
+  SLA2H_CHECK_ARG(bq == kT || Np == d.Nb);  // the prefix tail goes with 64-row query blocks
+  const Saved s(saved, d);
+  const FwdWs w(workspace, d, int8 != 0);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const int64_t nl = (int64_t)d.BH * d.Mq * d.J;
+  const int na = H * d.Mq;
+  const int64_t n = nl > na ? nl : na;
+  train_setup_kernel<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(
+      alpha_logit, na, s.alpha, lut, nl, T, d.J, Np, s.lut, stats, H);
+  SLA2H_TRY((int)hipGetLastError());
+  if (int8) {
+    SLA2H_TRY(sla2h_quant_train(q, k, v, dtype, B, H, L, kT, kT, w.q8, w.qs, w.k8, w.ks, w.v8f,
+                                w.vs, stream));
+    if (bq == kT) {
+      SLA2H_TRY(sla2h_sparse_fwd_qat(q, w.q8, w.qs, w.k8, w.ks, w.v8f, w.vs, lut, dtype, B, H, L,
+                                     kT, kT, Np, T, scale, s.o_s, s.lse, s.qphi, stream));
+    } else {
+      SLA2H_TRY(sla2h_quantize_trunc(q, dtype, (int64_t)d.BH, L, kT, bq, w.q8, w.qs, stream));
+      SLA2H_TRY(sla2h_sparse_fwd_int8(q, w.q8, w.qs, bq, w.k8, w.ks, w.v8f, w.vs, lut, dtype, B,
+                                      H, L, kT, bq, T, scale, s.o_s, s.lse, s.qphi, stream));
+    }
+    SLA2H_TRY(sla2h_linear_states_qat(k, v, dtype, B, H, L, kT, kT, w.Hb, w.zb, s.Hall, w.zall,
+                                      nullptr, stream));
+  } else {
+    SLA2H_TRY(sla2h_linear_states_qat(k, v, dtype, B, H, L, kT, kT, w.Hb, w.zb, s.Hall, w.zall,
+                                      w.vt, stream));
+    SLA2H_TRY(sla2h_sparse_fwd_1d(q, k, w.vt, s.lut, dtype, B, H, L, kT, bq, kT, d.J, scale,
+                                  s.o_s, s.lse, s.qphi, stream));
+  }
+  SLA2H_TRY(sla2h_complement(w.Hb, nullptr, w.zb, nullptr, s.lut, B, H, d.Mq, d.Nb, kT, d.J,
+                             w.bits, s.comp, stream));
+  // the reference's linear branch: score form up to 4 LUT columns, else state form
+  if (d.J <= 4)
+    SLA2H_TRY(sla2h_linear_mix_score(s.qphi, k, v, s.Hall, w.zall, s.lut, d.J, s.o_s, s.alpha,
+                                     d.Mq, dtype, B, H, L, kT, bq, eps_l, o, s.o_l, s.den,
+                                     stream));
+  else
+    SLA2H_TRY(sla2h_linear_mix_qat(s.qphi, s.comp, s.Hall, s.o_s, s.alpha, d.Mq, dtype, B, H, L,
+                                   kT, bq, eps_l, o, s.o_l, s.den, stream));
+  if (stats != nullptr) {
+    const int chunks = (int)((L + 4095) / 4096);
+    head_max_kernel<<<dim3(chunks, (unsigned)d.BH), 256, 0, st>>>(s.lse, L, H, stats);
+  }
+  return (int)hipGetLastError();
+}
+
+extern "C" size_t sla2h_train_bwd_workspace_bytes(int B, int H, int64_t L, int Np, int bq, int T) {
+  if (!dims_ok(0, B, H, L, Np, bq, T)) return 0;
+  return BwdWs(nullptr, Dims(B, H, L, Np, bq, T)).bytes;
+}
+
+extern "C" int sla2h_train_bwd(const void* q, const void* k, const void* v, const void* dout,
+                               const void* saved, int dtype, int B, int H, int64_t L, int Np,
+                               int bq, int T, float scale, void* workspace, void* dq, void* dk,
+                               void* dv, float* d_logit, void* stream) {
+  SLA2H_CHECK_ARG(q && k && v && dout && saved && workspace && dq && dk && dv && d_logit);
+  SLA2H_CHECK_ARG(dims_ok(dtype, B, H, L, Np, bq, T));
+  const Dims d(B, H, L, Np, bq, T);
+  const Saved s(const_cast<void*>(saved), d);
+  const BwdWs w(workspace, d);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  SLA2H_TRY(bwd_prep_segp(dout, s.o_s, s.o_l, s.den, s.qphi, s.alpha, d.Mq, dtype, B, H, L, bq,
+                          w.dos, w.delta, w.g16, w.s, w.segp, w.P, w.Pz, stream));
+  alpha_grad_kernel<<<(unsigned)((H * d.Mq + 255) / 256), 256, 0, st>>>(
+      w.segp, s.alpha, B, H, d.Nb, d.Mq, 1 << log2_of(bq), d_logit);
+  SLA2H_TRY((int)hipGetLastError());
+  SLA2H_TRY(sla2h_complement_bwd(w.P, w.Pz, s.lut, B, H, d.Nb, bq, d.J, w.bits, w.sel, w.comp,
+                                 stream));
+  SLA2H_TRY(sla2h_bwd_dq(q, k, v, w.dos, s.lse, w.delta, w.g16, w.s, s.comp, s.Hall, s.qphi,
+                         s.lut, dtype, B, H, L, kT, bq, d.J, scale, dq, stream));
+  return sla2h_bwd_dkdv(q, k, v, w.dos, s.lse, w.delta, w.sel, w.comp, dtype, B, H, L, kT, kT,
+                        scale, dk, dv, stream);
+}
+
+namespace sla2h {
+namespace {
+struct InferWs {
+  int8_t *q8, *k8, *v8f;
+  float *qs, *ks, *vs, *Hb, *zb, *lse;
+  uint16_t *vt, *o_s, *qphi;
+  unsigned char *bits, *comp;
+  size_t bytes;
+  InferWs(void* p, const Dims& d, bool int8) {
+    Carve c{static_cast<unsigned char*>(p)};
+    const size_t nb = d.BH * d.Nb;
+    if (int8) {
+      q8 = c.take<int8_t>(d.elems);
+      k8 = c.take<int8_t>(d.elems);
+      v8f = c.take<int8_t>(nb * kT * kT);
+      qs = c.take<float>(nb * 2);  // scales per 32 rows or more
+      ks = c.take<float>(nb);
+      vs = c.take<float>(nb);
+    }
+    vt = int8 ? nullptr : c.take<uint16_t>(nb * kT * kT);
+    Hb = c.take<float>(nb * kT * kT);
+    zb = c.take<float>(nb * kT);
+    lse = c.take<float>(d.rows);
+    o_s = c.take<uint16_t>(d.elems);
+    qphi = c.take<uint16_t>(d.elems);
+    bits = c.take<unsigned char>(sla2h_complement_workspace_bytes(d.B, d.H, d.Mq, d.Nb));
+    comp = c.take<unsigned char>(d.BH * d.Mq * kRecBytes);
+    bytes = c.used;
+  }
+};
+}  // namespace
+}  // namespace sla2h
+
+extern "C" size_t sla2h_sla2_infer_workspace_bytes(int B, int H, int64_t L, int bq, int T,
+                                                   int int8) {
+  const int Nb = (int)((L + kT - 1) / kT);
+  if (!dims_ok(0, B, H, L, Nb, bq, T)) return 0;
+  return InferWs(nullptr, Dims(B, H, L, Nb, bq, T), int8 != 0).bytes;
+}
+
+extern "C" int sla2h_sla2_infer(const void* q, const void* k, const void* v, const float* alpha,
+                                int alpha_stride, const int32_t* lut, int dtype, int B, int H,
+                                int64_t L, int bq, int T, int int8, int qblock, float scale,
+                                float eps_l, void* workspace, void* o, void* stream) {
+  SLA2H_CHECK_ARG(q && k && v && alpha && lut && workspace && o && L > 0);
+  const int Nb = (int)((L + kT - 1) / kT);
+  SLA2H_CHECK_ARG(dims_ok(dtype, B, H, L, Nb, bq, T));
+  const Dims d(B, H, L, Nb, bq, T);
+  const InferWs w(workspace, d, int8 != 0);
+  SLA2H_TRY(sla2h_hblocks_states(k, v, dtype, B, H, L, kT, kT, w.Hb, w.zb, nullptr, nullptr, w.vt,
+                                 stream));
+  if (int8) {
+    const int64_t bh = (int64_t)d.BH;
+    SLA2H_TRY(sla2h_quantize(q, dtype, bh, L, kT, qblock, w.q8, w.qs, stream));
+    SLA2H_TRY(sla2h_quantize(k, dtype, bh, L, kT, kT, w.k8, w.ks, stream));
+    SLA2H_TRY(sla2h_quantize_v8f(v, dtype, bh, L, kT, kT, w.v8f, w.vs, stream));
+    SLA2H_TRY(sla2h_sparse_fwd_int8(q, w.q8, w.qs, qblock, w.k8, w.ks, w.v8f, w.vs, lut, dtype, B,
+                                    H, L, kT, bq, T, scale, w.o_s, w.lse, w.qphi, stream));
+  } else {
+    SLA2H_TRY(sla2h_sparse_fwd_1d(q, k, w.vt, lut, dtype, B, H, L, kT, bq, kT, T, scale, w.o_s,
+                                  w.lse, w.qphi, stream));
+  }
+  SLA2H_TRY(sla2h_complement(w.Hb, nullptr, w.zb, nullptr, lut, B, H, d.Mq, Nb, kT, T, w.bits,
+                             w.comp, stream));
+  return sla2h_lin_fwd3(w.qphi, w.comp, w.o_s, alpha, alpha_stride, dtype, B, H, L, kT, bq, eps_l,
+                        o, stream);
+}

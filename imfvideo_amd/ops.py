@@ -32,7 +32,11 @@ def ctypes_ptr(t):
 
 
 def _stream(device):
-    return torch.cuda.current_stream(device).cuda_stream
+    # the raw handle of torch.cuda.current_stream(device), without building the
+    # Stream object (3.3 us a call, more than a launch)
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None
+                                              else index)
 
 
 def _need_gpu(*ts):
@@ -61,6 +65,30 @@ def _check_lut(lut, B, H, L):
     Mb = -(-L // E_TILE)
     if lut.dim() != 4 or tuple(lut.shape[:3]) != (B, H, Mb):
         raise ValueError(f"lut: expected (B, H, Mb, T) = ({B}, {H}, {Mb}, T), got {tuple(lut.shape)}")
+
+
+def _i32(lut):
+    return lut.to(torch.int32).contiguous()
+
+
+def _proj(p, dev):
+    """A (64, 64) projection as contiguous fp32 on dev, or None."""
+    if p is None:
+        return None
+    return p.detach().to(dev, torch.float32).contiguous()
+
+
+def _scratch(nbytes, dev):
+    return torch.empty(nbytes, device=dev, dtype=torch.uint8)
+
+
+def _same(ref, *ts):
+    """ValueError unless every tensor shares ref's shape, dtype and device."""
+    for t in ts:
+        if t.shape != ref.shape or t.dtype != ref.dtype or t.device != ref.device:
+            raise ValueError("operands must share shape, dtype and device: "
+                             f"{tuple(ref.shape)} {ref.dtype} {ref.device}, "
+                             f"{tuple(t.shape)} {t.dtype} {t.device}")
 
 
 def check_lut_ids(lut, Np):
@@ -273,6 +301,8 @@ def cube_jvp(q, k, v, dq, dk, dv, alpha, topk_frac, Np, prefix_len=0, proj_q=Non
     tan = dq is not None
     if tan:
         dq, dk, dv = (t.to(q.dtype).contiguous() for t in (dq, dk, dv))
+    if not return_aux:
+        return _cube_jvp_call(q, k, v, dq, dk, dv, alpha, topk_frac, Np, proj_q, proj_k, lut)
     q8, qs, k8, ks, qpool, kpool_t, kb = quant_pool_qk(q, k, Np, E, proj_q, proj_k, with_kb=True)
     if lut is None:
         T = topk_count(topk_frac, Np)
@@ -285,10 +315,45 @@ def cube_jvp(q, k, v, dq, dk, dv, alpha, topk_frac, Np, prefix_len=0, proj_q=Non
     comp = complement(st, lut, Np, check_ids=False)
     o, do = fwd_jvp(q, q8, k8, qs, ks, st, comp, alpha, lut, Np, dq if tan else None, kb=kb,
                     check_ids=False)
-    if return_aux:
-        aux = dict(q8=q8, qs=qs, k8=k8, ks=ks, kb=kb, qpool=qpool, kpool_t=kpool_t, lut=lut, T=T,
-                   comp=comp, **st)
-        return o, do, aux
+    aux = dict(q8=q8, qs=qs, k8=k8, ks=ks, kb=kb, qpool=qpool, kpool_t=kpool_t, lut=lut, T=T,
+               comp=comp, **st)
+    return o, do, aux
+
+
+def _cube_jvp_call(q, k, v, dq, dk, dv, alpha, topk_frac, Np, proj_q, proj_k, lut):
+    """cube_jvp without the intermediates: the same stages behind two native calls
+    around the routing, their buffers in one allocation."""
+    tan = dq is not None
+    _need_gpu(q, k, v, dq, dk, dv, alpha, lut)
+    q = _bhld(q, "q")
+    _same(q, k, v, *((dq, dk, dv) if tan else ()))
+    B, H, L, D = q.shape
+    dev, code = q.device, _dtype_code(q)
+    nb = -(-L // E_TILE)
+    alpha = _alpha_rows(alpha, H, nb, dev)
+    if lut is None:
+        T = topk_count(topk_frac, Np)
+    else:
+        lut = _i32(lut)
+        _check_lut(lut, B, H, L)
+        check_lut_ids(lut, Np)
+        T = lut.shape[-1]
+    pq, pk = _proj(proj_q, dev), _proj(proj_k, dev)
+    lib, st, scale = _lib.load(), _stream(dev), D ** -0.5
+    ws = _scratch(lib.sla2h_cube_jvp_workspace_bytes(B, H, L, Np, T, tan), dev)
+    qpool = torch.empty(B, H, nb, D, device=dev, dtype=torch.float32)
+    kpool_t = torch.empty(B, H, D, Np, device=dev, dtype=torch.float32)
+    _lib.check(lib.sla2h_cube_jvp_quant(
+        q.data_ptr(), k.data_ptr(), code, B, H, L, Np, T, tan, _ptr(pq), _ptr(pk), ws.data_ptr(),
+        qpool.data_ptr(), kpool_t.data_ptr(), st), "sla2h_cube_jvp_quant")
+    if lut is None:
+        lut = route_topk(qpool, kpool_t, T, scale)
+    o = torch.empty(B, H, L, D, device=dev, dtype=torch.float32)
+    do = torch.empty_like(o) if tan else None
+    _lib.check(lib.sla2h_cube_jvp_attn(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), _ptr(dq), _ptr(dk), _ptr(dv), alpha.data_ptr(),
+        alpha.stride(0), lut.data_ptr(), code, B, H, L, Np, T, scale, 1e-5, ws.data_ptr(),
+        o.data_ptr(), _ptr(do), st), "sla2h_cube_jvp_attn")
     return o, do
 
 
@@ -515,6 +580,50 @@ def train_bwd(q, k, v, alpha, fwd, do, scale=None, stage_events=None, bq=E_TILE)
     return dq, dk, dv, d_alpha
 
 
+def train_op_fwd(q, k, v, alpha_logit, lut, Np, bq=E_TILE, int8=True, stats=None, eps_l=1e-5):
+    """train_fwd / train_fwd_1d from the alpha logits (H, ceil(L/bq)) as one native
+    call -> (o, saved): saved is the buffer that train_op_bwd reads.  stats:
+    optional (H,) fp32 tensor that receives the per-head maximum of lse."""
+    _need_gpu(q, k, v, lut, stats)
+    q, k, v = (_bhld(t, n) for t, n in ((q, "q"), (k, "k"), (v, "v")))
+    _same(q, k, v)
+    B, H, L, D = q.shape
+    dev, Mq = q.device, -(-L // bq)
+    lut = _i32(lut)
+    if lut.dim() != 4 or tuple(lut.shape[:3]) != (B, H, Mq):
+        raise ValueError(f"lut: expected (B, H, {Mq}, T), got {tuple(lut.shape)}")
+    logit = _alpha_rows(alpha_logit, H, Mq, dev).contiguous()
+    T, lib = lut.shape[-1], _lib.load()
+    saved = _scratch(lib.sla2h_train_saved_bytes(B, H, L, Np, bq, T), dev)
+    ws = _scratch(lib.sla2h_train_fwd_workspace_bytes(B, H, L, Np, bq, T, int8), dev)
+    o = torch.empty_like(q)
+    _lib.check(lib.sla2h_train_fwd(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), logit.data_ptr(), lut.data_ptr(), _dtype_code(q),
+        B, H, L, Np, bq, T, int8, D ** -0.5, eps_l, saved.data_ptr(), ws.data_ptr(), o.data_ptr(),
+        _ptr(stats), _stream(dev)), "sla2h_train_fwd")
+    return o, saved
+
+
+def train_op_bwd(q, k, v, do, saved, Np, T, bq=E_TILE):
+    """Backward of train_op_fwd (T: its LUT's columns) as one native call ->
+    (dq, dk, dv) 16-bit and the gradient of the logits (H, ceil(L/bq)) fp32."""
+    _need_gpu(q, k, v, do, saved)
+    q, k, v = (t.contiguous() for t in (q, k, v))
+    B, H, L, D = q.shape
+    dev = q.device
+    do = do.to(q.dtype).contiguous()
+    _same(q, k, v, do)
+    lib = _lib.load()
+    ws = _scratch(lib.sla2h_train_bwd_workspace_bytes(B, H, L, Np, bq, T), dev)
+    dq, dk, dv = torch.empty_like(q), torch.empty_like(q), torch.empty_like(q)
+    dl = torch.empty(H, -(-L // bq), device=dev, dtype=torch.float32)
+    _lib.check(lib.sla2h_train_bwd(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), do.data_ptr(), saved.data_ptr(), _dtype_code(q),
+        B, H, L, Np, bq, T, D ** -0.5, ws.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+        dl.data_ptr(), _stream(dev)), "sla2h_train_bwd")
+    return dq, dk, dv, dl
+
+
 # ---------------------------------------------------------------------------
 # 1-D SLA2 blocks: query blocks of bq rows, key blocks of 64 rows
 # ---------------------------------------------------------------------------
@@ -584,6 +693,8 @@ def jvp_1d(q, k, v, dq, dk, dv, alpha, lut, bq, scale=None, eps_l=1e-5, return_a
     T = lut.shape[-1]
     alpha = _alpha_rows(alpha, H, mq, q.device)
     scale = D ** -0.5 if scale is None else scale
+    if not return_aux:
+        return _jvp16_call(q, k, v, dq, dk, dv, alpha, lut, nb, bq, scale, eps_l)
     st = linear_states(k, v, nb, dk, dv, with_sums=False)
     comp = complement(st, lut, nb, check_ids=False)
     o = torch.empty(B, H, L, D, device=q.device, dtype=torch.float32)
@@ -593,8 +704,22 @@ def jvp_1d(q, k, v, dq, dk, dv, alpha, lut, bq, scale=None, eps_l=1e-5, return_a
         alpha.data_ptr(), alpha.stride(0), lut.data_ptr(), _dtype_code(q), B, H, L, D, bq,
         E_TILE, T, float(scale), float(eps_l), o.data_ptr(), do.data_ptr(), _stream(q.device)),
         "sla2h_fwd_jvp_1d")
-    if return_aux:
-        return o, do, dict(comp=comp, **st)
+    return o, do, dict(comp=comp, **st)
+
+
+def _jvp16_call(q, k, v, dq, dk, dv, alpha, lut, Np, bq, scale, eps_l):
+    """The 16-bit-score JVP on checked operands as one native call -> (o, do) fp32."""
+    _same(q, k, v, dq, dk, dv)
+    B, H, L, D = q.shape
+    dev, T, lib = q.device, lut.shape[-1], _lib.load()
+    ws = _scratch(lib.sla2h_jvp16_workspace_bytes(B, H, L, Np, bq, T), dev)
+    o = torch.empty(B, H, L, D, device=dev, dtype=torch.float32)
+    do = torch.empty_like(o)
+    _lib.check(lib.sla2h_jvp16(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+        alpha.data_ptr(), alpha.stride(0), lut.data_ptr(), _dtype_code(q), B, H, L, Np, bq, T,
+        float(scale), float(eps_l), ws.data_ptr(), o.data_ptr(), do.data_ptr(), _stream(dev)),
+        "sla2h_jvp16")
     return o, do
 
 
@@ -635,17 +760,7 @@ def cube_jvp16(q, k, v, dq, dk, dv, alpha, lut, Np, scale=None, eps_l=1e-5):
     _check_lut(lut, B, H, L)
     alpha = _alpha_rows(alpha, H, nb, q.device)
     scale = D ** -0.5 if scale is None else scale
-    st = linear_states(k, v, Np, dk, dv, with_sums=False)
-    comp = complement(st, lut, Np, check_ids=False)
-    lut_aug = augment_lut(lut, Np, nb - Np)
-    o = torch.empty(B, H, L, D, device=q.device, dtype=torch.float32)
-    do = torch.empty_like(o)
-    _lib.check(_lib.load().sla2h_fwd_jvp_1d(
-        q.data_ptr(), dq.data_ptr(), st["kt"].data_ptr(), st["vt"].data_ptr(), comp.data_ptr(),
-        alpha.data_ptr(), alpha.stride(0), lut_aug.data_ptr(), _dtype_code(q), B, H, L, D,
-        E_TILE, E_TILE, lut_aug.shape[-1], float(scale), float(eps_l), o.data_ptr(),
-        do.data_ptr(), _stream(q.device)), "sla2h_fwd_jvp_1d")
-    return o, do
+    return _jvp16_call(q, k, v, dq, dk, dv, alpha, lut, Np, E_TILE, scale, eps_l)
 
 
 def train_fwd_1d(q, k, v, alpha, lut, bq, eps_l=1e-5, int8=False):
@@ -784,6 +899,8 @@ def sla2_infer(q, k, v, alpha, lut, bq, use_int8=True, qblock=None, eps_l=1e-5,
     B, H, L, D = q.shape
     nb = -(-L // E_TILE)
     lut = lut.to(torch.int32).contiguous()
+    if not return_parts:
+        return _sla2_infer_call(q, k, v, alpha, lut, bq, use_int8, qblock, eps_l)
     st = hblocks_states(k, v, with_vt=not use_int8)
     if use_int8:
         qb = bq if qblock is None else qblock
@@ -795,8 +912,25 @@ def sla2_infer(q, k, v, alpha, lut, bq, use_int8=True, qblock=None, eps_l=1e-5,
         o_s, lse, qphi = sparse_fwd_16(q, k, st["vt"], lut, bq)
     comp = complement(st, lut, nb, check_ids=False)
     o = lin_fwd3(qphi, comp, o_s, alpha, bq, eps_l)
-    if return_parts:
-        return o, dict(o_s=o_s, lse=lse, qphi=qphi, comp=comp, **st)
+    return o, dict(o_s=o_s, lse=lse, qphi=qphi, comp=comp, **st)
+
+
+def _sla2_infer_call(q, k, v, alpha, lut, bq, use_int8, qblock, eps_l):
+    """sla2_infer without the intermediates, as one native call."""
+    _same(q, k, v)
+    B, H, L, D = q.shape
+    dev, mq = q.device, -(-L // bq)
+    if lut.dim() != 4 or tuple(lut.shape[:3]) != (B, H, mq):
+        raise ValueError(f"lut: expected (B, H, {mq}, T), got {tuple(lut.shape)}")
+    alpha = _alpha_rows(alpha, H, mq, dev)
+    T, lib = lut.shape[-1], _lib.load()
+    use_int8 = bool(use_int8)
+    ws = _scratch(lib.sla2h_sla2_infer_workspace_bytes(B, H, L, bq, T, use_int8), dev)
+    o = torch.empty_like(q)
+    _lib.check(lib.sla2h_sla2_infer(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), alpha.data_ptr(), alpha.stride(0),
+        lut.data_ptr(), _dtype_code(q), B, H, L, bq, T, use_int8, bq if qblock is None else qblock,
+        D ** -0.5, float(eps_l), ws.data_ptr(), o.data_ptr(), _stream(dev)), "sla2h_sla2_infer")
     return o
 
 

@@ -30,6 +30,8 @@ COMPUTE_DTYPE = torch.bfloat16
 
 
 def _c16(x, dtype=None):
+    if x.dtype is dtype and x.is_contiguous():
+        return x
     if dtype is None:
         dtype = x.dtype if x.dtype in (torch.float16, torch.bfloat16) else COMPUTE_DTYPE
     return x.to(dtype).contiguous()
@@ -106,10 +108,10 @@ class _CubeQATFunction(torch.autograd.Function):
 
     Same argument list as the reference.  ``use_int8`` picks the INT8 or the
     16-bit sparse branch of the forward; the backward is the same 16-bit
-    recompute for both, as in the reference.  ``mask`` and ``a_index`` are
-    accepted and unused: the kernels derive the per-tile selection from
-    ``lut_aug`` on the device, and the alpha of a row is that of its 64-row
-    block.
+    recompute for both, as in the reference.  ``lut_aug``, ``mask`` and
+    ``a_index`` are accepted and unused: the kernels append the prefix tail to
+    ``lut`` and derive the per-tile selection from it on the device, and the
+    alpha of a row is that of its 64-row block.
     """
 
     @staticmethod
@@ -118,21 +120,25 @@ class _CubeQATFunction(torch.autograd.Function):
         assert E == ops.E_TILE, f"E must be {ops.E_TILE}, got {E}"
         B, H, L, D = qh.shape
         Np = -(-L // E) - n_tail
-        a = torch.sigmoid(alpha_logit.detach().float())
-        out = ops.train_fwd(qh, kh, vh, a, lut, Np, int8=bool(use_int8))
-        if stats_out is not None:
-            stats_out.copy_(out["lse"].amax(dim=(0, 2)))
-        ctx.save_for_backward(qh, kh, vh, a, out["o_s"], out["o_l"], out["lse"], out["den"],
-                              out["qphi"], out["Hall"], out["comp"], out["lut_aug"])
-        return out["o"]
+        qh, kh, vh = (t.contiguous() for t in (qh, kh, vh))
+        stats = stats_out
+        if stats is not None and not (stats.is_cuda and stats.device == qh.device
+                                      and stats.dtype == torch.float32
+                                      and tuple(stats.shape) == (H,) and stats.is_contiguous()):
+            stats = torch.empty(H, device=qh.device, dtype=torch.float32)
+        o, saved = ops.train_op_fwd(qh, kh, vh, alpha_logit, lut, Np, int8=bool(use_int8),
+                                    stats=stats)
+        if stats is not stats_out:
+            stats_out.copy_(stats)
+        ctx.Np, ctx.T = Np, lut.shape[-1]
+        ctx.save_for_backward(qh, kh, vh, saved)
+        return o
 
     @staticmethod
     def backward(ctx, do):
-        qh, kh, vh, a, o_s, o_l, lse, den, qphi, Hall, comp, lut_aug = ctx.saved_tensors
-        fwd = dict(o_s=o_s, o_l=o_l, lse=lse, den=den, qphi=qphi, Hall=Hall, comp=comp,
-                   lut_aug=lut_aug)
-        dq, dk, dv, d_alpha = ops.train_bwd(qh, kh, vh, a, fwd, do)
-        return (dq, dk, dv, d_alpha, None, None, None, None, None, None, None, None, None)
+        qh, kh, vh, saved = ctx.saved_tensors
+        grads = ops.train_op_bwd(qh, kh, vh, do, saved, ctx.Np, ctx.T)
+        return (*grads, None, None, None, None, None, None, None, None, None)
 
 
 class _RowsIn(torch.autograd.Function):
@@ -200,7 +206,7 @@ class SLA2CubeQATAttentionImpl(nn.Module):
     forward(q, k, v) takes (b, l, H, hd) tensors, moves them to tile order in
     fp16 (as the reference does), routes on them without gradient (so
     proj_q / proj_k never receive one), and runs the training-forward kernels
-    (``ops.train_fwd``: sparse branch, state-form linear branch, alpha mix),
+    (``ops.train_op_fwd``: sparse branch, linear branch, alpha mix),
     also under no_grad as the reference's guidance path does.  With gradients
     required the call goes through ``_CubeQATFunction`` (straight-through
     backward) and refreshes ``logit_max_log2`` (H,), the per-head maximum of
@@ -272,9 +278,8 @@ class SLA2CubeQATAttentionImpl(nn.Module):
         if needs_grad:
             if not hasattr(self, "logit_max_log2"):
                 self.logit_max_log2 = torch.zeros(H, device=qh.device, dtype=torch.float32)
-            lut_aug = ops.augment_lut(lut, self.Np, self.n_tail)
-            return _CubeQATFunction.apply(qh, kh, vh, self.alpha_logit, lut, lut_aug, None, T,
+            return _CubeQATFunction.apply(qh, kh, vh, self.alpha_logit, lut, None, None, T,
                                           self.E, self.use_int8, self.a_index, self.n_tail,
                                           self.logit_max_log2)
-        a = torch.sigmoid(self.alpha_logit.detach().float())
-        return ops.train_fwd(qh, kh, vh, a, lut, self.Np, int8=self.use_int8)["o"]
+        return ops.train_op_fwd(qh, kh, vh, self.alpha_logit, lut, self.Np,
+                                int8=bool(self.use_int8))[0]

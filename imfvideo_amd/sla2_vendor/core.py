@@ -39,20 +39,18 @@ class _SLA2Function(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, qh, kh, vh, alpha_logit, lut, bq, use_int8):
-        a = torch.sigmoid(alpha_logit.detach().float())
-        out = ops.train_fwd_1d(qh, kh, vh, a, lut, bq, int8=use_int8)
-        ctx.bq = bq
-        ctx.save_for_backward(qh, kh, vh, a, out["o_s"], out["o_l"], out["lse"], out["den"],
-                              out["qphi"], out["Hall"], out["comp"], out["lut_aug"])
-        return out["o"]
+        o, saved = ops.train_op_fwd(qh, kh, vh, alpha_logit, lut, -(-qh.shape[2] // ops.E_TILE),
+                                    bq=bq, int8=bool(use_int8))
+        ctx.bq, ctx.T = bq, lut.shape[-1]
+        ctx.save_for_backward(qh, kh, vh, saved)
+        return o
 
     @staticmethod
     def backward(ctx, do):
-        qh, kh, vh, a, o_s, o_l, lse, den, qphi, Hall, comp, lut_aug = ctx.saved_tensors
-        fwd = dict(o_s=o_s, o_l=o_l, lse=lse, den=den, qphi=qphi, Hall=Hall, comp=comp,
-                   lut_aug=lut_aug)
-        dq, dk, dv, d_alpha = ops.train_bwd(qh, kh, vh, a, fwd, do, bq=ctx.bq)
-        return dq, dk, dv, d_alpha, None, None, None
+        qh, kh, vh, saved = ctx.saved_tensors
+        grads = ops.train_op_bwd(qh, kh, vh, do, saved, -(-qh.shape[2] // ops.E_TILE), ctx.T,
+                                 bq=ctx.bq)
+        return (*grads, None, None, None)
 
 
 class SLA2(nn.Module):

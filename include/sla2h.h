@@ -728,6 +728,72 @@ size_t sla2h_linear_wgrad_workspace_bytes(int64_t rows, int M, int N);
 int sla2h_linear_wgrad(const void* dy, int64_t ldy, const void* x, int64_t ldx, int dtype,
                        int64_t rows, int M, int N, void* workspace, float* dw, void* stream);
 
+/* ---------------------------------------------------------------------
+ * Whole calls: the stages above in order on one stream, intermediates in one
+ * caller-owned workspace (256-byte aligned; *_bytes() returns 0 for
+ * sizes that the call refuses).  Np routable 64-row blocks; Nb = ceil(L/64), the
+ * other Nb - Np blocks are the prefix tail; bq query rows per LUT row.
+ * --------------------------------------------------------------------- */
+
+/*
+ * The cube op and its JVP (dq = dk = dv = d_o = NULL and tangent = 0: primal
+ * only): sla2h_cube_jvp_quant (sla2h_quant_pool_qk into the workspace, the pooled
+ * tiles to qpool / kpool_t), then the caller's routing (sla2h_route_topk or a LUT
+ * of its own), then sla2h_cube_jvp_attn (sla2h_linear_states, sla2h_complement,
+ * sla2h_fwd_jvp) with the same sizes and workspace.
+ */
+size_t sla2h_cube_jvp_workspace_bytes(int B, int H, int64_t L, int Np, int T, int tangent);
+int sla2h_cube_jvp_quant(const void* q, const void* k, int dtype, int B, int H, int64_t L, int Np,
+                         int T, int tangent, const float* proj_q, const float* proj_k,
+                         void* workspace, float* qpool, float* kpool_t, void* stream);
+int sla2h_cube_jvp_attn(const void* q, const void* k, const void* v, const void* dq,
+                        const void* dk, const void* dv, const float* alpha, int alpha_stride,
+                        const int32_t* lut, int dtype, int B, int H, int64_t L, int Np, int T,
+                        float scale, float eps_l, void* workspace, float* o, float* d_o,
+                        void* stream);
+
+/*
+ * The JVP with 16-bit scores: sla2h_linear_states, sla2h_complement and
+ * sla2h_fwd_jvp_1d over lut (B,H,ceil(L/bq),T) with the tail blocks appended
+ * (Np = Nb: the 1-D form, none).
+ */
+size_t sla2h_jvp16_workspace_bytes(int B, int H, int64_t L, int Np, int bq, int T);
+int sla2h_jvp16(const void* q, const void* k, const void* v, const void* dq, const void* dk,
+                const void* dv, const float* alpha, int alpha_stride, const int32_t* lut, int dtype,
+                int B, int H, int64_t L, int Np, int bq, int T, float scale, float eps_l,
+                void* workspace, float* o, float* d_o, void* stream);
+
+/*
+ * The training op: forward on given routing (cube: bq = 64; 1-D: Np = Nb) from the
+ * alpha logits (H, ceil(L/bq)), INT8 or 16-bit sparse branch, score-form linear
+ * branch up to 4 LUT columns.  `saved` holds what the backward reads; stats (H),
+ * optional, receives the per-head maximum of lse.  The backward writes dq, dk, dv
+ * (16-bit) and the gradient of the logits (H, ceil(L/bq)); it only reads `saved`.
+ * Replaces _CubeQATFunction (models/sla2_cube_qat.py:696-832).
+ */
+size_t sla2h_train_saved_bytes(int B, int H, int64_t L, int Np, int bq, int T);
+size_t sla2h_train_fwd_workspace_bytes(int B, int H, int64_t L, int Np, int bq, int T, int int8);
+int sla2h_train_fwd(const void* q, const void* k, const void* v, const float* alpha_logit,
+                    const int32_t* lut, int dtype, int B, int H, int64_t L, int Np, int bq, int T,
+                    int int8, float scale, float eps_l, void* saved, void* workspace, void* o,
+                    float* stats, void* stream);
+size_t sla2h_train_bwd_workspace_bytes(int B, int H, int64_t L, int Np, int bq, int T);
+int sla2h_train_bwd(const void* q, const void* k, const void* v, const void* dout,
+                    const void* saved, int dtype, int B, int H, int64_t L, int Np, int bq, int T,
+                    float scale, void* workspace, void* dq, void* dk, void* dv, float* d_logit,
+                    void* stream);
+
+/*
+ * The 1-D SLA2 inference forward on given routing: sla2h_hblocks_states, the
+ * quantisers (int8; Q per qblock rows) and sla2h_sparse_fwd_int8, or
+ * sla2h_sparse_fwd_1d, then sla2h_complement and sla2h_lin_fwd3.
+ */
+size_t sla2h_sla2_infer_workspace_bytes(int B, int H, int64_t L, int bq, int T, int int8);
+int sla2h_sla2_infer(const void* q, const void* k, const void* v, const float* alpha,
+                     int alpha_stride, const int32_t* lut, int dtype, int B, int H, int64_t L,
+                     int bq, int T, int int8, int qblock, float scale, float eps_l,
+                     void* workspace, void* o, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -454,3 +454,59 @@ def test_sla2_train_1d_config_shape():
             print(f"  h{h} {n} rel {rel_l2(a_, rb[n]):.2e}", flush=True)
             assert rel_l2(a_, rb[n]) < TOL_REL and max_abs(a_, rb[n]) < TOL_MAX * max(1, rb[n].abs().max())
         assert rel_l2(da[sl].cpu(), rb["d_alpha"]) < 1e-2
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,L,Np,bq,T", [(1, 1, 64, 1, 64, 1), (2, 3, 274, 4, 64, 2),
+                                           (1, 2, 700, 8, 64, 5), (2, 2, 583, 10, 128, 3),
+                                           (1, 3, 1000, 16, 256, 6), (1, 2, 640, 10, 64, 10)])
+@pytest.mark.parametrize("int8", [True, False])
+def test_native_calls_match_the_stages(dt, B, H, L, Np, bq, T, int8):
+    """The whole calls (one native entry each) against the same stages called one by
+    one: prefix tails of none, one and several blocks, score- and state-form
+    linear branch, every query block length.  Same kernels on the same values,
+    so outputs are equal to the bit; the alpha gradient sums the batches in
+    another order (fp32), and lse's per-head maximum is exact."""
+    from imfvideo_amd import ops
+    print("[case] native calls", dt, B, H, L, Np, bq, T, int8, flush=True)
+    g = torch.Generator().manual_seed(L + T)
+    x = [torch.randn(B, H, L, 64, generator=g).to(dt).cuda() for _ in range(6)]
+    q, k, v, do, dk, dv = x
+    nb, mq = -(-L // 64), -(-L // bq)
+    if bq == 64:  # a cube call: its prefix is at most the blocks past Np
+        assert Np <= L // 64 or Np == nb
+    lut = torch.stack([torch.randperm(Np, generator=g)[:T] for _ in range(B * H * mq)])
+    lut = lut.view(B, H, mq, T).to(torch.int32).cuda()
+    logit = torch.randn(H, mq, generator=g).cuda()
+    a = torch.sigmoid(logit)
+    stats = torch.zeros(H, device="cuda")
+    o, saved = ops.train_op_fwd(q, k, v, logit, lut, Np, bq, int8, stats)
+    if bq == 64:
+        ref = ops.train_fwd(q, k, v, a, lut, Np, int8=int8)
+    else:
+        assert Np == nb
+        ref = ops.train_fwd_1d(q, k, v, a, lut, bq, int8=int8)
+    assert torch.equal(o, ref["o"])
+    assert torch.equal(stats, ref["lse"].amax(dim=(0, 2)))
+    got = ops.train_op_bwd(q, k, v, do, saved, Np, T, bq)
+    want = ops.train_bwd(q, k, v, a, ref, do, bq=bq)
+    for n, gg, ww in zip(("dq", "dk", "dv"), got, want):
+        assert torch.equal(gg, ww), n
+    assert (got[3] - want[3]).abs().max() <= 1e-5 * want[3].abs().max()
+    again = ops.train_op_bwd(q, k, v, do, saved, Np, T, bq)
+    assert all(torch.equal(p, r) for p, r in zip(got, again))
+    if Np == nb:
+        f1 = ops.jvp_1d(q, k, v, do, dk, dv, a, lut, bq)
+        f2 = ops.jvp_1d(q, k, v, do, dk, dv, a, lut, bq, return_aux=True)
+        assert torch.equal(f1[0], f2[0]) and torch.equal(f1[1], f2[1])
+        assert torch.equal(ops.sla2_infer(q, k, v, a, lut, bq, use_int8=int8),
+                           ops.sla2_infer(q, k, v, a, lut, bq, use_int8=int8, return_parts=True)[0])
+    if bq == 64 and Np <= L // 64:
+        P = L - Np * 64
+        for tan in ((do, dk, dv), (None, None, None)):
+            for lut_ in (lut, None):
+                f1 = ops.cube_jvp(q, k, v, *tan, a, T / Np, Np, P, lut=lut_)
+                f2 = ops.cube_jvp(q, k, v, *tan, a, T / Np, Np, P, lut=lut_, return_aux=True)
+                assert torch.equal(f1[0], f2[0])
+                assert (f1[1] is None) == (tan[0] is None)
+                assert f1[1] is None or torch.equal(f1[1], f2[1])
