@@ -333,10 +333,10 @@ extern "C" int sla2h_train_fwd(const void* q, const void* k, const void* v,
   if (int8) {
     SLA2H_TRY(sla2h_quant_train(q, k, v, dtype, B, H, L, kT, kT, w.q8, w.qs, w.k8, w.ks, w.v8f,
                                 w.vs, stream));
-    if (bq == kT) {
+    if (bq == kT && (int64_t)Np * kT <= L) {
       SLA2H_TRY(sla2h_sparse_fwd_qat(q, w.q8, w.qs, w.k8, w.ks, w.v8f, w.vs, lut, dtype, B, H, L,
                                      kT, kT, Np, T, scale, s.o_s, s.lse, s.qphi, stream));
-    } else {
+    } else {  // query blocks over 64 rows, or a routable last block that is partial
       SLA2H_TRY(sla2h_quantize_trunc(q, dtype, (int64_t)d.BH, L, kT, bq, w.q8, w.qs, stream));
       SLA2H_TRY(sla2h_sparse_fwd_int8(q, w.q8, w.qs, bq, w.k8, w.ks, w.v8f, w.vs, lut, dtype, B,
                                       H, L, kT, bq, T, scale, s.o_s, s.lse, s.qphi, stream));
