@@ -40,6 +40,8 @@ struct TrainArgs {
   float* lse;
   uint16_t* qphi;
   float* os32 = nullptr;  // set: o_s is written here in fp32 instead of os
+  float* stats = nullptr;  // set: (H) running maximum of lse per head
+  int H = 1;
   int64_t L;
   int Nb, Np, Mb, T, n_tail, nwork, per_xcd;
   int Mq, qshift;  // LUT rows: query blocks of 64 << qshift rows
@@ -301,6 +303,8 @@ __global__ __launch_bounds__(256, 2) void sparse_fwd_qat_kernel(TrainArgs a) {
     }
     if (g == 0) a.lse[qkbase + qrow] = m_i + __log2f(lt);
   }
+  if (a.stats != nullptr)
+    wave_atomic_max(a.stats + bh % a.H, qok ? m_i + __log2f(lt) : -INFINITY);
 }
 
 // 16-bit variant of the same recurrence (_attn_fwd_qat without USE_INT8,
@@ -320,6 +324,8 @@ struct Fwd16Args {
   float* lse;
   uint16_t* qphi;
   float* os32 = nullptr;  // set: o_s is written here in fp32 instead of os
+  float* stats = nullptr;  // set: (H) running maximum of lse per head
+  int H = 1;
   int64_t L;
   int Nb, Mq, qshift, T, nwork, per_xcd;
   float c;  // fl32(scale * log2(e))
@@ -534,6 +540,8 @@ __global__ __launch_bounds__(256, 2) void sparse_fwd16_kernel(Fwd16Args a) {
     }
     if (g == 0) a.lse[qkbase + qrow] = m_i + __log2f(lt);
   }
+  if (a.stats != nullptr)
+    wave_atomic_max(a.stats + bh % a.H, qok ? m_i + __log2f(lt) : -INFINITY);
 }
 
 // Linear branch and mix of the training forward (_lin_fwd2 in its state form,
@@ -843,11 +851,11 @@ __global__ __launch_bounds__(256) void linear_mix_score_kernel(
 
 using namespace sla2h;
 
-extern "C" int sla2h_sparse_fwd_qat(const void* q, const int8_t* q8, const float* qs,
-                                    const int8_t* k8, const float* ks, const int8_t* v8f,
-                                    const float* vs, const int32_t* lut, int dtype, int B, int H,
-                                    int64_t L, int D, int E, int Np, int T, float scale,
-                                    void* o_s, float* lse, void* qphi, void* stream) {
+namespace sla2h {
+int sparse_fwd_qat_stats(const void* q, const int8_t* q8, const float* qs, const int8_t* k8,
+                         const float* ks, const int8_t* v8f, const float* vs, const int32_t* lut,
+                         int dtype, int B, int H, int64_t L, int D, int E, int Np, int T,
+                         float scale, void* o_s, float* lse, void* qphi, float* stats, void* stream) {
   SLA2H_CHECK_ARG(q && q8 && qs && k8 && ks && v8f && vs && lut && o_s && lse && qphi);
   SLA2H_CHECK_ARG(D == kT && E == kT);
   SLA2H_CHECK_ARG(dtype == SLA2H_DTYPE_F16 || dtype == SLA2H_DTYPE_BF16);
@@ -883,6 +891,8 @@ extern "C" int sla2h_sparse_fwd_qat(const void* q, const int8_t* q8, const float
   a.nwork = (int)nwork;
   a.per_xcd = (int)per_xcd;
   a.c2 = scale * 1.4426950408889634f;
+  a.stats = stats;
+  a.H = H;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int nblocks = (int)(8 * per_xcd);
   if (dtype == SLA2H_DTYPE_BF16)
@@ -890,6 +900,16 @@ extern "C" int sla2h_sparse_fwd_qat(const void* q, const int8_t* q8, const float
   else
     sparse_fwd_qat_kernel<F16><<<nblocks, 256, 0, st>>>(a);
   return (int)hipGetLastError();
+}
+}  // namespace sla2h
+
+extern "C" int sla2h_sparse_fwd_qat(const void* q, const int8_t* q8, const float* qs,
+                                    const int8_t* k8, const float* ks, const int8_t* v8f,
+                                    const float* vs, const int32_t* lut, int dtype, int B, int H,
+                                    int64_t L, int D, int E, int Np, int T, float scale, void* o_s,
+                                    float* lse, void* qphi, void* stream) {
+  return sparse_fwd_qat_stats(q, q8, qs, k8, ks, v8f, vs, lut, dtype, B, H, L, D, E, Np, T, scale,
+                              o_s, lse, qphi, nullptr, stream);
 }
 
 static int log2_exact(int x) {
@@ -904,11 +924,12 @@ static int log2_exact(int x) {
 // recurrence as above over every routable key block (the last one possibly
 // partial), LUT rows per query block of bq rows, Q scales per block of
 // qblock rows (bq for the unfused path, block_m for the fused one).
-extern "C" int sla2h_sparse_fwd_int8(const void* q, const int8_t* q8, const float* qs, int qblock,
-                                     const int8_t* k8, const float* ks, const int8_t* v8f,
-                                     const float* vs, const int32_t* lut, int dtype, int B, int H,
-                                     int64_t L, int D, int bq, int T, float scale, void* o_s,
-                                     float* lse, void* qphi, void* stream) {
+namespace sla2h {
+int sparse_fwd_int8_stats(const void* q, const int8_t* q8, const float* qs, int qblock,
+                          const int8_t* k8, const float* ks, const int8_t* v8f, const float* vs,
+                          const int32_t* lut, int dtype, int B, int H, int64_t L, int D, int bq,
+                          int T, float scale, void* o_s, float* lse, void* qphi, float* stats,
+                          void* stream) {
   SLA2H_CHECK_ARG(q && q8 && qs && k8 && ks && v8f && vs && lut && o_s && lse);
   SLA2H_CHECK_ARG(D == kT && (bq == 64 || bq == 128 || bq == 256));
   SLA2H_CHECK_ARG(qblock == 32 || qblock == 64 || qblock == 128 || qblock == 256);
@@ -944,6 +965,8 @@ extern "C" int sla2h_sparse_fwd_int8(const void* q, const int8_t* q8, const floa
   a.nwork = (int)nwork;
   a.per_xcd = (int)per_xcd;
   a.c2 = scale * 1.4426950408889634f;
+  a.stats = stats;
+  a.H = H;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int nblocks = (int)(8 * per_xcd);
   if (dtype == SLA2H_DTYPE_BF16)
@@ -951,6 +974,16 @@ extern "C" int sla2h_sparse_fwd_int8(const void* q, const int8_t* q8, const floa
   else
     sparse_fwd_qat_kernel<F16><<<nblocks, 256, 0, st>>>(a);
   return (int)hipGetLastError();
+}
+}  // namespace sla2h
+
+extern "C" int sla2h_sparse_fwd_int8(const void* q, const int8_t* q8, const float* qs, int qblock,
+                                     const int8_t* k8, const float* ks, const int8_t* v8f,
+                                     const float* vs, const int32_t* lut, int dtype, int B, int H,
+                                     int64_t L, int D, int bq, int T, float scale, void* o_s,
+                                     float* lse, void* qphi, void* stream) {
+  return sparse_fwd_int8_stats(q, q8, qs, qblock, k8, ks, v8f, vs, lut, dtype, B, H, L, D, bq, T,
+                               scale, o_s, lse, qphi, nullptr, stream);
 }
 
 extern "C" int sla2h_linear_mix_qat(const void* qphi, const void* comp, const float* Hall,
@@ -1144,10 +1177,10 @@ extern "C" int sla2h_lin_fwd3(const void* qphi, const void* comp, const void* o_
   return (int)hipGetLastError();
 }
 
-extern "C" int sla2h_sparse_fwd_1d(const void* q, const void* k, const void* vt, const int32_t* lut,
-                                   int dtype, int B, int H, int64_t L, int D, int bq, int bk,
-                                   int T, float scale, void* o_s, float* lse, void* qphi,
-                                   void* stream) {
+namespace sla2h {
+int sparse_fwd_1d_stats(const void* q, const void* k, const void* vt, const int32_t* lut, int dtype,
+                        int B, int H, int64_t L, int D, int bq, int bk, int T, float scale,
+                        void* o_s, float* lse, void* qphi, float* stats, void* stream) {
   SLA2H_CHECK_ARG(q && k && vt && lut && o_s && lse && qphi);
   SLA2H_CHECK_ARG(D == kT && bk == kT && (bq == 64 || bq == 128 || bq == 256));
   SLA2H_CHECK_ARG(dtype == SLA2H_DTYPE_F16 || dtype == SLA2H_DTYPE_BF16);
@@ -1173,6 +1206,8 @@ extern "C" int sla2h_sparse_fwd_1d(const void* q, const void* k, const void* vt,
   a.nwork = (int)nwork;
   a.per_xcd = (int)per_xcd;
   a.c = scale * 1.4426950408889634f;
+  a.stats = stats;
+  a.H = H;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int nblocks = (int)(8 * per_xcd);
   if (dtype == SLA2H_DTYPE_BF16)
@@ -1180,4 +1215,12 @@ extern "C" int sla2h_sparse_fwd_1d(const void* q, const void* k, const void* vt,
   else
     sparse_fwd16_kernel<F16><<<nblocks, 256, 0, st>>>(a);
   return (int)hipGetLastError();
+}
+}  // namespace sla2h
+
+extern "C" int sla2h_sparse_fwd_1d(const void* q, const void* k, const void* vt, const int32_t* lut,
+                                   int dtype, int B, int H, int64_t L, int D, int bq, int bk, int T,
+                                   float scale, void* o_s, float* lse, void* qphi, void* stream) {
+  return sparse_fwd_1d_stats(q, k, vt, lut, dtype, B, H, L, D, bq, bk, T, scale, o_s, lse, qphi,
+                             nullptr, stream);
 }

@@ -173,6 +173,29 @@ __device__ inline u32x2 buf_load8(__amdgpu_buffer_rsrc_t rs, int voff, int soff)
 // 2^x on the hardware exp unit (v_exp_f32); inputs here are <= 0 or -inf.
 __device__ inline float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// fp32 maximum by integer atomics: positive floats order as int, negative ones
+// in reverse as unsigned (NaN, made positive, above everything)
+__device__ inline void atomic_max_f32(float* p, float v) {
+  if (v != v) v = __builtin_bit_cast(float, 0x7fc00000);
+  if (__builtin_bit_cast(int, v) >= 0)
+    atomicMax(reinterpret_cast<int*>(p), __builtin_bit_cast(int, v));
+  else
+    atomicMin(reinterpret_cast<unsigned*>(p), __builtin_bit_cast(unsigned, v));
+}
+
+// *p = max(*p, v over the wave's lanes), NaN as torch.amax orders it; the
+// atomic only runs where the wave's maximum exceeds the value read.
+__device__ inline void wave_atomic_max(float* p, float v) {
+  const bool nan = __builtin_amdgcn_ballot_w64(v != v) != 0;
+#pragma unroll
+  for (int s = 32; s >= 1; s >>= 1) v = fmaxf(v, __shfl_xor(v, s, 64));
+  if (nan) v = __builtin_bit_cast(float, 0x7fc00000);
+  if (__lane_id() == 0) {
+    const float cur = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!(v <= cur)) atomic_max_f32(p, v);
+  }
+}
+
 // Ascending sort of the n tile ids of a visiting list in LDS (element i read
 // with get(i), written with set(i, id)).  Workgroups that visit their tiles in
 // ascending order sweep the key tiles of a head together and share them in

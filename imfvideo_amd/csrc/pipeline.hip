@@ -66,51 +66,59 @@ __global__ __launch_bounds__(256) void train_setup_kernel(const float* __restric
   }
 }
 
-// fp32 maximum by integer atomics: positive floats order as int, negative ones
-// in reverse as unsigned (NaN, made positive, above everything)
-__device__ inline void atomic_max_f32(float* p, float v) {
-  if (v != v) v = __builtin_bit_cast(float, 0x7fc00000);
-  if (__builtin_bit_cast(int, v) >= 0)
-    atomicMax(reinterpret_cast<int*>(p), __builtin_bit_cast(int, v));
-  else
-    atomicMin(reinterpret_cast<unsigned*>(p), __builtin_bit_cast(unsigned, v));
-}
-
-// stats[h] = max over batch and rows of lse (B, H, L); stats starts at -inf
-__global__ __launch_bounds__(256) void head_max_kernel(const float* __restrict__ lse, int64_t L,
-                                                      int H, float* __restrict__ stats) {
-  const float* src = lse + (int64_t)blockIdx.y * L;
-  float m = -INFINITY;
-  bool nan = false;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < L; i += (int64_t)gridDim.x * 256) {
-    const float x = src[i];
-    nan |= x != x;
-    m = fmaxf(m, x);
-  }
-#pragma unroll
-  for (int s = 32; s >= 1; s >>= 1) {
-    m = fmaxf(m, __shfl_xor(m, s, 64));
-    nan |= __shfl_xor((int)nan, s, 64) != 0;
-  }
-  if (nan) m = __builtin_bit_cast(float, 0x7fc00000);
-  if ((threadIdx.x & 63) == 0) atomic_max_f32(stats + blockIdx.y % H, m);
-}
-
-// d_logit[h][m] = seg a (1 - a), seg summed over the batches and the 64-row
-// blocks of query block m in order
-__global__ __launch_bounds__(256) void alpha_grad_kernel(const float* __restrict__ segp,
-                                                        const float* __restrict__ alpha, int B,
-                                                        int H, int Nb, int Mq, int sub,
-                                                        float* __restrict__ d) {
+// Two small jobs between bwd_prep and the backward's products.
+// Blocks y < BH: the selection bits seen from the key side, a transposition of
+// the forward's complement masks (cbits word (kc, mq): bit j = tile 32 kc + j not
+// routed by LUT row mq): sel[n][kcq] bit i = query block 32 kcq + i routes tile n,
+// and its complement over the real blocks, word (kcq, n), for the mask GEMM.
+// One thread per word; the 32 words it gathers are shared by the 32 tiles of a
+// kc.  (Clearing, scattering the LUT's columns with atomics and complementing
+// took three launches, 27 us at 16 heads x 468 blocks of 46 tiles.)
+// Blocks y == BH: d_logit[h][m] = seg a (1 - a), seg summed over the batches and
+// the 64-row blocks of query block m in order.
+struct SelArgs {
+  const uint32_t* cbits;
+  uint32_t* sel;
+  uint32_t* out;
+  const float* segp;
+  const float* alpha;
+  float* d;
+  int B, H, Nb, Mq, qshift, NC, MTf, MTb;  // 16 MT words per mask row, forward / backward
+};
+__global__ __launch_bounds__(256) void bwd_bits_kernel(SelArgs a) {
   const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= H * Mq) return;
-  const int h = i / Mq, m = i - h * Mq;
-  float s = 0.f;
-  for (int b = 0; b < B; ++b)
-    for (int n = m * sub; n < min(Nb, (m + 1) * sub); ++n)
-      s += segp[((int64_t)b * H + h) * Nb + n];
-  const float a = alpha[i];
-  d[i] = s * a * (1.0f - a);
+  const int BH = a.B * a.H;
+  if ((int)blockIdx.y == BH) {
+    const int sub = 1 << a.qshift;
+    for (int e = i; e < a.H * a.Mq; e += gridDim.x * 256) {
+      const int h = e / a.Mq, m = e - h * a.Mq;
+      float s = 0.f;
+      for (int b = 0; b < a.B; ++b)
+        for (int n = m * sub; n < min(a.Nb, (m + 1) * sub); ++n)
+          s += a.segp[((int64_t)b * a.H + h) * a.Nb + n];
+      const float al = a.alpha[e];
+      a.d[e] = s * al * (1.0f - al);
+    }
+    return;
+  }
+  const int bh = blockIdx.y;
+  const int mp = 16 * a.MTb;
+  if (i >= a.NC * mp) return;
+  const int kcq = i / mp, n = i - kcq * mp;
+  uint32_t routed = 0u, real = 0u;
+  if (n < a.Nb) {
+    const uint32_t* src = a.cbits + ((int64_t)bh * a.NC + (n >> 5)) * (16 * a.MTf);
+    const int left = a.Nb - 32 * kcq;
+    real = left >= 32 ? 0xffffffffu : ((1u << left) - 1u);
+#pragma unroll
+    for (int j = 0; j < 32; ++j) {
+      const int m = min(32 * kcq + j, a.Nb - 1);
+      routed |= ((~src[m >> a.qshift] >> (n & 31)) & 1u) << j;
+    }
+    routed &= real;
+    a.sel[((int64_t)bh * a.Nb + n) * a.NC + kcq] = routed;
+  }
+  a.out[(int64_t)bh * a.NC * mp + i] = ~routed & real;
 }
 
 struct JvpWs {
@@ -148,7 +156,7 @@ struct JvpWs {
 struct Saved {
   uint16_t *o_s, *o_l, *qphi;
   float *lse, *den, *Hall, *alpha;
-  unsigned char* comp;
+  unsigned char *comp, *bits;
   int32_t* lut;
   size_t bytes;
   Saved(void* p, const Dims& d) {
@@ -161,6 +169,7 @@ struct Saved {
     Hall = c.take<float>(d.BH * kT * kT);
     alpha = c.take<float>((size_t)d.H * d.Mq);
     comp = c.take<unsigned char>(d.BH * d.Mq * kRecBytes);
+    bits = c.take<unsigned char>(sla2h_complement_workspace_bytes(d.B, d.H, d.Mq, d.Nb));
     lut = c.take<int32_t>(d.BH * d.Mq * d.J);
     bytes = c.used;
   }
@@ -170,7 +179,6 @@ struct FwdWs {
   int8_t *q8, *k8, *v8f;
   float *qs, *ks, *vs, *Hb, *zb, *zall;
   uint16_t* vt;
-  unsigned char* bits;
   size_t bytes;
   FwdWs(void* p, const Dims& d, bool int8) {
     Carve c{static_cast<unsigned char*>(p)};
@@ -187,7 +195,6 @@ struct FwdWs {
     Hb = c.take<float>(nb * kT * kT);
     zb = c.take<float>(nb * kT);
     zall = c.take<float>(d.BH * kT);
-    bits = c.take<unsigned char>(sla2h_complement_workspace_bytes(d.B, d.H, d.Mq, d.Nb));
     bytes = c.used;
   }
 };
@@ -218,6 +225,27 @@ struct BwdWs {
 int log2_of(int x) { return x == 64 ? 0 : (x == 128 ? 1 : 2); }
 
 }  // namespace
+
+// attn_train.hip: the sparse forwards that also raise stats[h] (may be NULL) to
+// the maximum of lse over the head's rows
+int sparse_fwd_qat_stats(const void* q, const int8_t* q8, const float* qs, const int8_t* k8,
+                         const float* ks, const int8_t* v8f, const float* vs, const int32_t* lut,
+                         int dtype, int B, int H, int64_t L, int D, int E, int Np, int T,
+                         float scale, void* o_s, float* lse, void* qphi, float* stats,
+                         void* stream);
+int sparse_fwd_int8_stats(const void* q, const int8_t* q8, const float* qs, int qblock,
+                          const int8_t* k8, const float* ks, const int8_t* v8f, const float* vs,
+                          const int32_t* lut, int dtype, int B, int H, int64_t L, int D, int bq,
+                          int T, float scale, void* o_s, float* lse, void* qphi, float* stats,
+                          void* stream);
+int sparse_fwd_1d_stats(const void* q, const void* k, const void* vt, const int32_t* lut,
+                        int dtype, int B, int H, int64_t L, int D, int bq, int bk, int T,
+                        float scale, void* o_s, float* lse, void* qphi, float* stats,
+                        void* stream);
+
+// states.hip: the backward's complement records from given masks (word (kcq, n))
+int complement_gemm_bwd(const float* P, const float* Pz, const uint32_t* cbits, int BH, int Mb,
+                        void* comp, void* stream);
 
 // attn_bwd.hip: bwd_prep with each 64-row block's alpha segment sum stored to
 // segp[(b H + h) Nb + block] instead of added into seg
@@ -334,23 +362,24 @@ extern "C" int sla2h_train_fwd(const void* q, const void* k, const void* v,
     SLA2H_TRY(sla2h_quant_train(q, k, v, dtype, B, H, L, kT, kT, w.q8, w.qs, w.k8, w.ks, w.v8f,
                                 w.vs, stream));
     if (bq == kT && (int64_t)Np * kT <= L) {
-      SLA2H_TRY(sla2h_sparse_fwd_qat(q, w.q8, w.qs, w.k8, w.ks, w.v8f, w.vs, lut, dtype, B, H, L,
-                                     kT, kT, Np, T, scale, s.o_s, s.lse, s.qphi, stream));
+      SLA2H_TRY(sparse_fwd_qat_stats(q, w.q8, w.qs, w.k8, w.ks, w.v8f, w.vs, lut, dtype, B, H, L,
+                                     kT, kT, Np, T, scale, s.o_s, s.lse, s.qphi, stats, stream));
     } else {  // query blocks over 64 rows, or a routable last block that is partial
       SLA2H_TRY(sla2h_quantize_trunc(q, dtype, (int64_t)d.BH, L, kT, bq, w.q8, w.qs, stream));
-      SLA2H_TRY(sla2h_sparse_fwd_int8(q, w.q8, w.qs, bq, w.k8, w.ks, w.v8f, w.vs, lut, dtype, B,
-                                      H, L, kT, bq, T, scale, s.o_s, s.lse, s.qphi, stream));
+      SLA2H_TRY(sparse_fwd_int8_stats(q, w.q8, w.qs, bq, w.k8, w.ks, w.v8f, w.vs, lut, dtype, B,
+                                      H, L, kT, bq, T, scale, s.o_s, s.lse, s.qphi, stats,
+                                      stream));
     }
     SLA2H_TRY(sla2h_linear_states_qat(k, v, dtype, B, H, L, kT, kT, w.Hb, w.zb, s.Hall, w.zall,
                                       nullptr, stream));
   } else {
     SLA2H_TRY(sla2h_linear_states_qat(k, v, dtype, B, H, L, kT, kT, w.Hb, w.zb, s.Hall, w.zall,
                                       w.vt, stream));
-    SLA2H_TRY(sla2h_sparse_fwd_1d(q, k, w.vt, s.lut, dtype, B, H, L, kT, bq, kT, d.J, scale,
-                                  s.o_s, s.lse, s.qphi, stream));
+    SLA2H_TRY(sparse_fwd_1d_stats(q, k, w.vt, s.lut, dtype, B, H, L, kT, bq, kT, d.J, scale,
+                                  s.o_s, s.lse, s.qphi, stats, stream));
   }
   SLA2H_TRY(sla2h_complement(w.Hb, nullptr, w.zb, nullptr, s.lut, B, H, d.Mq, d.Nb, kT, d.J,
-                             w.bits, s.comp, stream));
+                             s.bits, s.comp, stream));
   // the reference's linear branch: score form up to 4 LUT columns, else state form
   if (d.J <= 4)
     SLA2H_TRY(sla2h_linear_mix_score(s.qphi, k, v, s.Hall, w.zall, s.lut, d.J, s.o_s, s.alpha,
@@ -359,11 +388,7 @@ extern "C" int sla2h_train_fwd(const void* q, const void* k, const void* v,
   else
     SLA2H_TRY(sla2h_linear_mix_qat(s.qphi, s.comp, s.Hall, s.o_s, s.alpha, d.Mq, dtype, B, H, L,
                                    kT, bq, eps_l, o, s.o_l, s.den, stream));
-  if (stats != nullptr) {
-    const int chunks = (int)((L + 4095) / 4096);
-    head_max_kernel<<<dim3(chunks, (unsigned)d.BH), 256, 0, st>>>(s.lse, L, H, stats);
-  }
-  return (int)hipGetLastError();
+  return 0;
 }
 
 extern "C" size_t sla2h_train_bwd_workspace_bytes(int B, int H, int64_t L, int Np, int bq, int T) {
@@ -383,11 +408,24 @@ extern "C" int sla2h_train_bwd(const void* q, const void* k, const void* v, cons
   hipStream_t st = static_cast<hipStream_t>(stream);
   SLA2H_TRY(bwd_prep_segp(dout, s.o_s, s.o_l, s.den, s.qphi, s.alpha, d.Mq, dtype, B, H, L, bq,
                           w.dos, w.delta, w.g16, w.s, w.segp, w.P, w.Pz, stream));
-  alpha_grad_kernel<<<(unsigned)((H * d.Mq + 255) / 256), 256, 0, st>>>(
-      w.segp, s.alpha, B, H, d.Nb, d.Mq, 1 << log2_of(bq), d_logit);
+  SelArgs b;
+  b.cbits = reinterpret_cast<const uint32_t*>(s.bits);
+  b.sel = w.sel;
+  b.out = reinterpret_cast<uint32_t*>(w.bits);
+  b.segp = w.segp;
+  b.alpha = s.alpha;
+  b.d = d_logit;
+  b.B = B;
+  b.H = H;
+  b.Nb = d.Nb;
+  b.Mq = d.Mq;
+  b.qshift = log2_of(bq);
+  b.NC = (d.Nb + 31) / 32;
+  b.MTf = (d.Mq + 15) / 16;
+  b.MTb = (d.Nb + 15) / 16;
+  bwd_bits_kernel<<<dim3((b.NC * 16 * b.MTb + 255) / 256, (unsigned)d.BH + 1), 256, 0, st>>>(b);
   SLA2H_TRY((int)hipGetLastError());
-  SLA2H_TRY(sla2h_complement_bwd(w.P, w.Pz, s.lut, B, H, d.Nb, bq, d.J, w.bits, w.sel, w.comp,
-                                 stream));
+  SLA2H_TRY(complement_gemm_bwd(w.P, w.Pz, b.out, (int)d.BH, d.Nb, w.comp, stream));
   SLA2H_TRY(sla2h_bwd_dq(q, k, v, w.dos, s.lse, w.delta, w.g16, w.s, s.comp, s.Hall, s.qphi,
                          s.lut, dtype, B, H, L, kT, bq, d.J, scale, dq, stream));
   return sla2h_bwd_dkdv(q, k, v, w.dos, s.lse, w.delta, w.sel, w.comp, dtype, B, H, L, kT, kT,

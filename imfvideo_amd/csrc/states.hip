@@ -688,6 +688,19 @@ __global__ __launch_bounds__(256) void sel_complement_kernel(const uint32_t* __r
   cbits[(int64_t)bh * NCq * MTp + idx] = wd;
 }
 
+namespace sla2h {
+// The mask GEMM of the backward: records of Mb key tiles from the partial states
+// [P | Pz] of Mb query blocks and the masks cbits.
+int complement_gemm_bwd(const float* P, const float* Pz, const uint32_t* cbits, int BH, int Mb,
+                        void* comp, void* stream) {
+  const int MT = (Mb + 15) / 16, NC = (Mb + 31) / 32;
+  dim3 grid(4160 / kCompCols, BH, (MT + kMaskSub - 1) / kMaskSub);
+  comp_gemm_kernel<false><<<grid, kCompThreads, 0, static_cast<hipStream_t>(stream)>>>(
+      P, nullptr, Pz, nullptr, cbits, Mb, Mb, MT, NC, static_cast<unsigned char*>(comp));
+  return (int)hipGetLastError();
+}
+}  // namespace sla2h
+
 extern "C" int sla2h_complement_bwd(const float* P, const float* Pz, const int32_t* lut_aug,
                                     int B, int H, int Mb, int bq, int J, void* workspace,
                                     uint32_t* sel, void* comp, void* stream) {
@@ -707,10 +720,7 @@ extern "C" int sla2h_complement_bwd(const float* P, const float* Pz, const int32
                                                                                MT * 16, cbits);
   int err = (int)hipGetLastError();
   if (err) return err;
-  dim3 grid(4160 / kCompCols, B * H, (MT + kMaskSub - 1) / kMaskSub);
-  comp_gemm_kernel<false><<<grid, kCompThreads, 0, st>>>(P, nullptr, Pz, nullptr, cbits, Mb, Mb,
-                                                         MT, NC, static_cast<unsigned char*>(comp));
-  return (int)hipGetLastError();
+  return complement_gemm_bwd(P, Pz, cbits, B * H, Mb, comp, stream);
 }
 
 extern "C" size_t sla2h_complement_workspace_bytes(int B, int H, int Mb, int Np) {
