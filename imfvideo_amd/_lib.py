@@ -89,8 +89,10 @@ SIGNATURES = {
     "sla2h_train_saved_bytes": (ctypes.c_size_t, [_c_int, _c_int, _c_i64, _c_int, _c_int, _c_int]),
     "sla2h_train_fwd_workspace_bytes": (ctypes.c_size_t, [_c_int, _c_int, _c_i64, _c_int, _c_int,
                                                           _c_int, _c_int]),
+    "sla2h_train_in": (_c_int, [_p, _p, _c_int, _p, _c_int, _c_int, _c_i64, _c_int, _p, _p, _p, _p,
+                                _p, _p, _p]),
     "sla2h_train_fwd": (_c_int, [_p, _p, _p, _p, _p, _c_int, _c_int, _c_int, _c_i64, _c_int,
-                                 _c_int, _c_int, _c_int, _c_f, _c_f, _p, _p, _p, _p, _p]),
+                                 _c_int, _c_int, _c_int, _c_int, _c_f, _c_f, _p, _p, _p, _p, _p]),
     "sla2h_train_bwd_workspace_bytes": (ctypes.c_size_t, [_c_int, _c_int, _c_i64, _c_int, _c_int,
                                                           _c_int]),
     "sla2h_train_bwd": (_c_int, [_p, _p, _p, _p, _p, _c_int, _c_int, _c_int, _c_i64, _c_int,

@@ -243,6 +243,12 @@ int sparse_fwd_1d_stats(const void* q, const void* k, const void* vt, const int3
                         float scale, void* o_s, float* lse, void* qphi, float* stats,
                         void* stream);
 
+// quant_route.hip: layout, INT8 operands and pooled tiles of q, k, v in one pass
+int launch_train_in(const void* const* x, const int64_t* strides, int dtype, const int64_t* idx,
+                    int B, int H, int64_t L, int Np, const float* proj_q, const float* proj_k,
+                    void* const* rows, int8_t* const* xq, float* const* xs, float* qpool,
+                    float* kpool_t, void* stream);
+
 // states.hip: the backward's complement records from given masks (word (kcq, n))
 int complement_gemm_bwd(const float* P, const float* Pz, const uint32_t* cbits, int BH, int Mb,
                         void* comp, void* stream);
@@ -340,10 +346,22 @@ extern "C" size_t sla2h_train_fwd_workspace_bytes(int B, int H, int64_t L, int N
   return FwdWs(nullptr, Dims(B, H, L, Np, bq, T), int8 != 0).bytes;
 }
 
+extern "C" int sla2h_train_in(const void* const* x, const int64_t* strides, int dtype,
+                              const int64_t* idx, int B, int H, int64_t L, int Np,
+                              const float* proj_q, const float* proj_k, void* const* rows,
+                              void* workspace, float* qpool, float* kpool_t, void* stream) {
+  SLA2H_CHECK_ARG(workspace && dims_ok(0, B, H, L, Np, kT, 1));
+  const FwdWs w(workspace, Dims(B, H, L, Np, kT, 1), true);
+  int8_t* const xq[3] = {w.q8, w.k8, w.v8f};
+  float* const xs[3] = {w.qs, w.ks, w.vs};
+  return launch_train_in(x, strides, dtype, idx, B, H, L, Np, proj_q, proj_k, rows, xq, xs, qpool,
+                         kpool_t, stream);
+}
+
 extern "C" int sla2h_train_fwd(const void* q, const void* k, const void* v,
                                const float* alpha_logit, const int32_t* lut, int dtype, int B,
-                               int H, int64_t L, int Np, int bq, int T, int int8, float scale,
-                               float eps_l, void* saved, void* workspace, void* o, float* stats,
+                               int H, int64_t L, int Np, int bq, int T, int int8, int quantised,
+                               float scale, float eps_l, void* saved, void* workspace, void* o, float* stats,
                                void* stream) {
   SLA2H_CHECK_ARG(q && k && v && alpha_logit && lut && saved && workspace && o);
   SLA2H_CHECK_ARG(dims_ok(dtype, B, H, L, Np, bq, T));
@@ -359,8 +377,9 @@ extern "C" int sla2h_train_fwd(const void* q, const void* k, const void* v,
       alpha_logit, na, s.alpha, lut, nl, T, d.J, Np, s.lut, stats, H);
   SLA2H_TRY((int)hipGetLastError());
   if (int8) {
-    SLA2H_TRY(sla2h_quant_train(q, k, v, dtype, B, H, L, kT, kT, w.q8, w.qs, w.k8, w.ks, w.v8f,
-                                w.vs, stream));
+    if (!quantised)
+      SLA2H_TRY(sla2h_quant_train(q, k, v, dtype, B, H, L, kT, kT, w.q8, w.qs, w.k8, w.ks, w.v8f,
+                                  w.vs, stream));
     if (bq == kT && (int64_t)Np * kT <= L) {
       SLA2H_TRY(sparse_fwd_qat_stats(q, w.q8, w.qs, w.k8, w.ks, w.v8f, w.vs, lut, dtype, B, H, L,
                                      kT, kT, Np, T, scale, s.o_s, s.lse, s.qphi, stats, stream));

@@ -16,6 +16,11 @@ namespace sla2h {
 
 constexpr int kTile = 64;  // E = D = 64
 
+// fp32 input "storage tag" (16-bit tags: common.h)
+struct F32In {
+  __device__ static inline float to_f32(float f) { return f; }
+};
+
 struct QuantPoolArgs {
   const uint16_t* x[2];   // (BH, L, 64) 16-bit
   int8_t* xq[2];          // (BH, L, 64)
@@ -300,6 +305,161 @@ __global__ __launch_bounds__(256) void quant_train_kernel(QuantTrainArgs a) {
     f[kb] = acc;
   }
   *reinterpret_cast<uint4*>(a.xq[2] + ((int64_t)bh * a.Nb + blk) * 4096 + tid * 16) =
+      make_uint4(f[0], f[1], f[2], f[3]);
+}
+
+// Everything the cube module's training forward does to q, k and v before the
+// attention, in one pass: token layout and fp16 cast (rows_in_kernel's), the
+// truncating INT8 law (quant_train_kernel's) and the router's pooled and
+// projected tiles of q and k (pool_pair_kernel's), equal to the bit.  One
+// (tensor, head, 64-row tile) per workgroup, heads fastest, thread tid = row tid
+// / 4, channels 16 (tid % 4) .. + 15; the pooling sums run in wave 0 from an
+// LDS copy.  HBM-bound: each element is read once; done in three launches the
+// rows were written, then read twice more (2 x 8 heads x 29,952 fp16 tokens 153 ->
+// 122 us, 8 heads x 8,269 bf16 tokens 33.9 -> 15.4 us).
+struct TrainInArgs {
+  const void* x[3];              // (B, L, H, 64), strides below
+  int64_t sb[3], st[3], sh[3];
+  const int64_t* idx;            // token of row l, or null
+  uint16_t* rows[3];             // (B, H, L, 64) fp16, or null
+  int8_t* xq[3];                 // q8, k8 (B, H, L, 64); v8f (B, H, Nb, 4096)
+  float* xs[3];                  // (B, H, Nb)
+  float* pool[2];                // (B, H, Nb, 64); (B, H, 64, Np)
+  const float* proj[2];
+  int B, H, Nb, Np;
+  int64_t L;
+};
+
+template <typename TS, typename Raw>
+__global__ __launch_bounds__(256) void train_in_kernel(TrainInArgs a) {
+  __shared__ __align__(16) uint16_t tile[kTile][kTile];
+  __shared__ __align__(16) int8_t q8t[kTile][kTile + 16];
+  __shared__ float red[4];
+  __shared__ float vec[kTile];
+  const int tid = threadIdx.x;
+  const int i = blockIdx.x;
+  const int h = i % a.H, i1 = i / a.H;
+  const int n = i1 % a.Nb, i2 = i1 / a.Nb;
+  const int b = i2 % a.B, t = i2 / a.B;
+  const int r = tid >> 2, c0 = (tid & 3) * 16;
+  const int64_t row = (int64_t)n * kTile + r;
+  const bool valid = row < a.L;
+  const int64_t bh = (int64_t)b * a.H + h;
+  const int64_t off = (bh * a.L + row) * kTile + c0;
+
+  uint32_t w16[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // the row segment in fp16
+  if (valid) {
+    int64_t tok = row;
+    if (a.idx != nullptr) {
+      tok = a.idx[row];
+      tok = tok < 0 ? 0 : (tok >= a.L ? a.L - 1 : tok);
+    }
+    const Raw* src = static_cast<const Raw*>(a.x[t]) + b * a.sb[t] + tok * a.st[t] + h * a.sh[t] + c0;
+    if constexpr (sizeof(Raw) == 4) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const float4 v = reinterpret_cast<const float4*>(src)[c];
+        w16[2 * c] = pack_pair<F16>(v.x, v.y);
+        w16[2 * c + 1] = pack_pair<F16>(v.z, v.w);
+      }
+    } else {
+      const uint4 u0 = reinterpret_cast<const uint4*>(src)[0], u1 = reinterpret_cast<const uint4*>(src)[1];
+      const uint32_t w[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        w16[k] = std::is_same<TS, F16>::value
+                     ? w[k]
+                     : pack_pair<F16>(TS::to_f32((uint16_t)(w[k] & 0xffff)),
+                                      TS::to_f32((uint16_t)(w[k] >> 16)));
+    }
+  }
+  const uint4 lo = make_uint4(w16[0], w16[1], w16[2], w16[3]);
+  const uint4 hi = make_uint4(w16[4], w16[5], w16[6], w16[7]);
+  if (valid && a.rows[t] != nullptr) {
+    uint4* dst = reinterpret_cast<uint4*>(a.rows[t] + off);
+    dst[0] = lo;
+    dst[1] = hi;
+  }
+  const bool pooled = t == 0 || (t == 1 && n < a.Np);
+  if (pooled) {
+    *reinterpret_cast<uint4*>(&tile[r][c0]) = lo;
+    *reinterpret_cast<uint4*>(&tile[r][c0 + 8]) = hi;
+  }
+  float xv[16];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    xv[2 * k] = F16::to_f32((uint16_t)(w16[k] & 0xffff));
+    xv[2 * k + 1] = F16::to_f32((uint16_t)(w16[k] >> 16));
+  }
+  float am = 0.f;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) am = fmaxf(am, fabsf(xv[k]));
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) am = fmaxf(am, __shfl_xor(am, m, 64));
+  if ((tid & 63) == 0) red[tid >> 6] = am;
+  __syncthreads();
+  am = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  const float s = am / 127.0f + 1e-12f;  // IEEE division, then add
+  const float rs = 1.0f / s;
+  uint32_t w8[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    int qv[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float x = xv[4 * k + e];
+      qv[e] = (int)(quotient(x, s, rs) + (x >= 0.f ? 0.5f : -0.5f));
+    }
+    w8[k] = pack_bytes(qv[0], qv[1], qv[2], qv[3]);
+  }
+  if (tid == 0) a.xs[t][bh * a.Nb + n] = s;
+  const uint4 q4 = make_uint4(w8[0], w8[1], w8[2], w8[3]);
+  if (t < 2) {
+    if (valid) *reinterpret_cast<uint4*>(a.xq[t] + off) = q4;
+    if (!pooled || tid >= kTile) return;
+    const int64_t rem = (t == 0 ? a.L : (int64_t)a.Np * kTile) - (int64_t)n * kTile;
+    const int cnt = rem < kTile ? (int)rem : kTile;
+    float acc = 0.f;
+    int rr = 0;
+    for (; rr + 16 <= cnt; rr += 16) {  // 16 LDS reads in flight, then the adds in row order
+      float xr[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) xr[u] = F16::to_f32(tile[rr + u][tid]);
+#pragma unroll
+      for (int u = 0; u < 16; ++u) acc = acc + xr[u];
+    }
+    for (; rr < cnt; ++rr) acc = acc + F16::to_f32(tile[rr][tid]);
+    float outv = acc / (float)cnt;
+    if (a.proj[t] != nullptr) {
+      vec[tid] = outv;
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      const float* pr = a.proj[t] + tid * kTile;  // out[e] = sum_d mean[d] P[e][d]
+      float p = 0.f;
+#pragma unroll 16
+      for (int d = 0; d < kTile; ++d) p = p + vec[d] * pr[d];
+      outv = p;
+    }
+    if (t)
+      a.pool[1][(bh * kTile + tid) * a.Np + n] = outv;
+    else
+      a.pool[0][(bh * a.Nb + n) * kTile + tid] = outv;
+    return;
+  }
+  // V: transpose to the fragment order through LDS (rows past L are zero)
+  *reinterpret_cast<uint4*>(&q8t[r][c0]) = q4;
+  __syncthreads();
+  const int ct = tid >> 6, lane = tid & 63, g = lane >> 4, rr = lane & 15;
+  uint32_t f[4];
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) {
+    uint32_t acc = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      acc |= ((uint32_t)(uint8_t)q8t[16 * kb + 4 * g + e][16 * ct + rr]) << (8 * e);
+    f[kb] = acc;
+  }
+  *reinterpret_cast<uint4*>(a.xq[2] + (bh * a.Nb + n) * 4096 + tid * 16) =
       make_uint4(f[0], f[1], f[2], f[3]);
 }
 
@@ -646,11 +806,6 @@ static int launch_quant_pool(const QuantPoolArgs& a, int ntens, int dtype, hipSt
 // one block of one (b, h) per workgroup, one thread per channel, sequential
 // fp32 sum over the block's real rows, then / count, then the optional
 // projection out[e] = sum_d mean[d] proj[e][d] (sequential, no contraction).
-// fp32 input "storage tag" for the pooling kernel (16-bit tags: common.h)
-struct F32In {
-  __device__ static inline float to_f32(float f) { return f; }
-};
-
 template <typename TS, typename Raw>
 __global__ __launch_bounds__(64) void pool_blocks_kernel(const Raw* __restrict__ x, int64_t L,
                                                         int blk, int nblk,
@@ -847,6 +1002,53 @@ extern "C" int sla2h_version(void) { return 1; }
 extern "C" const char* sla2h_error_string(int code) {
   return hipGetErrorString((hipError_t)code);
 }
+
+namespace sla2h {
+// x[t] (B, L, H, 64) of one dtype (2: fp32) with strides[3 t ..] of (b, l, h), 16-byte
+// aligned rows; rows[t] (fp16 rows in the op's layout) all given or all NULL.
+int launch_train_in(const void* const* x, const int64_t* strides, int dtype, const int64_t* idx,
+                    int B, int H, int64_t L, int Np, const float* proj_q, const float* proj_k,
+                    void* const* rows, int8_t* const* xq, float* const* xs, float* qpool,
+                    float* kpool_t, void* stream) {
+  const int64_t es = dtype == 2 ? 4 : 2;
+  SLA2H_CHECK_ARG(x && strides && qpool && kpool_t && B > 0 && H > 0 && L > 0);
+  SLA2H_CHECK_ARG(dtype == SLA2H_DTYPE_F16 || dtype == SLA2H_DTYPE_BF16 || dtype == 2);
+  SLA2H_CHECK_ARG(Np > 0 && (int64_t)Np * kTile <= L);
+  TrainInArgs a = {};
+  a.B = B;
+  a.H = H;
+  a.L = L;
+  a.Nb = (int)((L + kTile - 1) / kTile);
+  a.Np = Np;
+  a.idx = idx;
+  a.pool[0] = qpool;
+  a.pool[1] = kpool_t;
+  a.proj[0] = proj_q;
+  a.proj[1] = proj_k;
+  for (int t = 0; t < 3; ++t) {
+    SLA2H_CHECK_ARG(x[t] && (uintptr_t)x[t] % 16 == 0);
+    for (int d = 0; d < 3; ++d) SLA2H_CHECK_ARG(strides[3 * t + d] >= 0 && strides[3 * t + d] * es % 16 == 0);
+    a.x[t] = x[t];
+    a.sb[t] = strides[3 * t];
+    a.st[t] = strides[3 * t + 1];
+    a.sh[t] = strides[3 * t + 2];
+    a.rows[t] = rows == nullptr ? nullptr : static_cast<uint16_t*>(rows[t]);
+    SLA2H_CHECK_ARG(rows == nullptr || (rows[t] && (uintptr_t)rows[t] % 16 == 0));
+    a.xq[t] = xq[t];
+    a.xs[t] = xs[t];
+  }
+  const int64_t nwg = 3 * (int64_t)B * H * a.Nb;
+  SLA2H_CHECK_ARG(nwg < (1ll << 31));
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (dtype == 2)
+    train_in_kernel<F32In, float><<<(unsigned)nwg, 256, 0, st>>>(a);
+  else if (dtype == SLA2H_DTYPE_BF16)
+    train_in_kernel<BF16, uint16_t><<<(unsigned)nwg, 256, 0, st>>>(a);
+  else
+    train_in_kernel<F16, uint16_t><<<(unsigned)nwg, 256, 0, st>>>(a);
+  return (int)hipGetLastError();
+}
+}  // namespace sla2h
 
 extern "C" int sla2h_quant_train(const void* q, const void* k, const void* v, int dtype, int B,
                                  int H, int64_t L, int D, int E, int8_t* q8, float* qs, int8_t* k8,

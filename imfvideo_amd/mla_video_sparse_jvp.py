@@ -61,16 +61,19 @@ def _to16(x):
     return x if x.dtype in (torch.float16, torch.bfloat16) else x.to(torch.bfloat16)
 
 
-def route_tiles_fast(q, k, topk_frac, Np, E, prefix_len, proj_q=None, proj_k=None):
+def route_tiles_fast(q, k, topk_frac, Np, E, prefix_len, proj_q=None, proj_k=None, pooled=None):
     """Hard top-k router on pooled tiles (reference :532-566).
 
     q, k: (B, H, L, D) tile-major, 16-bit or fp32 (fp32 is pooled as given,
     unrounded).  Returns (lut (B,H,Mb,T) int32, T).  Rows of the LUT are
     ordered by descending score (the reference returns them unordered,
-    ``torch.topk(sorted=False)``).
+    ``torch.topk(sorted=False)``).  pooled: the pooled and projected tiles
+    (qpool, kpool_t) of the same q and k, if the caller has them (ops.train_in).
     """
     B, H, L, D = q.shape
-    if q.dtype == torch.float32 and k.dtype == torch.float32:
+    if pooled is not None:
+        qpool, kpool_t = pooled
+    elif q.dtype == torch.float32 and k.dtype == torch.float32:
         # the same pooling law (sequential fp32 row sums, / count, projection
         # as a sequential dot) on the unrounded inputs
         qpool = ops.pool_blocks(q, E, proj_q)

@@ -580,10 +580,33 @@ def train_bwd(q, k, v, alpha, fwd, do, scale=None, stage_events=None, bq=E_TILE)
     return dq, dk, dv, d_alpha
 
 
-def train_op_fwd(q, k, v, alpha_logit, lut, Np, bq=E_TILE, int8=True, stats=None, eps_l=1e-5):
+def train_in(xs, idx, Np, proj_q=None, proj_k=None, rows=True):
+    """The cube op's operands of q, k, v (B, L, H, 64) (rows_in_ok) in one pass ->
+    (rows, ws, qpool, kpool_t): rows the fp16 (B, H, L, 64) tensors of rows_in
+    (None without rows), ws train_op_fwd's workspace holding their INT8
+    operands, and the pooled tiles of pool_qk."""
+    x0 = xs[0]
+    B, L, H, D = x0.shape
+    dev, lib = x0.device, _lib.load()
+    outs = [torch.empty(B, H, L, D, device=dev, dtype=torch.float16) for _ in xs] if rows else None
+    ws = _scratch(lib.sla2h_train_fwd_workspace_bytes(B, H, L, Np, E_TILE, 1, 1), dev)
+    qpool = torch.empty(B, H, -(-L // E_TILE), D, device=dev, dtype=torch.float32)
+    kpool_t = torch.empty(B, H, D, Np, device=dev, dtype=torch.float32)
+    pq, pk = _proj(proj_q, dev), _proj(proj_k, dev)
+    _lib.check(lib.sla2h_train_in(
+        _ptrs(xs), (_lib._c_i64 * 9)(*(s for x in xs for s in x.stride()[:3])),
+        _SITU_DTYPES[x0.dtype], _ptr(idx), B, H, L, Np, _ptr(pq), _ptr(pk),
+        _ptrs(outs) if rows else None, ws.data_ptr(), qpool.data_ptr(), kpool_t.data_ptr(),
+        _stream(dev)), "sla2h_train_in")
+    return outs, ws, qpool, kpool_t
+
+
+def train_op_fwd(q, k, v, alpha_logit, lut, Np, bq=E_TILE, int8=True, stats=None, eps_l=1e-5,
+                 ws=None):
     """train_fwd / train_fwd_1d from the alpha logits (H, ceil(L/bq)) as one native
     call -> (o, saved): saved is the buffer that train_op_bwd reads.  stats:
-    optional (H,) fp32 tensor that receives the per-head maximum of lse."""
+    optional (H,) fp32 tensor that receives the per-head maximum of lse.  ws:
+    train_in's workspace of the same q, k, v (their INT8 operands)."""
     _need_gpu(q, k, v, lut, stats)
     q, k, v = (_bhld(t, n) for t, n in ((q, "q"), (k, "k"), (v, "v")))
     _same(q, k, v)
@@ -595,11 +618,14 @@ def train_op_fwd(q, k, v, alpha_logit, lut, Np, bq=E_TILE, int8=True, stats=None
     logit = _alpha_rows(alpha_logit, H, Mq, dev).contiguous()
     T, lib = lut.shape[-1], _lib.load()
     saved = _scratch(lib.sla2h_train_saved_bytes(B, H, L, Np, bq, T), dev)
-    ws = _scratch(lib.sla2h_train_fwd_workspace_bytes(B, H, L, Np, bq, T, int8), dev)
+    quantised = ws is not None
+    if not quantised:
+        ws = _scratch(lib.sla2h_train_fwd_workspace_bytes(B, H, L, Np, bq, T, int8), dev)
     o = torch.empty_like(q)
     _lib.check(lib.sla2h_train_fwd(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), logit.data_ptr(), lut.data_ptr(), _dtype_code(q),
-        B, H, L, Np, bq, T, int8, D ** -0.5, eps_l, saved.data_ptr(), ws.data_ptr(), o.data_ptr(),
+        B, H, L, Np, bq, T, int8, quantised, D ** -0.5, eps_l, saved.data_ptr(), ws.data_ptr(),
+        o.data_ptr(),
         _ptr(stats), _stream(dev)), "sla2h_train_fwd")
     return o, saved
 

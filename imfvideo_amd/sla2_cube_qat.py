@@ -111,12 +111,13 @@ class _CubeQATFunction(torch.autograd.Function):
     recompute for both, as in the reference.  ``lut_aug``, ``mask`` and
     ``a_index`` are accepted and unused: the kernels append the prefix tail to
     ``lut`` and derive the per-tile selection from it on the device, and the
-    alpha of a row is that of its 64-row block.
+    alpha of a row is that of its 64-row block.  ``ws``: ops.train_in's
+    workspace of the same operands, if the caller has it.
     """
 
     @staticmethod
     def forward(ctx, qh, kh, vh, alpha_logit, lut, lut_aug, mask, T, E, use_int8, a_index,
-                n_tail=1, stats_out=None):
+                n_tail=1, stats_out=None, ws=None):
         assert E == ops.E_TILE, f"E must be {ops.E_TILE}, got {E}"
         B, H, L, D = qh.shape
         Np = -(-L // E) - n_tail
@@ -127,7 +128,7 @@ class _CubeQATFunction(torch.autograd.Function):
                                       and tuple(stats.shape) == (H,) and stats.is_contiguous()):
             stats = torch.empty(H, device=qh.device, dtype=torch.float32)
         o, saved = ops.train_op_fwd(qh, kh, vh, alpha_logit, lut, Np, int8=bool(use_int8),
-                                    stats=stats)
+                                    stats=stats, ws=ws)
         if stats is not stats_out:
             stats_out.copy_(stats)
         ctx.Np, ctx.T = Np, lut.shape[-1]
@@ -138,7 +139,7 @@ class _CubeQATFunction(torch.autograd.Function):
     def backward(ctx, do):
         qh, kh, vh, saved = ctx.saved_tensors
         grads = ops.train_op_bwd(qh, kh, vh, do, saved, ctx.Np, ctx.T)
-        return (*grads, None, None, None, None, None, None, None, None, None)
+        return (*grads, *(None,) * 10)
 
 
 class _RowsIn(torch.autograd.Function):
@@ -165,6 +166,23 @@ class _RowsIn(torch.autograd.Function):
             for i, g in zip(have, outs):
                 grads[i] = g
         return (None, None, *grads)
+
+
+class _TrainIn(torch.autograd.Function):
+    """_RowsIn of q, k, v with the INT8 operands and the pooled tiles made in the
+    same pass (ops.train_in): (qh, kh, vh, ws, qpool, kpool_t)."""
+
+    @staticmethod
+    def forward(ctx, idx, inv, Np, proj_q, proj_k, *xs):
+        ctx.save_for_backward(idx, inv)
+        ctx.dtype = xs[0].dtype
+        rows, *rest = ops.train_in(xs, idx, Np, proj_q, proj_k)
+        ctx.mark_non_differentiable(*rest)
+        return (*rows, *rest)
+
+    @staticmethod
+    def backward(ctx, *ds):
+        return (None, None, None, *_RowsIn.backward(ctx, *ds[:3]))
 
 
 class _RowsOut(torch.autograd.Function):
@@ -252,10 +270,15 @@ class SLA2CubeQATAttentionImpl(nn.Module):
         own = (ops.plain_eager(q, k, v) and ops.rows_in_ok((q, k, v)) and self.perm.device == q.device
                and (self.pre_permuted or self.perm.numel() == q.shape[1]))
         perm, inv = (None, None) if self.pre_permuted else (self.perm, self.inv)
-        if own:
-            o = self.forward_tile_major(*_RowsIn.apply(perm, inv, q, k, v))
-        else:
+        if not own:
             o = self.forward_tile_major(tm(q), tm(k), tm(v))
+        elif (self._one_pass(q.shape[1]) and "forward_tile_major" not in self.__dict__
+              and type(self).forward_tile_major is SLA2CubeQATAttentionImpl.forward_tile_major):
+            qh, kh, vh, *pre = _TrainIn.apply(perm, inv, self.Np, self.proj_q.detach(),
+                                              self.proj_k.detach(), q, k, v)
+            o = self._op(qh, kh, vh, *pre)
+        else:
+            o = self.forward_tile_major(*_RowsIn.apply(perm, inv, q, k, v))
         if self.pre_permuted:
             return o.permute(0, 2, 1, 3).to(q.dtype)
         if own:
@@ -268,10 +291,26 @@ class SLA2CubeQATAttentionImpl(nn.Module):
         rows.  forward() is this between the reference's permute / .half() of
         q, k, v and the permute / cast back of o; a caller that keeps the
         sequence tile-major can build the operands and consume o directly."""
-        B, H, L, D = qh.shape
+        xs = [x.permute(0, 2, 1, 3) for x in (qh, kh, vh)]
+        pre = ()
+        if qh.dtype == torch.float16 and self._one_pass(qh.shape[2]) and ops.rows_in_ok(xs):
+            with torch.no_grad():
+                _, *pre = ops.train_in(xs, None, self.Np, self.proj_q, self.proj_k, rows=False)
+        return self._op(qh, kh, vh, *pre)
+
+    def _one_pass(self, L):
+        """ops.train_in can make this call's INT8 operands and pooled tiles."""
+        return (self.use_int8 and self.E == ops.E_TILE
+                and L == self.Np * self.E + self.prefix_len)
+
+    def _op(self, qh, kh, vh, ws=None, qpool=None, kpool_t=None):
+        """forward_tile_major on operands whose INT8 values and pooled tiles
+        (ops.train_in) are there already, or not."""
+        H = qh.shape[1]
         with torch.no_grad():
             lut, T = route_tiles_fast(qh, kh, self.topk_frac, self.Np, self.E, self.prefix_len,
-                                      proj_q=self.proj_q, proj_k=self.proj_k)
+                                      proj_q=self.proj_q, proj_k=self.proj_k,
+                                      pooled=None if ws is None else (qpool, kpool_t))
         needs_grad = torch.is_grad_enabled() and (
             qh.requires_grad or kh.requires_grad or vh.requires_grad
             or self.alpha_logit.requires_grad)
@@ -280,6 +319,6 @@ class SLA2CubeQATAttentionImpl(nn.Module):
                 self.logit_max_log2 = torch.zeros(H, device=qh.device, dtype=torch.float32)
             return _CubeQATFunction.apply(qh, kh, vh, self.alpha_logit, lut, None, None, T,
                                           self.E, self.use_int8, self.a_index, self.n_tail,
-                                          self.logit_max_log2)
+                                          self.logit_max_log2, ws)
         return ops.train_op_fwd(qh, kh, vh, self.alpha_logit, lut, self.Np,
-                                int8=bool(self.use_int8))[0]
+                                int8=bool(self.use_int8), ws=ws)[0]

@@ -766,7 +766,8 @@ int sla2h_jvp16(const void* q, const void* k, const void* v, const void* dq, con
 /*
  * The training op: forward on given routing (cube: bq = 64; 1-D: Np = Nb) from the
  * alpha logits (H, ceil(L/bq)), INT8 or 16-bit sparse branch, score-form linear
- * branch up to 4 LUT columns.  `saved` holds what the backward reads; stats (H),
+ * branch up to 4 LUT columns.  quantised: the workspace (of int8 = 1) already holds
+ * the INT8 operands, from sla2h_train_in.  `saved` holds what the backward reads; stats (H),
  * optional, receives the per-head maximum of lse.  The backward writes dq, dk, dv
  * (16-bit) and the gradient of the logits (H, ceil(L/bq)); it only reads `saved`.
  * Replaces _CubeQATFunction (models/sla2_cube_qat.py:696-832).
@@ -775,13 +776,24 @@ size_t sla2h_train_saved_bytes(int B, int H, int64_t L, int Np, int bq, int T);
 size_t sla2h_train_fwd_workspace_bytes(int B, int H, int64_t L, int Np, int bq, int T, int int8);
 int sla2h_train_fwd(const void* q, const void* k, const void* v, const float* alpha_logit,
                     const int32_t* lut, int dtype, int B, int H, int64_t L, int Np, int bq, int T,
-                    int int8, float scale, float eps_l, void* saved, void* workspace, void* o,
-                    float* stats, void* stream);
+                    int int8, int quantised, float scale, float eps_l, void* saved,
+                    void* workspace, void* o, float* stats, void* stream);
 size_t sla2h_train_bwd_workspace_bytes(int B, int H, int64_t L, int Np, int bq, int T);
 int sla2h_train_bwd(const void* q, const void* k, const void* v, const void* dout,
                     const void* saved, int dtype, int B, int H, int64_t L, int Np, int bq, int T,
                     float scale, void* workspace, void* dq, void* dk, void* dv, float* d_logit,
                     void* stream);
+
+/*
+ * The cube module's operands in one pass: x[t] = q, k, v (B, L, H, 64) of one dtype
+ * (0 / 1 / 2 = fp16 / bf16 / fp32), strides and idx as in sla2h_rows_in; writes
+ * the fp16 rows rows[t] (B, H, L, 64) unless rows is NULL, the truncating INT8
+ * operands of those rows into sla2h_train_fwd's workspace, and the router's
+ * qpool (B,H,Nb,64) and kpool_t (B,H,64,Np) of them (sla2h_pool_qk).
+ */
+int sla2h_train_in(const void* const* x, const int64_t* strides, int dtype, const int64_t* idx,
+                   int B, int H, int64_t L, int Np, const float* proj_q, const float* proj_k,
+                   void* const* rows, void* workspace, float* qpool, float* kpool_t, void* stream);
 
 /*
  * The 1-D SLA2 inference forward on given routing: sla2h_hblocks_states, the

@@ -508,3 +508,42 @@ def test_native_calls_match_the_stages(dt, B, H, L, Np, bq, T, int8):
                 assert torch.equal(f1[0], f2[0])
                 assert (f1[1] is None) == (tan[0] is None)
                 assert f1[1] is None or torch.equal(f1[1], f2[1])
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,L,H,Np", [(1, 64, 1, 1), (2, 274, 3, 4), (1, 1000, 2, 15), (1, 577, 5, 8)])
+@pytest.mark.parametrize("order", ["permuted", "tile_major"])
+def test_train_in_matches_the_separate_passes(dt, B, L, H, Np, order):
+    """The one-pass operands (fp16 rows, truncating INT8 values and scales, pooled
+    and projected tiles) against rows_in, quant_train and pool_qk: equal to the
+    bit, with a permutation and without, ragged and prefix blocks, zeros and
+    values up to the fp16 maximum."""
+    from imfvideo_amd import ops
+    print("[case] train_in", dt, B, L, H, Np, order, flush=True)
+    g = torch.Generator().manual_seed(L)
+    xs = [(torch.randn(B, L, H, 64, generator=g) * s).to(dt) for s in (1.0, 50.0, 0.01)]
+    xs[0][:, :64] = 0
+    xs[1][0, -1, 0, 3] = 65504.0
+    xs = [x.cuda() for x in xs]
+    idx = torch.randperm(L, generator=g).cuda() if order == "permuted" else None
+    pq, pk = (torch.randn(64, 64, generator=g).cuda() for _ in range(2))
+    rows, ws, qpool, kpool_t = ops.train_in(xs, idx, Np, pq, pk)
+    want = ops.rows_in(xs, idx)
+    for a, b in zip(rows, want):
+        assert torch.equal(a, b)
+    qz = ops.quant_train(*want)
+    off = 0
+    for name in ("q8", "k8", "v8f", "qs", "ks", "vs"):
+        t = qz[name]
+        n = t.numel() * t.element_size()
+        assert torch.equal(ws[off:off + n].view(t.dtype).view(t.shape), t), name
+        off += -(-n // 256) * 256
+    wq, wk = ops.pool_qk(want[0], want[1], 64, Np, pq, pk)
+    assert torch.equal(qpool, wq) and torch.equal(kpool_t, wk)
+    if order == "tile_major":
+        views = [x.permute(0, 2, 1, 3) for x in want]
+        none, ws2, qp2, kp2 = ops.train_in(views, None, Np, pq, pk, rows=False)
+        # (the alignment gaps between the buffers are not written)
+        n = L * B * H * 64
+        assert none is None and torch.equal(ws2[:n], ws[:n])
+        assert torch.equal(qp2, qpool) and torch.equal(kp2, kpool_t)
