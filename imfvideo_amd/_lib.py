@@ -100,7 +100,10 @@ SIGNATURES = {
     "sla2h_sla2_infer_workspace_bytes": (ctypes.c_size_t, [_c_int, _c_int, _c_i64, _c_int, _c_int,
                                                            _c_int]),
     "sla2h_sla2_infer": (_c_int, [_p, _p, _p, _p, _c_int, _p, _c_int, _c_int, _c_int, _c_i64,
-                                  _c_int, _c_int, _c_int, _c_int, _c_f, _c_f, _p, _p, _p]),
+                                  _c_int, _c_int, _c_int, _c_int, _c_int, _c_f, _c_f, _p, _p,
+                                  _p]),
+    "sla2h_sla2_infer_in": (_c_int, [_p, _p, _p, _c_int, _c_int, _c_int, _c_i64, _c_int, _p, _p,
+                                     _p, _p, _p, _p]),
     "sla2h_rows_in": (_c_int, [_p, _p, _c_int, _c_int, _p, _c_int, _c_int, _c_i64, _p, _p]),
     "sla2h_rows_out": (_c_int, [_p, _c_int, _c_int, _p, _c_int, _c_int, _c_i64, _p, _p]),
     "sla2h_linear_wgrad_workspace_bytes": (ctypes.c_size_t, [_c_i64, _c_int, _c_int]),

@@ -244,10 +244,10 @@ int sparse_fwd_1d_stats(const void* q, const void* k, const void* vt, const int3
                         void* stream);
 
 // quant_route.hip: layout, INT8 operands and pooled tiles of q, k, v in one pass
-int launch_train_in(const void* const* x, const int64_t* strides, int dtype, const int64_t* idx,
-                    int B, int H, int64_t L, int Np, const float* proj_q, const float* proj_k,
-                    void* const* rows, int8_t* const* xq, float* const* xs, float* qpool,
-                    float* kpool_t, void* stream);
+int launch_operands(const void* const* x, const int64_t* strides, int dtype, const int64_t* idx,
+                    int B, int H, int64_t L, int Np, int bq, int infer, const float* proj_q,
+                    const float* proj_k, void* const* rows, int8_t* const* xq, float* const* xs,
+                    float* qpool, float* kpool_t, void* stream);
 
 // states.hip: the backward's complement records from given masks (word (kcq, n))
 int complement_gemm_bwd(const float* P, const float* Pz, const uint32_t* cbits, int BH, int Mb,
@@ -354,8 +354,8 @@ extern "C" int sla2h_train_in(const void* const* x, const int64_t* strides, int 
   const FwdWs w(workspace, Dims(B, H, L, Np, kT, 1), true);
   int8_t* const xq[3] = {w.q8, w.k8, w.v8f};
   float* const xs[3] = {w.qs, w.ks, w.vs};
-  return launch_train_in(x, strides, dtype, idx, B, H, L, Np, proj_q, proj_k, rows, xq, xs, qpool,
-                         kpool_t, stream);
+  return launch_operands(x, strides, dtype, idx, B, H, L, Np, kT, 0, proj_q, proj_k, rows, xq, xs,
+                         qpool, kpool_t, stream);
 }
 
 extern "C" int sla2h_train_fwd(const void* q, const void* k, const void* v,
@@ -491,22 +491,41 @@ extern "C" size_t sla2h_sla2_infer_workspace_bytes(int B, int H, int64_t L, int 
   return InferWs(nullptr, Dims(B, H, L, Nb, bq, T), int8 != 0).bytes;
 }
 
+extern "C" int sla2h_sla2_infer_in(const void* q, const void* k, const void* v, int dtype, int B,
+                                   int H, int64_t L, int bq, const float* proj_q,
+                                   const float* proj_k, void* workspace, float* qpool,
+                                   float* kpool_t, void* stream) {
+  SLA2H_CHECK_ARG(workspace && L > 0);
+  const int Nb = (int)((L + kT - 1) / kT);
+  SLA2H_CHECK_ARG(dims_ok(dtype, B, H, L, Nb, bq, 1));
+  const InferWs w(workspace, Dims(B, H, L, Nb, bq, 1), true);
+  const void* const x[3] = {q, k, v};
+  const int64_t s[3] = {H * L * kT, kT, L * kT};
+  const int64_t strides[9] = {s[0], s[1], s[2], s[0], s[1], s[2], s[0], s[1], s[2]};
+  int8_t* const xq[3] = {w.q8, w.k8, w.v8f};
+  float* const xs[3] = {w.qs, w.ks, w.vs};
+  return launch_operands(x, strides, dtype, nullptr, B, H, L, Nb, bq, 1, proj_q, proj_k, nullptr,
+                         xq, xs, qpool, kpool_t, stream);
+}
+
 extern "C" int sla2h_sla2_infer(const void* q, const void* k, const void* v, const float* alpha,
                                 int alpha_stride, const int32_t* lut, int dtype, int B, int H,
-                                int64_t L, int bq, int T, int int8, int qblock, float scale,
-                                float eps_l, void* workspace, void* o, void* stream) {
+                                int64_t L, int bq, int T, int int8, int qblock, int quantised,
+                                float scale, float eps_l, void* workspace, void* o, void* stream) {
   SLA2H_CHECK_ARG(q && k && v && alpha && lut && workspace && o && L > 0);
   const int Nb = (int)((L + kT - 1) / kT);
-  SLA2H_CHECK_ARG(dims_ok(dtype, B, H, L, Nb, bq, T));
+  SLA2H_CHECK_ARG(dims_ok(dtype, B, H, L, Nb, bq, T) && (!quantised || (int8 && qblock == bq)));
   const Dims d(B, H, L, Nb, bq, T);
   const InferWs w(workspace, d, int8 != 0);
   SLA2H_TRY(sla2h_hblocks_states(k, v, dtype, B, H, L, kT, kT, w.Hb, w.zb, nullptr, nullptr, w.vt,
                                  stream));
   if (int8) {
     const int64_t bh = (int64_t)d.BH;
-    SLA2H_TRY(sla2h_quantize(q, dtype, bh, L, kT, qblock, w.q8, w.qs, stream));
-    SLA2H_TRY(sla2h_quantize(k, dtype, bh, L, kT, kT, w.k8, w.ks, stream));
-    SLA2H_TRY(sla2h_quantize_v8f(v, dtype, bh, L, kT, kT, w.v8f, w.vs, stream));
+    if (!quantised) {
+      SLA2H_TRY(sla2h_quantize(q, dtype, bh, L, kT, qblock, w.q8, w.qs, stream));
+      SLA2H_TRY(sla2h_quantize(k, dtype, bh, L, kT, kT, w.k8, w.ks, stream));
+      SLA2H_TRY(sla2h_quantize_v8f(v, dtype, bh, L, kT, kT, w.v8f, w.vs, stream));
+    }
     SLA2H_TRY(sla2h_sparse_fwd_int8(q, w.q8, w.qs, qblock, w.k8, w.ks, w.v8f, w.vs, lut, dtype, B,
                                     H, L, kT, bq, T, scale, w.o_s, w.lse, w.qphi, stream));
   } else {

@@ -308,92 +308,102 @@ __global__ __launch_bounds__(256) void quant_train_kernel(QuantTrainArgs a) {
       make_uint4(f[0], f[1], f[2], f[3]);
 }
 
-// Everything the cube module's training forward does to q, k and v before the
-// attention, in one pass: token layout and fp16 cast (rows_in_kernel's), the
-// truncating INT8 law (quant_train_kernel's) and the router's pooled and
-// projected tiles of q and k (pool_pair_kernel's), equal to the bit.  One
-// (tensor, head, 64-row tile) per workgroup, heads fastest, thread tid = row tid
-// / 4, channels 16 (tid % 4) .. + 15; the pooling sums run in wave 0 from an
-// LDS copy.  HBM-bound: each element is read once; done in three launches the
-// rows were written, then read twice more (2 x 8 heads x 29,952 fp16 tokens 153 ->
-// 122 us, 8 heads x 8,269 bf16 tokens 33.9 -> 15.4 us).
-struct TrainInArgs {
+// Everything done to q, k and v before the INT8 attention, in one pass: token
+// layout and 16-bit cast (rows_in_kernel's), the INT8 law (truncating as
+// quant_train_kernel, or with RND half away from zero as quant_rows_kernel) and
+// the router's pooled and projected blocks of q and k (pool_pair_kernel's), equal
+// to the bit.  q in blocks of 64 NB rows, k and v of 64; one (tensor, head, block)
+// per workgroup, heads fastest, thread tid = rows tid / 4 + 64 c, channels 16
+// (tid % 4) .. + 15; the pooling sums run in wave 0 from an LDS copy.  HBM-bound:
+// each element is read once.  Training, against three launches that wrote the
+// rows and read them twice more: 2 x 8 heads x 29,952 fp16 tokens 153 -> 122 us,
+// 8 heads x 8,269 bf16 tokens 33.9 -> 15.4 us.
+struct OperandArgs {
   const void* x[3];              // (B, L, H, 64), strides below
   int64_t sb[3], st[3], sh[3];
   const int64_t* idx;            // token of row l, or null
-  uint16_t* rows[3];             // (B, H, L, 64) fp16, or null
+  uint16_t* rows[3];             // (B, H, L, 64) 16-bit, or null
   int8_t* xq[3];                 // q8, k8 (B, H, L, 64); v8f (B, H, Nb, 4096)
-  float* xs[3];                  // (B, H, Nb)
-  float* pool[2];                // (B, H, Nb, 64); (B, H, 64, Np)
+  float* xs[3];                  // (B, H, blocks)
+  float* pool[2];                // (B, H, Mq, 64); (B, H, 64, Np)
   const float* proj[2];
-  int B, H, Nb, Np;
+  int B, H, Nb, Np, Mq;
   int64_t L;
 };
 
-template <typename TS, typename Raw>
-__global__ __launch_bounds__(256) void train_in_kernel(TrainInArgs a) {
-  __shared__ __align__(16) uint16_t tile[kTile][kTile];
+// TS: storage type of x, TR: the 16-bit type it is rounded to
+template <typename TS, typename Raw, typename TR, bool RND, int NB>
+__global__ __launch_bounds__(256) void operand_kernel(OperandArgs a) {
+  __shared__ __align__(16) uint16_t tile[64 * NB][kTile];
   __shared__ __align__(16) int8_t q8t[kTile][kTile + 16];
   __shared__ float red[4];
   __shared__ float vec[kTile];
   const int tid = threadIdx.x;
-  const int i = blockIdx.x;
+  int i = blockIdx.x;
+  const int nq = a.B * a.H * a.Mq, nk = a.B * a.H * a.Nb;
+  const int t = i < nq ? 0 : (i < nq + nk ? 1 : 2);
+  i -= t == 0 ? 0 : (t == 1 ? nq : nq + nk);
+  const int nblk = t == 0 ? a.Mq : a.Nb;  // blocks of this tensor per head
+  const int per = t == 0 ? kTile * NB : kTile;  // rows per block
   const int h = i % a.H, i1 = i / a.H;
-  const int n = i1 % a.Nb, i2 = i1 / a.Nb;
-  const int b = i2 % a.B, t = i2 / a.B;
+  const int n = i1 % nblk, b = i1 / nblk;
   const int r = tid >> 2, c0 = (tid & 3) * 16;
-  const int64_t row = (int64_t)n * kTile + r;
-  const bool valid = row < a.L;
   const int64_t bh = (int64_t)b * a.H + h;
-  const int64_t off = (bh * a.L + row) * kTile + c0;
-
-  uint32_t w16[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // the row segment in fp16
-  if (valid) {
-    int64_t tok = row;
-    if (a.idx != nullptr) {
-      tok = a.idx[row];
-      tok = tok < 0 ? 0 : (tok >= a.L ? a.L - 1 : tok);
-    }
-    const Raw* src = static_cast<const Raw*>(a.x[t]) + b * a.sb[t] + tok * a.st[t] + h * a.sh[t] + c0;
-    if constexpr (sizeof(Raw) == 4) {
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const float4 v = reinterpret_cast<const float4*>(src)[c];
-        w16[2 * c] = pack_pair<F16>(v.x, v.y);
-        w16[2 * c + 1] = pack_pair<F16>(v.z, v.w);
-      }
-    } else {
-      const uint4 u0 = reinterpret_cast<const uint4*>(src)[0], u1 = reinterpret_cast<const uint4*>(src)[1];
-      const uint32_t w[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
-#pragma unroll
-      for (int k = 0; k < 8; ++k)
-        w16[k] = std::is_same<TS, F16>::value
-                     ? w[k]
-                     : pack_pair<F16>(TS::to_f32((uint16_t)(w[k] & 0xffff)),
-                                      TS::to_f32((uint16_t)(w[k] >> 16)));
-    }
-  }
-  const uint4 lo = make_uint4(w16[0], w16[1], w16[2], w16[3]);
-  const uint4 hi = make_uint4(w16[4], w16[5], w16[6], w16[7]);
-  if (valid && a.rows[t] != nullptr) {
-    uint4* dst = reinterpret_cast<uint4*>(a.rows[t] + off);
-    dst[0] = lo;
-    dst[1] = hi;
-  }
+  const int64_t row0 = (int64_t)n * per + r;
+  const int64_t off = (bh * a.L + row0) * kTile + c0;
   const bool pooled = t == 0 || (t == 1 && n < a.Np);
-  if (pooled) {
-    *reinterpret_cast<uint4*>(&tile[r][c0]) = lo;
-    *reinterpret_cast<uint4*>(&tile[r][c0 + 8]) = hi;
-  }
-  float xv[16];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    xv[2 * k] = F16::to_f32((uint16_t)(w16[k] & 0xffff));
-    xv[2 * k + 1] = F16::to_f32((uint16_t)(w16[k] >> 16));
-  }
+
+  float xv[NB][16];
   float am = 0.f;
 #pragma unroll
-  for (int k = 0; k < 16; ++k) am = fmaxf(am, fabsf(xv[k]));
+  for (int c = 0; c < NB; ++c) {
+    if (c > 0 && t != 0) break;  // uniform
+    const int64_t row = row0 + 64 * c;
+    uint32_t w16[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // the row segment in 16 bits
+    if (row < a.L) {
+      int64_t tok = row;
+      if (a.idx != nullptr) {
+        tok = a.idx[row];
+        tok = tok < 0 ? 0 : (tok >= a.L ? a.L - 1 : tok);
+      }
+      const Raw* src = static_cast<const Raw*>(a.x[t]) + b * a.sb[t] + tok * a.st[t] + h * a.sh[t] + c0;
+      if constexpr (sizeof(Raw) == 4) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const float4 v = reinterpret_cast<const float4*>(src)[k];
+          w16[2 * k] = pack_pair<TR>(v.x, v.y);
+          w16[2 * k + 1] = pack_pair<TR>(v.z, v.w);
+        }
+      } else {
+        const uint4 u0 = reinterpret_cast<const uint4*>(src)[0], u1 = reinterpret_cast<const uint4*>(src)[1];
+        const uint32_t w[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          w16[k] = std::is_same<TS, TR>::value
+                       ? w[k]
+                       : pack_pair<TR>(TS::to_f32((uint16_t)(w[k] & 0xffff)),
+                                       TS::to_f32((uint16_t)(w[k] >> 16)));
+      }
+    }
+    const uint4 lo = make_uint4(w16[0], w16[1], w16[2], w16[3]);
+    const uint4 hi = make_uint4(w16[4], w16[5], w16[6], w16[7]);
+    if (row < a.L && a.rows[t] != nullptr) {
+      uint4* dst = reinterpret_cast<uint4*>(a.rows[t] + off + 64 * c * kTile);
+      dst[0] = lo;
+      dst[1] = hi;
+    }
+    if (pooled) {
+      *reinterpret_cast<uint4*>(&tile[r + 64 * c][c0]) = lo;
+      *reinterpret_cast<uint4*>(&tile[r + 64 * c][c0 + 8]) = hi;
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      xv[c][2 * k] = TR::to_f32((uint16_t)(w16[k] & 0xffff));
+      xv[c][2 * k + 1] = TR::to_f32((uint16_t)(w16[k] >> 16));
+    }
+#pragma unroll
+    for (int k = 0; k < 16; ++k) am = fmaxf(am, fabsf(xv[c][k]));
+  }
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) am = fmaxf(am, __shfl_xor(am, m, 64));
   if ((tid & 63) == 0) red[tid >> 6] = am;
@@ -401,34 +411,41 @@ __global__ __launch_bounds__(256) void train_in_kernel(TrainInArgs a) {
   am = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
   const float s = am / 127.0f + 1e-12f;  // IEEE division, then add
   const float rs = 1.0f / s;
-  uint32_t w8[4];
+  if (tid == 0) a.xs[t][bh * nblk + n] = s;
+  uint4 q4;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    int qv[4];
+  for (int c = 0; c < NB; ++c) {
+    if (c > 0 && t != 0) break;
+    uint32_t w8[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float x = xv[4 * k + e];
-      qv[e] = (int)(quotient(x, s, rs) + (x >= 0.f ? 0.5f : -0.5f));
+    for (int k = 0; k < 4; ++k) {
+      int qv[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float x = xv[c][4 * k + e];
+        const float y = quotient(x, s, rs);
+        qv[e] = RND ? round_away(y, x) : (int)(y + (x >= 0.f ? 0.5f : -0.5f));
+      }
+      w8[k] = pack_bytes(qv[0], qv[1], qv[2], qv[3]);
     }
-    w8[k] = pack_bytes(qv[0], qv[1], qv[2], qv[3]);
+    q4 = make_uint4(w8[0], w8[1], w8[2], w8[3]);
+    if (t < 2 && row0 + 64 * c < a.L)
+      *reinterpret_cast<uint4*>(a.xq[t] + off + 64 * c * kTile) = q4;
   }
-  if (tid == 0) a.xs[t][bh * a.Nb + n] = s;
-  const uint4 q4 = make_uint4(w8[0], w8[1], w8[2], w8[3]);
   if (t < 2) {
-    if (valid) *reinterpret_cast<uint4*>(a.xq[t] + off) = q4;
     if (!pooled || tid >= kTile) return;
-    const int64_t rem = (t == 0 ? a.L : (int64_t)a.Np * kTile) - (int64_t)n * kTile;
-    const int cnt = rem < kTile ? (int)rem : kTile;
+    const int64_t rem = (t == 0 ? a.L : min(a.L, (int64_t)a.Np * kTile)) - (int64_t)n * per;
+    const int cnt = rem < per ? (int)rem : per;
     float acc = 0.f;
     int rr = 0;
     for (; rr + 16 <= cnt; rr += 16) {  // 16 LDS reads in flight, then the adds in row order
       float xr[16];
 #pragma unroll
-      for (int u = 0; u < 16; ++u) xr[u] = F16::to_f32(tile[rr + u][tid]);
+      for (int u = 0; u < 16; ++u) xr[u] = TR::to_f32(tile[rr + u][tid]);
 #pragma unroll
       for (int u = 0; u < 16; ++u) acc = acc + xr[u];
     }
-    for (; rr < cnt; ++rr) acc = acc + F16::to_f32(tile[rr][tid]);
+    for (; rr < cnt; ++rr) acc = acc + TR::to_f32(tile[rr][tid]);
     float outv = acc / (float)cnt;
     if (a.proj[t] != nullptr) {
       vec[tid] = outv;
@@ -443,7 +460,7 @@ __global__ __launch_bounds__(256) void train_in_kernel(TrainInArgs a) {
     if (t)
       a.pool[1][(bh * kTile + tid) * a.Np + n] = outv;
     else
-      a.pool[0][(bh * a.Nb + n) * kTile + tid] = outv;
+      a.pool[0][(bh * a.Mq + n) * kTile + tid] = outv;
     return;
   }
   // V: transpose to the fragment order through LDS (rows past L are zero)
@@ -1005,21 +1022,25 @@ extern "C" const char* sla2h_error_string(int code) {
 
 namespace sla2h {
 // x[t] (B, L, H, 64) of one dtype (2: fp32) with strides[3 t ..] of (b, l, h), 16-byte
-// aligned rows; rows[t] (fp16 rows in the op's layout) all given or all NULL.
-int launch_train_in(const void* const* x, const int64_t* strides, int dtype, const int64_t* idx,
-                    int B, int H, int64_t L, int Np, const float* proj_q, const float* proj_k,
-                    void* const* rows, int8_t* const* xq, float* const* xs, float* qpool,
-                    float* kpool_t, void* stream) {
+// aligned rows.  infer = 0: the training operands (fp16 rows, all of rows[t] given or
+// rows NULL, truncating law, bq = 64); infer = 1: 16-bit x as it is, half away from
+// zero, q in blocks of bq rows, every key block pooled (Np = Nb).
+int launch_operands(const void* const* x, const int64_t* strides, int dtype, const int64_t* idx,
+                    int B, int H, int64_t L, int Np, int bq, int infer, const float* proj_q,
+                    const float* proj_k, void* const* rows, int8_t* const* xq, float* const* xs,
+                    float* qpool, float* kpool_t, void* stream) {
   const int64_t es = dtype == 2 ? 4 : 2;
   SLA2H_CHECK_ARG(x && strides && qpool && kpool_t && B > 0 && H > 0 && L > 0);
-  SLA2H_CHECK_ARG(dtype == SLA2H_DTYPE_F16 || dtype == SLA2H_DTYPE_BF16 || dtype == 2);
-  SLA2H_CHECK_ARG(Np > 0 && (int64_t)Np * kTile <= L);
-  TrainInArgs a = {};
+  SLA2H_CHECK_ARG(dtype == SLA2H_DTYPE_F16 || dtype == SLA2H_DTYPE_BF16 || (dtype == 2 && !infer));
+  SLA2H_CHECK_ARG(bq == 64 || (infer && (bq == 128 || bq == 256)));
+  OperandArgs a = {};
   a.B = B;
   a.H = H;
   a.L = L;
   a.Nb = (int)((L + kTile - 1) / kTile);
   a.Np = Np;
+  a.Mq = (int)((L + bq - 1) / bq);
+  SLA2H_CHECK_ARG(Np > 0 && (infer ? Np == a.Nb : (int64_t)Np * kTile <= L));
   a.idx = idx;
   a.pool[0] = qpool;
   a.pool[1] = kpool_t;
@@ -1037,15 +1058,24 @@ int launch_train_in(const void* const* x, const int64_t* strides, int dtype, con
     a.xq[t] = xq[t];
     a.xs[t] = xs[t];
   }
-  const int64_t nwg = 3 * (int64_t)B * H * a.Nb;
+  const int64_t nwg = (int64_t)B * H * (a.Mq + 2 * (int64_t)a.Nb);
   SLA2H_CHECK_ARG(nwg < (1ll << 31));
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (dtype == 2)
-    train_in_kernel<F32In, float><<<(unsigned)nwg, 256, 0, st>>>(a);
+  auto run = [&](auto kernel) { kernel<<<(unsigned)nwg, 256, 0, st>>>(a); };
+  auto run_infer = [&](auto ts) {
+    using TS = decltype(ts);
+    bq == 64 ? run(operand_kernel<TS, uint16_t, TS, true, 1>)
+             : (bq == 128 ? run(operand_kernel<TS, uint16_t, TS, true, 2>)
+                          : run(operand_kernel<TS, uint16_t, TS, true, 4>));
+  };
+  if (infer)
+    dtype == SLA2H_DTYPE_BF16 ? run_infer(BF16{}) : run_infer(F16{});
+  else if (dtype == 2)
+    run(operand_kernel<F32In, float, F16, false, 1>);
   else if (dtype == SLA2H_DTYPE_BF16)
-    train_in_kernel<BF16, uint16_t><<<(unsigned)nwg, 256, 0, st>>>(a);
+    run(operand_kernel<BF16, uint16_t, F16, false, 1>);
   else
-    train_in_kernel<F16, uint16_t><<<(unsigned)nwg, 256, 0, st>>>(a);
+    run(operand_kernel<F16, uint16_t, F16, false, 1>);
   return (int)hipGetLastError();
 }
 }  // namespace sla2h

@@ -912,13 +912,14 @@ def lin_fwd3(qphi, comp, o_s, alpha, bq, eps_l=1e-5):
 
 
 def sla2_infer(q, k, v, alpha, lut, bq, use_int8=True, qblock=None, eps_l=1e-5,
-               return_parts=False):
+               return_parts=False, ws=None):
     """SLA2 inference forward on given routing.
 
     q, k, v: (B,H,L,64) 16-bit, natural order; alpha (H, ceil(L/bq)) after the
     sigmoid; lut (B,H,ceil(L/bq),T) routed 64-row key blocks.  use_int8: the
     INT8 sparse branch with Q scales per qblock rows (default bq), else the
-    16-bit one.  Returns o (16-bit) [, dict of the intermediates].
+    16-bit one.  ws: sla2_infer_in's workspace of the same q, k, v and bq.
+    Returns o (16-bit) [, dict of the intermediates].
     """
     _need_gpu(q, k, v, lut)
     q, k, v = (_bhld(t, "qkv") for t in (q, k, v))
@@ -926,7 +927,7 @@ def sla2_infer(q, k, v, alpha, lut, bq, use_int8=True, qblock=None, eps_l=1e-5,
     nb = -(-L // E_TILE)
     lut = lut.to(torch.int32).contiguous()
     if not return_parts:
-        return _sla2_infer_call(q, k, v, alpha, lut, bq, use_int8, qblock, eps_l)
+        return _sla2_infer_call(q, k, v, alpha, lut, bq, use_int8, qblock, eps_l, ws)
     st = hblocks_states(k, v, with_vt=not use_int8)
     if use_int8:
         qb = bq if qblock is None else qblock
@@ -941,7 +942,25 @@ def sla2_infer(q, k, v, alpha, lut, bq, use_int8=True, qblock=None, eps_l=1e-5,
     return o, dict(o_s=o_s, lse=lse, qphi=qphi, comp=comp, **st)
 
 
-def _sla2_infer_call(q, k, v, alpha, lut, bq, use_int8, qblock, eps_l):
+def sla2_infer_in(q, k, v, bq, proj_q=None, proj_k=None):
+    """sla2_infer's INT8 operands and the router's pooled blocks of 16-bit q, k, v in
+    one pass -> (ws, qpool, kpool_t) (ws for sla2_infer; pool_qk's tensors)."""
+    _need_gpu(q, k, v)
+    q, k, v = (_bhld(t, "qkv") for t in (q, k, v))
+    _same(q, k, v)
+    B, H, L, D = q.shape
+    dev, lib, nb = q.device, _lib.load(), -(-L // E_TILE)
+    pq, pk = _proj(proj_q, dev), _proj(proj_k, dev)
+    ws = _scratch(lib.sla2h_sla2_infer_workspace_bytes(B, H, L, bq, 1, 1), dev)
+    qpool = torch.empty(B, H, -(-L // bq), D, device=dev, dtype=torch.float32)
+    kpool_t = torch.empty(B, H, D, nb, device=dev, dtype=torch.float32)
+    _lib.check(lib.sla2h_sla2_infer_in(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), _dtype_code(q), B, H, L, bq, _ptr(pq), _ptr(pk),
+        ws.data_ptr(), qpool.data_ptr(), kpool_t.data_ptr(), _stream(dev)), "sla2h_sla2_infer_in")
+    return ws, qpool, kpool_t
+
+
+def _sla2_infer_call(q, k, v, alpha, lut, bq, use_int8, qblock, eps_l, ws=None):
     """sla2_infer without the intermediates, as one native call."""
     _same(q, k, v)
     B, H, L, D = q.shape
@@ -950,13 +969,15 @@ def _sla2_infer_call(q, k, v, alpha, lut, bq, use_int8, qblock, eps_l):
         raise ValueError(f"lut: expected (B, H, {mq}, T), got {tuple(lut.shape)}")
     alpha = _alpha_rows(alpha, H, mq, dev)
     T, lib = lut.shape[-1], _lib.load()
-    use_int8 = bool(use_int8)
-    ws = _scratch(lib.sla2h_sla2_infer_workspace_bytes(B, H, L, bq, T, use_int8), dev)
+    use_int8, quantised = bool(use_int8), ws is not None
+    if not quantised:
+        ws = _scratch(lib.sla2h_sla2_infer_workspace_bytes(B, H, L, bq, T, use_int8), dev)
     o = torch.empty_like(q)
     _lib.check(lib.sla2h_sla2_infer(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), alpha.data_ptr(), alpha.stride(0),
         lut.data_ptr(), _dtype_code(q), B, H, L, bq, T, use_int8, bq if qblock is None else qblock,
-        D ** -0.5, float(eps_l), ws.data_ptr(), o.data_ptr(), _stream(dev)), "sla2h_sla2_infer")
+        quantised, D ** -0.5, float(eps_l), ws.data_ptr(), o.data_ptr(), _stream(dev)),
+        "sla2h_sla2_infer")
     return o
 
 

@@ -98,8 +98,16 @@ class SLA2(nn.Module):
         training = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad
                                                 or v.requires_grad)
         qh, kh, vh = (t.to(self.dtype).contiguous() for t in (q, k, v))
-        # the router scores the inputs in their own dtype (reference core.py:88)
-        lut, topk = self.router.route(q, k, self.topk)
+        # the router scores the inputs in their own dtype (reference core.py:88);
+        # where that is the op's, their pooled blocks come with the INT8 operands
+        ws = None
+        if (self.use_int8 and not self.fused and not training and D == ops.E_TILE
+                and q.dtype == k.dtype == self.dtype and q.shape == k.shape == v.shape
+                and qh.is_cuda and type(self.router) is Router
+                and "route" not in self.router.__dict__):
+            lut, topk, ws = self.router.route_quantised(qh, kh, vh, self.topk)
+        else:
+            lut, topk = self.router.route(q, k, self.topk)
         alpha_logit = self._get_alpha(H, -(-L // self.bq), q.device)
         if training:
             o = _SLA2Function.apply(qh, kh, vh, alpha_logit, lut, self.bq, self.use_int8)
@@ -111,7 +119,7 @@ class SLA2(nn.Module):
                 o = ops.sla2_infer_fused(qh, kh, vh, a.mean(0), lut, self.bq,
                                          use_int8=self.use_int8, block_m=self.block_m)
             else:
-                o = ops.sla2_infer(qh, kh, vh, a, lut, self.bq, use_int8=self.use_int8)
+                o = ops.sla2_infer(qh, kh, vh, a, lut, self.bq, use_int8=self.use_int8, ws=ws)
         if return_sparsity:
             return o.to(out_dtype), 1.0 - topk / -(-L // self.bk)
         return o.to(out_dtype)

@@ -78,6 +78,16 @@ class Router(nn.Module):
             return ops.route_1d(self._pool_input(q), self._pool_input(k), k_frac, self.bq,
                                 self.bk, pq, pk)
 
+    def route_quantised(self, qh, kh, vh, k_frac):
+        """route of 16-bit qh, kh with the inference op's INT8 operands made in the
+        same pass -> (lut, T, workspace for ops.sla2_infer)."""
+        pq = self.proj_q.weight if self.learnable else None
+        pk = self.proj_k.weight if self.learnable else None
+        with torch.no_grad():
+            ws, qpool, kpool_t = ops.sla2_infer_in(qh, kh, vh, self.bq, pq, pk)
+            T = ops.topk_count(k_frac, kpool_t.shape[-1])
+            return ops.route_topk(qpool, kpool_t, T, qh.shape[-1] ** -0.5), T, ws
+
     def forward(self, q, k, k_frac, soft=False, need_mask=True):
         """Returns (mask, lut, topk, pc): mask (B,H,Mb,Nb) int8 hard mask (the soft
         mask when soft=True), lut (B,H,Mb,topk) int32, pc the block scores."""

@@ -803,8 +803,18 @@ int sla2h_train_in(const void* const* x, const int64_t* strides, int dtype, cons
 size_t sla2h_sla2_infer_workspace_bytes(int B, int H, int64_t L, int bq, int T, int int8);
 int sla2h_sla2_infer(const void* q, const void* k, const void* v, const float* alpha,
                      int alpha_stride, const int32_t* lut, int dtype, int B, int H, int64_t L,
-                     int bq, int T, int int8, int qblock, float scale, float eps_l,
+                     int bq, int T, int int8, int qblock, int quantised, float scale, float eps_l,
                      void* workspace, void* o, void* stream);
+
+/*
+ * Its INT8 operands (sla2h_quantize per bq rows of q and 64 of k, sla2h_quantize_v8f)
+ * in the workspace (of int8 = 1; then quantised = 1, qblock = bq), and the
+ * router's pooled blocks qpool (B,H,ceil(L/bq),64) and kpool_t (B,H,64,Nb)
+ * (sla2h_pool_qk), in one pass over q, k, v.
+ */
+int sla2h_sla2_infer_in(const void* q, const void* k, const void* v, int dtype, int B, int H,
+                        int64_t L, int bq, const float* proj_q, const float* proj_k,
+                        void* workspace, float* qpool, float* kpool_t, void* stream);
 
 #ifdef __cplusplus
 }

@@ -288,3 +288,34 @@ def test_sla2_infer_edge_shapes(L, topk, bq, int8):
           flush=True)
     assert torch.isfinite(got).all()
     assert max_abs(got, ref["o"]) < TOL_MAX and rel_l2(got, ref["o"]) < TOL_REL
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,L", [(1, 1, 40), (2, 3, 583), (1, 2, 1024)])
+@pytest.mark.parametrize("bq", [64, 128, 256])
+def test_infer_in_matches_the_separate_passes(dt, B, H, L, bq):
+    """The inference operands in one pass (INT8 q per bq rows, k, v fragments, pooled
+    and projected blocks) against the quantisers and pool_qk: the pooled blocks
+    equal to the bit, and the op's output from the one-pass operands equal to
+    the one that quantises by itself."""
+    from imfvideo_amd import ops
+    print("[case] infer_in", dt, B, H, L, bq, flush=True)
+    g = torch.Generator().manual_seed(L + bq)
+    q, k, v = (torch.randn(B, H, L, 64, generator=g).to(dt).cuda() for _ in range(3))
+    pq, pk = (torch.randn(64, 64, generator=g).cuda() for _ in range(2))
+    nb, mq = -(-L // 64), -(-L // bq)
+    ws, qpool, kpool_t = ops.sla2_infer_in(q, k, v, bq, pq, pk)
+    wq, wk = ops.pool_qk(q, k, bq, nb, pq, pk)
+    assert torch.equal(qpool, wq) and torch.equal(kpool_t, wk)
+    off = 0
+    v8f, vs = ops.quantize_v8f(v)
+    (q8, qs), (k8, ks) = ops.quantize(q, bq), ops.quantize(k)
+    room = {"qs": 2 * B * H * nb * 4}  # the q scales' buffer holds 32-row blocks
+    for name, t in (("q8", q8), ("k8", k8), ("v8f", v8f), ("qs", qs), ("ks", ks), ("vs", vs)):
+        n = t.numel() * t.element_size()
+        assert torch.equal(ws[off:off + n].view(t.dtype).view(t.shape), t), name
+        off += -(-room.get(name, n) // 256) * 256
+    T = max(1, nb // 4)
+    lut = ops.route_topk(qpool, kpool_t, T, 0.125)
+    a = torch.rand(H, mq, generator=g).cuda()
+    assert torch.equal(ops.sla2_infer(q, k, v, a, lut, bq, ws=ws), ops.sla2_infer(q, k, v, a, lut, bq))
