@@ -199,15 +199,6 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(PrepArgs a) {
     a.Pz[((int64_t)bh * a.Nb + blk) * kT + tid] = (zp[0][tid] + zp[1][tid]) + (zp[2][tid] + zp[3][tid]);
 }
 
-// gfx950 transposing LDS read (ds_read_b64_tr_b16): within each group of 16
-// lanes, lane j receives element j % 4 of the 8 bytes addressed by lanes
-// j / 4, 4 + j / 4, 8 + j / 4 and 12 + j / 4 of its group, in that order.
-__device__ inline u32x2 lds_read_tr16(const void* p) {
-  typedef short v4s __attribute__((ext_vector_type(4)));
-  const v4s v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)p);
-  return __builtin_bit_cast(u32x2, v);
-}
-
 // ---------------------------------------------------------------------------
 // dq: one 64-row query block per workgroup; wave w owns keys 16w..16w+15 of
 // every tile of the augmented LUT and all 64 queries.  Per tile and query

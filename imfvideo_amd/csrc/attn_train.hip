@@ -555,7 +555,11 @@ __global__ __launch_bounds__(256, 2) void sparse_fwd16_kernel(Fwd16Args a) {
 // The complement record holds sum over the tiles NOT in lut_aug of
 // phi(K_j)^T V_j; H_i = record + (htot16 - htot) with htot = sum over all tiles
 // (the same sum, in another fp32 order).  Wave w owns queries 16w..16w+15;
-// lane (g, r) holds query r, output channels 16 ct + 4g + i.
+// lane (g, r) holds query r, output channels 16 g .. + 15.  HBM-bound (49 KB per
+// block: record, phi(q), o_s, o, o_l).  With all loads issued first, H_i staged
+// row-major (16-byte LDS writes, transposing reads) and 16-byte row accesses:
+// 16 heads x 468 blocks 112 -> 73 us (5.0 TB/s); before, H_i went to LDS
+// transposed by 2-byte writes and phi(q) and o_s were loaded where used.
 constexpr int kRecH = 0, kRecZ = 32768, kRecBytes = 33280;
 
 // INFER: the inference law of _lin_fwd3 (models/sla2_vendor/kernel_linear.py:
@@ -569,45 +573,59 @@ __global__ __launch_bounds__(256) void linear_mix_qat_kernel(
     const float* __restrict__ Hall, const uint16_t* __restrict__ o_s,
     const float* __restrict__ alpha, int alpha_stride, int64_t L, int Mq, int qshift, int H,
     float eps_l, uint16_t* __restrict__ o, uint16_t* __restrict__ o_l, float* __restrict__ den_out) {
-  __shared__ __align__(16) uint16_t hT[kT][kT + 8];  // [value channel][key channel]
+  __shared__ __align__(16) uint16_t hs[kT][kT + 8];  // H_i [key channel d][value channel]
   __shared__ float zs[kT];
 
   const int m = blockIdx.x, bh = blockIdx.y, h = bh % H;
   const int mq = m >> qshift;  // record and alpha of this 64-row block's query block
   const int tid = threadIdx.x;
-  const unsigned char* rec = comp + ((int64_t)bh * Mq + mq) * kRecBytes;
-  {
-    const int d = tid >> 2, v0 = (tid & 3) * 16;
-    const f32x4* hr = reinterpret_cast<const f32x4*>(rec + kRecH) + (d * kT + v0) / 4;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const f32x4 x = hr[c];
-      if (INFER) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) hT[v0 + 4 * c + i][d] = T16::from_f32(x[i]);
-      } else {
-        const f32x4 t = reinterpret_cast<const f32x4*>(Hall + (int64_t)bh * kT * kT + d * kT + v0)[c];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float t16 = T16::to_f32(T16::from_f32(t[i]));
-          hT[v0 + 4 * c + i][d] = T16::from_f32(x[i] + (t16 - t[i]));
-        }
-      }
-    }
-    if (tid < kT) zs[tid] = reinterpret_cast<const float*>(rec + kRecZ)[tid];
-  }
-  __syncthreads();
-
   const int w = tid >> 6, l = tid & 63, r = l & 15, g = l >> 4;
+  const unsigned char* rec = comp + ((int64_t)bh * Mq + mq) * kRecBytes;
   const int64_t qrow = (int64_t)m * kT + 16 * w + r;
   const bool qok = qrow < L;
   const int64_t rowoff = ((int64_t)bh * L + qrow) * kT;
-  u32x4 qb[2];
+  const int d = tid >> 2, v0 = (tid & 3) * 16;
+
+  // every load of the block up front
+  f32x4 x[4], t[4];
+  u32x4 qb[2], sv[2];  // phi(q) channels 32 ks + 8 g ..; o_s channels 16 g ..
+#pragma unroll
+  for (int c = 0; c < 4; ++c) x[c] = reinterpret_cast<const f32x4*>(rec + kRecH)[(d * kT + v0) / 4 + c];
+  if (!INFER) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      t[c] = reinterpret_cast<const f32x4*>(Hall + (int64_t)bh * kT * kT + d * kT + v0)[c];
+  }
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    qb[k] = qok ? *reinterpret_cast<const u32x4*>(qphi + rowoff + 32 * k + 8 * g)
+                : u32x4{0, 0, 0, 0};
+    sv[k] = qok ? *reinterpret_cast<const u32x4*>(o_s + rowoff + 16 * g + 8 * k)
+                : u32x4{0, 0, 0, 0};
+  }
+  if (tid < kT) zs[tid] = reinterpret_cast<const float*>(rec + kRecZ)[tid];
+  const float af = alpha[(int64_t)h * alpha_stride + mq];
+
+#pragma unroll
+  for (int c = 0; c < 4; c += 2) {
+    u32x4 hw;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      float y[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        y[i] = INFER ? x[c + k][i]
+                     : x[c + k][i] + (T16::to_f32(T16::from_f32(t[c + k][i])) - t[c + k][i]);
+      hw[2 * k] = pack_pair<T16>(y[0], y[1]);
+      hw[2 * k + 1] = pack_pair<T16>(y[2], y[3]);
+    }
+    *reinterpret_cast<u32x4*>(&hs[d][v0 + 4 * c]) = hw;
+  }
+  __syncthreads();
+
   float dn = 0.f;
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) {
-    qb[ks] = qok ? *reinterpret_cast<const u32x4*>(qphi + rowoff + 32 * ks + 8 * g)
-                 : u32x4{0, 0, 0, 0};
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       dn += T16::to_f32((uint16_t)(qb[ks][e] & 0xffff)) * zs[32 * ks + 8 * g + 2 * e];
@@ -617,43 +635,53 @@ __global__ __launch_bounds__(256) void linear_mix_qat_kernel(
   dn = sum_over_groups(dn);
   dn = dn >= 0.f ? dn + eps_l : dn - eps_l;
   const float rdn = 1.f / dn;
-  const float af = alpha[(int64_t)h * alpha_stride + mq];
   const float a16 = INFER ? af : T16::to_f32(T16::from_f32(af));
   const float b16 = INFER ? 1.f - af : T16::to_f32(T16::from_f32(1.f - a16));
+  // Product ct: output row 4 g + i is value channel 16 g + 4 ct + i, so that a lane
+  // ends up with 16 consecutive channels of its query.  The A operand (H^T rows
+  // of those channels) is read transposed: lane (g, r) addresses row 32 ks + 8 g +
+  // r / 4 (and + 4), channels 16 (r % 4) + 4 ct .. + 3.
+  uint32_t ow[8], lw[8];
 #pragma unroll
   for (int ct = 0; ct < 4; ++ct) {
     f32x4 num = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      const u32x4 av = *reinterpret_cast<const u32x4*>(&hT[16 * ct + r][32 * ks + 8 * g]);
-      num = mfma_16x16x32<T16>(av, qb[ks], num);
+      const uint16_t* src = &hs[32 * ks + 8 * g + (r >> 2)][16 * (r & 3) + 4 * ct];
+      const u32x2 lo = lds_read_tr16(src), hi = lds_read_tr16(src + 4 * (kT + 8));
+      num = mfma_16x16x32<T16>(u32x4{lo.x, lo.y, hi.x, hi.y}, qb[ks], num);
     }
-    if (qok) {
-      const int64_t oo = rowoff + 16 * ct + 4 * g;
-      const uint2 sv = *reinterpret_cast<const uint2*>(o_s + oo);
-      const uint32_t sw[2] = {sv.x, sv.y};
-      float ol[4], ov[4];
+    float ol[4], ov[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float os16 = T16::to_f32((uint16_t)(sw[i >> 1] >> (16 * (i & 1))));
-        if (INFER) {
-          ol[i] = num[i] * rdn;
-          ov[i] = a16 * os16 + b16 * ol[i];
-        } else {
-          ol[i] = T16::to_f32(T16::from_f32(num[i] * rdn));
-          const float x = T16::to_f32(T16::from_f32(a16 * os16));
-          const float y = T16::to_f32(T16::from_f32(b16 * ol[i]));
-          ov[i] = x + y;
-        }
+    for (int i = 0; i < 4; ++i) {
+      const int e = 4 * ct + i;  // channel 16 g + e
+      const float os16 = T16::to_f32((uint16_t)(sv[e >> 3][(e >> 1) & 3] >> (16 * (e & 1))));
+      if (INFER) {
+        ol[i] = num[i] * rdn;
+        ov[i] = a16 * os16 + b16 * ol[i];
+      } else {
+        ol[i] = T16::to_f32(T16::from_f32(num[i] * rdn));
+        const float xx = T16::to_f32(T16::from_f32(a16 * os16));
+        const float yy = T16::to_f32(T16::from_f32(b16 * ol[i]));
+        ov[i] = xx + yy;
       }
-      *reinterpret_cast<uint2*>(o + oo) =
-          make_uint2(pack_pair<T16>(ov[0], ov[1]), pack_pair<T16>(ov[2], ov[3]));
-      if (o_l != nullptr)
-        *reinterpret_cast<uint2*>(o_l + oo) =
-            make_uint2(pack_pair<T16>(ol[0], ol[1]), pack_pair<T16>(ol[2], ol[3]));
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      ow[2 * ct + k] = pack_pair<T16>(ov[2 * k], ov[2 * k + 1]);
+      lw[2 * ct + k] = pack_pair<T16>(ol[2 * k], ol[2 * k + 1]);
     }
   }
-  if (qok && g == 0 && den_out != nullptr) den_out[(int64_t)bh * L + qrow] = dn;
+  if (!qok) return;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int64_t oo = rowoff + 16 * g + 8 * k;
+    *reinterpret_cast<u32x4*>(o + oo) = u32x4{ow[4 * k], ow[4 * k + 1], ow[4 * k + 2], ow[4 * k + 3]};
+    if (o_l != nullptr)
+      *reinterpret_cast<u32x4*>(o_l + oo) =
+          u32x4{lw[4 * k], lw[4 * k + 1], lw[4 * k + 2], lw[4 * k + 3]};
+  }
+  if (g == 0 && den_out != nullptr) den_out[(int64_t)bh * L + qrow] = dn;
 }
 
 // Score form of the same linear branch (_lin_fwd2 with SCORE_FORM,

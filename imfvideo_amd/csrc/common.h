@@ -170,6 +170,15 @@ __device__ inline u32x2 buf_load8(__amdgpu_buffer_rsrc_t rs, int voff, int soff)
   return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, voff, soff, 0));
 }
 
+// gfx950 transposing LDS read (ds_read_b64_tr_b16): within each group of 16
+// lanes, lane j receives element j % 4 of the 8 bytes addressed by lanes
+// j / 4, 4 + j / 4, 8 + j / 4 and 12 + j / 4 of its group, in that order.
+__device__ inline u32x2 lds_read_tr16(const void* p) {
+  typedef short v4s __attribute__((ext_vector_type(4)));
+  const v4s v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)p);
+  return __builtin_bit_cast(u32x2, v);
+}
+
 // 2^x on the hardware exp unit (v_exp_f32); inputs here are <= 0 or -inf.
 __device__ inline float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
