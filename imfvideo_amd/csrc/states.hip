@@ -32,17 +32,26 @@ constexpr size_t kRecBytes = 2 * 16384 + 2 * 256;
 // half vanishes.  RH (the inference states of _hblocks): H is stored
 // rounded to the 16-bit type, as the reference keeps HALL in V's dtype.  The
 // value operand tiles are written when vt is not NULL.
+//
+// HBM-bound at scale, by the LDS pipe and latency below.  Rows go to LDS as
+// they are (16-byte writes) and the operands, the fragment-ordered value tile
+// included, come out transposed (ds_read_b64_tr_b16); the column sums exchange
+// 15 values per lane; H is computed as H^T for 16-byte stores.  Against 2-byte
+// transposed LDS writes (4-way bank conflicts), 64 cross-lane exchanges per
+// sum and 4-byte stores, us: 8 heads x 468 tiles with tangent 68.6 -> 62.0 (370
+// MB, 6.0 TB/s), primal 35.1 -> 28.7, training 16 x 468 60.5 -> 44.4, 4 x 64 with
+// tangent 13.1 -> 10.2.
 template <typename T16, bool TAN, bool ROUND = false, bool RH = false>
 __global__ __launch_bounds__(256) void linear_states_kernel(
     const uint16_t* __restrict__ K, const uint16_t* __restrict__ dK,
     const uint16_t* __restrict__ V, const uint16_t* __restrict__ dV, int64_t L, int Np, int Nb,
     float* __restrict__ Hb, float* __restrict__ dHb, float* __restrict__ zb,
     float* __restrict__ dzb, uint16_t* __restrict__ vt, uint16_t* __restrict__ kt) {
-  // phi^T, then (tangent, second phase) dphi^T: one buffer keeps the LDS
-  // footprint at four workgroups per CU
-  __shared__ __align__(16) uint16_t phiT[2][kT][kLds];   // [hi/lo][d][r]
-  __shared__ __align__(16) uint16_t vT[kT][kLds];        // [c][r]
-  __shared__ __align__(16) uint16_t dvT[kT][kLds];
+  // phi rows (hi, lo), then (tangent, second phase) dphi rows: one buffer keeps
+  // the LDS footprint at four workgroups per CU
+  __shared__ __align__(16) uint16_t ph[2][kT][kLds];   // [hi/lo][r][d]
+  __shared__ __align__(16) uint16_t vs[kT][kLds];      // [r][c]
+  __shared__ __align__(16) uint16_t dvs[TAN ? kT : 1][kLds];
   __shared__ float zred[2][4][kT];
 
   const int tid = threadIdx.x;
@@ -50,63 +59,96 @@ __global__ __launch_bounds__(256) void linear_states_kernel(
   const int bh = blockIdx.y;
   const int r = tid >> 2;
   const int c0 = (tid & 3) * 16;
+  const int w = tid >> 6, l = tid & 63, lr = l & 15, g = l >> 4;
   const int64_t row = (int64_t)n * kT + r;
   const bool valid = row < L;
   const int64_t off = ((int64_t)bh * L + row) * kT + c0;
 
-  auto load16 = [&](const uint16_t* src, uint16_t* dst) {
-    if (valid) {
-      const uint4* s = reinterpret_cast<const uint4*>(src + off);
-      uint4 u0 = s[0], u1 = s[1];
-      uint32_t w[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
+  struct Row16 {  // 16 consecutive 16-bit values of one row
+    u32x4 u[2];
+  };
+  auto load16 = [&](const uint16_t* src) {
+    Row16 x;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        dst[2 * i] = (uint16_t)(w[i] & 0xffff);
-        dst[2 * i + 1] = (uint16_t)(w[i] >> 16);
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) dst[i] = 0;
-    }
+    for (int k = 0; k < 2; ++k)
+      x.u[k] = valid ? reinterpret_cast<const u32x4*>(src + off)[k] : u32x4{0, 0, 0, 0};
+    return x;
+  };
+  auto store16 = [&](uint16_t* dst, const Row16& x) {
+    reinterpret_cast<u32x4*>(dst)[0] = x.u[0];
+    reinterpret_cast<u32x4*>(dst)[1] = x.u[1];
+  };
+  auto val = [](const Row16& x, int i) {
+    return T16::to_f32((uint16_t)(x.u[i >> 3][(i >> 1) & 3] >> (16 * (i & 1))));
   };
 
-  uint16_t vb[16], dvb[16];
-  load16(V, vb);
-  if (TAN) load16(dV, dvb);
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    vT[c0 + i][r] = vb[i];
-    if (TAN) dvT[c0 + i][r] = dvb[i];
-  }
-
   const bool states = n < Np;  // uniform over the workgroup
-  uint16_t kb[16], dkb[16];
+  const Row16 vb = load16(V);
+  Row16 dvb, kb, dkb;
+  if (TAN) dvb = load16(dV);
   if (states || TAN) {
-    load16(K, kb);
-    if (TAN) load16(dK, dkb);
+    kb = load16(K);
+    if (TAN) dkb = load16(dK);
   }
-  if (TAN) {  // key-operand fragments of this thread's 16 columns: 2 x (K, dK) chunks
+  store16(&vs[r][c0], vb);
+  if (TAN) {
+    store16(&dvs[r][c0], dvb);
+    // key-operand fragments of this thread's 16 columns: 2 x (K, dK) chunks
     const int kw = r >> 4, rr = r & 15, ksd = c0 >> 5, g0 = (c0 & 31) >> 3;
     unsigned char* base = reinterpret_cast<unsigned char*>(kt) + ((int64_t)bh * Nb + n) * 16384;
 #pragma unroll
     for (int h2 = 0; h2 < 2; ++h2) {
       const int lane = (g0 + h2) * 16 + rr;
-      uint4 kv, dkv;
-      kv.x = pack2(kb[8 * h2 + 0], kb[8 * h2 + 1]); kv.y = pack2(kb[8 * h2 + 2], kb[8 * h2 + 3]);
-      kv.z = pack2(kb[8 * h2 + 4], kb[8 * h2 + 5]); kv.w = pack2(kb[8 * h2 + 6], kb[8 * h2 + 7]);
-      dkv.x = pack2(dkb[8 * h2 + 0], dkb[8 * h2 + 1]); dkv.y = pack2(dkb[8 * h2 + 2], dkb[8 * h2 + 3]);
-      dkv.z = pack2(dkb[8 * h2 + 4], dkb[8 * h2 + 5]); dkv.w = pack2(dkb[8 * h2 + 6], dkb[8 * h2 + 7]);
-      *reinterpret_cast<uint4*>(base + ((kw * 4 + ksd) * 64 + lane) * 16) = kv;
-      *reinterpret_cast<uint4*>(base + ((kw * 4 + ksd + 2) * 64 + lane) * 16) = dkv;
+      *reinterpret_cast<u32x4*>(base + ((kw * 4 + ksd) * 64 + lane) * 16) = kb.u[h2];
+      *reinterpret_cast<u32x4*>(base + ((kw * 4 + ksd + 2) * 64 + lane) * 16) = dkb.u[h2];
     }
   }
+  // x rows as hi + lo halves of the 16-bit type
+  auto store_split = [&](const float (&x)[16]) {
+    Row16 hi, lo;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t hw = pack_pair<T16>(x[2 * e], x[2 * e + 1]);
+      hi.u[e >> 2][e & 3] = hw;
+      lo.u[e >> 2][e & 3] = pack_pair<T16>(x[2 * e] - T16::to_f32((uint16_t)(hw & 0xffff)),
+                                           x[2 * e + 1] - T16::to_f32((uint16_t)(hw >> 16)));
+    }
+    store16(&ph[0][r][c0], hi);
+    if (!ROUND) store16(&ph[1][r][c0], lo);
+  };
+  // Column sums over the wave's 16 rows: a lane holds 16 columns of one row, so
+  // each step halves both the rows to add and the columns a lane keeps (15
+  // exchanges instead of 64), leaving one column per lane: c0 + 8 b5 + 4 b4 + 2
+  // b3 + b2 of its lane bits.
+  auto col_sum = [&](const float (&x)[16]) {
+    float a8[8], a4[4], a2[2];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const auto s = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, x[i]),
+                                                      __builtin_bit_cast(unsigned, x[i + 8]), false, false);
+      a8[i] = __builtin_bit_cast(float, (unsigned)s[0]) + __builtin_bit_cast(float, (unsigned)s[1]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const auto s = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a8[i]),
+                                                      __builtin_bit_cast(unsigned, a8[i + 4]), false, false);
+      a4[i] = __builtin_bit_cast(float, (unsigned)s[0]) + __builtin_bit_cast(float, (unsigned)s[1]);
+    }
+    const bool b3 = (l & 8) != 0, b2 = (l & 4) != 0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      a2[i] = (b3 ? a4[i + 2] : a4[i]) + __shfl_xor(b3 ? a4[i] : a4[i + 2], 8, 64);
+    return (b2 ? a2[1] : a2[0]) + __shfl_xor(b2 ? a2[0] : a2[1], 4, 64);
+  };
+  const int zcol = c0 + ((l >> 5) & 1) * 8 + ((l >> 4) & 1) * 4 + ((l >> 3) & 1) * 2 + ((l >> 2) & 1);
+
   float dphi[16];
   if (states) {
     float x[16], phi[16];
     float mx = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      x[i] = T16::to_f32(kb[i]);
+      x[i] = val(kb, i);
       mx = fmaxf(mx, x[i]);
     }
     mx = fmaxf(mx, __shfl_xor(mx, 1, 64));
@@ -124,11 +166,11 @@ __global__ __launch_bounds__(256) void linear_states_kernel(
     if (TAN) {
       float dot = 0.f;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) dot += phi[i] * T16::to_f32(dkb[i]);
+      for (int i = 0; i < 16; ++i) dot += phi[i] * val(dkb, i);
       dot += __shfl_xor(dot, 1, 64);
       dot += __shfl_xor(dot, 2, 64);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) dphi[i] = phi[i] * (T16::to_f32(dkb[i]) - dot);
+      for (int i = 0; i < 16; ++i) dphi[i] = phi[i] * (val(dkb, i) - dot);
     }
     if (!valid) {  // padding rows of a ragged last tile stay inert
 #pragma unroll
@@ -138,47 +180,35 @@ __global__ __launch_bounds__(256) void linear_states_kernel(
 #pragma unroll
       for (int i = 0; i < 16; ++i) phi[i] = T16::to_f32(T16::from_f32(phi[i]));
     }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const uint16_t hi = T16::from_f32(phi[i]);
-      phiT[0][c0 + i][r] = hi;
-      phiT[1][c0 + i][r] = T16::from_f32(phi[i] - T16::to_f32(hi));
-    }
-    // column sums over the 64 rows: 16 rows per wave by shuffles, then LDS
-    const int w = tid >> 6;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      float s = phi[i];
-      float ds = TAN ? dphi[i] : 0.f;
-#pragma unroll
-      for (int m = 4; m <= 32; m <<= 1) {
-        s += __shfl_xor(s, m, 64);
-        if (TAN) ds += __shfl_xor(ds, m, 64);
-      }
-      if ((tid & 63) < 4) {
-        zred[0][w][c0 + i] = s;
-        if (TAN) zred[1][w][c0 + i] = ds;
-      }
-    }
+    store_split(phi);
+    zred[0][w][zcol] = col_sum(phi);
+    if (TAN) zred[1][w][zcol] = col_sum(dphi);
   }
   __syncthreads();
 
-  // value-operand tile in fragment order: thread -> (ct, w, r), 4 lane groups g
+  // Four consecutive rows 16 vw + 4 g .. + 3 of one column 16 ct + lr, read
+  // transposed: half a K = 32 operand (rows 4 g .. and 16 + 4 g .. of a 32-row
+  // step are the K slots of lane group g, in both operands).
+  auto quad = [&](const uint16_t (*m)[kLds], int ct, int vw) {
+    return lds_read_tr16(&m[16 * vw + 4 * g + (lr >> 2)][16 * ct + 4 * (lr & 3)]);
+  };
+  auto frag = [&](const uint16_t (*m)[kLds], int ct, int ks) {
+    const u32x2 lo = quad(m, ct, 2 * ks), hi = quad(m, ct, 2 * ks + 1);
+    return u32x4{lo.x, lo.y, hi.x, hi.y};
+  };
+
+  // value-operand tile in fragment order: wave w writes column tile w
   if (vt != nullptr) {
-    const int ct = tid >> 6, vw = (tid >> 4) & 3, rr = tid & 15;
-    const int c = 16 * ct + rr;
     unsigned char* base = reinterpret_cast<unsigned char*>(vt) +
                           ((int64_t)bh * Nb + n) * (TAN ? 16384 : 8192);
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int lane = g * 16 + rr;
-      const int k0 = 16 * vw + 4 * g;
-      const uint2 a = *reinterpret_cast<const uint2*>(&vT[c][k0]);
+    for (int vw = 0; vw < 4; ++vw) {
+      const u32x2 a = quad(vs, w, vw);
       if (TAN) {
-        const uint2 b = *reinterpret_cast<const uint2*>(&dvT[c][k0]);
-        *reinterpret_cast<uint4*>(base + ((ct * 4 + vw) * 64 + lane) * 16) = make_uint4(a.x, a.y, b.x, b.y);
+        const u32x2 b = quad(dvs, w, vw);
+        *reinterpret_cast<u32x4*>(base + ((w * 4 + vw) * 64 + l) * 16) = u32x4{a.x, a.y, b.x, b.y};
       } else {
-        *reinterpret_cast<uint2*>(base + ((ct * 4 + vw) * 64 + lane) * 8) = a;
+        *reinterpret_cast<u32x2*>(base + ((w * 4 + vw) * 64 + l) * 8) = a;
       }
     }
   }
@@ -190,64 +220,58 @@ __global__ __launch_bounds__(256) void linear_states_kernel(
     if (TAN) dzb[zo] = (zred[1][0][tid] + zred[1][1][tid]) + (zred[1][2][tid] + zred[1][3][tid]);
   }
 
-  // Hb[d][v] = sum_r phi[r][d] V[r][v]: wave w owns d rows 16w..16w+15.
-  const int w = tid >> 6, l = tid & 63, lr = l & 15, g = l >> 4;
-  const int drow = 16 * w + lr;
+  // Hb[d][v] = sum_r phi[r][d] V[r][v] as H^T = V^T phi: wave w owns d 16w ..
+  // 16w + 15, lane (g, lr) holds v = 16 ct + 4 g .. + 3 of d = 16w + lr (16-byte
+  // stores).
   f32x4 acc[4], dacc[4];
 #pragma unroll
-  for (int vt_ = 0; vt_ < 4; ++vt_) {
-    acc[vt_] = f32x4{0.f, 0.f, 0.f, 0.f};
-    dacc[vt_] = acc[vt_];
-  }
+  for (int ct = 0; ct < 4; ++ct) acc[ct] = dacc[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
   // phase 1: H = phi^T V and the phi^T dV half of dH
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) {
-    const int k0 = 32 * ks + 8 * g;
-    const u32x4 ah = *reinterpret_cast<const u32x4*>(&phiT[0][drow][k0]);
-    const u32x4 al = *reinterpret_cast<const u32x4*>(&phiT[1][drow][k0]);
+    const u32x4 bh_ = frag(ph[0], w, ks);
+    u32x4 bl = bh_;
+    if (!ROUND) bl = frag(ph[1], w, ks);
 #pragma unroll
-    for (int vt_ = 0; vt_ < 4; ++vt_) {
-      const u32x4 bv = *reinterpret_cast<const u32x4*>(&vT[16 * vt_ + lr][k0]);
-      acc[vt_] = mfma_16x16x32<T16>(ah, bv, acc[vt_]);
-      if (!ROUND) acc[vt_] = mfma_16x16x32<T16>(al, bv, acc[vt_]);
+    for (int ct = 0; ct < 4; ++ct) {
+      const u32x4 av = frag(vs, ct, ks);
+      acc[ct] = mfma_16x16x32<T16>(av, bh_, acc[ct]);
+      if (!ROUND) acc[ct] = mfma_16x16x32<T16>(av, bl, acc[ct]);
       if (TAN) {
-        const u32x4 bdv = *reinterpret_cast<const u32x4*>(&dvT[16 * vt_ + lr][k0]);
-        dacc[vt_] = mfma_16x16x32<T16>(ah, bdv, dacc[vt_]);
-        dacc[vt_] = mfma_16x16x32<T16>(al, bdv, dacc[vt_]);
+        const u32x4 adv = frag(dvs, ct, ks);
+        dacc[ct] = mfma_16x16x32<T16>(adv, bh_, dacc[ct]);
+        dacc[ct] = mfma_16x16x32<T16>(adv, bl, dacc[ct]);
       }
     }
   }
-  if (TAN) {  // phase 2: dphi^T replaces phi^T; dH += dphi^T V
+  if (TAN) {  // phase 2: dphi replaces phi; dH += dphi^T V
     __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const uint16_t dhi = T16::from_f32(dphi[i]);
-      phiT[0][c0 + i][r] = dhi;
-      phiT[1][c0 + i][r] = T16::from_f32(dphi[i] - T16::to_f32(dhi));
-    }
+    store_split(dphi);
     __syncthreads();
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      const int k0 = 32 * ks + 8 * g;
-      const u32x4 dah = *reinterpret_cast<const u32x4*>(&phiT[0][drow][k0]);
-      const u32x4 dal = *reinterpret_cast<const u32x4*>(&phiT[1][drow][k0]);
+      const u32x4 bh_ = frag(ph[0], w, ks), bl = frag(ph[1], w, ks);
 #pragma unroll
-      for (int vt_ = 0; vt_ < 4; ++vt_) {
-        const u32x4 bv = *reinterpret_cast<const u32x4*>(&vT[16 * vt_ + lr][k0]);
-        dacc[vt_] = mfma_16x16x32<T16>(dah, bv, dacc[vt_]);
-        dacc[vt_] = mfma_16x16x32<T16>(dal, bv, dacc[vt_]);
+      for (int ct = 0; ct < 4; ++ct) {
+        const u32x4 av = frag(vs, ct, ks);
+        dacc[ct] = mfma_16x16x32<T16>(av, bh_, dacc[ct]);
+        dacc[ct] = mfma_16x16x32<T16>(av, bl, dacc[ct]);
       }
     }
   }
-  const int64_t hbase = ((int64_t)bh * Np + n) * kT * kT;
+  const int64_t hbase = ((int64_t)bh * Np + n) * kT * kT + (16 * w + lr) * kT + 4 * g;
 #pragma unroll
-  for (int vt_ = 0; vt_ < 4; ++vt_) {
+  for (int ct = 0; ct < 4; ++ct) {
+    f32x4 x = acc[ct];
+    if (RH) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int64_t o = hbase + (int64_t)(16 * w + 4 * g + i) * kT + 16 * vt_ + lr;
-      Hb[o] = RH ? T16::to_f32(T16::from_f32(acc[vt_][i])) : acc[vt_][i];
-      if (TAN) dHb[o] = dacc[vt_][i];
+      for (int i = 0; i < 4; ++i) {
+        const float e = x[i];
+        x[i] = T16::to_f32(T16::from_f32(e));
+      }
     }
+    *reinterpret_cast<f32x4*>(Hb + hbase + 16 * ct) = x;
+    if (TAN) *reinterpret_cast<f32x4*>(dHb + hbase + 16 * ct) = dacc[ct];
   }
 }
 
