@@ -112,7 +112,6 @@ __global__ __launch_bounds__(256, TAN ? 2 : 3) void fwd_jvp_kernel(FwdArgs a) {
   __shared__ __align__(16) float mbuf[4][8][64][4];
   // key tiles of this query block in visiting order: (tile id, key scale)
   __shared__ int2 tiles[kMaxTiles];
-  __shared__ int ragged_last;  // the partial key tile was moved to the end of the routed list
   __shared__ float wmax[2][4];  // per wave: max kb, max ks over the block's key tiles
   __shared__ int redo;          // a row of the static-shift pass came out below its range
 
@@ -126,7 +125,6 @@ __global__ __launch_bounds__(256, TAN ? 2 : 3) void fwd_jvp_kernel(FwdArgs a) {
   for (int kk = (int)(blockIdx.x >> 3); kk < a.per_xcd; kk += slots) {
     const int logical = (blockIdx.x & 7) * a.per_xcd + kk;
     if (logical >= a.nwork) break;  // uniform: the whole workgroup leaves
-    __syncthreads();  // the previous unit's LDS is free
     // integer division runs on the VALU: pin the (uniform) results to SGPRs so
     // that every pointer and buffer descriptor derived from them stays scalar
     const int bh = __builtin_amdgcn_readfirstlane(logical / a.Mb);
@@ -149,83 +147,80 @@ __global__ __launch_bounds__(256, TAN ? 2 : 3) void fwd_jvp_kernel(FwdArgs a) {
     const int64_t blk = (qkbase + q0) * kTa;
 
     // ---- query side: INT8 and 16-bit [dQ|Q] B operands staged once in LDS,
-    // wave w loading sub-tile w.
+    // wave w loading sub-tile w.  The loads of a unit (and its LUT row's, by wave
+    // 0) are issued before the barrier that frees the previous unit's LDS.
+    const int mq = m >> a.qshift;  // LUT row, alpha and record of this query block
+    const int32_t* lrow = a.lut + ((int64_t)bh * a.Mq + mq) * a.T;
+    const int J = a.T + a.n_tail;
+    const bool short_list = a.T <= 64;  // the routed list fits the lanes of wave 0
+    auto clamp_id = [&](int n) { return n < 0 ? 0 : (n >= a.Nb ? a.Nb - 1 : n); };
+    int nid = 0x7fffffff;  // wave 0, short list: this lane's routed tile
+    if (short_list && w == 0 && l < a.T) nid = clamp_id(lrow[l]);
     {
       const int64_t row = q0 + 16 * w + r;
       const bool ok = row < L;
       const int ro = (16 * w + r) * kTa;
-      if (!S16)
-        q8sh[w][l] = ok ? *reinterpret_cast<const i32x4*>(a.q8 + blk + ro + 16 * g)
-                        : i32x4{0, 0, 0, 0};
+      i32x4 v8 = i32x4{0, 0, 0, 0};
+      u32x4 v16[4];  // dQ in ks 0,1, Q in ks 2,3
+      if (!S16 && ok) v8 = *reinterpret_cast<const i32x4*>(a.q8 + blk + ro + 16 * g);
       if (TAN) {
 #pragma unroll
-        for (int part = 0; part < 2; ++part) {  // dQ in ks 0,1, Q in ks 2,3
-          const uint16_t* src = part ? a.q : a.dq;
+        for (int ks = 0; ks < 4; ++ks)
+          v16[ks] = ok ? *reinterpret_cast<const u32x4*>((ks < 2 ? a.dq : a.q) + blk + ro +
+                                                         32 * (ks & 1) + 8 * g)
+                       : u32x4{0, 0, 0, 0};
+      }
+      __syncthreads();  // the previous unit's LDS is free
+      if (!S16) q8sh[w][l] = v8;
+      if (TAN) {
 #pragma unroll
-          for (int ks = 0; ks < 2; ++ks) {
-            u32x4 v = ok ? *reinterpret_cast<const u32x4*>(src + blk + ro + 32 * ks + 8 * g)
-                         : u32x4{0, 0, 0, 0};
-            if (PRE) v = scale_bf16x8(v, a.scale);
-            qsh[w][ks + 2 * part][l] = v;
-          }
-        }
+        for (int ks = 0; ks < 4; ++ks)
+          qsh[w][ks][l] = PRE ? scale_bf16x8(v16[ks], a.scale) : v16[ks];
       }
     }
-    const int mq = m >> a.qshift;  // LUT row, alpha and record of this query block
-    const int32_t* lrow = a.lut + ((int64_t)bh * a.Mq + mq) * a.T;
-    const int J = a.T + a.n_tail;
-    for (int j = tid; j < J; j += 256) {
-      int n = j < a.T ? lrow[j] : a.Np + (j - a.T);
-      n = n < 0 ? 0 : (n >= a.Nb ? a.Nb - 1 : n);  // out-of-range ids are clamped
-      tiles[j].x = n;
-    }
-    __syncthreads();
-    // routed tiles in ascending id order (the prefix tails stay at the end)
-    sort_ids_ascending(
-        a.T, tid, [&](int i) { return tiles[i].x; }, [&](int i, int v) { tiles[i].x = v; },
-        reinterpret_cast<int*>(&mbuf[0][0][0][0]));
-    // A partial key tile (1-D blocks over a ragged L) can sit anywhere in a routed
-    // list: move it to the end, where the masked one-tile path handles it.
-    int Tu = a.T;
-    if (a.ragged >= 0) {
-      if (tid == 0) {
-        int found = 0;
-        for (int j = 0; j < a.T; ++j) {
-          if (tiles[j].x == a.ragged) {
-            const int2 t = tiles[j];
-            tiles[j] = tiles[a.T - 1];
-            tiles[a.T - 1] = t;
-            found = 1;
-            break;
-          }
-        }
-        ragged_last = found;
-      }
-      __syncthreads();
-      Tu = a.T - ragged_last;
-    }
-    // key scales of the tiles in visiting order; the barrier that publishes
-    // them comes after the first key loads are issued (their latencies overlap)
-    if (!S16) {
-      float kbm = 0.f, ksm = 0.f;
-      for (int j = tid; j < J; j += 256) {
-        const int64_t ti = (int64_t)bh * a.Nb + tiles[j].x;
+    // Visiting list: the routed tiles in ascending id order, each with its key
+    // scale, then the prefix tails; a partial key tile (1-D blocks over a ragged L)
+    // has the largest id, so it ends the routed list, where the masked one-tile
+    // path handles it.
+    float kbm = 0.f, ksm = 0.f;  // this lane's largest kb, ks
+    auto put = [&](int j, int n) {
+      int ys = 0;
+      if (!S16) {
+        const int64_t ti = (int64_t)bh * a.Nb + n;
         const float ksj = a.ks[ti];
-        tiles[j].y = __builtin_bit_cast(int, ksj);
+        ys = __builtin_bit_cast(int, ksj);
         ksm = fmaxf(ksm, ksj);
         if (a.kb != nullptr) kbm = fmaxf(kbm, a.kb[ti]);
       }
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) {
-        kbm = fmaxf(kbm, __shfl_xor(kbm, o, 64));
-        ksm = fmaxf(ksm, __shfl_xor(ksm, o, 64));
+      tiles[j] = make_int2(n, ys);
+    };
+    if (short_list) {
+      if (w == 0) {
+        const int c = wave_rank(nid, l, a.T);
+        if (l < a.T) put(c, nid);
       }
+      for (int j = a.T + tid; j < J; j += 256) put(j, clamp_id(a.Np + (j - a.T)));
+    } else {
+      for (int j = tid; j < J; j += 256)
+        tiles[j].x = clamp_id(j < a.T ? lrow[j] : a.Np + (j - a.T));
+      __syncthreads();
+      sort_ids_ascending(
+          a.T, tid, [&](int i) { return tiles[i].x; }, [&](int i, int v) { tiles[i].x = v; },
+          reinterpret_cast<int*>(&mbuf[0][0][0][0]));
+      for (int j = tid; j < J; j += 256) put(j, tiles[j].x);
+    }
+    if (!S16) {
+      kbm = wave_max(kbm);
+      ksm = wave_max(ksm);
       if (l == 0) {
         wmax[0][w] = kbm;
         wmax[1][w] = ksm;
       }
       if (tid == 0) redo = 0;
     }
+    __syncthreads();  // operands, list, scales and block maxima are in LDS
+    int Tu = a.T;
+    if (a.ragged >= 0 && __builtin_amdgcn_readfirstlane(tiles[a.T - 1].x) == a.ragged) --Tu;
     const float sq = S16 ? 1.f : a.qs[(int64_t)bh * a.Nb + m];
     // log2-domain score factor of key tile j: (sq * sk_j) * scale * log2(e)
     auto tile_c = [&](int j) {
@@ -519,7 +514,6 @@ __global__ __launch_bounds__(256, TAN ? 2 : 3) void fwd_jvp_kernel(FwdArgs a) {
     // while the prefetch stays in flight.
     KeyRegs ka_, kb_;
     load_keys(0, 0, ka_);
-    __syncthreads();  // key scales in tiles[].y, block maxima in wmax
     // Per-block choice of the static shift (uniform): kb given, every score
     // factor c_j <= 2^-9; M_i = ||q8_i|| qs scale log2(e) max_j kb_j.
     bool exact = true;

@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/sla2h.h"
 
 namespace sla2h {
@@ -205,27 +207,50 @@ __device__ inline void wave_atomic_max(float* p, float v) {
   }
 }
 
+// Maximum over the 64 lanes, VALU only (DPP rotations within rows of 16, then the
+// row-swap permutes); every lane gets it.
+__device__ inline float wave_max(float v) {
+  auto ror = [](float x, auto n) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
+                                         0, __builtin_bit_cast(int, x), 0x120 + decltype(n)::value,
+                                         0xf, 0xf, false));
+  };
+  v = fmaxf(v, ror(v, std::integral_constant<int, 8>{}));
+  v = fmaxf(v, ror(v, std::integral_constant<int, 4>{}));
+  v = fmaxf(v, ror(v, std::integral_constant<int, 2>{}));
+  v = fmaxf(v, ror(v, std::integral_constant<int, 1>{}));
+  return max_over_groups(v);
+}
+
+// Ascending rank of lane l's id among the ids of lanes 0 .. n - 1 (n <= 64), ties by
+// lane: one scalar broadcast and compare per id, where a bitonic sort takes 21
+// dependent cross-lane exchanges.
+__device__ inline int wave_rank(int v, int l, int n) {
+  int c = 0;
+  for (int j = 0; j < n; j += 4) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int nj = __builtin_amdgcn_readlane(v, j + u);  // j + u <= 63
+      c += (j + u < n && (nj < v || (nj == v && j + u < l))) ? 1 : 0;
+    }
+  }
+  return c;
+}
+
 // Ascending sort of the n tile ids of a visiting list in LDS (element i read
 // with get(i), written with set(i, id)).  Workgroups that visit their tiles in
 // ascending order sweep the key tiles of a head together and share them in
-// the XCD's L2.  Up to 64 ids: a bitonic sort in the registers of wave 0
-// (threads 0..63); more: rank by counting into tmp (n ints of LDS), ties by
-// position.  Called by every thread of a 256-thread workgroup after the list
-// is complete in LDS (barrier included); ends with a barrier.
+// the XCD's L2.  Rank by counting: up to 64 ids in the registers of wave 0
+// (threads 0..63), more into tmp (n ints of LDS); ties by position.  Called by
+// every thread of a 256-thread workgroup after the list is complete in LDS
+// (barrier included); ends with a barrier.
 template <typename Get, typename Set>
 __device__ inline void sort_ids_ascending(int n, int tid, Get get, Set set, int* tmp) {
   if (n <= 64) {
     if (tid < 64) {
-      int v = tid < n ? get(tid) : 0x7fffffff;
-#pragma unroll
-      for (int k = 2; k <= 64; k <<= 1) {
-#pragma unroll
-        for (int jj = k >> 1; jj > 0; jj >>= 1) {
-          const int o = __shfl_xor(v, jj);
-          v = (((tid & jj) == 0) == ((tid & k) == 0)) ? min(v, o) : max(v, o);
-        }
-      }
-      if (tid < n) set(tid, v);
+      const int v = tid < n ? get(tid) : 0x7fffffff;
+      const int c = wave_rank(v, tid, n);
+      if (tid < n) set(c, v);
     }
   } else {
     for (int j = tid; j < n; j += 256) {
