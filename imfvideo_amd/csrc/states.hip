@@ -323,7 +323,8 @@ __global__ __launch_bounds__(256) void states_sum_kernel(const float* __restrict
 // (Mb x Np, 0/1) and S = [Hb | dHb | zb | dzb] (Np x 8320 columns, fp32).  S
 // is split into bf16 hi + lo halves (about 16 significant bits) and the
 // products accumulate in fp32 on MFMA; the mask is exact in bf16.  The H
-// columns run in comp_gemm_kernel, the z columns in comp_mask_kernel.
+// columns run in comp_gemm_kernel, the z columns in comp_mask_kernel (small
+// calls: all of it in comp_gemm_kernel, see kFusedMaskWords).
 //
 // Record of (b,h,m), kRecBytes bytes, fp32:
 //   [0, 16384) Hc[d][v] row-major, [16384, 32768) dHc, [32768, 33024) zc,
@@ -332,6 +333,18 @@ __global__ __launch_bounds__(256) void states_sum_kernel(const float* __restrict
 constexpr int kMaskSub = 32;  // 16-row mask sub-tiles per GEMM workgroup (512 rows)
 constexpr int kCompCols = 64;  // state columns per GEMM workgroup
 constexpr int kCompThreads = 512;  // 8 waves
+// One launch for masks, z and H columns where that is the faster one: the
+// workgroups of each column tile build the same mask, so it pays while the
+// launch it saves costs more than that.  Measured (two launches -> one, us):
+// 4 heads x 5 query blocks, 4 tiles, tangent 9.0 -> 5.4; 4 x 64, T = 6 of 64,
+// 9.2 -> 8.1; 8 x 64, T = 16 of 64, primal 9.7 -> 8.4.  Past the lines: two
+// waves of workgroups, 24 x 32, T = 3 of 64, 22.2 -> 24.1; 2048 LUT entries a
+// workgroup, 4 x 64, T = 32 of 64, 9.3 -> 11.3; four mask words, 8 x 130,
+// T = 12 of 128, 12.9 -> 14.4; 8 x 300, T = 3 of 32, 12.7 -> 13.1.
+constexpr int kFusedMaskWords = 3;        // 32 tiles each
+constexpr int kFusedMaskRows = 96;        // query blocks
+constexpr int kFusedMaskEntries = 1024;   // LUT entries of a workgroup's rows
+constexpr int kFusedMaskGroups = 520;     // workgroups: two a CU, and the last few
 
 // 8 mask bits -> the 8 bf16 A-operand slots (1.0 where set)
 __device__ __forceinline__ u32x4 expand_mask8(uint32_t b) {
@@ -438,13 +451,19 @@ __global__ __launch_bounds__(512) void comp_mask_kernel(const int32_t* __restric
 // column c, splits them into bf16 hi + lo and writes half a B-operand
 // fragment of each with one 8-byte LDS store.  The A operand (0/1 mask)
 // comes from the row's mask byte, one 16-entry nibble table read per half.
-template <bool TAN>
+//
+// MASK: the workgroup builds the mask words of its rows itself, in LDS, from
+// the LUT (and the one of column tile 0 also stores them to cbits_out), and the
+// z columns are two more column tiles: no comp_mask_kernel before it.
+template <bool TAN, bool MASK>
 __global__ __launch_bounds__(kCompThreads, 4) void comp_gemm_kernel(
     const float* __restrict__ Hb, const float* __restrict__ dHb, const float* __restrict__ zb,
     const float* __restrict__ dzb, const uint32_t* __restrict__ cbits, int Mb, int Np, int MT,
-    int NC, unsigned char* __restrict__ comp) {
+    int NC, unsigned char* __restrict__ comp, const int32_t* __restrict__ lut, int T,
+    uint32_t* __restrict__ cbits_out) {
+  extern __shared__ uint32_t lbits[];  // MASK: [kc][local row], 16 kMaskSub rows
   __shared__ __align__(16) uint16_t sb[2][2][kCompCols][40];  // [buf][hi/lo][column][n] (+pad)
-  __shared__ __align__(16) uint32_t mw[2][16 * kMaskSub];    // [buf][local row] mask words
+  __shared__ __align__(16) uint32_t mw[2][MASK ? 1 : 16 * kMaskSub];  // [buf][local row] mask words
   // mask nibble -> four bf16 operand slots: 16 entries of 8 bytes occupy 32 distinct LDS
   // banks, so lanes reading different entries never conflict
   __shared__ __align__(16) u32x2 mexp[16];
@@ -473,11 +492,35 @@ __global__ __launch_bounds__(kCompThreads, 4) void comp_gemm_kernel(
   }
   // tile rows n >= Np and mask words past the head read as 0 (buffer range check)
   const auto rs = make_rsrc(src + (int64_t)bh * Np * stride, (int64_t)Np * stride * 4);
-  const auto rb = make_rsrc(cbits + (int64_t)bh * NC * MTp, (int64_t)NC * MTp * 4);
+  const auto rb = make_rsrc(MASK ? reinterpret_cast<const uint32_t*>(lut)
+                                 : cbits + (int64_t)bh * NC * MTp, (int64_t)NC * MTp * 4);
 
   if (tid < 16) {
     const u32x4 e = expand_mask8(tid);
     mexp[tid] = u32x2{e[0], e[1]};
+  }
+
+  if constexpr (MASK) {
+    constexpr int kRows = 16 * kMaskSub;
+    const int rows = min(kRows, MTp - m0);
+    for (int i = tid; i < NC * kRows; i += kCompThreads) lbits[i] = 0u;
+    __syncthreads();
+    const int real = min(rows, Mb - m0);  // rows of real query blocks
+    const int32_t* lrow = lut + ((int64_t)bh * Mb + m0) * T;
+    for (int i = tid; i < real * T; i += kCompThreads) {
+      const int row = i / T;
+      const int n = lrow[i];
+      if ((unsigned)n < (unsigned)Np) atomicOr(&lbits[(n >> 5) * kRows + row], 1u << (n & 31));
+    }
+    __syncthreads();
+    for (int i = tid; i < NC * kRows; i += kCompThreads) {
+      const int kc = i / kRows, row = i - kc * kRows;
+      const int nv = Np - 32 * kc;  // real tiles in this word
+      const uint32_t valid = nv >= 32 ? 0xffffffffu : ((1u << nv) - 1u);
+      const uint32_t wd = row < real ? (~lbits[i] & valid) : 0u;
+      lbits[i] = wd;
+      if (c0 == 0 && row < rows) cbits_out[((int64_t)bh * NC + kc) * MTp + m0 + row] = wd;
+    }
   }
 
   f32x4 acc[4][4];
@@ -497,7 +540,7 @@ __global__ __launch_bounds__(kCompThreads, 4) void comp_gemm_kernel(
     for (int j = 0; j < 4; ++j)
       c.x[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
                                              rs, xoff + (32 * kc + j) * stride * 4, 0, 0));
-    c.mk = __builtin_amdgcn_raw_buffer_load_b32(rb, (kc * MTp + m0 + tid) * 4, 0, 0);
+    if (!MASK) c.mk = __builtin_amdgcn_raw_buffer_load_b32(rb, (kc * MTp + m0 + tid) * 4, 0, 0);
   };
   auto store_chunk = [&](int buf, const Chunk& c) {
     u32x2 hi, lo;
@@ -510,10 +553,10 @@ __global__ __launch_bounds__(kCompThreads, 4) void comp_gemm_kernel(
     }
     *reinterpret_cast<u32x2*>(&sb[buf][0][l][4 * w]) = hi;
     *reinterpret_cast<u32x2*>(&sb[buf][1][l][4 * w]) = lo;
-    mw[buf][tid] = c.mk;
+    if (!MASK) mw[buf][tid] = c.mk;
   };
-  const unsigned char* mwb = reinterpret_cast<const unsigned char*>(&mw[0][0]);
-  auto compute = [&](int buf) {
+  const unsigned char* mwb = reinterpret_cast<const unsigned char*>(MASK ? lbits : &mw[0][0]);
+  auto compute = [&](int buf, int kc) {
     u32x4 bhi[4], blo[4];
 #pragma unroll
     for (int ct = 0; ct < 4; ++ct) {
@@ -524,7 +567,7 @@ __global__ __launch_bounds__(kCompThreads, 4) void comp_gemm_kernel(
     for (int s = 0; s < 4; ++s) {
       const int lt = w + 8 * s;  // local 16-row tile; uniform per wave
       if (mt0 + lt < MT) {
-        const uint32_t mb = mwb[(buf * 16 * kMaskSub + lt * 16 + r) * 4 + g];
+        const uint32_t mb = mwb[((MASK ? kc : buf) * 16 * kMaskSub + lt * 16 + r) * 4 + g];
         const u32x2 alo = mexp[mb & 15u], ahi = mexp[mb >> 4];
         const u32x4 am = u32x4{alo.x, alo.y, ahi.x, ahi.y};
 #pragma unroll
@@ -544,12 +587,12 @@ __global__ __launch_bounds__(kCompThreads, 4) void comp_gemm_kernel(
   for (int kc = 0; kc < NC; kc += 2) {
     // chunk kc in buffer 0, chunk kc+1 in registers cb
     load_chunk(kc + 2, ca);
-    compute(0);
+    compute(0, kc);
     store_chunk(1, cb);  // buffer 1 was last read before the previous barrier
     __syncthreads();
     if (kc + 1 >= NC) break;
     load_chunk(kc + 3, cb);
-    compute(1);
+    compute(1, kc + 1);
     store_chunk(0, ca);
     __syncthreads();
   }
@@ -719,8 +762,9 @@ int complement_gemm_bwd(const float* P, const float* Pz, const uint32_t* cbits, 
                         void* comp, void* stream) {
   const int MT = (Mb + 15) / 16, NC = (Mb + 31) / 32;
   dim3 grid(4160 / kCompCols, BH, (MT + kMaskSub - 1) / kMaskSub);
-  comp_gemm_kernel<false><<<grid, kCompThreads, 0, static_cast<hipStream_t>(stream)>>>(
-      P, nullptr, Pz, nullptr, cbits, Mb, Mb, MT, NC, static_cast<unsigned char*>(comp));
+  comp_gemm_kernel<false, false><<<grid, kCompThreads, 0, static_cast<hipStream_t>(stream)>>>(
+      P, nullptr, Pz, nullptr, cbits, Mb, Mb, MT, NC, static_cast<unsigned char*>(comp), nullptr, 0,
+      nullptr);
   return (int)hipGetLastError();
 }
 }  // namespace sla2h
@@ -801,18 +845,33 @@ extern "C" int sla2h_complement(const float* Hb, const float* dHb, const float* 
   hipStream_t st = static_cast<hipStream_t>(stream);
   auto cbits = static_cast<uint32_t*>(workspace);
   auto out = static_cast<unsigned char*>(comp);
+  const unsigned groups = (unsigned)((MT + kMaskSub - 1) / kMaskSub);
+  const int tiles = (tan ? 8320 : 4160) / kCompCols;
+  if (NC <= kFusedMaskWords && Mb <= kFusedMaskRows && (int64_t)Mb * T <= kFusedMaskEntries &&
+      (int64_t)tiles * B * H <= kFusedMaskGroups) {  // so one group of rows
+    dim3 grid(tiles, B * H, groups);
+    const size_t shmem = (size_t)NC * 16 * kMaskSub * 4;
+    if (tan)
+      comp_gemm_kernel<true, true><<<grid, kCompThreads, shmem, st>>>(
+          Hb, dHb, zb, dzb, nullptr, Mb, Np, MT, NC, out, lut, T, cbits);
+    else
+      comp_gemm_kernel<false, true><<<grid, kCompThreads, shmem, st>>>(
+          Hb, nullptr, zb, nullptr, nullptr, Mb, Np, MT, NC, out, lut, T, cbits);
+    return (int)hipGetLastError();
+  }
   // mask bits plus the z parts of the records; the GEMM takes the H parts only
   // (128 or 64 column tiles per head: whole rounds of workgroups)
   comp_mask_kernel<<<dim3(MT, B * H), tan ? 512 : 256, (size_t)16 * NC * 4, st>>>(
       lut, Mb, Np, T, MT, NC, cbits, zb, dzb, out);
   int err = (int)hipGetLastError();
   if (err) return err;
-  const int ncols = tan ? 8192 : 4096;
-  dim3 grid(ncols / kCompCols, B * H, (MT + kMaskSub - 1) / kMaskSub);
+  dim3 grid((tan ? 8192 : 4096) / kCompCols, B * H, groups);
   if (tan)
-    comp_gemm_kernel<true><<<grid, kCompThreads, 0, st>>>(Hb, dHb, zb, dzb, cbits, Mb, Np, MT, NC, out);
+    comp_gemm_kernel<true, false><<<grid, kCompThreads, 0, st>>>(
+        Hb, dHb, zb, dzb, cbits, Mb, Np, MT, NC, out, nullptr, 0, nullptr);
   else
-    comp_gemm_kernel<false><<<grid, kCompThreads, 0, st>>>(Hb, nullptr, zb, nullptr, cbits, Mb, Np, MT, NC, out);
+    comp_gemm_kernel<false, false><<<grid, kCompThreads, 0, st>>>(
+        Hb, nullptr, zb, nullptr, cbits, Mb, Np, MT, NC, out, nullptr, 0, nullptr);
   return (int)hipGetLastError();
 }
 

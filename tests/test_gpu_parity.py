@@ -113,6 +113,36 @@ def test_linear_states_and_complement():
     assert rel_l2(zc, wz) < 1e-5
 
 
+@pytest.mark.parametrize("tan", [False, True])
+@pytest.mark.parametrize("BH,Mb,Np,T", [
+    (1, 1, 1, 1), (2, 3, 4, 4), (4, 17, 31, 5), (4, 32, 32, 32), (4, 31, 33, 33), (4, 64, 64, 16),
+    (4, 60, 64, 17), (4, 96, 96, 10), (4, 97, 96, 10), (3, 65, 97, 5), (5, 40, 65, 6),
+    (8, 64, 64, 6), (9, 64, 64, 6)])
+def test_complement_one_launch_sizes(BH, Mb, Np, T, tan):
+    """Both sides of the lines at which complement builds the masks inside the
+    GEMM, against a float64 sum.  Bound, elementwise: the bf16 hi + lo split
+    leaves 2^-16 of each term, and Np fp32 additions of two products each."""
+    say(f"complement {BH}x{Mb} Np={Np} T={T} tan={tan}")
+    from imfvideo_amd import ops
+    gen = torch.Generator().manual_seed(Mb * 1000 + Np)
+    rnd = lambda *s: torch.randn(*s, generator=gen)
+    st = {"Hb": rnd(1, BH, Np, 64, 64), "zb": rnd(1, BH, Np, 64)}
+    if tan:
+        st |= {"dHb": rnd(1, BH, Np, 64, 64), "dzb": rnd(1, BH, Np, 64)}
+    lut = torch.stack([torch.randperm(Np, generator=gen)[:T] for _ in range(BH * Mb)])
+    keep = torch.ones(BH * Mb, Np, dtype=torch.float64).scatter_(1, lut, 0.0).view(1, BH, Mb, Np)
+    rec = ops.complement({n: cuda(t) for n, t in st.items()},
+                         cuda(lut.int().view(1, BH, Mb, T)), Np).cpu()
+    for n, at, size in (("Hb", 0, 16384), ("dHb", 16384, 16384), ("zb", 32768, 256),
+                        ("dzb", 33024, 256)):
+        if n not in st:
+            continue
+        got = rec[..., at:at + size].contiguous().view(torch.float32).double()
+        src = st[n].double().reshape(1, BH, Np, -1)
+        err = (got - keep @ src).abs()
+        assert (err <= (2.0 ** -16 + 2 * Np * 2.0 ** -24) * (keep @ src.abs())).all(), n
+
+
 def config_inputs(cfg, heads=None):
     """Config 1: (1,4,4096) fp32 N(0,1) -> bf16, seed 1.  Config 2/3: (1,8,29952), seed 2/3."""
     if cfg == 1:
