@@ -1162,6 +1162,309 @@ void attn_in_dispatch(int lo_dt, int hi_dt, F&& f) {
 }  // namespace sla2h
 
 // ---------------------------------------------------------------------------
+// The same operands straight from the projections' outputs: q (B, L, H, 64) =
+// [nope | rope], kv (B, L, H, 96) = [k nope | v] and the key band kr (B, L, 32)
+// that the heads share, all of one 16-bit type, through the per-head RMSNorm of
+// the nope halves (models/imf_dit_video.py:121-133) and RoPE of the others
+// (266-284), with the roundings of those stages: the normalised value to the
+// 16-bit type before its fp32 weight, the rotated one to the 16-bit type.
+// Backward: dq, dkv and dkr whole (no concatenation after it), dw as one partial
+// row per workgroup, then col_sum_kernel.  HBM-bound: q, kv, kr and the operands
+// cross memory once each way; as norms, rotations, operand copies and
+// concatenations the halves crossed it three to five times, partly in fp32.
+// Eight threads a (token, head): lanes 0..3 of them hold the nope half (the row
+// sums are two lane exchanges), 4..7 the rope half; heads before tokens, so a
+// token's heads are read and written contiguously on the projections' side.
+// 16,384 tokens x 8 heads, bf16, against those stages: 57 -> 19.4 us forward (92 MB,
+// 4.7 TB/s), 116 -> 34 us backward (135 MB; 30 us of it mla_in_bwd, 47 when the
+// thread of head 0 read the other heads' band gradients itself, one dependent
+// chain a row, and a workgroup had twice the rows in flight).
+// ---------------------------------------------------------------------------
+namespace sla2h {
+namespace {
+
+struct MlaIn {
+  const void *q, *kv, *kr;       // kr unused by the backward
+  int64_t kr_sb, kr_st;          // strides of kr's batches and tokens, in elements
+  const float *wq, *wk;          // (32) norm weights
+  float eps_q, eps_k;
+  const float *cos_t, *sin_t;    // (L, 16)
+  int H, L, rows;                // rows = B L H
+};
+
+constexpr int kMlaPasses = 2, kMlaRows = 32 * kMlaPasses;  // rows of a backward workgroup
+
+__device__ inline u32x4 ld_raw(const void* p, int64_t i) {
+  return *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(p) + i);
+}
+template <int DT>
+__device__ inline void expand8(u32x4 v, float (&x)[8]) {
+  using T16 = typename std::conditional<DT == SLA2H_DTYPE_BF16, BF16, F16>::type;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    x[2 * e] = T16::to_f32((uint16_t)(v[e] & 0xffff));
+    x[2 * e + 1] = T16::to_f32((uint16_t)(v[e] >> 16));
+  }
+}
+
+// RMSNorm of the 32 channels of a row, eight a lane over four lanes
+template <int DT>
+__device__ inline void mla_norm(float (&x)[8], const float (&w)[8], float eps) {
+  float ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) ss += x[e] * x[e];
+  const float r = 1.f / sqrtf(group_sum<4>(ss) / 32.f + eps);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = round_to<DT>(x[e] * r) * w[e];
+}
+
+// its backward: x the input, dy the output gradient -> dx in x, dw terms added
+template <int DT>
+__device__ inline void mla_norm_bwd(float (&x)[8], const float (&dy)[8], const float (&w)[8],
+                                    float eps, float (&dw)[8]) {
+  float ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) ss += x[e] * x[e];
+  const float r = 1.f / sqrtf(group_sum<4>(ss) / 32.f + eps);
+  float g[8], gx = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    g[e] = round_to<DT>(dy[e] * w[e]);
+    gx += g[e] * x[e];
+    dw[e] += round_to<DT>(x[e] * r) * dy[e];
+  }
+  const float mgx = group_sum<4>(gx) / 32.f;
+  const float r3 = r * r * r;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = r * g[e] - x[e] * r3 * mgx;
+}
+
+// four channel pairs by the angles c + i sgn s, rounded to the 16-bit type
+template <int DT>
+__device__ inline void mla_rope(float (&x)[8], const float4& c, const float4& s, float sgn) {
+  const float cv[4] = {c.x, c.y, c.z, c.w}, sv[4] = {s.x, s.y, s.z, s.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float re = x[2 * i], im = x[2 * i + 1], sn = sgn * sv[i];
+    x[2 * i] = round_to<DT>(re * cv[i] - im * sn);
+    x[2 * i + 1] = round_to<DT>(re * sn + im * cv[i]);
+  }
+}
+
+template <int DT>
+__global__ __launch_bounds__(256) void mla_in_fwd_kernel(MlaIn a, uint16_t* __restrict__ qh,
+                                                         uint16_t* __restrict__ kh,
+                                                         uint16_t* __restrict__ vh) {
+  const int row = blockIdx.x * 32 + (threadIdx.x >> 3), c8 = threadIdx.x & 7;
+  if (row >= a.rows) return;
+  const int tok = row / a.H, h = row - tok * a.H;
+  const int b = tok / a.L, t = tok - b * a.L;
+  const int64_t oi = ((int64_t)(b * a.H + h) * a.L + t) * 64 + 8 * c8;
+  const u32x4 rq = ld_raw(a.q, (int64_t)row * 64 + 8 * c8);
+  const u32x4 rv = ld_raw(a.kv, (int64_t)row * 96 + 32 + 8 * c8);
+  const u32x4 rk = c8 < 4 ? ld_raw(a.kv, (int64_t)row * 96 + 8 * c8)
+                          : ld_raw(a.kr, b * a.kr_sb + t * a.kr_st + 8 * (c8 - 4));
+  float q[8], k[8], v[8];
+  expand8<DT>(rq, q);
+  expand8<DT>(rk, k);
+  expand8<DT>(rv, v);
+  if (c8 < 4) {
+    float w[8];
+    ld8f(a.wq, 8 * c8, w);
+    mla_norm<DT>(q, w, a.eps_q);
+    ld8f(a.wk, 8 * c8, w);
+    mla_norm<DT>(k, w, a.eps_k);
+  } else {
+    const float4 c = *reinterpret_cast<const float4*>(a.cos_t + (int64_t)t * 16 + 4 * (c8 - 4));
+    const float4 s = *reinterpret_cast<const float4*>(a.sin_t + (int64_t)t * 16 + 4 * (c8 - 4));
+    mla_rope<DT>(q, c, s, 1.f);
+    mla_rope<DT>(k, c, s, 1.f);
+  }
+  st8<SLA2H_DTYPE_F16>(qh, oi, q);
+  st8<SLA2H_DTYPE_F16>(kh, oi, k);
+  st8<SLA2H_DTYPE_F16>(vh, oi, v);
+}
+
+template <int DT>
+__global__ __launch_bounds__(256) void mla_in_bwd_kernel(MlaIn a, const uint16_t* __restrict__ dqh,
+                                                         const uint16_t* __restrict__ dkh,
+                                                         const uint16_t* __restrict__ dvh,
+                                                         void* __restrict__ dq,
+                                                         void* __restrict__ dkv,
+                                                         void* __restrict__ dkr,
+                                                         float* __restrict__ DWP) {
+  constexpr int P = kMlaPasses;
+  __shared__ float part[4][64];
+  __shared__ __align__(16) uint16_t band[kMlaRows][32];  // round(dk) of the rope halves
+  const int c8 = threadIdx.x & 7, w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const bool nope = c8 < 4;
+  const bool whole = kMlaRows % a.H == 0;  // no token's heads cross a workgroup
+  const int row0 = blockIdx.x * kMlaRows + (threadIdx.x >> 3);
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  u32x4 gq[P], gk[P], gv[P], xq[P], xk[P];  // all passes' rows in flight
+  float4 cs[P], sn[P];
+#pragma unroll
+  for (int k = 0; k < P; ++k) {
+    const int row = row0 + 32 * k;
+    gq[k] = gk[k] = gv[k] = xq[k] = xk[k] = zero;
+    cs[k] = sn[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (row >= a.rows) continue;
+    const int tok = row / a.H, h = row - tok * a.H;
+    const int b = tok / a.L, t = tok - b * a.L;
+    const int64_t oi = ((int64_t)(b * a.H + h) * a.L + t) * 64 + 8 * c8;
+    gq[k] = ld_raw(dqh, oi);
+    gk[k] = ld_raw(dkh, oi);
+    gv[k] = ld_raw(dvh, oi);
+    if (nope) {
+      xq[k] = ld_raw(a.q, (int64_t)row * 64 + 8 * c8);
+      xk[k] = ld_raw(a.kv, (int64_t)row * 96 + 8 * c8);
+    } else {
+      cs[k] = *reinterpret_cast<const float4*>(a.cos_t + (int64_t)t * 16 + 4 * (c8 - 4));
+      sn[k] = *reinterpret_cast<const float4*>(a.sin_t + (int64_t)t * 16 + 4 * (c8 - 4));
+    }
+  }
+  float wq[8] = {}, wk[8] = {}, dwq[8] = {}, dwk[8] = {};
+  if (nope) {
+    ld8f(a.wq, 8 * c8, wq);
+    ld8f(a.wk, 8 * c8, wk);
+  }
+#pragma unroll
+  for (int k = 0; k < P; ++k) {
+    const int row = row0 + 32 * k;
+    if (row >= a.rows) break;  // the same for a row's eight threads
+    float g[8], x[8];
+    if (nope) {
+      expand8<SLA2H_DTYPE_F16>(gq[k], g);
+      expand8<DT>(xq[k], x);
+      mla_norm_bwd<DT>(x, g, wq, a.eps_q, dwq);
+      st8<DT>(dq, (int64_t)row * 64 + 8 * c8, x);
+      expand8<SLA2H_DTYPE_F16>(gk[k], g);
+      expand8<DT>(xk[k], x);
+      mla_norm_bwd<DT>(x, g, wk, a.eps_k, dwk);
+      st8<DT>(dkv, (int64_t)row * 96 + 8 * c8, x);
+    } else {
+      expand8<SLA2H_DTYPE_F16>(gq[k], g);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) g[e] = round_to<DT>(g[e]);
+      mla_rope<DT>(g, cs[k], sn[k], -1.f);
+      st8<DT>(dq, (int64_t)row * 64 + 8 * c8, g);
+      expand8<SLA2H_DTYPE_F16>(gk[k], x);
+      st8<DT>(&band[(threadIdx.x >> 3) + 32 * k][0], 8 * (c8 - 4), x);
+    }
+    expand8<SLA2H_DTYPE_F16>(gv[k], x);
+    st8<DT>(dkv, (int64_t)row * 96 + 32 + 8 * c8, x);
+  }
+  __syncthreads();
+  // the shared band: its heads' 16-bit gradients summed in head order, rounded,
+  // rotated back; four threads a token, over the tokens whose head 0 is here
+  {
+    const int first = blockIdx.x * kMlaRows, last = min(first + kMlaRows, a.rows);
+    const int tok0 = (first + a.H - 1) / a.H, tok1 = (last + a.H - 1) / a.H;
+    const int c = threadIdx.x & 3;
+    for (int tok = tok0 + (threadIdx.x >> 2); tok < tok1; tok += 64) {
+      const int b = tok / a.L, t = tok - b * a.L;
+      const float4 cv = *reinterpret_cast<const float4*>(a.cos_t + (int64_t)t * 16 + 4 * c);
+      const float4 sv = *reinterpret_cast<const float4*>(a.sin_t + (int64_t)t * 16 + 4 * c);
+      float acc[8] = {};
+      for (int h = 0; h < a.H; ++h) {
+        float x[8];
+        if (whole) {
+          ld8<DT>(&band[tok * a.H + h - first][0], 8 * c, x);
+        } else {
+          ld8<SLA2H_DTYPE_F16>(dkh, ((int64_t)(b * a.H + h) * a.L + t) * 64 + 32 + 8 * c, x);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) x[e] = round_to<DT>(x[e]);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] += x[e];
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] = round_to<DT>(acc[e]);
+      mla_rope<DT>(acc, cv, sv, -1.f);
+      st8<DT>(dkr, (int64_t)tok * 32 + 8 * c, acc);
+    }
+  }
+  // the wave's eight rows of a pass (lanes l, l ^ 8, ...), then its four waves
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+#pragma unroll
+    for (int m = 8; m < 64; m <<= 1) {
+      dwq[e] += __shfl_xor(dwq[e], m, 64);
+      dwk[e] += __shfl_xor(dwk[e], m, 64);
+    }
+  if (l < 4)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      part[w][8 * l + e] = dwq[e];
+      part[w][32 + 8 * l + e] = dwk[e];
+    }
+  __syncthreads();
+  const int c = threadIdx.x;
+  if (c < 64)
+    DWP[(int64_t)blockIdx.x * 64 + c] = (part[0][c] + part[1][c]) + (part[2][c] + part[3][c]);
+}
+
+bool mla_in_ok(const MlaIn& a, int dtype, int B, int H, int64_t L) {
+  return a.q && a.kv && a.wq && a.wk && a.cos_t && a.sin_t && dt_ok(dtype, false) && B > 0 &&
+         H > 0 && L > 0 && L < (1ll << 31) && (int64_t)B * H < (1ll << 31) &&
+         (int64_t)B * L * H <= (1ll << 31) - 1 - kMlaRows && aligned16(a.q) &&
+         aligned16(a.kv) && aligned16(a.wq) && aligned16(a.wk) && aligned16(a.cos_t) &&
+         aligned16(a.sin_t);
+}
+unsigned mla_in_groups(int64_t rows) { return (unsigned)((rows + kMlaRows - 1) / kMlaRows); }
+
+}  // namespace
+}  // namespace sla2h
+
+extern "C" int sla2h_mla_in_fwd(const void* q, const void* kv, const void* kr, int64_t kr_sb,
+                                int64_t kr_st, int dtype, int B, int64_t L, int H, const float* wq,
+                                const float* wk, float eps_q, float eps_k, const float* cos_t,
+                                const float* sin_t, void* qh, void* kh, void* vh, void* stream) {
+  MlaIn a{q, kv, kr, kr_sb, kr_st, wq, wk, eps_q, eps_k, cos_t, sin_t, H, (int)L, 0};
+  SLA2H_CHECK_ARG(mla_in_ok(a, dtype, B, H, L) && half_ok(kr, dtype, kr_sb, kr_st, 0));
+  SLA2H_CHECK_ARG(qh && kh && vh && aligned16(qh) && aligned16(kh) && aligned16(vh));
+  a.rows = (int)(B * L * H);
+  const unsigned grid = (unsigned)(((int64_t)a.rows + 31) / 32);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  uint16_t *o0 = static_cast<uint16_t*>(qh), *o1 = static_cast<uint16_t*>(kh),
+           *o2 = static_cast<uint16_t*>(vh);
+  if (dtype == SLA2H_DTYPE_BF16)
+    mla_in_fwd_kernel<SLA2H_DTYPE_BF16><<<grid, 256, 0, st>>>(a, o0, o1, o2);
+  else
+    mla_in_fwd_kernel<SLA2H_DTYPE_F16><<<grid, 256, 0, st>>>(a, o0, o1, o2);
+  return (int)hipGetLastError();
+}
+
+extern "C" size_t sla2h_mla_in_bwd_workspace_bytes(int B, int64_t L, int H) {
+  return B > 0 && L > 0 && H > 0 ? (size_t)mla_in_groups((int64_t)B * L * H) * 64 * 4 : 0;
+}
+
+extern "C" int sla2h_mla_in_bwd(const void* dqh, const void* dkh, const void* dvh, const void* q,
+                                const void* kv, int dtype, int B, int64_t L, int H,
+                                const float* wq, const float* wk, float eps_q, float eps_k,
+                                const float* cos_t, const float* sin_t, void* dq, void* dkv,
+                                void* dkr, float* dw, float* workspace, void* stream) {
+  MlaIn a{q, kv, nullptr, 0, 0, wq, wk, eps_q, eps_k, cos_t, sin_t, H, (int)L, 0};
+  SLA2H_CHECK_ARG(mla_in_ok(a, dtype, B, H, L));
+  for (const void* p : {dqh, dkh, dvh, (const void*)dq, (const void*)dkv, (const void*)dkr})
+    SLA2H_CHECK_ARG(p && aligned16(p));
+  SLA2H_CHECK_ARG(dw && workspace);
+  a.rows = (int)(B * L * H);
+  const unsigned grid = mla_in_groups(a.rows);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const uint16_t *g0 = static_cast<const uint16_t*>(dqh), *g1 = static_cast<const uint16_t*>(dkh),
+                 *g2 = static_cast<const uint16_t*>(dvh);
+  if (dtype == SLA2H_DTYPE_BF16)
+    mla_in_bwd_kernel<SLA2H_DTYPE_BF16><<<grid, 256, 0, st>>>(a, g0, g1, g2, dq, dkv, dkr, workspace);
+  else
+    mla_in_bwd_kernel<SLA2H_DTYPE_F16><<<grid, 256, 0, st>>>(a, g0, g1, g2, dq, dkv, dkr, workspace);
+  const int err = (int)hipGetLastError();
+  if (err) return err;
+  col_sum_kernel<<<64, 256, 0, st>>>(workspace, grid, 64, dw);
+  return (int)hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
 // Token layout of the cube op: (B, L, H, 64) tensors in model order <-> the
 // op's (B, H, L, 64) fp16 rows in tile order, one pass for up to three tensors.
 // idx[l] is the token of the source that goes to row l (NULL: l itself).

@@ -365,6 +365,53 @@ class _AttnInFunction(torch.autograd.Function):
         return tuple(grads)
 
 
+class _MlaInFunction(torch.autograd.Function):
+    """_AttnInFunction with the per-head norms and the rotations in the same
+    kernel, from the projections' outputs q (B, L, H, 64), kv (B, L, H, 96) and the
+    shared key band k_rope (B, L, 32); the backward writes their gradients whole."""
+
+    @staticmethod
+    def forward(ctx, q, kv, k_rope, wq, wk, eps_q, eps_k, rope_cos, rope_sin):
+        from . import ops
+        ctx.eps = eps_q, eps_k
+        ctx.save_for_backward(q, kv, wq, wk, rope_cos, rope_sin)
+        return tuple(ops.mla_in_fwd(q, kv, k_rope, wq, wk, eps_q, eps_k, rope_cos, rope_sin))
+
+    @staticmethod
+    def backward(ctx, dqh, dkh, dvh):
+        from . import ops
+        q, kv, wq, wk, rope_cos, rope_sin = ctx.saved_tensors
+        return (*ops.mla_in_bwd(dqh, dkh, dvh, q, kv, wq, wk, *ctx.eps, rope_cos, rope_sin),
+                None, None, None, None)
+
+
+def _plain_norm(m):
+    """m is an RMSNorm of 32 channels whose call is its forward and nothing else."""
+    return (type(m) is RMSNorm and "forward" not in m.__dict__ and not m._forward_hooks
+            and not m._forward_pre_hooks and not m._backward_hooks and not m._backward_pre_hooks
+            and not nn.modules.module._has_any_global_hook() and m.weight.dtype == torch.float32
+            and m.weight.is_cuda and tuple(m.weight.shape) == (32,) and m.weight.is_contiguous()
+            and m.weight.data_ptr() % 16 == 0)
+
+
+def _mla_in_ok(attn, q, kv, k_rope, rope_cos, rope_sin):
+    """The operands of this call can come from _MlaInFunction: what
+    _tile_major_operands_ok asks of the halves, on the projections' outputs of one
+    16-bit dtype, with plain norms and fp32 angles, in eager reverse mode."""
+    from . import ops
+    dn = attn.qk_nope_head_dim
+    return (q.dtype in (torch.float16, torch.bfloat16) and q.dtype == kv.dtype == k_rope.dtype
+            and q.is_contiguous() and kv.is_contiguous() and q.shape[1] > 0
+            and _tile_major_operands_ok(attn.attn_impl, q[..., :dn], q[..., dn:], kv[..., :dn],
+                                        k_rope.unsqueeze(2), kv[..., dn:])
+            and _plain_norm(attn.q_norm) and _plain_norm(attn.k_norm)
+            and all(t.is_cuda and t.dtype == torch.float32 and t.is_contiguous()
+                    and tuple(t.shape) == (q.shape[1], 16) and t.data_ptr() % 16 == 0
+                    for t in (rope_cos, rope_sin))
+            and ops.plain_eager(q, kv, k_rope, attn.q_norm.weight, attn.k_norm.weight, rope_cos,
+                                rope_sin))
+
+
 class _AttnGateFunction(torch.autograd.Function):
     """round16(fp32(o) * sigmoid(g)) from a tile-major SLA2 op's fp16 output o
     (B, H, L, 64): the reference's permute / .to(float32) of o, its fp32 gate
@@ -452,27 +499,37 @@ class MLAAttention(nn.Module):
         H = self.num_heads
         dn, dr, dv = self.qk_nope_head_dim, self.qk_rope_head_dim, self.v_head_dim
         q = self.q_b_proj(self.q_a_layernorm(self.q_a_proj(xq))).reshape(b, l, H, dn + dr)
-        q_nope, q_rope = q.split([dn, dr], dim=-1)
         kv_latent, k_rope = self.kv_a_proj(xkv).split([self.kv_lora_rank, dr], dim=-1)
         kv = self.kv_b_proj(self.kv_a_layernorm(kv_latent)).reshape(b, l, H, dn + dv)
-        k_nope, v = kv.split([dn, dv], dim=-1)
-        q_nope, k_nope = self.q_norm(q_nope), self.k_norm(k_nope)
-        q_rope = apply_rotary_pos_emb(q_rope, rope_cos, rope_sin)
-        k_rope = apply_rotary_pos_emb(k_rope.unsqueeze(2), rope_cos, rope_sin)
-        if _tile_major_operands_ok(self.attn_impl, q_nope, q_rope, k_nope, k_rope, v):
-            # the op's fp16 tile-major operands straight from the halves, and
-            # (under autocast) its output through the gate into the projection
-            qh, kh, vh = _AttnInFunction.apply(q_nope, q_rope, k_nope, k_rope, v)
-            o = self.attn_impl.forward_tile_major(qh, kh, vh)
+        heads = None
+        if _mla_in_ok(self, q, kv, k_rope, rope_cos, rope_sin):
+            # the op's fp16 tile-major operands straight from the projections
+            heads = _MlaInFunction.apply(q, kv, k_rope, self.q_norm.weight, self.k_norm.weight,
+                                         float(self.q_norm.eps), float(self.k_norm.eps), rope_cos,
+                                         rope_sin)
+            dtype = torch.float32
+        else:
+            q_nope, q_rope = q.split([dn, dr], dim=-1)
+            k_nope, v = kv.split([dn, dv], dim=-1)
+            q_nope, k_nope = self.q_norm(q_nope), self.k_norm(k_nope)
+            q_rope = apply_rotary_pos_emb(q_rope, rope_cos, rope_sin)
+            k_rope = apply_rotary_pos_emb(k_rope.unsqueeze(2), rope_cos, rope_sin)
+            if _tile_major_operands_ok(self.attn_impl, q_nope, q_rope, k_nope, k_rope, v):
+                # ... or from the halves
+                heads = _AttnInFunction.apply(q_nope, q_rope, k_nope, k_rope, v)
+                dtype = torch.promote_types(q_nope.dtype, q_rope.dtype)
+        if heads is not None:
+            # (under autocast) the op's output goes through the gate into the projection
+            o = self.attn_impl.forward_tile_major(*heads)
             if self.use_output_gate:
                 g = self.g_proj(xg)
                 if (torch.is_autocast_enabled("cuda") and g.dtype == torch.get_autocast_dtype("cuda")
                         and g.dtype in (torch.float16, torch.bfloat16) and g.is_contiguous()
                         and g.data_ptr() % 16 == 0):
                     return self.out_proj(_AttnGateFunction.apply(o, g))
-                attn = o.permute(0, 2, 1, 3).to(torch.promote_types(q_nope.dtype, q_rope.dtype))
+                attn = o.permute(0, 2, 1, 3).to(dtype)
                 return self.out_proj(attn.reshape(b, l, H * dv) * torch.sigmoid(g))
-            attn = o.permute(0, 2, 1, 3).to(torch.promote_types(q_nope.dtype, q_rope.dtype))
+            attn = o.permute(0, 2, 1, 3).to(dtype)
             return self.out_proj(attn.reshape(b, l, H * dv))
         k_rope = k_rope.expand(b, l, H, dr)
         q = torch.cat([q_nope, q_rope], dim=-1)

@@ -1173,6 +1173,51 @@ def attn_in_bwd(dout, dlo, dhi):
         _stream(dout.device)), "sla2h_attn_in_bwd")
 
 
+def mla_in_fwd(q, kv, kr, wq, wk, eps_q, eps_k, cos_t, sin_t):
+    """(qh, kh, vh) (B, H, L, 64) fp16 from q (B, L, H, 64) = [nope | rope], kv
+    (B, L, H, 96) = [k nope | v] and the heads' shared key band kr (B, L, 32), one
+    16-bit dtype: RMSNorm of the nope halves, RoPE of the others, the operand
+    layout and its cast in one pass."""
+    _need_gpu(q, kv, kr, wq, wk, cos_t, sin_t)
+    B, L, H, _ = q.shape
+    if (q.dtype not in _F16_CODES or not q.dtype == kv.dtype == kr.dtype
+            or tuple(q.shape) != (B, L, H, 64) or tuple(kv.shape) != (B, L, H, 96)
+            or tuple(kr.shape) != (B, L, 32) or kr.stride(-1) != 1
+            or not (q.is_contiguous() and kv.is_contiguous())):
+        raise ValueError("mla_in_fwd: expected contiguous (B, L, H, 64) q, (B, L, H, 96) kv and "
+                         "(B, L, 32) kr of one 16-bit dtype")
+    if tuple(cos_t.shape) != (L, 16) or tuple(sin_t.shape) != (L, 16) or not (
+            wq.numel() == wk.numel() == 32) or any(
+            t.dtype != torch.float32 or not t.is_contiguous() for t in (wq, wk, cos_t, sin_t)):
+        raise ValueError("mla_in_fwd: expected contiguous fp32 (32) weights and (L, 16) angles")
+    out = [torch.empty(B, H, L, 64, device=q.device, dtype=torch.float16) for _ in range(3)]
+    _lib.check(_lib.load().sla2h_mla_in_fwd(
+        q.data_ptr(), kv.data_ptr(), kr.data_ptr(), kr.stride(0), kr.stride(1),
+        _F16_CODES[q.dtype], B, L, H, wq.data_ptr(), wk.data_ptr(), float(eps_q), float(eps_k),
+        cos_t.data_ptr(), sin_t.data_ptr(), *(t.data_ptr() for t in out), _stream(q.device)),
+        "sla2h_mla_in_fwd")
+    return out
+
+
+def mla_in_bwd(dqh, dkh, dvh, q, kv, wq, wk, eps_q, eps_k, cos_t, sin_t):
+    """(dq, dkv, dkr, dwq, dwk) of mla_in_fwd for its outputs' fp16 gradients."""
+    _need_gpu(dqh, dkh, dvh, q, kv, wq, wk, cos_t, sin_t)
+    B, L, H, _ = q.shape
+    dqh, dkh, dvh = (d.to(torch.float16).contiguous() for d in (dqh, dkh, dvh))
+    dq, dkv = torch.empty_like(q), torch.empty_like(kv)
+    dkr = torch.empty(B, L, 32, device=q.device, dtype=q.dtype)
+    dw = torch.empty(64, device=q.device, dtype=torch.float32)
+    lib = _lib.load()
+    ws = torch.empty(lib.sla2h_mla_in_bwd_workspace_bytes(B, L, H), device=q.device,
+                     dtype=torch.uint8)
+    _lib.check(lib.sla2h_mla_in_bwd(
+        dqh.data_ptr(), dkh.data_ptr(), dvh.data_ptr(), q.data_ptr(), kv.data_ptr(),
+        _F16_CODES[q.dtype], B, L, H, wq.data_ptr(), wk.data_ptr(), float(eps_q), float(eps_k),
+        cos_t.data_ptr(), sin_t.data_ptr(), dq.data_ptr(), dkv.data_ptr(), dkr.data_ptr(),
+        dw.data_ptr(), ws.data_ptr(), _stream(q.device)), "sla2h_mla_in_bwd")
+    return dq, dkv, dkr, dw[:32], dw[32:]
+
+
 def attn_gate_fwd(o, g):
     """round16(fp32(o) sigmoid16(g)) as (B, L, H * 64) in g's dtype, from the
     op's (B, H, L, 64) fp16 output o and the gate logits g (B, L, H * 64)."""

@@ -373,6 +373,29 @@ int sla2h_attn_in_bwd(const void* dout, void* dlo, int lo_dtype, int64_t lo_sb, 
                       int64_t hi_sh, int B, int H, int64_t L, void* stream);
 
 /*
+ * The same three operands straight from the projections' outputs, all of one
+ * 16-bit dtype: q (B, L, H, 64) = [nope | rope], kv (B, L, H, 96) = [k nope | v],
+ * both contiguous, and kr, the (B, L, 32) key band the heads share (kr_sb, kr_st:
+ * its batch and token strides in elements; 16-byte multiples).  wq, wk: (32) fp32
+ * weights of the nope halves' RMSNorm; cos_t, sin_t: (L, 16) fp32 angles of the
+ * RoPE of the others (replaces models/imf_dit_video.py:121-133 and 266-284 on
+ * the heads, the cat and the permute / .half()).  qh, kh, vh: (B, H, L, 64) fp16.
+ * Backward: dqh, dkh, dvh (B, H, L, 64) fp16 -> dq, dkv (as q, kv), dkr
+ * (B, L, 32) contiguous, dw (64) fp32: the gradients of wq and of wk.
+ * workspace: sla2h_mla_in_bwd_workspace_bytes.
+ */
+int sla2h_mla_in_fwd(const void* q, const void* kv, const void* kr, int64_t kr_sb, int64_t kr_st,
+                     int dtype, int B, int64_t L, int H, const float* wq, const float* wk,
+                     float eps_q, float eps_k, const float* cos_t, const float* sin_t, void* qh,
+                     void* kh, void* vh, void* stream);
+size_t sla2h_mla_in_bwd_workspace_bytes(int B, int64_t L, int H);
+int sla2h_mla_in_bwd(const void* dqh, const void* dkh, const void* dvh, const void* q,
+                     const void* kv, int dtype, int B, int64_t L, int H, const float* wq,
+                     const float* wk, float eps_q, float eps_k, const float* cos_t,
+                     const float* sin_t, void* dq, void* dkv, void* dkr, float* dw,
+                     float* workspace, void* stream);
+
+/*
  * The output gate after a tile-major SLA2 op under autocast: replaces
  * o.permute(0, 2, 1, 3).to(float32) (models/sla2_cube_qat.py:397-400), the
  * gate attn * torch.sigmoid(g) in fp32 (models/imf_dit_video.py:466) and the

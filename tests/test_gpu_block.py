@@ -395,6 +395,75 @@ def test_attn_operands_and_gate_match_torch(dt):
         assert not bad.any()
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,L,H", [(1, 1, 1), (1, 3, 5), (2, 43, 3), (1, 16, 8), (2, 333, 8),
+                                   (3, 129, 16)])
+def test_mla_in_matches_the_separate_stages(B, L, H, dt):
+    """Norm, RoPE and operand layout in one kernel against the same in separate
+    ones, both ways.  The roundings are the same ones, so an element differs
+    only where a contracted fp32 expression falls on the other side of a
+    rounding: the next value of the 16-bit type (at most 2 ULP relative), rarely;
+    where two terms of up to 32 cancel, by their fp32 rounding, 2^-18.  The
+    weight gradients are fp32 sums of B L H terms in another order."""
+    from imfvideo_amd.imf_dit_video import (_AttnInFunction, _MlaInFunction, _RMSNormFunction,
+                                            _RopeFunction)
+    say("mla_in", dt, B, L, H)
+    g = torch.Generator().manual_seed(B * 1000 + L)
+    rnd = lambda *s: torch.randn(*s, generator=g)
+    q, kv = rnd(B, L, H, 64).to(dt).cuda(), rnd(B, L, H, 96).to(dt).cuda()
+    kva = rnd(B, L, 64 + 32).to(dt).cuda()
+    wq, wk = (1 + 0.2 * rnd(32)).cuda(), (1 + 0.2 * rnd(32)).cuda()
+    ang = 3 * rnd(L, 16)
+    cos, sin = torch.cos(ang).cuda(), torch.sin(ang).cuda()
+    dys = [rnd(B, H, L, 64).half().cuda() for _ in range(3)]
+
+    def run(fused):
+        xs = [t.clone().requires_grad_(True) for t in (q, kv, kva, wq, wk)]
+        q_, kv_, band, a, b = xs[0], xs[1], xs[2][..., 64:], xs[3], xs[4]
+        if fused:
+            out = _MlaInFunction.apply(q_, kv_, band, a, b, 1e-6, 1e-5, cos, sin)
+        else:
+            out = _AttnInFunction.apply(_RMSNormFunction.apply(q_[..., :32], a, 1e-6),
+                                        _RopeFunction.apply(q_[..., 32:], cos, sin),
+                                        _RMSNormFunction.apply(kv_[..., :32], b, 1e-5),
+                                        _RopeFunction.apply(band.unsqueeze(2), cos, sin),
+                                        kv_[..., 32:])
+        torch.autograd.backward(out, dys)
+        return [t.detach() for t in out], [x.grad for x in xs]
+
+    (o1, g1), (o0, g0) = run(True), run(False)
+    for i, (x, y) in enumerate(zip(o1 + g1[:3], o0 + g0[:3])):
+        assert x.dtype == y.dtype and x.shape == y.shape
+        x, y = x.float(), y.float()
+        assert bool(((x - y).abs() <= 2 * ULP[dt] * y.abs() + 2.0 ** -18).all()), i
+        assert (x != y).float().mean() < 0.01, i
+    for x, y, n, gr in ((g1[3], g0[3], q, dys[0]), (g1[4], g0[4], kv, dys[1])):
+        # |normalised value| <= sqrt(32)
+        bound = 2 * B * L * H * 2.0 ** -24 * 32 ** 0.5 * gr[..., :32].float().abs().sum((0, 1, 2))
+        assert bool(((x - y).abs() <= bound).all())
+
+
+def test_mla_in_leaves_hooked_norms_alone():
+    """A hook on a head norm runs: the one-kernel operands step aside for it."""
+    from functools import partial
+    import imfvideo_amd.imf_dit_video as M
+    from imfvideo_amd.sla2_cube_qat import SLA2CubeQATAttentionImpl
+    impl = partial(SLA2CubeQATAttentionImpl, seq_len=128, num_heads=2, grid=(4, 4, 8),
+                   tile=(4, 4, 4), topk=0.5, pre_permuted=True)
+    attn = M.MLAAttention(64, 2, 32, 32, 32, 32, 64, attn_impl=impl).cuda()
+    x = torch.randn(1, 128, 64, device="cuda")
+    cos, sin = (t.cuda() for t in M.precompute_axial_rope_3d(32, (4, 4, 8), 0,
+                                                             axis_dims=(8, 12, 12)))
+    calls = []
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        a = attn(x, cos, sin)
+        h = attn.k_norm.register_forward_hook(lambda m, i, o: calls.append(1) or o * 0)
+        b = attn(x, cos, sin)
+        h.remove()
+        c = attn(x, cos, sin)
+    assert calls == [1] and torch.equal(a, c) and not torch.equal(a, b)
+
+
 def test_block_fused_attention_path_matches_eager_layout():
     """A TransformerBlock under bf16 autocast with the fused attention operand /
     gate path and the same block on the eager cat / permute / gate path: outputs
