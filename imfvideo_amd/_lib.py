@@ -83,10 +83,10 @@ SIGNATURES = {
                                     _c_f, _p, _p, _p]),
     "sla2h_cube_jvp_workspace_bytes": (ctypes.c_size_t, [_c_int, _c_int, _c_i64, _c_int, _c_int,
                                                          _c_int]),
-    "sla2h_cube_jvp_quant": (_c_int, [_p, _p, _c_int, _c_int, _c_int, _c_i64, _c_int, _c_int,
+    "sla2h_cube_jvp_quant": (_c_int, [_p, _p, _p, _p, _p, _c_int, _c_int, _c_int, _c_i64, _c_int,
                                       _c_int, _p, _p, _p, _p, _p, _p]),
-    "sla2h_cube_jvp_attn": (_c_int, [_p, _p, _p, _p, _p, _p, _p, _c_int, _p, _c_int, _c_int,
-                                     _c_int, _c_i64, _c_int, _c_int, _c_f, _c_f, _p, _p, _p, _p]),
+    "sla2h_cube_jvp_attn": (_c_int, [_p, _p, _p, _c_int, _p, _c_int, _c_int, _c_int, _c_i64, _c_int,
+                                     _c_int, _c_f, _c_f, _p, _p, _p, _p]),
     "sla2h_jvp16_workspace_bytes": (ctypes.c_size_t, [_c_int, _c_int, _c_i64, _c_int, _c_int,
                                                       _c_int]),
     "sla2h_jvp16": (_c_int, [_p, _p, _p, _p, _p, _p, _p, _c_int, _p, _c_int, _c_int, _c_int,

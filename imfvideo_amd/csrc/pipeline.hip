@@ -8,6 +8,7 @@
 // On small shapes the op is bound by the host: per stage a Python wrapper, its
 // output allocations and its launch.  One call per pass leaves the launches.
 #include "common.h"
+#include "quant_pool.h"
 
 namespace sla2h {
 
@@ -249,6 +250,12 @@ int launch_operands(const void* const* x, const int64_t* strides, int dtype, con
                     const float* proj_k, void* const* rows, int8_t* const* xq, float* const* xs,
                     float* qpool, float* kpool_t, void* stream);
 
+// states.hip: INT8 operands, pooled tiles and linear states of the cube op
+int quant_states(const QuantPoolArgs& a, const void* k, const void* dk, const void* v,
+                 const void* dv, int dtype, int B, int H, int Np, const float* proj_q,
+                 const float* proj_k, float* Hb, float* dHb, float* zb, float* dzb, void* vt,
+                 void* kt, void* stream);
+
 // states.hip: the backward's complement records from given masks (word (kcq, n))
 int complement_gemm_bwd(const float* P, const float* Pz, const uint32_t* cbits, int BH, int Mb,
                         void* comp, void* stream);
@@ -276,28 +283,28 @@ extern "C" size_t sla2h_cube_jvp_workspace_bytes(int B, int H, int64_t L, int Np
   return JvpWs(nullptr, Dims(B, H, L, Np, kT, T), tangent != 0, true).bytes;
 }
 
-extern "C" int sla2h_cube_jvp_quant(const void* q, const void* k, int dtype, int B, int H,
-                                    int64_t L, int Np, int T, int tangent, const float* proj_q,
-                                    const float* proj_k, void* workspace, float* qpool,
-                                    float* kpool_t, void* stream) {
-  SLA2H_CHECK_ARG(workspace && dims_ok(dtype, B, H, L, Np, kT, T));
-  const JvpWs w(workspace, Dims(B, H, L, Np, kT, T), tangent != 0, true);
-  return sla2h_quant_pool_qk(q, k, dtype, B, H, L, kT, kT, Np, proj_q, proj_k, w.q8, w.qs, w.k8,
-                             w.ks, qpool, kpool_t, w.kb, stream);
+extern "C" int sla2h_cube_jvp_quant(const void* q, const void* k, const void* v, const void* dk,
+                                    const void* dv, int dtype, int B, int H, int64_t L, int Np,
+                                    int T, const float* proj_q, const float* proj_k,
+                                    void* workspace, float* qpool, float* kpool_t, void* stream) {
+  SLA2H_CHECK_ARG(q && k && v && workspace && qpool && kpool_t && dims_ok(dtype, B, H, L, Np, kT, T));
+  SLA2H_CHECK_ARG((dk == nullptr) == (dv == nullptr));
+  SLA2H_CHECK_ARG((int64_t)B * H * 2 <= 65535 && (int64_t)Np * kT <= L);
+  const JvpWs w(workspace, Dims(B, H, L, Np, kT, T), dk != nullptr, true);
+  const QuantPoolArgs a = quant_pool_qk_args(q, k, B * H, L, Np, proj_q, proj_k, w.q8, w.qs, w.k8,
+                                             w.ks, qpool, kpool_t, w.kb);
+  return quant_states(a, k, dk, v, dv, dtype, B, H, Np, proj_q, proj_k, w.Hb, w.dHb, w.zb, w.dzb,
+                      w.vt, w.kt, stream);
 }
 
-extern "C" int sla2h_cube_jvp_attn(const void* q, const void* k, const void* v, const void* dq,
-                                   const void* dk, const void* dv, const float* alpha,
+extern "C" int sla2h_cube_jvp_attn(const void* q, const void* dq, const float* alpha,
                                    int alpha_stride, const int32_t* lut, int dtype, int B, int H,
                                    int64_t L, int Np, int T, float scale, float eps_l,
                                    void* workspace, float* o, float* d_o, void* stream) {
   SLA2H_CHECK_ARG(workspace && lut && dims_ok(dtype, B, H, L, Np, kT, T));
   const bool tan = dq != nullptr;
-  SLA2H_CHECK_ARG(!tan || (dk && dv && d_o));
+  SLA2H_CHECK_ARG(!tan || d_o);
   const JvpWs w(workspace, Dims(B, H, L, Np, kT, T), tan, true);
-  SLA2H_TRY(sla2h_linear_states(k, tan ? dk : nullptr, v, tan ? dv : nullptr, dtype, B, H, L, kT,
-                                kT, Np, w.Hb, w.dHb, w.zb, w.dzb, nullptr, nullptr, nullptr,
-                                nullptr, w.vt, w.kt, stream));
   const int Mb = (int)((L + kT - 1) / kT);
   SLA2H_TRY(sla2h_complement(w.Hb, w.dHb, w.zb, w.dzb, lut, B, H, Mb, Np, kT, T, w.bits, w.comp,
                              stream));

@@ -7,6 +7,7 @@
 //   global sums    models/sla2_cube_qat.py:645-648
 //   complement     models/sla2_cube_qat.py:510-523, 570-578
 #include "common.h"
+#include "quant_pool.h"
 
 #include <mutex>
 
@@ -41,22 +42,28 @@ constexpr size_t kRecBytes = 2 * 16384 + 2 * 256;
 // sum and 4-byte stores, us: 8 heads x 468 tiles with tangent 68.6 -> 62.0 (370
 // MB, 6.0 TB/s), primal 35.1 -> 28.7, training 16 x 468 60.5 -> 44.4, 4 x 64 with
 // tangent 13.1 -> 10.2.
-template <typename T16, bool TAN, bool ROUND = false, bool RH = false>
-__global__ __launch_bounds__(256) void linear_states_kernel(
+template <bool TAN>
+struct StatesLds {  // 16-byte aligned
+  // phi rows (hi, lo), then (tangent, second phase) dphi rows: one buffer keeps
+  // the LDS footprint at four workgroups per CU
+  uint16_t ph[2][kT][kLds];   // [hi/lo][r][d]
+  uint16_t vs[kT][kLds];      // [r][c]
+  uint16_t dvs[TAN ? kT : 1][kLds];
+  float zred[2][4][kT];
+};
+
+template <typename T16, bool TAN, bool ROUND, bool RH>
+__device__ __forceinline__ void linear_states_tile(
     const uint16_t* __restrict__ K, const uint16_t* __restrict__ dK,
     const uint16_t* __restrict__ V, const uint16_t* __restrict__ dV, int64_t L, int Np, int Nb,
     float* __restrict__ Hb, float* __restrict__ dHb, float* __restrict__ zb,
-    float* __restrict__ dzb, uint16_t* __restrict__ vt, uint16_t* __restrict__ kt) {
-  // phi rows (hi, lo), then (tangent, second phase) dphi rows: one buffer keeps
-  // the LDS footprint at four workgroups per CU
-  __shared__ __align__(16) uint16_t ph[2][kT][kLds];   // [hi/lo][r][d]
-  __shared__ __align__(16) uint16_t vs[kT][kLds];      // [r][c]
-  __shared__ __align__(16) uint16_t dvs[TAN ? kT : 1][kLds];
-  __shared__ float zred[2][4][kT];
-
+    float* __restrict__ dzb, uint16_t* __restrict__ vt, uint16_t* __restrict__ kt, int n, int bh,
+    StatesLds<TAN>& lds) {
+  auto& ph = lds.ph;
+  auto& vs = lds.vs;
+  auto& dvs = lds.dvs;
+  auto& zred = lds.zred;
   const int tid = threadIdx.x;
-  const int n = blockIdx.x;
-  const int bh = blockIdx.y;
   const int r = tid >> 2;
   const int c0 = (tid & 3) * 16;
   const int w = tid >> 6, l = tid & 63, lr = l & 15, g = l >> 4;
@@ -273,6 +280,45 @@ __global__ __launch_bounds__(256) void linear_states_kernel(
     *reinterpret_cast<f32x4*>(Hb + hbase + 16 * ct) = x;
     if (TAN) *reinterpret_cast<f32x4*>(dHb + hbase + 16 * ct) = dacc[ct];
   }
+}
+
+template <typename T16, bool TAN, bool ROUND = false, bool RH = false>
+__global__ __launch_bounds__(256) void linear_states_kernel(
+    const uint16_t* __restrict__ K, const uint16_t* __restrict__ dK,
+    const uint16_t* __restrict__ V, const uint16_t* __restrict__ dV, int64_t L, int Np, int Nb,
+    float* __restrict__ Hb, float* __restrict__ dHb, float* __restrict__ zb,
+    float* __restrict__ dzb, uint16_t* __restrict__ vt, uint16_t* __restrict__ kt) {
+  __shared__ __align__(16) StatesLds<TAN> lds;
+  linear_states_tile<T16, TAN, ROUND, RH>(K, dK, V, dV, L, Np, Nb, Hb, dHb, zb, dzb, vt, kt,
+                                          blockIdx.x, blockIdx.y, lds);
+}
+
+// (batch, head, block) tiles that one grid of three workgroups each holds (2^32 threads)
+constexpr int64_t kFusedStatesTiles = 1 << 22;
+
+// The states and, independent of them, the INT8 quantisation and pooling of q
+// and k in one launch: workgroups 0 .. BH Nb - 1 take a states tile each (the
+// longer ones first), the others a quantisation tile.  The quantisation is bound
+// by its barrier and pooling chain, the states by HBM, so they fill each other's
+// gaps, and a small call saves a launch.  As two launches -> one, us: 4 heads x 5
+// tiles 11.1 -> 6.0, 4 x 64 13.0 -> 8.2, 8 x 130 27.8 -> 22.1, 8 x 468 91.3 -> 86.3,
+// 16 x 218 93.6 -> 89.7 (tangent); primal 8 x 468 49.6 -> 47.8.
+template <typename T16, bool TAN>
+__global__ __launch_bounds__(256) void quant_states_kernel(
+    QuantPoolArgs a, int ntiles, const uint16_t* __restrict__ K, const uint16_t* __restrict__ dK,
+    const uint16_t* __restrict__ V, const uint16_t* __restrict__ dV, int Np,
+    float* __restrict__ Hb, float* __restrict__ dHb, float* __restrict__ zb,
+    float* __restrict__ dzb, uint16_t* __restrict__ vt, uint16_t* __restrict__ kt) {
+  constexpr size_t kBytes = sizeof(StatesLds<TAN>) > sizeof(QuantPoolLds) ? sizeof(StatesLds<TAN>)
+                                                                          : sizeof(QuantPoolLds);
+  __shared__ __align__(16) unsigned char lds[kBytes];
+  const int ns = a.BH * a.Nb, i = blockIdx.x;
+  if (i < ns)
+    linear_states_tile<T16, TAN, false, false>(K, dK, V, dV, a.L, Np, a.Nb, Hb, dHb, zb, dzb, vt, kt,
+                                               i % a.Nb, i / a.Nb,
+                                               *reinterpret_cast<StatesLds<TAN>*>(lds));
+  else
+    quant_pool_tiles<T16>(a, ntiles, i - ns, gridDim.x - ns, *reinterpret_cast<QuantPoolLds*>(lds));
 }
 
 // Global sums over the Np tiles in a fixed order (deterministic): four
@@ -874,6 +920,40 @@ extern "C" int sla2h_complement(const float* Hb, const float* dHb, const float* 
         Hb, nullptr, zb, nullptr, cbits, Mb, Np, MT, NC, out, nullptr, 0, nullptr);
   return (int)hipGetLastError();
 }
+
+namespace sla2h {
+
+// sla2h_quant_pool_qk (a) and sla2h_linear_states without the global sums, in one
+// launch where its grid holds them.
+int quant_states(const QuantPoolArgs& a, const void* k, const void* dk, const void* v,
+                 const void* dv, int dtype, int B, int H, int Np, const float* proj_q,
+                 const float* proj_k, float* Hb, float* dHb, float* zb, float* dzb, void* vt,
+                 void* kt, void* stream) {
+  const int64_t ns = (int64_t)a.BH * a.Nb;
+  if (ns <= kFusedStatesTiles) {
+    SLA2H_CHECK_ARG(k && v && Hb && zb && vt && Np > 0 && (int64_t)Np * kT <= a.L);
+    SLA2H_CHECK_ARG(dtype == SLA2H_DTYPE_F16 || dtype == SLA2H_DTYPE_BF16);
+    if (dk) SLA2H_CHECK_ARG(dv && dHb && dzb && kt);
+    auto run = [&](auto kernel) {
+      kernel<<<(unsigned)(3 * ns), 256, 0, static_cast<hipStream_t>(stream)>>>(
+          a, (int)(2 * ns), static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(dk),
+          static_cast<const uint16_t*>(v), static_cast<const uint16_t*>(dv), Np, Hb, dHb, zb, dzb,
+          static_cast<uint16_t*>(vt), static_cast<uint16_t*>(kt));
+      return (int)hipGetLastError();
+    };
+    if (dtype == SLA2H_DTYPE_BF16)
+      return dk ? run(quant_states_kernel<BF16, true>) : run(quant_states_kernel<BF16, false>);
+    return dk ? run(quant_states_kernel<F16, true>) : run(quant_states_kernel<F16, false>);
+  }
+  const int err = sla2h_quant_pool_qk(a.x[0], a.x[1], dtype, B, H, a.L, kT, kT, Np, proj_q, proj_k,
+                                      a.xq[0], a.xs[0], a.xq[1], a.xs[1], a.pool[0], a.pool[1],
+                                      a.kb[1], stream);
+  if (err) return err;
+  return sla2h_linear_states(k, dk, v, dv, dtype, B, H, a.L, kT, kT, Np, Hb, dHb, zb, dzb, nullptr,
+                             nullptr, nullptr, nullptr, vt, kt, stream);
+}
+
+}  // namespace sla2h
 
 extern "C" int sla2h_complement_noalloc(const float* Hb, const float* dHb, const float* zb,
                                         const float* dzb, const int32_t* lut, int B, int H,

@@ -344,16 +344,16 @@ def _cube_jvp_call(q, k, v, dq, dk, dv, alpha, topk_frac, Np, proj_q, proj_k, lu
     qpool = torch.empty(B, H, nb, D, device=dev, dtype=torch.float32)
     kpool_t = torch.empty(B, H, D, Np, device=dev, dtype=torch.float32)
     _lib.check(lib.sla2h_cube_jvp_quant(
-        q.data_ptr(), k.data_ptr(), code, B, H, L, Np, T, tan, _ptr(pq), _ptr(pk), ws.data_ptr(),
-        qpool.data_ptr(), kpool_t.data_ptr(), st), "sla2h_cube_jvp_quant")
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), *((_ptr(dk), _ptr(dv)) if tan else (None, None)),
+        code, B, H, L, Np, T, _ptr(pq), _ptr(pk), ws.data_ptr(), qpool.data_ptr(), kpool_t.data_ptr(), st),
+        "sla2h_cube_jvp_quant")
     if lut is None:
         lut = route_topk(qpool, kpool_t, T, scale)
     o = torch.empty(B, H, L, D, device=dev, dtype=torch.float32)
     do = torch.empty_like(o) if tan else None
     _lib.check(lib.sla2h_cube_jvp_attn(
-        q.data_ptr(), k.data_ptr(), v.data_ptr(), _ptr(dq), _ptr(dk), _ptr(dv), alpha.data_ptr(),
-        alpha.stride(0), lut.data_ptr(), code, B, H, L, Np, T, scale, 1e-5, ws.data_ptr(),
-        o.data_ptr(), _ptr(do), st), "sla2h_cube_jvp_attn")
+        q.data_ptr(), _ptr(dq), alpha.data_ptr(), alpha.stride(0), lut.data_ptr(), code, B, H, L,
+        Np, T, scale, 1e-5, ws.data_ptr(), o.data_ptr(), _ptr(do), st), "sla2h_cube_jvp_attn")
     return o, do
 
 

@@ -759,18 +759,18 @@ int sla2h_linear_wgrad(const void* dy, int64_t ldy, const void* x, int64_t ldx, 
  * --------------------------------------------------------------------- */
 
 /*
- * The cube op and its JVP (dq = dk = dv = d_o = NULL and tangent = 0: primal
- * only): sla2h_cube_jvp_quant (sla2h_quant_pool_qk into the workspace, the pooled
- * tiles to qpool / kpool_t), then the caller's routing (sla2h_route_topk or a LUT
- * of its own), then sla2h_cube_jvp_attn (sla2h_linear_states, sla2h_complement,
- * sla2h_fwd_jvp) with the same sizes and workspace.
+ * The cube op and its JVP (dq = dk = dv = d_o = NULL: primal only):
+ * sla2h_cube_jvp_quant (sla2h_quant_pool_qk and sla2h_linear_states into the
+ * workspace, the pooled tiles to qpool / kpool_t), then the caller's routing
+ * (sla2h_route_topk or a LUT of its own), then sla2h_cube_jvp_attn
+ * (sla2h_complement, sla2h_fwd_jvp) with the same sizes and workspace.
  */
 size_t sla2h_cube_jvp_workspace_bytes(int B, int H, int64_t L, int Np, int T, int tangent);
-int sla2h_cube_jvp_quant(const void* q, const void* k, int dtype, int B, int H, int64_t L, int Np,
-                         int T, int tangent, const float* proj_q, const float* proj_k,
-                         void* workspace, float* qpool, float* kpool_t, void* stream);
-int sla2h_cube_jvp_attn(const void* q, const void* k, const void* v, const void* dq,
-                        const void* dk, const void* dv, const float* alpha, int alpha_stride,
+int sla2h_cube_jvp_quant(const void* q, const void* k, const void* v, const void* dk,
+                         const void* dv, int dtype, int B, int H, int64_t L, int Np, int T,
+                         const float* proj_q, const float* proj_k, void* workspace, float* qpool,
+                         float* kpool_t, void* stream);
+int sla2h_cube_jvp_attn(const void* q, const void* dq, const float* alpha, int alpha_stride,
                         const int32_t* lut, int dtype, int B, int H, int64_t L, int Np, int T,
                         float scale, float eps_l, void* workspace, float* o, float* d_o,
                         void* stream);

@@ -113,6 +113,27 @@ def test_linear_states_and_complement():
     assert rel_l2(zc, wz) < 1e-5
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,Np,P", [(1, 1, 0), (3, 1, 1), (2, 7, 65), (4, 33, 0), (8, 130, 77)])
+def test_quant_and_states_in_one_launch(H, Np, P, dt):
+    """The operands of a whole call (INT8 values and pooled tiles beside the linear
+    states, one launch), with router projections, against the stages one by one:
+    the same arithmetic, so equal to the bit."""
+    say(f"quant + states {H}x{Np} P={P} {dt}")
+    from imfvideo_amd import ops
+    gen = torch.Generator().manual_seed(Np * 100 + P)
+    rnd = lambda *s: torch.randn(*s, generator=gen)
+    x = [cuda(rnd(1, H, Np * 64 + P, 64).to(dt)) for _ in range(6)]
+    a = cuda(torch.sigmoid(rnd(H, -(-(Np * 64 + P) // 64))))
+    pq, pk = cuda(rnd(64, 64)), cuda(rnd(64, 64))
+    for ins in (x, x[:3] + [None] * 3):
+        f1 = ops.cube_jvp(*ins, a, 0.3, Np, P, pq, pk)
+        f2 = ops.cube_jvp(*ins, a, 0.3, Np, P, pq, pk, return_aux=True)
+        assert torch.equal(f1[0], f2[0])
+        assert (f1[1] is None) == (ins[3] is None)
+        assert f1[1] is None or torch.equal(f1[1], f2[1])
+
+
 @pytest.mark.parametrize("tan", [False, True])
 @pytest.mark.parametrize("BH,Mb,Np,T", [
     (1, 1, 1, 1), (2, 3, 4, 4), (4, 17, 31, 5), (4, 32, 32, 32), (4, 31, 33, 33), (4, 64, 64, 16),
