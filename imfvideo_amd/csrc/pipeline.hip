@@ -250,6 +250,14 @@ int launch_operands(const void* const* x, const int64_t* strides, int dtype, con
                     const float* proj_k, void* const* rows, int8_t* const* xq, float* const* xs,
                     float* qpool, float* kpool_t, void* stream);
 
+// states.hip: sla2h_linear_states_qat without the sums over the tiles, and
+// sla2h_complement with them
+int linear_states_train(const void* k, const void* v, int dtype, int B, int H, int64_t L, int D,
+                        int E, float* Hb, float* zb, void* vt, void* stream);
+int complement_sums(const float* Hb, const float* dHb, const float* zb, const float* dzb,
+                    const int32_t* lut, int B, int H, int Mb, int Np, int D, int T,
+                    void* workspace, void* comp, float* Hall, float* zall, void* stream);
+
 // states.hip: INT8 operands, pooled tiles and linear states of the cube op
 int quant_states(const QuantPoolArgs& a, const void* k, const void* dk, const void* v,
                  const void* dv, int dtype, int B, int H, int Np, const float* proj_q,
@@ -396,16 +404,15 @@ extern "C" int sla2h_train_fwd(const void* q, const void* k, const void* v,
                                       H, L, kT, bq, T, scale, s.o_s, s.lse, s.qphi, stats,
                                       stream));
     }
-    SLA2H_TRY(sla2h_linear_states_qat(k, v, dtype, B, H, L, kT, kT, w.Hb, w.zb, s.Hall, w.zall,
-                                      nullptr, stream));
+    SLA2H_TRY(linear_states_train(k, v, dtype, B, H, L, kT, kT, w.Hb, w.zb, nullptr, stream));
   } else {
-    SLA2H_TRY(sla2h_linear_states_qat(k, v, dtype, B, H, L, kT, kT, w.Hb, w.zb, s.Hall, w.zall,
-                                      w.vt, stream));
+    SLA2H_TRY(linear_states_train(k, v, dtype, B, H, L, kT, kT, w.Hb, w.zb, w.vt, stream));
     SLA2H_TRY(sparse_fwd_1d_stats(q, k, w.vt, s.lut, dtype, B, H, L, kT, bq, kT, d.J, scale,
                                   s.o_s, s.lse, s.qphi, stats, stream));
   }
-  SLA2H_TRY(sla2h_complement(w.Hb, nullptr, w.zb, nullptr, s.lut, B, H, d.Mq, d.Nb, kT, d.J,
-                             s.bits, s.comp, stream));
+  // (zall: the score form's)
+  SLA2H_TRY(complement_sums(w.Hb, nullptr, w.zb, nullptr, s.lut, B, H, d.Mq, d.Nb, kT, d.J, s.bits,
+                            s.comp, s.Hall, d.J <= 4 ? w.zall : nullptr, stream));
   // the reference's linear branch: score form up to 4 LUT columns, else state form
   if (d.J <= 4)
     SLA2H_TRY(sla2h_linear_mix_score(s.qphi, k, v, s.Hall, w.zall, s.lut, d.J, s.o_s, s.alpha,

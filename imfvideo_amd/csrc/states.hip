@@ -321,9 +321,12 @@ __global__ __launch_bounds__(256) void quant_states_kernel(
     quant_pool_tiles<T16>(a, ntiles, i - ns, gridDim.x - ns, *reinterpret_cast<QuantPoolLds*>(lds));
 }
 
-// Global sums over the Np tiles in a fixed order (deterministic): four
-// contiguous ranges of tiles summed in sequence by four threads of a column,
-// then ((r0 + r1) + (r2 + r3)).  64 columns per workgroup of 256 threads.
+// Global sums over the Np tiles in a fixed order (deterministic): eight partial
+// sums of a column, partial w over tiles 32 c + 4 w .. + 3 of every group c of 32
+// in order, four at a time as (x0 + x1) + (x2 + x3); then ((p0 + p1) + (p2 + p3))
+// + ((p4 + p5) + (p6 + p7)).  It is the order in which comp_gemm_kernel sums
+// (SUM below), so both give the same bits.  64 columns per workgroup of 256
+// threads, two partials a thread.
 // Column index e spans [Hb 4096 | dHb 4096 | zb 64 | dzb 64].
 __global__ __launch_bounds__(256) void states_sum_kernel(const float* __restrict__ Hb,
                                                         const float* __restrict__ dHb,
@@ -333,7 +336,7 @@ __global__ __launch_bounds__(256) void states_sum_kernel(const float* __restrict
                                                         float* __restrict__ dHall,
                                                         float* __restrict__ zall,
                                                         float* __restrict__ dzall) {
-  __shared__ float part[4][64];
+  __shared__ float part[8][64];
   const int c = threadIdx.x & 63, part_id = threadIdx.x >> 6;
   const int e = blockIdx.x * 64 + c;
   const int bh = blockIdx.y;
@@ -350,16 +353,23 @@ __global__ __launch_bounds__(256) void states_sum_kernel(const float* __restrict
     src = dzb; dst = dzall; stride = 64; col = e - 8256;
   }
   if (src == nullptr) return;  // uniform: a workgroup never spans two parts
-  const int chunk = (Np + 3) / 4;
-  const int n0 = part_id * chunk, n1 = min(Np, n0 + chunk);
   const float* p = src + (int64_t)bh * Np * stride + col;
-  float acc = 0.f;
-#pragma unroll 8
-  for (int nn = n0; nn < n1; ++nn) acc += p[(int64_t)nn * stride];
-  part[part_id][c] = acc;
+  float acc[2] = {0.f, 0.f};
+  auto at = [&](int n) { return n < Np ? p[(int64_t)n * stride] : 0.f; };
+#pragma unroll 4
+  for (int n0 = 4 * part_id; n0 < Np; n0 += 32)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int n = n0 + 16 * u;
+      acc[u] += (at(n) + at(n + 1)) + (at(n + 2) + at(n + 3));
+    }
+  part[part_id][c] = acc[0];
+  part[part_id + 4][c] = acc[1];
   __syncthreads();
   if (part_id == 0)
-    dst[(int64_t)bh * stride + col] = (part[0][c] + part[1][c]) + (part[2][c] + part[3][c]);
+    dst[(int64_t)bh * stride + col] =
+        ((part[0][c] + part[1][c]) + (part[2][c] + part[3][c])) +
+        ((part[4][c] + part[5][c]) + (part[6][c] + part[7][c]));
 }
 
 // ---------------------------------------------------------------------------
@@ -501,12 +511,18 @@ __global__ __launch_bounds__(512) void comp_mask_kernel(const int32_t* __restric
 // MASK: the workgroup builds the mask words of its rows itself, in LDS, from
 // the LUT (and the one of column tile 0 also stores them to cbits_out), and the
 // z columns are two more column tiles: no comp_mask_kernel before it.
-template <bool TAN, bool MASK>
+//
+// SUM (training): the column sums over all tiles as well, Hall and (may be NULL)
+// zall, in fp32 from the rows that the staging holds anyway, where
+// states_sum_kernel read them again: 16 heads x 468 tiles 25 us, 4 x 64 tiles
+// 4 us and a launch; the GEMM takes the same time.
+template <bool TAN, bool MASK, bool SUM = false>
 __global__ __launch_bounds__(kCompThreads, 4) void comp_gemm_kernel(
     const float* __restrict__ Hb, const float* __restrict__ dHb, const float* __restrict__ zb,
     const float* __restrict__ dzb, const uint32_t* __restrict__ cbits, int Mb, int Np, int MT,
     int NC, unsigned char* __restrict__ comp, const int32_t* __restrict__ lut, int T,
-    uint32_t* __restrict__ cbits_out) {
+    uint32_t* __restrict__ cbits_out, float* __restrict__ Hall, float* __restrict__ zall) {
+  __shared__ float psum[SUM ? 2 : 1][SUM ? 8 : 1][kCompCols];
   extern __shared__ uint32_t lbits[];  // MASK: [kc][local row], 16 kMaskSub rows
   __shared__ __align__(16) uint16_t sb[2][2][kCompCols][40];  // [buf][hi/lo][column][n] (+pad)
   __shared__ __align__(16) uint32_t mw[2][MASK ? 1 : 16 * kMaskSub];  // [buf][local row] mask words
@@ -588,7 +604,9 @@ __global__ __launch_bounds__(kCompThreads, 4) void comp_gemm_kernel(
                                              rs, xoff + (32 * kc + j) * stride * 4, 0, 0));
     if (!MASK) c.mk = __builtin_amdgcn_raw_buffer_load_b32(rb, (kc * MTp + m0 + tid) * 4, 0, 0);
   };
-  auto store_chunk = [&](int buf, const Chunk& c) {
+  float sum = 0.f;
+  auto store_chunk = [&](int buf, const Chunk& c, int kc) {
+    if (SUM && kc < NC) sum += (c.x[0] + c.x[1]) + (c.x[2] + c.x[3]);
     u32x2 hi, lo;
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
@@ -628,19 +646,51 @@ __global__ __launch_bounds__(kCompThreads, 4) void comp_gemm_kernel(
   Chunk ca, cb;
   load_chunk(0, ca);
   load_chunk(1, cb);
-  store_chunk(0, ca);
+  store_chunk(0, ca, 0);
   __syncthreads();
   for (int kc = 0; kc < NC; kc += 2) {
     // chunk kc in buffer 0, chunk kc+1 in registers cb
     load_chunk(kc + 2, ca);
     compute(0, kc);
-    store_chunk(1, cb);  // buffer 1 was last read before the previous barrier
+    store_chunk(1, cb, kc + 1);  // buffer 1 was last read before the previous barrier
     __syncthreads();
     if (kc + 1 >= NC) break;
     load_chunk(kc + 3, cb);
     compute(1, kc + 1);
-    store_chunk(0, ca);
+    store_chunk(0, ca, kc + 2);
     __syncthreads();
+  }
+
+  if constexpr (SUM) {
+    // with the masks the z columns are a column tile of their own; otherwise the
+    // first column tile's workgroup sums them too
+    const bool zsum = !MASK && c0 == 0 && zall != nullptr;
+    psum[0][w][l] = sum;
+    if (zsum) {
+      const auto rz = make_rsrc(zb + (int64_t)bh * Np * 64, (int64_t)Np * 256);
+      float zs = 0.f;
+#pragma unroll 4
+      for (int kc = 0; kc < NC; ++kc) {
+        float x[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          x[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                               rz, (32 * kc + 4 * w + j) * 256 + 4 * l, 0, 0));
+        zs += (x[0] + x[1]) + (x[2] + x[3]);
+      }
+      psum[1][w][l] = zs;
+    }
+    __syncthreads();
+    if (w < 2 && blockIdx.z == 0) {
+      float* dst = w == 0 ? (part == 0 ? Hall + (int64_t)bh * 4096 + col0
+                                       : (zall != nullptr ? zall + (int64_t)bh * 64 : nullptr))
+                          : (zsum ? zall + (int64_t)bh * 64 : nullptr);
+      if (dst != nullptr) {
+        const auto& p = psum[w];
+        dst[l] = ((p[0][l] + p[1][l]) + (p[2][l] + p[3][l])) +
+                 ((p[4][l] + p[5][l]) + (p[6][l] + p[7][l]));
+      }
+    }
   }
 
   // records: lane (g, r) element i = C[16 mt + 4g + i][c0 + 16 ct + r]; 16
@@ -711,10 +761,12 @@ extern "C" int sla2h_linear_states(const void* k, const void* dk, const void* v,
   return (int)hipGetLastError();
 }
 
-extern "C" int sla2h_linear_states_qat(const void* k, const void* v, int dtype, int B, int H,
-                                       int64_t L, int D, int E, float* Hb, float* zb, float* Hall,
-                                       float* zall, void* vt, void* stream) {
-  SLA2H_CHECK_ARG(k && v && Hb && zb && Hall && zall);
+namespace sla2h {
+
+// sla2h_linear_states_qat without the sums over the tiles
+int linear_states_train(const void* k, const void* v, int dtype, int B, int H, int64_t L, int D,
+                        int E, float* Hb, float* zb, void* vt, void* stream) {
+  SLA2H_CHECK_ARG(k && v && Hb && zb);
   SLA2H_CHECK_ARG(D == kT && E == kT);
   SLA2H_CHECK_ARG(dtype == SLA2H_DTYPE_F16 || dtype == SLA2H_DTYPE_BF16);
   SLA2H_CHECK_ARG(B > 0 && H > 0 && B * H <= 65535 && L > 0);
@@ -727,10 +779,21 @@ extern "C" int sla2h_linear_states_qat(const void* k, const void* v, int dtype, 
     linear_states_kernel<BF16, false, true><<<grid, 256, 0, st>>>(K, nullptr, V, nullptr, L, Nb, Nb, Hb, nullptr, zb, nullptr, static_cast<uint16_t*>(vt), nullptr);
   else
     linear_states_kernel<F16, false, true><<<grid, 256, 0, st>>>(K, nullptr, V, nullptr, L, Nb, Nb, Hb, nullptr, zb, nullptr, static_cast<uint16_t*>(vt), nullptr);
-  int err = (int)hipGetLastError();
+  return (int)hipGetLastError();
+}
+
+}  // namespace sla2h
+
+extern "C" int sla2h_linear_states_qat(const void* k, const void* v, int dtype, int B, int H,
+                                       int64_t L, int D, int E, float* Hb, float* zb, float* Hall,
+                                       float* zall, void* vt, void* stream) {
+  SLA2H_CHECK_ARG(Hall && zall);
+  const int err = linear_states_train(k, v, dtype, B, H, L, D, E, Hb, zb, vt, stream);
   if (err) return err;
+  const int Nb = (int)((L + E - 1) / E);
   dim3 g2(8320 / 64, B * H);
-  states_sum_kernel<<<g2, 256, 0, st>>>(Hb, nullptr, zb, nullptr, Nb, Hall, nullptr, zall, nullptr);
+  states_sum_kernel<<<g2, 256, 0, static_cast<hipStream_t>(stream)>>>(Hb, nullptr, zb, nullptr, Nb,
+                                                                      Hall, nullptr, zall, nullptr);
   return (int)hipGetLastError();
 }
 
@@ -810,7 +873,7 @@ int complement_gemm_bwd(const float* P, const float* Pz, const uint32_t* cbits, 
   dim3 grid(4160 / kCompCols, BH, (MT + kMaskSub - 1) / kMaskSub);
   comp_gemm_kernel<false, false><<<grid, kCompThreads, 0, static_cast<hipStream_t>(stream)>>>(
       P, nullptr, Pz, nullptr, cbits, Mb, Mb, MT, NC, static_cast<unsigned char*>(comp), nullptr, 0,
-      nullptr);
+      nullptr, nullptr, nullptr);
   return (int)hipGetLastError();
 }
 }  // namespace sla2h
@@ -877,16 +940,19 @@ int complement_scratch(void** out) {
 }
 }  // namespace
 
-extern "C" int sla2h_complement(const float* Hb, const float* dHb, const float* zb,
-                                const float* dzb, const int32_t* lut, int B, int H, int Mb,
-                                int Np, int D, int T, void* workspace, void* comp,
-                                void* stream) {
+namespace sla2h {
+
+// sla2h_complement; with Hall (primal only) the sums of Hb and, where zall is
+// given, of zb over the tiles as well
+int complement_sums(const float* Hb, const float* dHb, const float* zb, const float* dzb,
+                    const int32_t* lut, int B, int H, int Mb, int Np, int D, int T,
+                    void* workspace, void* comp, float* Hall, float* zall, void* stream) {
   SLA2H_CHECK_ARG(Hb && zb && lut && comp && workspace);
   SLA2H_CHECK_ARG(D == kT);
   SLA2H_CHECK_ARG(B > 0 && H > 0 && B * H <= 65535 && Mb > 0 && Np > 0 && Np <= 4096);
   SLA2H_CHECK_ARG(T >= 1 && T <= Np);
   const bool tan = dHb != nullptr;
-  if (tan) SLA2H_CHECK_ARG(dzb);
+  if (tan) SLA2H_CHECK_ARG(dzb && !Hall);
   const int MT = (Mb + 15) / 16, NC = (Np + 31) / 32;
   hipStream_t st = static_cast<hipStream_t>(stream);
   auto cbits = static_cast<uint32_t*>(workspace);
@@ -899,10 +965,13 @@ extern "C" int sla2h_complement(const float* Hb, const float* dHb, const float* 
     const size_t shmem = (size_t)NC * 16 * kMaskSub * 4;
     if (tan)
       comp_gemm_kernel<true, true><<<grid, kCompThreads, shmem, st>>>(
-          Hb, dHb, zb, dzb, nullptr, Mb, Np, MT, NC, out, lut, T, cbits);
+          Hb, dHb, zb, dzb, nullptr, Mb, Np, MT, NC, out, lut, T, cbits, nullptr, nullptr);
+    else if (Hall)
+      comp_gemm_kernel<false, true, true><<<grid, kCompThreads, shmem, st>>>(
+          Hb, nullptr, zb, nullptr, nullptr, Mb, Np, MT, NC, out, lut, T, cbits, Hall, zall);
     else
       comp_gemm_kernel<false, true><<<grid, kCompThreads, shmem, st>>>(
-          Hb, nullptr, zb, nullptr, nullptr, Mb, Np, MT, NC, out, lut, T, cbits);
+          Hb, nullptr, zb, nullptr, nullptr, Mb, Np, MT, NC, out, lut, T, cbits, nullptr, nullptr);
     return (int)hipGetLastError();
   }
   // mask bits plus the z parts of the records; the GEMM takes the H parts only
@@ -914,11 +983,24 @@ extern "C" int sla2h_complement(const float* Hb, const float* dHb, const float* 
   dim3 grid((tan ? 8192 : 4096) / kCompCols, B * H, groups);
   if (tan)
     comp_gemm_kernel<true, false><<<grid, kCompThreads, 0, st>>>(
-        Hb, dHb, zb, dzb, cbits, Mb, Np, MT, NC, out, nullptr, 0, nullptr);
+        Hb, dHb, zb, dzb, cbits, Mb, Np, MT, NC, out, nullptr, 0, nullptr, nullptr, nullptr);
+  else if (Hall)
+    comp_gemm_kernel<false, false, true><<<grid, kCompThreads, 0, st>>>(
+        Hb, nullptr, zb, nullptr, cbits, Mb, Np, MT, NC, out, nullptr, 0, nullptr, Hall, zall);
   else
     comp_gemm_kernel<false, false><<<grid, kCompThreads, 0, st>>>(
-        Hb, nullptr, zb, nullptr, cbits, Mb, Np, MT, NC, out, nullptr, 0, nullptr);
+        Hb, nullptr, zb, nullptr, cbits, Mb, Np, MT, NC, out, nullptr, 0, nullptr, nullptr, nullptr);
   return (int)hipGetLastError();
+}
+
+}  // namespace sla2h
+
+extern "C" int sla2h_complement(const float* Hb, const float* dHb, const float* zb,
+                                const float* dzb, const int32_t* lut, int B, int H, int Mb,
+                                int Np, int D, int T, void* workspace, void* comp,
+                                void* stream) {
+  return complement_sums(Hb, dHb, zb, dzb, lut, B, H, Mb, Np, D, T, workspace, comp, nullptr,
+                         nullptr, stream);
 }
 
 namespace sla2h {

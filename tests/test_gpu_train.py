@@ -456,6 +456,30 @@ def test_sla2_train_1d_config_shape():
         assert rel_l2(da[sl].cpu(), rb["d_alpha"]) < 1e-2
 
 
+@pytest.mark.parametrize("H,nb,T", [(9, 3, 1), (2, 33, 4), (1, 97, 2), (3, 130, 12), (1, 64, 16),
+                                    (1, 520, 3)])
+def test_state_sums_beside_the_complement(H, nb, T):
+    """The whole call takes the sums of the states over the tiles from the
+    complement GEMM (masks inside it or not, one and two groups of query blocks,
+    zall for the score form), the stages from their own kernel, in the same fp32
+    order: outputs and gradients equal to the bit."""
+    from imfvideo_amd import ops
+    print("[case] state sums", H, nb, T, flush=True)
+    g = torch.Generator().manual_seed(nb + T)
+    L = nb * 64
+    q, k, v, do = (torch.randn(1, H, L, 64, generator=g).half().cuda() for _ in range(4))
+    lut = torch.stack([torch.randperm(nb, generator=g)[:T] for _ in range(H * nb)])
+    lut = lut.view(1, H, nb, T).to(torch.int32).cuda()
+    logit = torch.randn(H, nb, generator=g).cuda()
+    o, saved = ops.train_op_fwd(q, k, v, logit, lut, nb)
+    a = torch.sigmoid(logit)
+    ref = ops.train_fwd(q, k, v, a, lut, nb)
+    assert torch.equal(o, ref["o"])
+    got = ops.train_op_bwd(q, k, v, do, saved, nb, T)
+    want = ops.train_bwd(q, k, v, a, ref, do)
+    assert all(torch.equal(x, y) for x, y in zip(got[:3], want[:3]))
+
+
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,H,L,Np,bq,T", [(1, 1, 64, 1, 64, 1), (2, 3, 274, 4, 64, 2),
                                            (1, 2, 700, 8, 64, 5), (2, 2, 583, 10, 128, 3),
