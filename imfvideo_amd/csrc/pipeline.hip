@@ -9,6 +9,7 @@
 // output allocations and its launch.  One call per pass leaves the launches.
 #include "common.h"
 #include "quant_pool.h"
+#include "train_setup.h"
 
 namespace sla2h {
 
@@ -49,22 +50,10 @@ bool dims_ok(int dtype, int B, int H, int64_t L, int Np, int bq, int T) {
          (int64_t)(Np - 1) * kT < L && (bq == 64 || bq == 128 || bq == 256) && T >= 1 && T <= Np;
 }
 
-// alpha = sigmoid(logit); LUT rows with the tail blocks Np .. Nb - 1 appended;
-// stats = -inf.  Each part may be absent (n = 0 or NULL).
-__global__ __launch_bounds__(256) void train_setup_kernel(const float* __restrict__ logit, int na,
-                                                         float* __restrict__ alpha,
-                                                         const int32_t* __restrict__ lut,
-                                                         int64_t nl, int T, int J, int Np,
-                                                         int32_t* __restrict__ lut_aug,
-                                                         float* __restrict__ stats, int H) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < na) alpha[i] = 1.0f / (1.0f + expf(-logit[i]));
-  if (stats != nullptr && i < H) stats[i] = -INFINITY;
-  if (i < nl) {
-    const int64_t row = i / J;
-    const int j = (int)(i - row * J);
-    lut_aug[i] = j < T ? lut[row * T + j] : Np + (j - T);
-  }
+constexpr int64_t kEarlyStates = 2560;  // tiles: 40 MB of states
+
+__global__ __launch_bounds__(256) void train_setup_kernel(TrainSetup a) {
+  train_setup(a, (int64_t)blockIdx.x * 256 + threadIdx.x);
 }
 
 // Two small jobs between bwd_prep and the backward's products.
@@ -250,10 +239,10 @@ int launch_operands(const void* const* x, const int64_t* strides, int dtype, con
                     const float* proj_k, void* const* rows, int8_t* const* xq, float* const* xs,
                     float* qpool, float* kpool_t, void* stream);
 
-// states.hip: sla2h_linear_states_qat without the sums over the tiles, and
-// sla2h_complement with them
-int linear_states_train(const void* k, const void* v, int dtype, int B, int H, int64_t L, int D,
-                        int E, float* Hb, float* zb, void* vt, void* stream);
+// states.hip: sla2h_linear_states_qat without the sums over the tiles and the
+// setup of a training forward, in one launch; sla2h_complement with the sums
+int states_and_setup(const void* k, const void* v, int dtype, int B, int H, int64_t L, float* Hb,
+                     float* zb, void* vt, const TrainSetup& setup, void* stream);
 int complement_sums(const float* Hb, const float* dHb, const float* zb, const float* dzb,
                     const int32_t* lut, int B, int H, int Mb, int Np, int D, int T,
                     void* workspace, void* comp, float* Hall, float* zall, void* stream);
@@ -342,7 +331,7 @@ extern "C" int sla2h_jvp16(const void* q, const void* k, const void* v, const vo
   if (d.J > T) {
     const int64_t nl = (int64_t)d.BH * d.Mq * d.J;
     train_setup_kernel<<<(unsigned)((nl + 255) / 256), 256, 0, st>>>(
-        nullptr, 0, nullptr, lut, nl, T, d.J, Np, w.lut, nullptr, 0);
+        TrainSetup{nullptr, 0, nullptr, lut, nl, T, d.J, Np, w.lut, nullptr, 0});
     SLA2H_TRY((int)hipGetLastError());
     lut = w.lut;
   }
@@ -384,13 +373,25 @@ extern "C" int sla2h_train_fwd(const void* q, const void* k, const void* v,
   SLA2H_CHECK_ARG(bq == kT || Np == d.Nb);  // the prefix tail goes with 64-row query blocks
   const Saved s(saved, d);
   const FwdWs w(workspace, d, int8 != 0);
-  hipStream_t st = static_cast<hipStream_t>(stream);
   const int64_t nl = (int64_t)d.BH * d.Mq * d.J;
   const int na = H * d.Mq;
-  const int64_t n = nl > na ? nl : na;
-  train_setup_kernel<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(
-      alpha_logit, na, s.alpha, lut, nl, T, d.J, Np, s.lut, stats, H);
-  SLA2H_TRY((int)hipGetLastError());
+  // stats, alpha and the whole LUT rows, beside the states (w.vt: the 16-bit sparse
+  // kernel's).  Large INT8 calls keep the states behind the sparse kernel, next to
+  // the complement that reads them while they are still in the caches, and the
+  // setup in a launch of its own.  States behind -> before the sparse kernel, us a
+  // forward: 256 tiles 37.3 -> 34.9, 1040 83.8 -> 82.8, 2048 161.8 -> 159.6; 3200
+  // 302.6 -> 307.3, 7488 722 -> 735.
+  const TrainSetup setup{alpha_logit, na, s.alpha, lut, nl, T, d.J, Np, s.lut, stats, H};
+  const bool late = int8 && (int64_t)d.BH * d.Nb > kEarlyStates;
+  if (late) {
+    const int64_t n = nl > na ? nl : na;
+    train_setup_kernel<<<(unsigned)((n + 255) / 256), 256, 0, static_cast<hipStream_t>(stream)>>>(
+        setup);
+    SLA2H_TRY((int)hipGetLastError());
+  } else {
+    SLA2H_TRY(states_and_setup(k, v, dtype, B, H, L, w.Hb, w.zb, int8 ? nullptr : w.vt, setup,
+                               stream));
+  }
   if (int8) {
     if (!quantised)
       SLA2H_TRY(sla2h_quant_train(q, k, v, dtype, B, H, L, kT, kT, w.q8, w.qs, w.k8, w.ks, w.v8f,
@@ -404,9 +405,9 @@ extern "C" int sla2h_train_fwd(const void* q, const void* k, const void* v,
                                       H, L, kT, bq, T, scale, s.o_s, s.lse, s.qphi, stats,
                                       stream));
     }
-    SLA2H_TRY(linear_states_train(k, v, dtype, B, H, L, kT, kT, w.Hb, w.zb, nullptr, stream));
+    if (late)
+      SLA2H_TRY(states_and_setup(k, v, dtype, B, H, L, w.Hb, w.zb, nullptr, TrainSetup{}, stream));
   } else {
-    SLA2H_TRY(linear_states_train(k, v, dtype, B, H, L, kT, kT, w.Hb, w.zb, w.vt, stream));
     SLA2H_TRY(sparse_fwd_1d_stats(q, k, w.vt, s.lut, dtype, B, H, L, kT, bq, kT, d.J, scale,
                                   s.o_s, s.lse, s.qphi, stats, stream));
   }

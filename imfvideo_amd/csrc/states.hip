@@ -8,6 +8,7 @@
 //   complement     models/sla2_cube_qat.py:510-523, 570-578
 #include "common.h"
 #include "quant_pool.h"
+#include "train_setup.h"
 
 #include <mutex>
 
@@ -319,6 +320,21 @@ __global__ __launch_bounds__(256) void quant_states_kernel(
                                                *reinterpret_cast<StatesLds<TAN>*>(lds));
   else
     quant_pool_tiles<T16>(a, ntiles, i - ns, gridDim.x - ns, *reinterpret_cast<QuantPoolLds*>(lds));
+}
+
+// The training states and, independent of them, the call's setup (2.9 us as a
+// launch of its own): workgroups BH Nb .. take 256 of its elements each.
+template <typename T16>
+__global__ __launch_bounds__(256) void states_setup_kernel(
+    const uint16_t* __restrict__ K, const uint16_t* __restrict__ V, int64_t L, int Nb, int ns,
+    float* __restrict__ Hb, float* __restrict__ zb, uint16_t* __restrict__ vt, TrainSetup setup) {
+  __shared__ __align__(16) StatesLds<false> lds;
+  const int i = blockIdx.x;
+  if (i < ns)
+    linear_states_tile<T16, false, true, false>(K, nullptr, V, nullptr, L, Nb, Nb, Hb, nullptr, zb,
+                                                nullptr, vt, nullptr, i % Nb, i / Nb, lds);
+  else
+    train_setup(setup, (int64_t)(i - ns) * 256 + threadIdx.x);
 }
 
 // Global sums over the Np tiles in a fixed order (deterministic): eight partial
@@ -763,10 +779,36 @@ extern "C" int sla2h_linear_states(const void* k, const void* dk, const void* v,
 
 namespace sla2h {
 
-// sla2h_linear_states_qat without the sums over the tiles
-int linear_states_train(const void* k, const void* v, int dtype, int B, int H, int64_t L, int D,
-                        int E, float* Hb, float* zb, void* vt, void* stream) {
+// sla2h_linear_states_qat without the sums over the tiles, and a training
+// forward's setup
+int states_and_setup(const void* k, const void* v, int dtype, int B, int H, int64_t L, float* Hb,
+                     float* zb, void* vt, const TrainSetup& setup, void* stream) {
   SLA2H_CHECK_ARG(k && v && Hb && zb);
+  SLA2H_CHECK_ARG(dtype == SLA2H_DTYPE_F16 || dtype == SLA2H_DTYPE_BF16);
+  SLA2H_CHECK_ARG(B > 0 && H > 0 && B * H <= 65535 && L > 0);
+  const int Nb = (int)((L + kT - 1) / kT);
+  const int64_t ns = (int64_t)B * H * Nb;
+  int64_t n = setup.nl > setup.na ? setup.nl : setup.na;
+  if (setup.stats != nullptr && n < setup.H) n = setup.H;
+  const int64_t grid = ns + (n + 255) / 256;
+  SLA2H_CHECK_ARG(grid < (1 << 24));  // 2^32 threads
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  auto K = static_cast<const uint16_t*>(k);
+  auto V = static_cast<const uint16_t*>(v);
+  auto VT = static_cast<uint16_t*>(vt);
+  if (dtype == SLA2H_DTYPE_BF16)
+    states_setup_kernel<BF16><<<(unsigned)grid, 256, 0, st>>>(K, V, L, Nb, (int)ns, Hb, zb, VT, setup);
+  else
+    states_setup_kernel<F16><<<(unsigned)grid, 256, 0, st>>>(K, V, L, Nb, (int)ns, Hb, zb, VT, setup);
+  return (int)hipGetLastError();
+}
+
+}  // namespace sla2h
+
+extern "C" int sla2h_linear_states_qat(const void* k, const void* v, int dtype, int B, int H,
+                                       int64_t L, int D, int E, float* Hb, float* zb, float* Hall,
+                                       float* zall, void* vt, void* stream) {
+  SLA2H_CHECK_ARG(k && v && Hb && zb && Hall && zall);
   SLA2H_CHECK_ARG(D == kT && E == kT);
   SLA2H_CHECK_ARG(dtype == SLA2H_DTYPE_F16 || dtype == SLA2H_DTYPE_BF16);
   SLA2H_CHECK_ARG(B > 0 && H > 0 && B * H <= 65535 && L > 0);
@@ -779,21 +821,10 @@ int linear_states_train(const void* k, const void* v, int dtype, int B, int H, i
     linear_states_kernel<BF16, false, true><<<grid, 256, 0, st>>>(K, nullptr, V, nullptr, L, Nb, Nb, Hb, nullptr, zb, nullptr, static_cast<uint16_t*>(vt), nullptr);
   else
     linear_states_kernel<F16, false, true><<<grid, 256, 0, st>>>(K, nullptr, V, nullptr, L, Nb, Nb, Hb, nullptr, zb, nullptr, static_cast<uint16_t*>(vt), nullptr);
-  return (int)hipGetLastError();
-}
-
-}  // namespace sla2h
-
-extern "C" int sla2h_linear_states_qat(const void* k, const void* v, int dtype, int B, int H,
-                                       int64_t L, int D, int E, float* Hb, float* zb, float* Hall,
-                                       float* zall, void* vt, void* stream) {
-  SLA2H_CHECK_ARG(Hall && zall);
-  const int err = linear_states_train(k, v, dtype, B, H, L, D, E, Hb, zb, vt, stream);
+  const int err = (int)hipGetLastError();
   if (err) return err;
-  const int Nb = (int)((L + E - 1) / E);
   dim3 g2(8320 / 64, B * H);
-  states_sum_kernel<<<g2, 256, 0, static_cast<hipStream_t>(stream)>>>(Hb, nullptr, zb, nullptr, Nb,
-                                                                      Hall, nullptr, zall, nullptr);
+  states_sum_kernel<<<g2, 256, 0, st>>>(Hb, nullptr, zb, nullptr, Nb, Hall, nullptr, zall, nullptr);
   return (int)hipGetLastError();
 }
 

@@ -457,12 +457,12 @@ def test_sla2_train_1d_config_shape():
 
 
 @pytest.mark.parametrize("H,nb,T", [(9, 3, 1), (2, 33, 4), (1, 97, 2), (3, 130, 12), (1, 64, 16),
-                                    (1, 520, 3)])
+                                    (1, 520, 3), (5, 513, 6)])
 def test_state_sums_beside_the_complement(H, nb, T):
     """The whole call takes the sums of the states over the tiles from the
     complement GEMM (masks inside it or not, one and two groups of query blocks,
-    zall for the score form), the stages from their own kernel, in the same fp32
-    order: outputs and gradients equal to the bit."""
+    zall for the score form; states before and, from 2,561 tiles, behind the sparse
+    kernel), the stages from their own kernel, in the same fp32 order: outputs and gradients equal to the bit."""
     from imfvideo_amd import ops
     print("[case] state sums", H, nb, T, flush=True)
     g = torch.Generator().manual_seed(nb + T)
