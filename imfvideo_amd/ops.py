@@ -78,6 +78,11 @@ def _proj(p, dev):
     return p.detach().to(dev, torch.float32).contiguous()
 
 
+def aligned(t, nbytes):
+    """t, or a copy of it where its data is not aligned to nbytes."""
+    return t if t.data_ptr() % nbytes == 0 else t.clone()
+
+
 def _scratch(nbytes, dev):
     return torch.empty(nbytes, device=dev, dtype=torch.uint8)
 

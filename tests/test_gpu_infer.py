@@ -319,3 +319,22 @@ def test_infer_in_matches_the_separate_passes(dt, B, H, L, bq):
     lut = ops.route_topk(qpool, kpool_t, T, 0.125)
     a = torch.rand(H, mq, generator=g).cuda()
     assert torch.equal(ops.sla2_infer(q, k, v, a, lut, bq, ws=ws), ops.sla2_infer(q, k, v, a, lut, bq))
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("which", ["q", "k", "v", "qkv"])
+def test_sla2_takes_unaligned_operands(dt, which):
+    """Contiguous views at an odd storage offset (not 16-byte aligned) give what
+    aligned tensors of the same values give."""
+    from imfvideo_amd.sla2_vendor import SLA2
+    print("[case] unaligned operands", dt, which, flush=True)
+    torch.manual_seed(5)
+    m = SLA2(64, topk=0.3, use_bf16=dt == torch.bfloat16).cuda()
+    xs = [torch.randn(1, 2, 583, 64, device="cuda").to(dt) for _ in range(3)]
+    off = []
+    for name, x in zip("qkv", xs):
+        flat = torch.empty(x.numel() + 1, device="cuda", dtype=dt)
+        flat[1:] = x.flatten()
+        off.append(flat[1:].view(x.shape) if name in which else x)
+    with torch.no_grad():
+        assert torch.equal(m(*off), m(*xs))
