@@ -681,7 +681,7 @@ def pool_qk(q, k, bq, Nk, proj_q=None, proj_k=None, bk=E_TILE):
     """pool_blocks of 16-bit q over bq rows (B,H,ceil(L/bq),64) and of k's first Nk
     blocks of 64 rows, transposed (B,H,64,Nk), in one launch."""
     _need_gpu(q, k, proj_q, proj_k)
-    q, k = _bhld(q, "q"), _bhld(k, "k")
+    q, k = (aligned(_bhld(t, n), 4) for t, n in ((q, "q"), (k, "k")))  # 4-byte accesses
     if q.shape != k.shape or q.dtype != k.dtype:
         raise ValueError("q and k must share shape and dtype")
     B, H, L, D = q.shape

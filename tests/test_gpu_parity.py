@@ -689,3 +689,23 @@ def test_pool_qk_matches_pool_blocks(dt, BH, L, bq, short, proj):
         want = O.project_pool(O.pool_tiles(q.cpu().float(), -(-L // bq), L, block=bq),
                               None if pq is None else pq.cpu())
         assert np.array_equal(qp.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_routers_take_unaligned_rows(dt):
+    """q and k off 4-byte alignment (contiguous views at an odd storage offset) route
+    as aligned tensors of the same values, in the 1-D and in the cube router."""
+    from imfvideo_amd import ops
+    from imfvideo_amd.mla_video_sparse_jvp import route_tiles_fast
+    print("[case] unaligned router rows", dt, flush=True)
+    g = torch.Generator().manual_seed(9)
+    q, k = (torch.randn(1, 2, 583, 64, generator=g).to(dt).cuda() for _ in range(2))
+    off = []
+    for x in (q, k):
+        flat = torch.empty(x.numel() + 1, device="cuda", dtype=dt)
+        flat[1:] = x.flatten()
+        off.append(flat[1:].view(x.shape))
+    for a, b in ((off, (q, k)), ((off[0], k), (q, k)), ((q, off[1]), (q, k))):
+        assert torch.equal(ops.route_1d(*a, 0.4, 128)[0], ops.route_1d(*b, 0.4, 128)[0])
+        assert torch.equal(route_tiles_fast(*a, 0.4, 8, 64, 71)[0],
+                           route_tiles_fast(*b, 0.4, 8, 64, 71)[0])
