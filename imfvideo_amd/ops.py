@@ -680,14 +680,13 @@ def pool_blocks(x, blk, proj=None, transposed=False):
 def pool_qk(q, k, bq, Nk, proj_q=None, proj_k=None, bk=E_TILE):
     """pool_blocks of 16-bit q over bq rows (B,H,ceil(L/bq),64) and of k's first Nk
     blocks of 64 rows, transposed (B,H,64,Nk), in one launch."""
-    _need_gpu(q, k, proj_q, proj_k)
+    _need_gpu(q, k)
     q, k = (aligned(_bhld(t, n), 4) for t, n in ((q, "q"), (k, "k")))  # 4-byte accesses
     if q.shape != k.shape or q.dtype != k.dtype:
         raise ValueError("q and k must share shape and dtype")
     B, H, L, D = q.shape
     dev = q.device
-    pq, pk = (None if p is None else p.detach().to(dev, torch.float32).contiguous()
-              for p in (proj_q, proj_k))
+    pq, pk = _proj(proj_q, dev), _proj(proj_k, dev)
     qpool = torch.empty(B, H, -(-L // bq), D, device=dev, dtype=torch.float32)
     kpool_t = torch.empty(B, H, D, Nk, device=dev, dtype=torch.float32)
     _lib.check(_lib.load().sla2h_pool_qk(
@@ -703,6 +702,7 @@ def route_1d(q, k, topk_frac, bq, bk=E_TILE, proj_q=None, proj_k=None):
     B, H, L, D = q.shape
     nb = -(-L // bk)
     T = max(1, min(nb, int(topk_frac * nb)))
+    _need_gpu(q, k, proj_q, proj_k)
     if q.dtype == k.dtype and q.dtype in _F16_CODES and q.shape == k.shape:
         qpool, kpool_t = pool_qk(q, k, bq, nb, proj_q, proj_k)
     else:

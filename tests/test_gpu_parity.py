@@ -709,3 +709,23 @@ def test_routers_take_unaligned_rows(dt):
         assert torch.equal(ops.route_1d(*a, 0.4, 128)[0], ops.route_1d(*b, 0.4, 128)[0])
         assert torch.equal(route_tiles_fast(*a, 0.4, 8, 64, 71)[0],
                            route_tiles_fast(*b, 0.4, 8, 64, 71)[0])
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
+def test_cube_router_takes_projections_from_the_host(dt):
+    """route_tiles_fast moves the projections of 16-bit q and k to their device; the
+    pooling kernels that route_1d and fp32 inputs call refuse them, as ever."""
+    from imfvideo_amd import ops
+    from imfvideo_amd.mla_video_sparse_jvp import route_tiles_fast
+    print("[case] host projections", dt, flush=True)
+    g = torch.Generator().manual_seed(10)
+    q, k = (torch.randn(1, 2, 583, 64, generator=g).to(dt).cuda() for _ in range(2))
+    pq, pk = (torch.randn(64, 64, generator=g) for _ in range(2))
+    want = route_tiles_fast(q, k, 0.4, 8, 64, 71, pq.cuda(), pk.cuda())[0]
+    if dt == torch.float32:
+        with pytest.raises(RuntimeError):
+            route_tiles_fast(q, k, 0.4, 8, 64, 71, pq, pk)
+    else:
+        assert torch.equal(route_tiles_fast(q, k, 0.4, 8, 64, 71, pq, pk)[0], want)
+    with pytest.raises(RuntimeError):
+        ops.route_1d(q, k, 0.4, 128, proj_q=pq, proj_k=pk)
