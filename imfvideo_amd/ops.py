@@ -1405,8 +1405,12 @@ def _ptrs(ts):
 # ---------------------------------------------------------------------------
 def linear_wgrad_ok(rows, M, N):
     """Sizes that sla2h_linear_wgrad takes: M and N multiples of 8, 32-bit byte offsets."""
-    return (rows > 0 and M > 0 and N > 0 and M % 8 == 0 and N % 8 == 0
-            and (rows + 144) * max(M, N) * 2 + 256 < 2 ** 31)
+    return rows > 0 and M > 0 and N > 0 and M % 8 == 0 and N % 8 == 0 and _offsets32(rows, max(M, N))
+
+
+def _offsets32(rows, ld):
+    """The weight gradient's byte offsets into rows of ld 16-bit elements fit 32 bits."""
+    return (rows + 144) * ld * 2 + 256 < 2 ** 31
 
 
 def linear_wgrad(dy, x):
@@ -1419,7 +1423,7 @@ def linear_wgrad(dy, x):
     dy2, M, ldy = _rows16(dy)
     x2, N, ldx = _rows16(x)
     rows = x2.shape[0]
-    if not linear_wgrad_ok(rows, max(M, ldy), max(N, ldx)):
+    if not linear_wgrad_ok(rows, M, N):
         raise ValueError(f"linear_wgrad: unsupported sizes {tuple(dy.shape)}, {tuple(x.shape)}")
     lib = _lib.load()
     dw = torch.empty(M, N, device=x.device, dtype=torch.float32)
@@ -1432,9 +1436,10 @@ def linear_wgrad(dy, x):
 
 
 def _rows16(t):
-    """_rows_view with 16-byte aligned rows (copied when they are not)."""
+    """_rows_view with 16-byte aligned rows and 32-bit byte offsets (copied when the
+    data or the row stride does not give them)."""
     v, F, s = _rows_view(t)
-    if v.data_ptr() % 16 or s % 8:
+    if v.data_ptr() % 16 or s % 8 or not _offsets32(v.shape[0], s):
         v = v.clone(memory_format=torch.contiguous_format)
         s = F
     return v, F, s

@@ -248,3 +248,19 @@ def test_caller_lut_ids_are_checked():
         x[0, 0, 1, 0] = bad
         with pytest.raises(ValueError):
             ops.check_lut_ids(x, 4)
+
+
+def test_weight_gradient_rows_of_a_wide_tensor_are_copied():
+    """A column slice whose row stride passes the weight gradient's 32-bit byte
+    offsets, while its width does not, is made contiguous: whatever the sizes
+    rule admits in the forward is taken in the backward.  One whose offsets fit
+    stays a view.  (Meta tensors: sizes and strides only.)"""
+    from imfvideo_amd import ops
+    wide = torch.empty(70000, 16384, dtype=torch.bfloat16, device="meta")
+    x = wide[:, :512]
+    assert ops.linear_wgrad_ok(70000, 512, 512) and not ops.linear_wgrad_ok(70000, 16384, 512)
+    assert ops._rows16(x)[1:] == (512, 512) and ops._rows16(x)[0].is_contiguous()
+    assert ops._rows16(x.view(7, 10000, 512))[1:] == (512, 512)
+    most = (2 ** 31 - 256 - 1) // 2 // 16384 - 144  # rows whose offsets fit
+    assert ops._rows16(wide[:most, :512])[2] == 16384
+    assert ops._rows16(wide[:most + 1, :512])[2] == 512
