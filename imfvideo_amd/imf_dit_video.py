@@ -35,17 +35,21 @@ class _LinearFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy):
+        from . import ops
         x, w16 = ctx.saved_tensors
         need_x, need_w = ctx.needs_input_grad
         if torch.is_grad_enabled():  # create_graph: torch ops, differentiable again
             if ctx.weight._version != ctx.version:
                 raise RuntimeError("a linear layer's weight was modified in place before its "
                                    "double backward")
-            dw = dy.flatten(0, -2).t() @ x.flatten(0, -2) if need_w else None
-            return (dy @ ctx.weight.to(x.dtype) if need_x else None,
-                    dw.to(ctx.weight.dtype) if need_w else None)
-        from . import ops
-        return dy @ w16 if need_x else None, ops.linear_wgrad(dy, x) if need_w else None
+            w16 = ctx.weight.to(x.dtype)
+        dx = dy @ w16 if need_x else None
+        if not need_w:
+            return dx, None
+        if torch.is_grad_enabled() or not ops.plain_eager(dy):  # batched gradients (vmap) too
+            dw = dy.reshape(-1, dy.shape[-1]).t() @ x.reshape(-1, x.shape[-1])
+            return dx, dw.to(ctx.weight.dtype)
+        return dx, ops.linear_wgrad(dy, x)
 
 
 # Weights of at most this many 128 x 128 tiles take the split-row gradient

@@ -46,10 +46,12 @@ def _need_gpu(*ts):
 
 
 def plain_eager(*ts):
-    """Plain tensors (no subclass) in eager mode, outside torch.func transforms,
-    forward-mode AD, tracing and compilation: what the autograd Functions that
-    replace torch's own ops are for."""
-    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in ts)
+    """Plain tensors (no subclass, none that is_grads_batched made a batch of) in
+    eager mode, outside torch.func transforms, forward-mode AD, tracing and
+    compilation: what the autograd Functions that replace torch's own ops are
+    for."""
+    return (all(type(t) in (torch.Tensor, torch.nn.Parameter)
+                and not torch._C._functorch.is_legacy_batchedtensor(t) for t in ts)
             and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
             and not torch._C._are_functorch_transforms_active()
             and torch.autograd.forward_ad._current_level < 0)

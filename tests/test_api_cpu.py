@@ -264,3 +264,23 @@ def test_weight_gradient_rows_of_a_wide_tensor_are_copied():
     most = (2 ** 31 - 256 - 1) // 2 // 16384 - 144  # rows whose offsets fit
     assert ops._rows16(wide[:most, :512])[2] == 16384
     assert ops._rows16(wide[:most + 1, :512])[2] == 512
+
+
+def test_linear_takes_batched_gradients():
+    """The block's linear under is_grads_batched (backward under vmap), where the
+    weight gradient's kernel cannot read dy: the same products in torch, one
+    gradient at a time or batched."""
+    from imfvideo_amd.imf_dit_video import _LinearFunction
+    g = torch.Generator().manual_seed(12)
+    x = torch.randn(2, 5, 16, generator=g).to(torch.bfloat16).requires_grad_()
+    w = torch.randn(8, 16, generator=g).requires_grad_()
+    dys = torch.randn(3, 2, 5, 8, generator=g).to(torch.bfloat16)
+    y = _LinearFunction.apply(x, w)
+    dx, dw = torch.autograd.grad(y, [x, w], dys, is_grads_batched=True, retain_graph=True)
+    w16 = w.detach().to(torch.bfloat16).requires_grad_()
+    ref = torch.nn.functional.linear(x, w16)
+    assert dw.dtype == torch.float32
+    for i in range(3):
+        rx, rw = torch.autograd.grad(ref, [x, w16], dys[i], retain_graph=True)
+        assert torch.allclose(dx[i].float(), rx.float(), rtol=2.0 ** -7, atol=1e-3)
+        assert torch.allclose(dw[i], rw.float(), rtol=2.0 ** -7, atol=1e-3)

@@ -572,3 +572,27 @@ def test_linear_module_matches_nn_linear(shape):
     with torch.autocast("cuda", dtype=torch.bfloat16):
         j0, j1 = (torch.func.jvp(m, (x,), (x,))[1] for m in (own, ref))
     assert torch.equal(j0, j1)
+
+
+def test_linear_module_batched_gradients():
+    """is_grads_batched through the block's linear on the GPU: each row of the batch
+    is nn.Linear's gradient, the weight's within the 16-bit rounding of both."""
+    from imfvideo_amd.imf_dit_video import scaled_variance_linear
+    say("linear module, batched gradients")
+    torch.manual_seed(2)
+    own = scaled_variance_linear(64, 96, bias=False).cuda()
+    ref = torch.nn.Linear(64, 96, bias=False).cuda()
+    ref.load_state_dict(own.state_dict())
+    x = torch.randn(2, 65, 64, device="cuda")
+    dys = torch.randn(3, 2, 65, 96, device="cuda", dtype=torch.bfloat16)
+    res = []
+    for m in (own, ref):
+        xi = x.clone().requires_grad_()
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = m(xi)
+        res.append(torch.autograd.grad(y, [xi, m.weight], dys, is_grads_batched=True))
+    (dx0, dw0), (dx1, dw1) = res
+    assert dx0.shape == dx1.shape and dw0.shape == dw1.shape and dw0.dtype == dw1.dtype
+    # one bf16 rounding of each (2^-8) plus fp32 summation order
+    assert bool(((dx0 - dx1).abs() <= 2.0 ** -7 * dx1.abs() + 1e-4).all())
+    assert bool(((dw0 - dw1).abs() <= 2.0 ** -7 * dw1.abs() + 1e-4).all())
