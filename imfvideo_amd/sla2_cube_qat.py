@@ -281,7 +281,7 @@ class SLA2CubeQATAttentionImpl(nn.Module):
             o = self.forward_tile_major(*_RowsIn.apply(perm, inv, q, k, v))
         if self.pre_permuted:
             return o.permute(0, 2, 1, 3).to(q.dtype)
-        if own:
+        if own and ops.rows_out_ok(o, q):
             return _RowsOut.apply(inv, perm, q.dtype, o)[0]
         return o[:, :, self.inv].permute(0, 2, 1, 3).to(q.dtype)
 

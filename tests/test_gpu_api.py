@@ -321,3 +321,40 @@ def test_module_token_layout_matches_torch(dt, layout, pre_permuted):
     assert o.dtype == want.dtype and torch.equal(o, want)
     for g, gw in zip(grads, torch.autograd.grad(want, xs, do)):
         assert g.dtype == gw.dtype and torch.equal(g, gw)
+
+
+@pytest.mark.parametrize("kind", ["fp32", "bf16", "wider", "unaligned", "strided"])
+def test_module_with_its_own_tile_major_op(kind):
+    """A forward_tile_major of the caller's own may return rows of another dtype,
+    width or layout than the op's: the output and the gradients are torch's
+    permute / cast / index of what it returned."""
+    from imfvideo_amd.sla2_cube_qat import SLA2CubeQATAttentionImpl
+    print("[case] own tile-major op", kind, flush=True)
+    torch.manual_seed(6)
+    B, H, grid, P = 1, 3, (4, 8, 8), 18
+    L = 256 + P
+    mod = SLA2CubeQATAttentionImpl(64, L, H, grid, topk=0.5).cuda()
+
+    def op(q, k, v):
+        o = q * 2 + k * v
+        if kind == "fp32":
+            return o.float() * 1.0001
+        if kind == "bf16":
+            return o.to(torch.bfloat16)
+        if kind == "wider":
+            return torch.cat([o, q], -1)
+        if kind == "unaligned":
+            flat = torch.zeros(o.numel() + 1, device=o.device, dtype=o.dtype)
+            return flat.index_copy(0, torch.arange(1, o.numel() + 1, device=o.device),
+                                   o.flatten())[1:].view(o.shape)
+        return torch.stack([o, q], -1)[..., 0]
+
+    mod.forward_tile_major = op
+    xs = [torch.randn(B, L, H, 64, device="cuda").requires_grad_() for _ in range(3)]
+    rows = [x.permute(0, 2, 1, 3)[:, :, mod.perm].half().contiguous() for x in xs]
+    want = op(*rows)[:, :, mod.inv].permute(0, 2, 1, 3).to(xs[0].dtype)
+    o = mod(*xs)
+    assert o.dtype == want.dtype and torch.equal(o, want)
+    do = torch.randn_like(want)
+    for g, gw in zip(torch.autograd.grad(o, xs, do), torch.autograd.grad(want, xs, do)):
+        assert torch.equal(g, gw)
