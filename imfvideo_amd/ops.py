@@ -1372,6 +1372,13 @@ def rows_in_ok(xs):
     return True
 
 
+def token_index_ok(idx, x):
+    """idx can be rows_in's / rows_out's for x (B, L, H, 64): one int64 per token,
+    contiguous, on x's device (torch's index takes other forms)."""
+    return (idx.dtype == torch.int64 and tuple(idx.shape) == (x.shape[1],)
+            and idx.is_contiguous() and idx.device == x.device)
+
+
 def rows_in(xs, idx):
     """1 to 3 (B, L, H, 64) tensors (rows_in_ok) -> (B, H, L, 64) fp16, row l from
     token idx[l] (int64 on their device; None: l itself)."""

@@ -267,8 +267,9 @@ class SLA2CubeQATAttentionImpl(nn.Module):
 
         # one kernel for the three operands (and one for the output) where they
         # are plain GPU tensors with 16-byte rows; else the torch form
-        own = (ops.plain_eager(q, k, v) and ops.rows_in_ok((q, k, v)) and self.perm.device == q.device
-               and (self.pre_permuted or self.perm.numel() == q.shape[1]))
+        own = (ops.plain_eager(q, k, v) and ops.rows_in_ok((q, k, v))
+               and (self.pre_permuted or all(ops.token_index_ok(i, q)
+                                             for i in (self.perm, self.inv))))
         perm, inv = (None, None) if self.pre_permuted else (self.perm, self.inv)
         if not own:
             o = self.forward_tile_major(tm(q), tm(k), tm(v))

@@ -284,3 +284,15 @@ def test_linear_takes_batched_gradients():
         rx, rw = torch.autograd.grad(ref, [x, w16], dys[i], retain_graph=True)
         assert torch.allclose(dx[i].float(), rx.float(), rtol=2.0 ** -7, atol=1e-3)
         assert torch.allclose(dw[i], rw.float(), rtol=2.0 ** -7, atol=1e-3)
+
+
+def test_token_index_forms():
+    """The layout kernels read their index as L contiguous int64 values on the
+    operands' device; every other form goes through torch's index."""
+    from imfvideo_amd import ops
+    x = torch.empty(2, 6, 3, 64)
+    idx = torch.arange(6)
+    assert ops.token_index_ok(idx, x)
+    for bad in (idx.int(), idx[:5], torch.arange(12)[::2], idx.view(2, 3), idx.to("meta"),
+                torch.ones(6, dtype=torch.bool)):
+        assert not ops.token_index_ok(bad, x)

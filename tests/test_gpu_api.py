@@ -358,3 +358,21 @@ def test_module_with_its_own_tile_major_op(kind):
     do = torch.randn_like(want)
     for g, gw in zip(torch.autograd.grad(o, xs, do), torch.autograd.grad(want, xs, do)):
         assert torch.equal(g, gw)
+
+
+def test_module_with_another_index_form():
+    """The module's permutation as int32 or strided values gives what the int64 one
+    gives (torch's index takes them; the layout kernels read int64)."""
+    from imfvideo_amd.sla2_cube_qat import SLA2CubeQATAttentionImpl
+    print("[case] permutation forms", flush=True)
+    torch.manual_seed(7)
+    B, H, grid, P = 1, 2, (4, 8, 8), 18
+    mod = SLA2CubeQATAttentionImpl(64, 256 + P, H, grid, topk=0.5).cuda()
+    xs = [torch.randn(B, 256 + P, H, 64, device="cuda") for _ in range(3)]
+    perm, inv = mod.perm, mod.inv
+    with torch.no_grad():
+        want = mod(*xs)
+        for p, i in ((perm.int(), inv), (perm, inv.int()),
+                     (perm.repeat_interleave(2)[::2], inv.repeat_interleave(2)[::2])):
+            mod.perm, mod.inv = p, i
+            assert torch.equal(mod(*xs), want)
