@@ -161,7 +161,10 @@ class _RowsIn(torch.autograd.Function):
                                   for d in ds))
         have = [i for i, d in enumerate(ds) if d is not None]
         grads = [None] * len(ds)
-        if have:
+        if not ops.plain_eager(*(ds[i] for i in have)):  # batched gradients
+            for i in have:
+                grads[i] = ds[i][:, :, inv].permute(0, 2, 1, 3).to(ctx.dtype)
+        elif have:
             outs = _RowsOut.apply(inv, idx, ctx.dtype, *(ds[i].contiguous() for i in have))
             for i, g in zip(have, outs):
                 grads[i] = g
@@ -199,7 +202,10 @@ class _RowsOut(torch.autograd.Function):
         idx, inv = ctx.saved_tensors
         have = [i for i, d in enumerate(ds) if d is not None]
         grads = [None] * len(ds)
-        if have:
+        if not ops.plain_eager(*(ds[i] for i in have)):  # batched gradients
+            for i in have:
+                grads[i] = ds[i].permute(0, 2, 1, 3)[:, :, inv].half()
+        elif have:
             xs = [ds[i] for i in have]
             if not ops.rows_in_ok(xs):
                 xs = [x.clone(memory_format=torch.contiguous_format) for x in xs]

@@ -376,3 +376,21 @@ def test_module_with_another_index_form():
                      (perm.repeat_interleave(2)[::2], inv.repeat_interleave(2)[::2])):
             mod.perm, mod.inv = p, i
             assert torch.equal(mod(*xs), want)
+
+
+@pytest.mark.parametrize("pre_permuted", [False, True])
+def test_module_layout_takes_batched_gradients(pre_permuted):
+    """is_grads_batched through the module's layout kernels (around a differentiable
+    op of the caller's own): each row of the batch is that gradient by itself."""
+    from imfvideo_amd.sla2_cube_qat import SLA2CubeQATAttentionImpl
+    print("[case] layout, batched gradients", pre_permuted, flush=True)
+    torch.manual_seed(8)
+    mod = SLA2CubeQATAttentionImpl(64, 274, 2, (4, 8, 8), topk=0.5, pre_permuted=pre_permuted).cuda()
+    mod.forward_tile_major = lambda q, k, v: q * 2 + k * v
+    xs = [torch.randn(1, 274, 2, 64, device="cuda").requires_grad_() for _ in range(3)]
+    o = mod(*xs)
+    dos = torch.randn(3, *o.shape, device="cuda")
+    got = torch.autograd.grad(o, xs, dos, is_grads_batched=True, retain_graph=True)
+    for i in range(3):
+        for g, gw in zip(got, torch.autograd.grad(o, xs, dos[i], retain_graph=True)):
+            assert torch.equal(g[i], gw)
