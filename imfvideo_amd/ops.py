@@ -1395,18 +1395,17 @@ def rows_in(xs, idx):
 
 def rows_out_ok(o, q):
     """o can go through rows_out as the op's output for token-order input q
-    (B, L, H, 64): fp16 rows (B, H, L, 64) on q's device, 16-byte aligned (a
-    forward_tile_major of the caller's own may return others)."""
+    (B, L, H, 64): fp16 rows (B, H, L, 64) on q's device (a forward_tile_major of
+    the caller's own may return others)."""
     B, L, H, D = q.shape
     return (plain_eager(o) and o.device == q.device and o.dtype == torch.float16
-            and tuple(o.shape) == (B, H, L, D)
-            and (o.data_ptr() % 16 == 0 or not o.is_contiguous()))
+            and tuple(o.shape) == (B, H, L, D))
 
 
 def rows_out(xs, idx, dtype):
     """1 to 3 (B, H, L, 64) fp16 tensors -> (B, L, H, 64) contiguous in dtype, token
     l from row idx[l]."""
-    xs = [x.contiguous() for x in xs]
+    xs = [aligned(x.contiguous(), 16) for x in xs]
     B, H, L, D = xs[0].shape
     outs = [torch.empty(B, L, H, D, device=x.device, dtype=dtype) for x in xs]
     _lib.check(_lib.load().sla2h_rows_out(

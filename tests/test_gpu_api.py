@@ -394,3 +394,25 @@ def test_module_layout_takes_batched_gradients(pre_permuted):
     for i in range(3):
         for g, gw in zip(got, torch.autograd.grad(o, xs, dos[i], retain_graph=True)):
             assert torch.equal(g[i], gw)
+
+
+def test_module_layout_takes_unaligned_gradients():
+    """The gradient of the operand rows as a contiguous view off 16 bytes (here the
+    tail of a concatenation's) goes through the layout's backward."""
+    from imfvideo_amd.sla2_cube_qat import SLA2CubeQATAttentionImpl
+    print("[case] unaligned gradients of the rows", flush=True)
+    torch.manual_seed(9)
+    mod = SLA2CubeQATAttentionImpl(64, 274, 2, (4, 8, 8), topk=0.5).cuda()
+    one = torch.ones(1, device="cuda", dtype=torch.float16)
+
+    def op(q, k, v):
+        flat = torch.cat([one, q.reshape(-1)])
+        return (flat * 2)[1:].view(q.shape) + k * v
+
+    mod.forward_tile_major = op
+    xs = [torch.randn(1, 274, 2, 64, device="cuda").requires_grad_() for _ in range(3)]
+    do = torch.randn(1, 274, 2, 64, device="cuda")
+    got = torch.autograd.grad(mod(*xs), xs, do)
+    mod.forward_tile_major = lambda q, k, v: q * 2 + k * v
+    for g, gw in zip(got, torch.autograd.grad(mod(*xs), xs, do)):
+        assert torch.equal(g, gw)
