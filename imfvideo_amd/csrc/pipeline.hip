@@ -167,7 +167,7 @@ struct Saved {
 
 struct FwdWs {
   int8_t *q8, *k8, *v8f;
-  float *qs, *ks, *vs, *Hb, *zb, *zall;
+  float *qs, *ks, *vs, *Hb, *zb, *zall, *lse_max;
   uint16_t* vt;
   size_t bytes;
   FwdWs(void* p, const Dims& d, bool int8) {
@@ -185,6 +185,7 @@ struct FwdWs {
     Hb = c.take<float>(nb * kT * kT);
     zb = c.take<float>(nb * kT);
     zall = c.take<float>(d.BH * kT);
+    lse_max = c.take<float>(d.H);
     bytes = c.used;
   }
 };
@@ -245,7 +246,8 @@ int states_and_setup(const void* k, const void* v, int dtype, int B, int H, int6
                      float* zb, void* vt, const TrainSetup& setup, void* stream);
 int complement_sums(const float* Hb, const float* dHb, const float* zb, const float* dzb,
                     const int32_t* lut, int B, int H, int Mb, int Np, int D, int T,
-                    void* workspace, void* comp, float* Hall, float* zall, void* stream);
+                    void* workspace, void* comp, float* Hall, float* zall, const float* lse_max,
+                    float* stats, void* stream);
 
 // states.hip: INT8 operands, pooled tiles and linear states of the cube op
 int quant_states(const QuantPoolArgs& a, const void* k, const void* dk, const void* v,
@@ -381,7 +383,11 @@ extern "C" int sla2h_train_fwd(const void* q, const void* k, const void* v,
   // setup in a launch of its own.  States behind -> before the sparse kernel, us a
   // forward: 256 tiles 37.3 -> 34.9, 1040 83.8 -> 82.8, 2048 161.8 -> 159.6; 3200
   // 302.6 -> 307.3, 7488 722 -> 735.
-  const TrainSetup setup{alpha_logit, na, s.alpha, lut, nl, T, d.J, Np, s.lut, stats, H};
+  // The sparse kernels raise the maxima of lse in the workspace and the complement
+  // copies them out when they are whole: the caller's buffer only ever receives one
+  // call's values, also where calls of several streams share it.
+  float* const lse_max = stats != nullptr ? w.lse_max : nullptr;
+  const TrainSetup setup{alpha_logit, na, s.alpha, lut, nl, T, d.J, Np, s.lut, lse_max, H};
   const bool late = int8 && (int64_t)d.BH * d.Nb > kEarlyStates;
   if (late) {
     const int64_t n = nl > na ? nl : na;
@@ -398,22 +404,22 @@ extern "C" int sla2h_train_fwd(const void* q, const void* k, const void* v,
                                   w.vs, stream));
     if (bq == kT && (int64_t)Np * kT <= L) {
       SLA2H_TRY(sparse_fwd_qat_stats(q, w.q8, w.qs, w.k8, w.ks, w.v8f, w.vs, lut, dtype, B, H, L,
-                                     kT, kT, Np, T, scale, s.o_s, s.lse, s.qphi, stats, stream));
+                                     kT, kT, Np, T, scale, s.o_s, s.lse, s.qphi, lse_max, stream));
     } else {  // query blocks over 64 rows, or a routable last block that is partial
       SLA2H_TRY(sla2h_quantize_trunc(q, dtype, (int64_t)d.BH, L, kT, bq, w.q8, w.qs, stream));
       SLA2H_TRY(sparse_fwd_int8_stats(q, w.q8, w.qs, bq, w.k8, w.ks, w.v8f, w.vs, lut, dtype, B,
-                                      H, L, kT, bq, T, scale, s.o_s, s.lse, s.qphi, stats,
+                                      H, L, kT, bq, T, scale, s.o_s, s.lse, s.qphi, lse_max,
                                       stream));
     }
     if (late)
       SLA2H_TRY(states_and_setup(k, v, dtype, B, H, L, w.Hb, w.zb, nullptr, TrainSetup{}, stream));
   } else {
     SLA2H_TRY(sparse_fwd_1d_stats(q, k, w.vt, s.lut, dtype, B, H, L, kT, bq, kT, d.J, scale,
-                                  s.o_s, s.lse, s.qphi, stats, stream));
+                                  s.o_s, s.lse, s.qphi, lse_max, stream));
   }
   // (zall: the score form's)
   SLA2H_TRY(complement_sums(w.Hb, nullptr, w.zb, nullptr, s.lut, B, H, d.Mq, d.Nb, kT, d.J, s.bits,
-                            s.comp, s.Hall, d.J <= 4 ? w.zall : nullptr, stream));
+                            s.comp, s.Hall, d.J <= 4 ? w.zall : nullptr, lse_max, stats, stream));
   // the reference's linear branch: score form up to 4 LUT columns, else state form
   if (d.J <= 4)
     SLA2H_TRY(sla2h_linear_mix_score(s.qphi, k, v, s.Hall, w.zall, s.lut, d.J, s.o_s, s.alpha,

@@ -531,13 +531,15 @@ __global__ __launch_bounds__(512) void comp_mask_kernel(const int32_t* __restric
 // SUM (training): the column sums over all tiles as well, Hall and (may be NULL)
 // zall, in fp32 from the rows that the staging holds anyway, where
 // states_sum_kernel read them again: 16 heads x 468 tiles 25 us, 4 x 64 tiles
-// 4 us and a launch; the GEMM takes the same time.
+// 4 us and a launch; the GEMM takes the same time.  Its first workgroup also copies
+// the call's finished lse maxima to the caller's buffer (stats, may be NULL).
 template <bool TAN, bool MASK, bool SUM = false>
 __global__ __launch_bounds__(kCompThreads, 4) void comp_gemm_kernel(
     const float* __restrict__ Hb, const float* __restrict__ dHb, const float* __restrict__ zb,
     const float* __restrict__ dzb, const uint32_t* __restrict__ cbits, int Mb, int Np, int MT,
     int NC, unsigned char* __restrict__ comp, const int32_t* __restrict__ lut, int T,
-    uint32_t* __restrict__ cbits_out, float* __restrict__ Hall, float* __restrict__ zall) {
+    uint32_t* __restrict__ cbits_out, float* __restrict__ Hall, float* __restrict__ zall,
+    const float* __restrict__ lse_max, float* __restrict__ stats, int nstats) {
   __shared__ float psum[SUM ? 2 : 1][SUM ? 8 : 1][kCompCols];
   extern __shared__ uint32_t lbits[];  // MASK: [kc][local row], 16 kMaskSub rows
   __shared__ __align__(16) uint16_t sb[2][2][kCompCols][40];  // [buf][hi/lo][column][n] (+pad)
@@ -678,6 +680,8 @@ __global__ __launch_bounds__(kCompThreads, 4) void comp_gemm_kernel(
   }
 
   if constexpr (SUM) {
+    if (stats != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0)
+      for (int i = tid; i < nstats; i += kCompThreads) stats[i] = lse_max[i];
     // with the masks the z columns are a column tile of their own; otherwise the
     // first column tile's workgroup sums them too
     const bool zsum = !MASK && c0 == 0 && zall != nullptr;
@@ -904,7 +908,7 @@ int complement_gemm_bwd(const float* P, const float* Pz, const uint32_t* cbits, 
   dim3 grid(4160 / kCompCols, BH, (MT + kMaskSub - 1) / kMaskSub);
   comp_gemm_kernel<false, false><<<grid, kCompThreads, 0, static_cast<hipStream_t>(stream)>>>(
       P, nullptr, Pz, nullptr, cbits, Mb, Mb, MT, NC, static_cast<unsigned char*>(comp), nullptr, 0,
-      nullptr, nullptr, nullptr);
+      nullptr, nullptr, nullptr, nullptr, nullptr, 0);
   return (int)hipGetLastError();
 }
 }  // namespace sla2h
@@ -974,11 +978,13 @@ int complement_scratch(void** out) {
 namespace sla2h {
 
 // sla2h_complement; with Hall (primal only) the sums of Hb and, where zall is
-// given, of zb over the tiles as well
+// given, of zb over the tiles as well, and with stats (H) a copy of lse_max there
 int complement_sums(const float* Hb, const float* dHb, const float* zb, const float* dzb,
                     const int32_t* lut, int B, int H, int Mb, int Np, int D, int T,
-                    void* workspace, void* comp, float* Hall, float* zall, void* stream) {
+                    void* workspace, void* comp, float* Hall, float* zall, const float* lse_max,
+                    float* stats, void* stream) {
   SLA2H_CHECK_ARG(Hb && zb && lut && comp && workspace);
+  SLA2H_CHECK_ARG(!stats || (Hall && lse_max));
   SLA2H_CHECK_ARG(D == kT);
   SLA2H_CHECK_ARG(B > 0 && H > 0 && B * H <= 65535 && Mb > 0 && Np > 0 && Np <= 4096);
   SLA2H_CHECK_ARG(T >= 1 && T <= Np);
@@ -996,13 +1002,16 @@ int complement_sums(const float* Hb, const float* dHb, const float* zb, const fl
     const size_t shmem = (size_t)NC * 16 * kMaskSub * 4;
     if (tan)
       comp_gemm_kernel<true, true><<<grid, kCompThreads, shmem, st>>>(
-          Hb, dHb, zb, dzb, nullptr, Mb, Np, MT, NC, out, lut, T, cbits, nullptr, nullptr);
+          Hb, dHb, zb, dzb, nullptr, Mb, Np, MT, NC, out, lut, T, cbits, nullptr, nullptr,
+          nullptr, nullptr, 0);
     else if (Hall)
       comp_gemm_kernel<false, true, true><<<grid, kCompThreads, shmem, st>>>(
-          Hb, nullptr, zb, nullptr, nullptr, Mb, Np, MT, NC, out, lut, T, cbits, Hall, zall);
+          Hb, nullptr, zb, nullptr, nullptr, Mb, Np, MT, NC, out, lut, T, cbits, Hall, zall,
+          lse_max, stats, H);
     else
       comp_gemm_kernel<false, true><<<grid, kCompThreads, shmem, st>>>(
-          Hb, nullptr, zb, nullptr, nullptr, Mb, Np, MT, NC, out, lut, T, cbits, nullptr, nullptr);
+          Hb, nullptr, zb, nullptr, nullptr, Mb, Np, MT, NC, out, lut, T, cbits, nullptr, nullptr,
+          nullptr, nullptr, 0);
     return (int)hipGetLastError();
   }
   // mask bits plus the z parts of the records; the GEMM takes the H parts only
@@ -1014,13 +1023,16 @@ int complement_sums(const float* Hb, const float* dHb, const float* zb, const fl
   dim3 grid((tan ? 8192 : 4096) / kCompCols, B * H, groups);
   if (tan)
     comp_gemm_kernel<true, false><<<grid, kCompThreads, 0, st>>>(
-        Hb, dHb, zb, dzb, cbits, Mb, Np, MT, NC, out, nullptr, 0, nullptr, nullptr, nullptr);
+        Hb, dHb, zb, dzb, cbits, Mb, Np, MT, NC, out, nullptr, 0, nullptr, nullptr, nullptr,
+        nullptr, nullptr, 0);
   else if (Hall)
     comp_gemm_kernel<false, false, true><<<grid, kCompThreads, 0, st>>>(
-        Hb, nullptr, zb, nullptr, cbits, Mb, Np, MT, NC, out, nullptr, 0, nullptr, Hall, zall);
+        Hb, nullptr, zb, nullptr, cbits, Mb, Np, MT, NC, out, nullptr, 0, nullptr, Hall, zall,
+        lse_max, stats, H);
   else
     comp_gemm_kernel<false, false><<<grid, kCompThreads, 0, st>>>(
-        Hb, nullptr, zb, nullptr, cbits, Mb, Np, MT, NC, out, nullptr, 0, nullptr, nullptr, nullptr);
+        Hb, nullptr, zb, nullptr, cbits, Mb, Np, MT, NC, out, nullptr, 0, nullptr, nullptr, nullptr,
+        nullptr, nullptr, 0);
   return (int)hipGetLastError();
 }
 
@@ -1031,7 +1043,7 @@ extern "C" int sla2h_complement(const float* Hb, const float* dHb, const float* 
                                 int Np, int D, int T, void* workspace, void* comp,
                                 void* stream) {
   return complement_sums(Hb, dHb, zb, dzb, lut, B, H, Mb, Np, D, T, workspace, comp, nullptr,
-                         nullptr, stream);
+                         nullptr, nullptr, nullptr, stream);
 }
 
 namespace sla2h {

@@ -612,8 +612,10 @@ def train_op_fwd(q, k, v, alpha_logit, lut, Np, bq=E_TILE, int8=True, stats=None
                  ws=None):
     """train_fwd / train_fwd_1d from the alpha logits (H, ceil(L/bq)) as one native
     call -> (o, saved): saved is the buffer that train_op_bwd reads.  stats:
-    optional (H,) fp32 tensor that receives the per-head maximum of lse.  ws:
-    train_in's workspace of the same q, k, v (their INT8 operands)."""
+    optional (H,) fp32 tensor that receives the per-head maximum of lse in one
+    store behind the sparse kernel (of calls that share it on several streams, the
+    last one's values).  ws: train_in's workspace of the same q, k, v (their INT8
+    operands)."""
     _need_gpu(q, k, v, lut, stats)
     q, k, v = (_bhld(t, n) for t, n in ((q, "q"), (k, "k"), (v, "v")))
     _same(q, k, v)
@@ -632,8 +634,9 @@ def train_op_fwd(q, k, v, alpha_logit, lut, Np, bq=E_TILE, int8=True, stats=None
     _lib.check(lib.sla2h_train_fwd(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), logit.data_ptr(), lut.data_ptr(), _dtype_code(q),
         B, H, L, Np, bq, T, int8, quantised, D ** -0.5, eps_l, saved.data_ptr(), ws.data_ptr(),
-        o.data_ptr(),
-        _ptr(stats), _stream(dev)), "sla2h_train_fwd")
+        o.data_ptr(), _ptr(stats), _stream(dev)), "sla2h_train_fwd")
+    if stats is not None:
+        torch.autograd.graph.increment_version(stats)  # as an in-place op of torch's does
     return o, saved
 
 

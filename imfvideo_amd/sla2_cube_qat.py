@@ -234,7 +234,8 @@ class SLA2CubeQATAttentionImpl(nn.Module):
     also under no_grad as the reference's guidance path does.  With gradients
     required the call goes through ``_CubeQATFunction`` (straight-through
     backward) and refreshes ``logit_max_log2`` (H,), the per-head maximum of
-    the sparse branch's lse, for the QK-Clip step.
+    the sparse branch's lse, for the QK-Clip step: the values of one call, of the
+    last one to finish where forwards run on several streams.
     """
 
     TILE_MAJOR = True

@@ -791,7 +791,8 @@ int sla2h_jvp16(const void* q, const void* k, const void* v, const void* dq, con
  * alpha logits (H, ceil(L/bq)), INT8 or 16-bit sparse branch, score-form linear
  * branch up to 4 LUT columns.  quantised: the workspace (of int8 = 1) already holds
  * the INT8 operands, from sla2h_train_in.  `saved` holds what the backward reads; stats (H),
- * optional, receives the per-head maximum of lse.  The backward writes dq, dk, dv
+ * optional, receives the per-head maximum of lse, written once behind the sparse
+ * kernel.  The backward writes dq, dk, dv
  * (16-bit) and the gradient of the logits (H, ceil(L/bq)); it only reads `saved`.
  * Replaces _CubeQATFunction (models/sla2_cube_qat.py:696-832).
  */

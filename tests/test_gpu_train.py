@@ -571,3 +571,29 @@ def test_train_in_matches_the_separate_passes(dt, B, L, H, Np, order):
         n = L * B * H * 64
         assert none is None and torch.equal(ws2[:n], ws[:n])
         assert torch.equal(qp2, qpool) and torch.equal(kp2, kpool_t)
+
+
+@pytest.mark.parametrize("T,int8", [(1, True), (6, True), (1, False), (6, False)])
+def test_lse_maxima_replace_the_buffer_as_a_whole(T, int8):
+    """The caller's buffer of lse maxima only ever receives a finished call's values:
+    a call that is refused half-way (a prefix tail over the sparse kernel's 1,024
+    tiles, after the setup ran) leaves it as it was, a good one replaces it and
+    counts as an in-place change."""
+    from imfvideo_amd import ops
+    print("[case] lse maxima", T, int8, flush=True)
+    g = torch.Generator().manual_seed(T)
+    H = 2
+    stats = torch.full((H,), 123.0, device="cuda")
+    q, k, v = (torch.randn(1, H, 64 * 1060, 64, generator=g).half().cuda() for _ in range(3))
+    logit = torch.zeros(H, 1060, device="cuda")
+    lut = torch.arange(T, dtype=torch.int32).expand(1, H, 1060, T).contiguous().cuda()
+    with pytest.raises(RuntimeError):
+        ops.train_op_fwd(q, k, v, logit, lut, T, 64, int8, stats)
+    torch.cuda.synchronize()
+    assert stats.tolist() == [123.0] * H
+    n, nb = 64 * 12, 12
+    q, k, v = (t[:, :, :n].contiguous() for t in (q, k, v))
+    lut, logit, version = lut[:, :, :nb].contiguous(), logit[:, :nb], stats._version
+    ops.train_op_fwd(q, k, v, logit, lut, nb, 64, int8, stats)
+    ref = ops.train_fwd(q, k, v, torch.sigmoid(logit), lut, nb, int8=int8)
+    assert torch.equal(stats, ref["lse"].amax(dim=(0, 2))) and stats._version > version
