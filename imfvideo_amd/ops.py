@@ -955,7 +955,7 @@ def sla2_infer(q, k, v, alpha, lut, bq, use_int8=True, qblock=None, eps_l=1e-5,
 def sla2_infer_in(q, k, v, bq, proj_q=None, proj_k=None):
     """sla2_infer's INT8 operands and the router's pooled blocks of 16-bit q, k, v in
     one pass -> (ws, qpool, kpool_t) (ws for sla2_infer; pool_qk's tensors)."""
-    _need_gpu(q, k, v)
+    _need_gpu(q, k, v, proj_q, proj_k)
     q, k, v = (_bhld(t, "qkv") for t in (q, k, v))
     _same(q, k, v)
     B, H, L, D = q.shape

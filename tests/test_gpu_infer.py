@@ -338,3 +338,14 @@ def test_sla2_takes_unaligned_operands(dt, which):
         off.append(flat[1:].view(x.shape) if name in which else x)
     with torch.no_grad():
         assert torch.equal(m(*off), m(*xs))
+
+
+@pytest.mark.parametrize("int8", [True, False])
+def test_sla2_refuses_a_router_on_the_host(int8):
+    """Router projections left on the CPU are an error with either sparse branch."""
+    from imfvideo_amd.sla2_vendor import SLA2
+    print("[case] router on the host", int8, flush=True)
+    m = SLA2(64, topk=0.3, use_int8=int8)
+    xs = [torch.randn(1, 2, 583, 64, device="cuda").half() for _ in range(3)]
+    with torch.no_grad(), pytest.raises(RuntimeError):
+        m(*xs)
