@@ -21,6 +21,20 @@ __all__ = ["RMSNorm", "SituAndMul", "SwiGLUMlp", "MLAAttention", "TransformerBlo
            "sdpa_math_attention"]
 
 
+class _CastOf(torch.autograd.Function):
+    """w16 as the 16-bit copy that it is of weight, for a double backward: its value
+    is that of the cast's time, its gradient goes to weight."""
+
+    @staticmethod
+    def forward(ctx, weight, w16):
+        ctx.dtype = weight.dtype
+        return w16.view_as(w16)
+
+    @staticmethod
+    def backward(ctx, d):
+        return d.to(ctx.dtype), None
+
+
 class _LinearFunction(torch.autograd.Function):
     """x @ weight^T for a 16-bit x and an fp32 weight, as nn.Linear under a 16-bit
     autocast, with the weight gradient from sla2h_linear_wgrad: fp32, summed
@@ -30,7 +44,7 @@ class _LinearFunction(torch.autograd.Function):
     def forward(ctx, x, weight):
         w16 = weight.to(x.dtype)
         ctx.save_for_backward(x, w16)
-        ctx.weight, ctx.version = weight, weight._version
+        ctx.weight = weight  # a double backward's link; its value is not read
         return F.linear(x, w16)
 
     @staticmethod
@@ -39,10 +53,7 @@ class _LinearFunction(torch.autograd.Function):
         x, w16 = ctx.saved_tensors
         need_x, need_w = ctx.needs_input_grad
         if torch.is_grad_enabled():  # create_graph: torch ops, differentiable again
-            if ctx.weight._version != ctx.version:
-                raise RuntimeError("a linear layer's weight was modified in place before its "
-                                   "double backward")
-            w16 = ctx.weight.to(x.dtype)
+            w16 = _CastOf.apply(ctx.weight, w16)
         dx = dy @ w16 if need_x else None
         if not need_w:
             return dx, None

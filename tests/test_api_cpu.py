@@ -296,3 +296,26 @@ def test_token_index_forms():
     for bad in (idx.int(), idx[:5], torch.arange(12)[::2], idx.view(2, 3), idx.to("meta"),
                 torch.ones(6, dtype=torch.bool)):
         assert not ops.token_index_ok(bad, x)
+
+
+def test_linear_double_backward_after_a_weight_update():
+    """A weight changed in place between the forward and its create_graph backward
+    (an optimizer step): as nn.Linear under autocast, the backward is at the
+    forward's 16-bit copy and its gradient reaches the weight."""
+    from imfvideo_amd.imf_dit_video import _LinearFunction
+    g = torch.Generator().manual_seed(13)
+    x0 = torch.randn(6, 16, generator=g)
+    w0 = torch.randn(8, 16, generator=g)
+    got = []
+    for own in (True, False):
+        x, w = x0.clone().requires_grad_(), torch.nn.Parameter(w0.clone())
+        with torch.autocast("cpu", dtype=torch.bfloat16):
+            y = (_LinearFunction.apply(x.to(torch.bfloat16), w) if own
+                 else torch.nn.functional.linear(x, w))
+        with torch.no_grad():
+            w.add_(1.0)
+        dx, dw = torch.autograd.grad(y.float().pow(2).sum(), [x, w], create_graph=True)
+        ddx, ddw = torch.autograd.grad(dx.pow(2).sum() + dw.pow(2).sum(), [x, w], create_graph=True)
+        got.append((dx.detach(), dw.detach(), ddx, ddw))
+    for a, b in zip(*got):
+        assert a.dtype == b.dtype and (a - b).norm() <= 2e-2 * b.norm()
