@@ -251,9 +251,8 @@ int complement_sums(const float* Hb, const float* dHb, const float* zb, const fl
 
 // states.hip: INT8 operands, pooled tiles and linear states of the cube op
 int quant_states(const QuantPoolArgs& a, const void* k, const void* dk, const void* v,
-                 const void* dv, int dtype, int B, int H, int Np, const float* proj_q,
-                 const float* proj_k, float* Hb, float* dHb, float* zb, float* dzb, void* vt,
-                 void* kt, void* stream);
+                 const void* dv, int dtype, int Np, float* Hb, float* dHb, float* zb, float* dzb,
+                 void* vt, void* kt, void* stream);
 
 // states.hip: the backward's complement records from given masks (word (kcq, n))
 int complement_gemm_bwd(const float* P, const float* Pz, const uint32_t* cbits, int BH, int Mb,
@@ -292,8 +291,7 @@ extern "C" int sla2h_cube_jvp_quant(const void* q, const void* k, const void* v,
   const JvpWs w(workspace, Dims(B, H, L, Np, kT, T), dk != nullptr, true);
   const QuantPoolArgs a = quant_pool_qk_args(q, k, B * H, L, Np, proj_q, proj_k, w.q8, w.qs, w.k8,
                                              w.ks, qpool, kpool_t, w.kb);
-  return quant_states(a, k, dk, v, dv, dtype, B, H, Np, proj_q, proj_k, w.Hb, w.dHb, w.zb, w.dzb,
-                      w.vt, w.kt, stream);
+  return quant_states(a, k, dk, v, dv, dtype, Np, w.Hb, w.dHb, w.zb, w.dzb, w.vt, w.kt, stream);
 }
 
 extern "C" int sla2h_cube_jvp_attn(const void* q, const void* dq, const float* alpha,

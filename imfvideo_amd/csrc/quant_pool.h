@@ -1,7 +1,7 @@
 // INT8 quantisation and router pooling of q and k tiles: the body that
-// quant_pool_kernel and, for small calls, quant_states_kernel run.  Every fp32
-// product and sum rounds separately, in the order written, whatever the
-// translation unit's contraction mode.
+// quant_pool_kernel and quant_states_kernel run.  Every fp32 product and sum
+// rounds separately, in the order written, whatever the translation unit's
+// contraction mode.
 #pragma once
 
 #include "common.h"

@@ -294,7 +294,9 @@ __global__ __launch_bounds__(256) void linear_states_kernel(
                                           blockIdx.x, blockIdx.y, lds);
 }
 
-// (batch, head, block) tiles that one grid of three workgroups each holds (2^32 threads)
+// (batch, head, block) tiles that one grid of three workgroups each holds (2^32
+// threads).  No call comes near: their fp32 states alone would take 69 GB, the
+// whole primal call over 400 GB.
 constexpr int64_t kFusedStatesTiles = 1 << 22;
 
 // The states and, independent of them, the INT8 quantisation and pooling of q
@@ -1049,33 +1051,25 @@ extern "C" int sla2h_complement(const float* Hb, const float* dHb, const float* 
 namespace sla2h {
 
 // sla2h_quant_pool_qk (a) and sla2h_linear_states without the global sums, in one
-// launch where its grid holds them.
+// launch.
 int quant_states(const QuantPoolArgs& a, const void* k, const void* dk, const void* v,
-                 const void* dv, int dtype, int B, int H, int Np, const float* proj_q,
-                 const float* proj_k, float* Hb, float* dHb, float* zb, float* dzb, void* vt,
-                 void* kt, void* stream) {
+                 const void* dv, int dtype, int Np, float* Hb, float* dHb, float* zb, float* dzb,
+                 void* vt, void* kt, void* stream) {
   const int64_t ns = (int64_t)a.BH * a.Nb;
-  if (ns <= kFusedStatesTiles) {
-    SLA2H_CHECK_ARG(k && v && Hb && zb && vt && Np > 0 && (int64_t)Np * kT <= a.L);
-    SLA2H_CHECK_ARG(dtype == SLA2H_DTYPE_F16 || dtype == SLA2H_DTYPE_BF16);
-    if (dk) SLA2H_CHECK_ARG(dv && dHb && dzb && kt);
-    auto run = [&](auto kernel) {
-      kernel<<<(unsigned)(3 * ns), 256, 0, static_cast<hipStream_t>(stream)>>>(
-          a, (int)(2 * ns), static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(dk),
-          static_cast<const uint16_t*>(v), static_cast<const uint16_t*>(dv), Np, Hb, dHb, zb, dzb,
-          static_cast<uint16_t*>(vt), static_cast<uint16_t*>(kt));
-      return (int)hipGetLastError();
-    };
-    if (dtype == SLA2H_DTYPE_BF16)
-      return dk ? run(quant_states_kernel<BF16, true>) : run(quant_states_kernel<BF16, false>);
-    return dk ? run(quant_states_kernel<F16, true>) : run(quant_states_kernel<F16, false>);
-  }
-  const int err = sla2h_quant_pool_qk(a.x[0], a.x[1], dtype, B, H, a.L, kT, kT, Np, proj_q, proj_k,
-                                      a.xq[0], a.xs[0], a.xq[1], a.xs[1], a.pool[0], a.pool[1],
-                                      a.kb[1], stream);
-  if (err) return err;
-  return sla2h_linear_states(k, dk, v, dv, dtype, B, H, a.L, kT, kT, Np, Hb, dHb, zb, dzb, nullptr,
-                             nullptr, nullptr, nullptr, vt, kt, stream);
+  SLA2H_CHECK_ARG(ns <= kFusedStatesTiles);
+  SLA2H_CHECK_ARG(k && v && Hb && zb && vt && Np > 0 && (int64_t)Np * kT <= a.L);
+  SLA2H_CHECK_ARG(dtype == SLA2H_DTYPE_F16 || dtype == SLA2H_DTYPE_BF16);
+  if (dk) SLA2H_CHECK_ARG(dv && dHb && dzb && kt);
+  auto run = [&](auto kernel) {
+    kernel<<<(unsigned)(3 * ns), 256, 0, static_cast<hipStream_t>(stream)>>>(
+        a, (int)(2 * ns), static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(dk),
+        static_cast<const uint16_t*>(v), static_cast<const uint16_t*>(dv), Np, Hb, dHb, zb, dzb,
+        static_cast<uint16_t*>(vt), static_cast<uint16_t*>(kt));
+    return (int)hipGetLastError();
+  };
+  if (dtype == SLA2H_DTYPE_BF16)
+    return dk ? run(quant_states_kernel<BF16, true>) : run(quant_states_kernel<BF16, false>);
+  return dk ? run(quant_states_kernel<F16, true>) : run(quant_states_kernel<F16, false>);
 }
 
 }  // namespace sla2h
