@@ -50,6 +50,7 @@ bool dims_ok(int dtype, int B, int H, int64_t L, int Np, int bq, int T) {
          (int64_t)(Np - 1) * kT < L && (bq == 64 || bq == 128 || bq == 256) && T >= 1 && T <= Np;
 }
 
+constexpr int kScoreFormCols = 4;  // LUT columns up to which the linear branch is in score form
 constexpr int64_t kEarlyStates = 2560;  // tiles: 40 MB of states
 
 __global__ __launch_bounds__(256) void train_setup_kernel(TrainSetup a) {
@@ -417,9 +418,10 @@ extern "C" int sla2h_train_fwd(const void* q, const void* k, const void* v,
   }
   // (zall: the score form's)
   SLA2H_TRY(complement_sums(w.Hb, nullptr, w.zb, nullptr, s.lut, B, H, d.Mq, d.Nb, kT, d.J, s.bits,
-                            s.comp, s.Hall, d.J <= 4 ? w.zall : nullptr, lse_max, stats, stream));
-  // the reference's linear branch: score form up to 4 LUT columns, else state form
-  if (d.J <= 4)
+                            s.comp, s.Hall, d.J <= kScoreFormCols ? w.zall : nullptr, lse_max,
+                            stats, stream));
+  // the reference's linear branch: score form for few LUT columns, else state form
+  if (d.J <= kScoreFormCols)
     SLA2H_TRY(sla2h_linear_mix_score(s.qphi, k, v, s.Hall, w.zall, s.lut, d.J, s.o_s, s.alpha,
                                      d.Mq, dtype, B, H, L, kT, bq, eps_l, o, s.o_l, s.den,
                                      stream));

@@ -448,7 +448,7 @@ def linear_mix_qat(qphi, comp, Hall, o_s, alpha, eps_l=1e-5, bq=E_TILE):
     return o, o_l, den
 
 
-SCORE_FORM_MAX_J = 4
+SCORE_FORM_MAX_J = 4  # the native calls': kScoreFormCols of csrc/pipeline.hip
 
 
 def linear_mix_score(qphi, k, v, st, lut, o_s, alpha, eps_l=1e-5, bq=E_TILE):

@@ -94,3 +94,12 @@ def test_no_alloc_capacity_at_the_29952_token_shape():
     assert lib.sla2h_complement_workspace_bytes(1, 1, 468, 468) == 28_800
     assert lib.sla2h_complement_workspace_bytes(1, 145, 468, 468) <= cap
     assert lib.sla2h_complement_workspace_bytes(1, 146, 468, 468) > cap
+
+
+def test_score_form_limit_is_one_number():
+    """The stage functions and the native calls switch the linear branch's form at
+    the same number of LUT columns."""
+    src = open(os.path.join(os.path.dirname(_lib.__file__), "csrc", "pipeline.hip")).read()
+    limit, = re.findall(r"constexpr int kScoreFormCols = (\d+);", src)
+    assert int(limit) == ops.SCORE_FORM_MAX_J
+    assert len(re.findall(r"\bJ <= ", src)) == len(re.findall(r"J <= kScoreFormCols", src)) == 2
