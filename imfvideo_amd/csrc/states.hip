@@ -409,16 +409,22 @@ constexpr int kCompCols = 64;  // state columns per GEMM workgroup
 constexpr int kCompThreads = 512;  // 8 waves
 // One launch for masks, z and H columns where that is the faster one: the
 // workgroups of each column tile build the same mask, so it pays while the
-// launch it saves costs more than that.  Measured (two launches -> one, us):
-// 4 heads x 5 query blocks, 4 tiles, tangent 9.0 -> 5.4; 4 x 64, T = 6 of 64,
-// 9.2 -> 8.1; 8 x 64, T = 16 of 64, primal 9.7 -> 8.4.  Past the lines: two
-// waves of workgroups, 24 x 32, T = 3 of 64, 22.2 -> 24.1; 2048 LUT entries a
-// workgroup, 4 x 64, T = 32 of 64, 9.3 -> 11.3; four mask words, 8 x 130,
-// T = 12 of 128, 12.9 -> 14.4; 8 x 300, T = 3 of 32, 12.7 -> 13.1.
+// launch it saves costs more than that.  Measured (two launches -> one, us; 130
+// workgroups a head with tangent, 65 without):
+//   heads x query blocks   4, tangent     6            8            12
+//   5, T = 2 of 4        7.3 ->  5.3   7.9 ->  6.0   8.7 ->  7.3  10.3 ->  9.6
+//   32, T = 3 of 32      7.4 ->  5.9   8.6 ->  7.0   9.5 ->  8.5  11.5 -> 11.1
+//   64, T = 6 of 64      8.8 ->  7.7  11.0 ->  9.3  12.3 -> 12.3  15.9 -> 16.3
+//   64, T = 16 of 64     9.2 ->  9.1  10.9 -> 10.2  12.1 -> 13.4  15.6 -> 17.4
+//   96, T = 10 of 96    10.5 -> 10.8  13.8 -> 12.6  15.9 -> 16.4  20.3 -> 21.6
+// (primal: the same at twice the heads, within 0.8), so up to 780 workgroups; the
+// two launches' GEMM is at its best at 512, two a CU.  Past the other lines, 2048
+// LUT entries a workgroup, 4 x 64, T = 32 of 64, 9.3 -> 11.3; four mask words, 8 x
+// 130, T = 12 of 128, 12.9 -> 14.4; 8 x 300, T = 3 of 32, 12.7 -> 13.1.
 constexpr int kFusedMaskWords = 3;        // 32 tiles each
 constexpr int kFusedMaskRows = 96;        // query blocks
 constexpr int kFusedMaskEntries = 1024;   // LUT entries of a workgroup's rows
-constexpr int kFusedMaskGroups = 520;     // workgroups: two a CU, and the last few
+constexpr int kFusedMaskGroups = 780;     // workgroups
 
 // 8 mask bits -> the 8 bf16 A-operand slots (1.0 where set)
 __device__ __forceinline__ u32x4 expand_mask8(uint32_t b) {

@@ -729,3 +729,28 @@ def test_cube_router_takes_projections_from_the_host(dt):
         assert torch.equal(route_tiles_fast(q, k, 0.4, 8, 64, 71, pq, pk)[0], want)
     with pytest.raises(RuntimeError):
         ops.route_1d(q, k, 0.4, 128, proj_q=pq, proj_k=pk)
+
+
+@pytest.mark.parametrize("Mb,Np,T", [(5, 4, 2), (64, 64, 16), (96, 96, 10)])
+@pytest.mark.parametrize("BH,tan", [(6, True), (12, False)])
+def test_complement_forms_agree_at_the_workgroup_line(BH, tan, Mb, Np, T):
+    """BH heads take the masks inside the GEMM, one head more takes two launches: the
+    records of the heads they share are equal to the bit."""
+    say(f"complement forms {BH}x{Mb} Np={Np} T={T} tan={tan}")
+    from imfvideo_amd import ops
+    gen = torch.Generator().manual_seed(Mb + BH)
+    rnd = lambda *s: torch.randn(*s, generator=gen).cuda()
+    names = {"Hb": (Np, 64, 64), "zb": (Np, 64)}
+    if tan:
+        names |= {"dHb": (Np, 64, 64), "dzb": (Np, 64)}
+    st = {n: rnd(1, BH + 1, *s) for n, s in names.items()}
+    lut = torch.stack([torch.randperm(Np, generator=gen)[:T] for _ in range((BH + 1) * Mb)])
+    lut = lut.int().view(1, BH + 1, Mb, T).cuda()
+    two = ops.complement(st, lut, Np)[:, :BH]
+    one = ops.complement({n: t[:, :BH].contiguous() for n, t in st.items()},
+                         lut[:, :BH].contiguous(), Np)
+    if not tan:  # a primal call leaves the tangent halves of the records alone
+        keep = torch.ones(two.shape[-1], dtype=torch.bool, device="cuda")
+        keep[16384:32768] = keep[33024:] = False
+        two, one = two[..., keep], one[..., keep]
+    assert torch.equal(one, two)
