@@ -65,9 +65,14 @@ class _LinearFunction(torch.autograd.Function):
 
 # Weights of at most this many 128 x 128 tiles take the split-row gradient
 # kernel: with few output tiles the library's kernel for the same product leaves
-# most CUs idle (2048 x 512, 64 tiles: 110 us against 46 us at 16,384 rows, 284
-# against 157 us at 59,904), with many it is as fast or faster (4096 x 1024, 256
-# tiles: 555 against 622 us at 59,904 rows).
+# most CUs idle.  Library product and cast against this kernel, us, bf16 rows x
+# (output x input) widths: 4,096 x (160 x 512), 8 tiles, 31 against 16; 16,384 x (512 x
+# 512), 16 tiles, 104 against 25; (2048 x 512), 64 tiles, 107 against 45 at 16,384 and 283
+# against 151 at 59,904 rows.  It is ahead at every row count from 64 to 131,072 up to
+# 128 tiles (1024 x 2048 at 131,072: 848 against 677), behind at long ones from 144
+# (1536 x 1536 at 131,072: 851 against 964; 4096 x 1024 at 59,904: 574 against 647).
+# Weights of 65 to 128 tiles stay with the library all the same: their gradients
+# would change from 16-bit rounded to fp32 sums.
 _WGRAD_MAX_TILES = 64
 
 
