@@ -596,3 +596,37 @@ def test_linear_module_batched_gradients():
     # one bf16 rounding of each (2^-8) plus fp32 summation order
     assert bool(((dx0 - dx1).abs() <= 2.0 ** -7 * dx1.abs() + 1e-4).all())
     assert bool(((dw0 - dw1).abs() <= 2.0 ** -7 * dw1.abs() + 1e-4).all())
+
+
+# Largest relative error of each output of a block over nine inputs (three sizes, three
+# seeds) against float64 with the routing of the run, times about three.  y and dx
+# are mostly the residual; every other gradient is a product of operands behind
+# several bf16 roundings (2^-9 rms each): 4.8e-3 to 8.3e-3 for the MLP, the v path
+# and the scales, 1.7e-2 behind the softmax's backward (q and k).
+BLOCK_BOUND = {"y": 1.5e-4, "dx": 1.5e-4, "logit_max_log2": 3e-3}
+BLOCK_BOUND_QK = ("attn.q_a_proj", "attn.q_b_proj", "attn.q_a_layernorm", "attn.q_norm", "attn.k_norm")
+
+
+@pytest.mark.parametrize("dims,seed", [((1, 4, 16, 16), 4), ((2, 8, 16, 20), 5), ((1, 12, 24, 20), 6)])
+def test_block_outputs_against_float64(dims, seed, monkeypatch):
+    """A training step of the whole block, every output by itself: the float64 side
+    takes the tiles that the run routed, so that a rerouted tile (which moves the
+    attention weights' gradients by 5 to 20 %) does not hide an error."""
+    from imfvideo_amd import ops
+    from perf import cases
+    say("block against float64", dims, seed)
+    B, gt, gh, gw = dims
+    c = dict(kind="block_train", dtype="bf16", B=B, H=8, gt=gt, gh=gh, gw=gw, P=0, topk=0.1,
+             tile_major=True)
+    luts, route = [], ops.route_topk
+    monkeypatch.setattr(ops, "route_topk", lambda *a, **k: luts.append(route(*a, **k)) or luts[-1])
+    got = cases.run(cases.prepare(c, seed))
+    lut, = luts
+    monkeypatch.setattr(cases, "_lut", lambda *a: lut.flatten(0, 1).long())
+    want = cases.exact(c, seed)
+    assert got.keys() == want.keys()
+    for n, w in want.items():
+        err = ((got[n].double() - w).norm() / w.norm()).item()
+        bound = BLOCK_BOUND.get(n, 5e-2 if n.startswith(BLOCK_BOUND_QK) else 2.5e-2)
+        print(f"  {n:28s} {err:.2e} (bound {bound:.1e})", flush=True)
+        assert err <= bound, n
