@@ -57,7 +57,7 @@ class _LinearFunction(torch.autograd.Function):
         dx = dy @ w16 if need_x else None
         if not need_w:
             return dx, None
-        if torch.is_grad_enabled() or not ops.plain_eager(dy):  # batched gradients (vmap) too
+        if torch.is_grad_enabled() or ops.batched(dy):
             dw = dy.reshape(-1, dy.shape[-1]).t() @ x.reshape(-1, x.shape[-1])
             return dx, dw.to(ctx.weight.dtype)
         return dx, ops.linear_wgrad(dy, x)

@@ -46,15 +46,23 @@ def _need_gpu(*ts):
 
 
 def plain_eager(*ts):
-    """Plain tensors (no subclass, none that is_grads_batched made a batch of) in
-    eager mode, outside torch.func transforms, forward-mode AD, tracing and
-    compilation: what the autograd Functions that replace torch's own ops are
-    for."""
-    return (all(type(t) in (torch.Tensor, torch.nn.Parameter)
-                and not torch._C._functorch.is_legacy_batchedtensor(t) for t in ts)
+    """Plain tensors (no subclass) in eager mode, outside torch.func transforms,
+    forward-mode AD, tracing and compilation: what the autograd Functions that
+    replace torch's own ops are for."""
+    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in ts)
             and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
             and not torch._C._are_functorch_transforms_active()
             and torch.autograd.forward_ad._current_level < 0)
+
+
+_transforms_active = torch._C._are_functorch_transforms_active
+_is_batch = torch._C._functorch.is_legacy_batchedtensor
+
+
+def batched(*ts):
+    """A backward under vmap (is_grads_batched, torch.func.vmap around
+    autograd.grad): its gradients have no storage that a kernel could read."""
+    return _transforms_active() or any(map(_is_batch, ts))
 
 
 def _bhld(t, name):
@@ -1378,8 +1386,8 @@ def rows_in_ok(xs):
 def token_index_ok(idx, x):
     """idx can be rows_in's / rows_out's for x (B, L, H, 64): one int64 per token,
     contiguous, on x's device (torch's index takes other forms)."""
-    return (idx.dtype == torch.int64 and tuple(idx.shape) == (x.shape[1],)
-            and idx.is_contiguous() and idx.device == x.device)
+    return (idx.dtype is torch.int64 and idx.shape == x.shape[1:2] and idx.is_contiguous()
+            and idx.device == x.device)
 
 
 def rows_in(xs, idx):
@@ -1401,8 +1409,8 @@ def rows_out_ok(o, q):
     (B, L, H, 64): fp16 rows (B, H, L, 64) on q's device (a forward_tile_major of
     the caller's own may return others)."""
     B, L, H, D = q.shape
-    return (plain_eager(o) and o.device == q.device and o.dtype == torch.float16
-            and tuple(o.shape) == (B, H, L, D))
+    return (type(o) is torch.Tensor and o.dtype is torch.float16 and o.device == q.device
+            and o.shape == (B, H, L, D))
 
 
 def rows_out(xs, idx, dtype):

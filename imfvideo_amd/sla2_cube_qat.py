@@ -161,7 +161,7 @@ class _RowsIn(torch.autograd.Function):
                                   for d in ds))
         have = [i for i, d in enumerate(ds) if d is not None]
         grads = [None] * len(ds)
-        if not ops.plain_eager(*(ds[i] for i in have)):  # batched gradients
+        if ops.batched(*(ds[i] for i in have)):
             for i in have:
                 grads[i] = ds[i][:, :, inv].permute(0, 2, 1, 3).to(ctx.dtype)
         elif have:
@@ -202,7 +202,7 @@ class _RowsOut(torch.autograd.Function):
         idx, inv = ctx.saved_tensors
         have = [i for i, d in enumerate(ds) if d is not None]
         grads = [None] * len(ds)
-        if not ops.plain_eager(*(ds[i] for i in have)):  # batched gradients
+        if ops.batched(*(ds[i] for i in have)):
             for i in have:
                 grads[i] = ds[i].permute(0, 2, 1, 3)[:, :, inv].half()
         elif have:

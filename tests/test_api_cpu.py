@@ -267,9 +267,9 @@ def test_weight_gradient_rows_of_a_wide_tensor_are_copied():
 
 
 def test_linear_takes_batched_gradients():
-    """The block's linear under is_grads_batched (backward under vmap), where the
-    weight gradient's kernel cannot read dy: the same products in torch, one
-    gradient at a time or batched."""
+    """The block's linear under is_grads_batched and under vmap around autograd.grad,
+    where the weight gradient's kernel cannot read dy: the same products in torch,
+    one gradient at a time or batched."""
     from imfvideo_amd.imf_dit_video import _LinearFunction
     g = torch.Generator().manual_seed(12)
     x = torch.randn(2, 5, 16, generator=g).to(torch.bfloat16).requires_grad_()
@@ -277,6 +277,8 @@ def test_linear_takes_batched_gradients():
     dys = torch.randn(3, 2, 5, 8, generator=g).to(torch.bfloat16)
     y = _LinearFunction.apply(x, w)
     dx, dw = torch.autograd.grad(y, [x, w], dys, is_grads_batched=True, retain_graph=True)
+    vx, vw = torch.func.vmap(lambda d: torch.autograd.grad(y, [x, w], d, retain_graph=True))(dys)
+    assert torch.equal(vx, dx) and torch.equal(vw, dw)
     w16 = w.detach().to(torch.bfloat16).requires_grad_()
     ref = torch.nn.functional.linear(x, w16)
     assert dw.dtype == torch.float32
