@@ -178,6 +178,7 @@ class _TrainIn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, idx, inv, Np, proj_q, proj_k, *xs):
         ctx.save_for_backward(idx, inv)
+        ctx.set_materialize_grads(False)  # no zero gradients of the size of the workspace
         ctx.dtype = xs[0].dtype
         rows, *rest = ops.train_in(xs, idx, Np, proj_q, proj_k)
         ctx.mark_non_differentiable(*rest)

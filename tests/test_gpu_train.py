@@ -597,3 +597,24 @@ def test_lse_maxima_replace_the_buffer_as_a_whole(T, int8):
     ops.train_op_fwd(q, k, v, logit, lut, nb, 64, int8, stats)
     ref = ops.train_fwd(q, k, v, torch.sigmoid(logit), lut, nb, int8=int8)
     assert torch.equal(stats, ref["lse"].amax(dim=(0, 2))) and stats._version > version
+
+
+@pytest.mark.parametrize("pre_permuted", [False, True])
+def test_no_gradients_for_the_forward_workspace(pre_permuted, monkeypatch):
+    """The forward's workspace and pooled tiles take no gradient: autograd makes no
+    zero-filled tensors of their sizes (hundreds of MB at full length) for the
+    backward of the module's operands."""
+    from imfvideo_amd import sla2_cube_qat as M
+    print("[case] workspace gradients", pre_permuted, flush=True)
+    seen, backward = [], M._TrainIn.backward
+
+    def spy(ctx, *ds):
+        seen.append([d is None for d in ds])
+        return backward(ctx, *ds)
+
+    monkeypatch.setattr(M._TrainIn, "backward", staticmethod(spy))
+    mod = M.SLA2CubeQATAttentionImpl(64, 274, 2, (4, 8, 8), topk=0.5, pre_permuted=pre_permuted).cuda()
+    xs = [torch.randn(1, 274, 2, 64, device="cuda").requires_grad_() for _ in range(3)]
+    grads = torch.autograd.grad(mod(*xs).float().pow(2).sum(), xs)
+    assert seen == [[False] * 3 + [True] * 3]
+    assert all(g.abs().sum() > 0 for g in grads)
