@@ -206,7 +206,7 @@ int sla2h_pool_blocks(const void* x, int dtype, int64_t BH, int64_t L, int D, in
  * (B,H,ceil(L/bq),64) = means over bq rows, kpool_t (B,H,64,Nk) = means over the
  * first Nk blocks of bk = 64 rows, transposed, each after its optional projection;
  * sla2h_pool_blocks' arithmetic and order.  A block that reaches past L (only
- * the last one can) averages its real rows.
+ * the last one can) averages its real rows.  q and k 4-byte aligned, qpool 8-byte.
  */
 int sla2h_pool_qk(const void* q, const void* k, int dtype, int B, int H, int64_t L, int D, int bq,
                   int bk, int Nk, const float* proj_q, const float* proj_k, float* qpool,
@@ -834,7 +834,7 @@ int sla2h_sla2_infer(const void* q, const void* k, const void* v, const float* a
  * Its INT8 operands (sla2h_quantize per bq rows of q and 64 of k, sla2h_quantize_v8f)
  * in the workspace (of int8 = 1; then quantised = 1, qblock = bq), and the
  * router's pooled blocks qpool (B,H,ceil(L/bq),64) and kpool_t (B,H,64,Nb)
- * (sla2h_pool_qk), in one pass over q, k, v.
+ * (sla2h_pool_qk), in one pass over q, k, v (16-byte aligned).
  */
 int sla2h_sla2_infer_in(const void* q, const void* k, const void* v, int dtype, int B, int H,
                         int64_t L, int bq, const float* proj_q, const float* proj_k,
