@@ -52,12 +52,13 @@ class _LinearFunction(torch.autograd.Function):
         from . import ops
         x, w16 = ctx.saved_tensors
         need_x, need_w = ctx.needs_input_grad
-        if torch.is_grad_enabled():  # create_graph: torch ops, differentiable again
+        again = torch.is_grad_enabled()  # create_graph: torch ops, differentiable again
+        if again:
             w16 = _CastOf.apply(ctx.weight, w16)
         dx = dy @ w16 if need_x else None
         if not need_w:
             return dx, None
-        if torch.is_grad_enabled() or ops.batched(dy):
+        if again or ops.batched(dy):
             dw = dy.reshape(-1, dy.shape[-1]).t() @ x.reshape(-1, x.shape[-1])
             return dx, dw.to(ctx.weight.dtype)
         return dx, ops.linear_wgrad(dy, x)

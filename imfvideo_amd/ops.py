@@ -1383,11 +1383,15 @@ def rows_in_ok(xs):
     return True
 
 
-def token_index_ok(idx, x):
-    """idx can be rows_in's / rows_out's for x (B, L, H, 64): one int64 per token,
-    contiguous, on x's device (torch's index takes other forms)."""
-    return (idx.dtype is torch.int64 and idx.shape == x.shape[1:2] and idx.is_contiguous()
-            and idx.device == x.device)
+def token_index_ok(x, *idx):
+    """Each idx can be rows_in's / rows_out's for x (B, L, H, 64): one int64 per
+    token, contiguous, on x's device (torch's index takes other forms)."""
+    L, dev = x.shape[1], x.device
+    for i in idx:
+        if not (i.dtype is torch.int64 and i.dim() == 1 and i.numel() == L and i.is_contiguous()
+                and i.device == dev):
+            return False
+    return True
 
 
 def rows_in(xs, idx):
@@ -1432,14 +1436,14 @@ def _ptrs(ts):
 # ---------------------------------------------------------------------------
 # DiT block, training backward: weight gradients of the linear layers
 # ---------------------------------------------------------------------------
+# (rows + 144) * row stride, in 16-bit elements, stays below this: 32-bit byte offsets
+_WGRAD_SPAN = 2 ** 30 - 128
+
+
 def linear_wgrad_ok(rows, M, N):
     """Sizes that sla2h_linear_wgrad takes: M and N multiples of 8, 32-bit byte offsets."""
-    return rows > 0 and M > 0 and N > 0 and M % 8 == 0 and N % 8 == 0 and _offsets32(rows, max(M, N))
-
-
-def _offsets32(rows, ld):
-    """The weight gradient's byte offsets into rows of ld 16-bit elements fit 32 bits."""
-    return (rows + 144) * ld * 2 + 256 < 2 ** 31
+    return (rows > 0 and M > 0 and N > 0 and M % 8 == 0 and N % 8 == 0
+            and (rows + 144) * max(M, N) < _WGRAD_SPAN)
 
 
 def linear_wgrad(dy, x):
@@ -1468,7 +1472,7 @@ def _rows16(t):
     """_rows_view with 16-byte aligned rows and 32-bit byte offsets (copied when the
     data or the row stride does not give them)."""
     v, F, s = _rows_view(t)
-    if v.data_ptr() % 16 or s % 8 or not _offsets32(v.shape[0], s):
+    if v.data_ptr() % 16 or s % 8 or (v.shape[0] + 144) * s >= _WGRAD_SPAN:
         v = v.clone(memory_format=torch.contiguous_format)
         s = F
     return v, F, s

@@ -275,10 +275,9 @@ class SLA2CubeQATAttentionImpl(nn.Module):
 
         # one kernel for the three operands (and one for the output) where they
         # are plain GPU tensors with 16-byte rows; else the torch form
-        own = (ops.plain_eager(q, k, v) and ops.rows_in_ok((q, k, v))
-               and (self.pre_permuted or all(ops.token_index_ok(i, q)
-                                             for i in (self.perm, self.inv))))
         perm, inv = (None, None) if self.pre_permuted else (self.perm, self.inv)
+        own = (ops.plain_eager(q, k, v) and ops.rows_in_ok((q, k, v))
+               and (self.pre_permuted or ops.token_index_ok(q, perm, inv)))
         if not own:
             o = self.forward_tile_major(tm(q), tm(k), tm(v))
         elif (self._one_pass(q.shape[1]) and "forward_tile_major" not in self.__dict__
@@ -288,9 +287,10 @@ class SLA2CubeQATAttentionImpl(nn.Module):
             o = self._op(qh, kh, vh, *pre)
         else:
             o = self.forward_tile_major(*_RowsIn.apply(perm, inv, q, k, v))
+            own = ops.rows_out_ok(o, q)
         if self.pre_permuted:
             return o.permute(0, 2, 1, 3).to(q.dtype)
-        if own and ops.rows_out_ok(o, q):
+        if own:
             return _RowsOut.apply(inv, perm, q.dtype, o)[0]
         return o[:, :, self.inv].permute(0, 2, 1, 3).to(q.dtype)
 

@@ -105,7 +105,8 @@ class SLA2(nn.Module):
                 and q.dtype == k.dtype == self.dtype and q.shape == k.shape == v.shape
                 and qh.is_cuda and type(self.router) is Router
                 and "route" not in self.router.__dict__):
-            qh, kh, vh = (ops.aligned(t, 16) for t in (qh, kh, vh))  # 16-byte accesses
+            if (qh.data_ptr() | kh.data_ptr() | vh.data_ptr()) % 16:  # its accesses
+                qh, kh, vh = (ops.aligned(t, 16) for t in (qh, kh, vh))
             lut, topk, ws = self.router.route_quantised(qh, kh, vh, self.topk)
         else:
             lut, topk = self.router.route(q, k, self.topk)

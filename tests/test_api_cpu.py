@@ -294,10 +294,10 @@ def test_token_index_forms():
     from imfvideo_amd import ops
     x = torch.empty(2, 6, 3, 64)
     idx = torch.arange(6)
-    assert ops.token_index_ok(idx, x)
+    assert ops.token_index_ok(x, idx) and ops.token_index_ok(x, idx, idx.flip(0))
     for bad in (idx.int(), idx[:5], torch.arange(12)[::2], idx.view(2, 3), idx.to("meta"),
                 torch.ones(6, dtype=torch.bool)):
-        assert not ops.token_index_ok(bad, x)
+        assert not ops.token_index_ok(x, bad) and not ops.token_index_ok(x, idx, bad)
 
 
 def test_linear_double_backward_after_a_weight_update():
